@@ -1,13 +1,15 @@
-// Linear layers of the fp32 build:  y[T, N] (=|+=) alpha x[T, K] . W[N, K]^T  in IEEE fp32 on the vector ALUs, plain, per
-// head (a batch of small matrices) or per expert (token tiles of a routing plan).  64 x 64 output blocks, operands staged
-// through LDS, sums in ascending k.
+// Linear layers of the fp32 build:  y[T, N] (=|+=) alpha x[T, K] . W[N, K]^T  in IEEE fp32 on the matrix cores
+// (v_mfma_f32_16x16x4_f32: products and sums in fp32), plain, per head (a batch of small matrices) or per expert (token tiles
+// of a routing plan).
+#include <type_traits>
+
 #include "common.h"
 #include "moe.h"
 
 namespace {
 
-constexpr int FB = 64;       // block side
-constexpr int FK = 16;       // k per stage
+constexpr int FB = 64;       // tokens of a block
+constexpr int FW = 8;        // waves of a workgroup
 
 struct F32Linear {
   float* y;
@@ -19,11 +21,199 @@ struct F32Linear {
   float alpha;
   int accumulate, act;       // act: MLORA_ACT_*
   int gather, scatter, top;  // expert tiles (blockIdx.y = tile): gather: x row = entry / top; scatter: y row = entry
+  int vec;                   // rows of y can be stored 16 bytes at a time
 };
 
-__global__ __launch_bounds__(256) void linear_f32_kernel(F32Linear a, MoePlan plan, int grouped) {
-  __shared__ float xs[FK][FB + 4], ws[FK][FB + 4];
-  const int n0 = blockIdx.x * FB;
+// The fp32 16 x 16 x 4 product takes one element per lane: a lane holds 4 consecutive k of its row, element e of the four
+// k-groups of 16 lanes is one MFMA (any order of k serves, as long as both operands have the same).
+//
+// At T x K x N = 299 x 2048 x 2048: 49 us (51 TFLOP/s), 1 x 2048 x 11264: 23 us (3.9 TB/s), 4096 x 2048 x 11264: 1715 us
+// (110 TFLOP/s).  The vector ALUs (64 x 64 blocks, both operands staged through LDS behind two barriers per 16 k): 122, 139,
+// 2415 us.
+
+// Adds the sums of the waves that share K, in their order, and stores.  red [KW][tiles][lane]: four rows n of a token; tile = row
+// tile * RT + token tile.
+template <int KW, int TILES, int RT>
+__device__ __forceinline__ void f32_store(const F32Linear& a, const MoePlan& plan, int grouped, float* __restrict__ y, int n0, int t0, int t1,
+                                          const f32x4* red) {
+  for (int o = threadIdx.x; o < TILES * 64; o += FW * WAVE) {
+    const int tile = o >> 6, l = o & 63;
+    f32x4 v = red[o];
+#pragma unroll
+    for (int q = 1; q < KW; ++q) v += red[q * TILES * 64 + o];
+    int t = t0 + tile % RT * 16 + (l & 15);
+    const int n = n0 + tile / RT * 16 + (l >> 4) * 4;
+    if (t >= t1 || n >= a.N) continue;
+    if (grouped && a.scatter) t = plan.perm[t];
+    float* p = y + t * a.ldy + n;
+    v *= a.alpha;
+    if (a.act == MLORA_ACT_RELU2) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        v[r] = fmaxf(v[r], 0.f);
+        v[r] *= v[r];
+      }
+    }
+    if (a.vec && n + 4 <= a.N) {
+      f32x4* q = reinterpret_cast<f32x4*>(p);
+      *q = a.accumulate ? *q + v : v;
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (n + r < a.N) p[r] = a.accumulate ? p[r] + v[r] : v[r];
+    }
+  }
+}
+
+__device__ __forceinline__ f32x4 mfma_f32(const f32x4& w, const f32x4& x, f32x4 c) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_16x16x4f32(w[e], x[e], c, 0, 0, 0);
+  return c;
+}
+
+// 16 weight rows per workgroup, up to 64 tokens (RT tiles of 16, as many as the block has): all eight waves share K, 32 k at a
+// time in turn, so that together they read whole lines.  Operands go straight into registers, D stages ahead.  For few tokens
+// or rows: bound by the stream of W and its latency; x is read again by every workgroup, through the first two cache levels.
+template <int RT>
+__device__ __forceinline__ void f32_thin(const F32Linear& a, const MoePlan& plan, int grouped, const float* __restrict__ x, const float* __restrict__ W,
+                                         float* __restrict__ y, int n0, int t0, int t1, f32x4* red) {
+  constexpr int D = RT == 1 ? 4 : RT <= 3 ? 3 : 2;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
+  const float* wp = W + (size_t)(n0 + r16 < a.N ? n0 + r16 : a.N - 1) * a.K + g * 4;
+  const float* xp[RT];
+#pragma unroll
+  for (int j = 0; j < RT; ++j) {
+    int t = t0 + j * 16 + r16;
+    t = t < t1 ? t : t1 - 1;
+    if (grouped && a.gather) t = plan.perm[t] / a.top;
+    xp[j] = x + t * a.ldx + g * 4;
+  }
+  f32x4 acc[RT], wf[D][2], xf[D][RT][2];
+#pragma unroll
+  for (int j = 0; j < RT; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int steps = (a.K + 31) / 32;              // of 32 k; the last one may have 16
+  auto load = [&](auto S, int p) {
+    constexpr int s = decltype(S)::value;
+    const int k = (p < steps ? p : 0) * 32, k1 = k + 16 < a.K ? k + 16 : k;     // past the end: valid addresses, not multiplied
+    wf[s][0] = *reinterpret_cast<const f32x4*>(wp + k);
+    wf[s][1] = *reinterpret_cast<const f32x4*>(wp + k1);
+#pragma unroll
+    for (int j = 0; j < RT; ++j) {
+      xf[s][j][0] = *reinterpret_cast<const f32x4*>(xp[j] + k);
+      xf[s][j][1] = *reinterpret_cast<const f32x4*>(xp[j] + k1);
+    }
+  };
+  auto turn = [&](auto S, int p) {
+    constexpr int s = decltype(S)::value;
+    load(std::integral_constant<int, (s + D - 1) % D>(), p + (D - 1) * FW);
+    if (p >= steps) return;                       // uniform
+#pragma unroll
+    for (int j = 0; j < RT; ++j) acc[j] = mfma_f32(wf[s][0], xf[s][j][0], acc[j]);
+    if (p * 32 + 16 < a.K) {
+#pragma unroll
+      for (int j = 0; j < RT; ++j) acc[j] = mfma_f32(wf[s][1], xf[s][j][1], acc[j]);
+    }
+  };
+  load(std::integral_constant<int, 0>(), wave);
+  if constexpr (D > 2) load(std::integral_constant<int, 1>(), wave + FW);
+  if constexpr (D > 3) load(std::integral_constant<int, 2>(), wave + 2 * FW);
+  for (int p = wave; p < steps; p += D * FW) {
+    turn(std::integral_constant<int, 0>(), p);
+    turn(std::integral_constant<int, 1>(), p + FW);
+    if constexpr (D > 2) turn(std::integral_constant<int, 2>(), p + 2 * FW);
+    if constexpr (D > 3) turn(std::integral_constant<int, 3>(), p + 3 * FW);
+  }
+#pragma unroll
+  for (int j = 0; j < RT; ++j) red[(wave * RT + j) * 64 + lane] = acc[j];
+  __syncthreads();
+  f32_store<FW, RT, RT>(a, plan, grouped, y, n0, t0, t1, red);
+}
+
+// FN * 16 weight rows by up to 64 tokens: four waves share the rows (FN / 4 tiles each, all tokens), twice, for the two halves
+// of every 64 k.  Both operands go from global memory straight into an LDS ring (fragments of 16 rows x 16 k as the lanes read
+// them) that is NST - 1 stages of 64 k ahead, one bare barrier per stage.  Bound by the matrix cores (157 TFLOP/s nominal).
+template <int FN, int RT>
+__device__ __forceinline__ void f32_wide(const F32Linear& a, const MoePlan& plan, int grouped, const float* __restrict__ x, const float* __restrict__ W,
+                                         float* __restrict__ y, int n0, int t0, int t1, f32x4* smem) {
+  constexpr int NST = FN == 4 ? 4 : 3, RW = FN / 4, SF = FN + RT, LF = 4 * SF, LQ = (LF + FW - 1) / FW;   // fragments: of 16 k, of a stage, per loading wave
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
+  // fragment f = wave + 8 q of a stage: 16 k number f / SF, there weight tile or (behind those) token tile f % SF
+  const float* src[LQ];
+  int fk[LQ], fd[LQ];
+#pragma unroll
+  for (int q = 0; q < LQ; ++q) {
+    int f = wave + FW * q;
+    f = f < LF ? f : LF - 1;                      // (twice the same: every wave has LQ requests per stage)
+    fk[q] = f / SF * 16;
+    fd[q] = f;
+    f -= f / SF * SF;
+    if (f < FN) {
+      const int n = n0 + f * 16 + r16;
+      src[q] = W + (size_t)(n < a.N ? n : a.N - 1) * a.K + g * 4;
+    } else {
+      int t = t0 + (f - FN) * 16 + r16;
+      t = t < t1 ? t : t1 - 1;
+      if (grouped && a.gather) t = plan.perm[t] / a.top;
+      src[q] = x + t * a.ldx + g * 4;
+    }
+  }
+  const int nst = (a.K + 63) / 64;
+  int slot = 0;                                   // of the stage requested next
+  auto request = [&](int s) {
+#pragma unroll
+    for (int q = 0; q < LQ; ++q) {
+      const int k = s * 64 + fk[q];               // past the end: a valid address, not multiplied
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[q] + (k < a.K ? k : 0)),
+                                       (__attribute__((address_space(3))) void*)(smem + (slot * LF + fd[q]) * 64), 16, 0, 0);
+    }
+    slot = slot + 1 < NST ? slot + 1 : 0;
+  };
+  const int rg = wave & 3, kh = wave >> 2;
+  f32x4 acc[RW][RT];
+#pragma unroll
+  for (int i = 0; i < RW; ++i)
+#pragma unroll
+    for (int j = 0; j < RT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < NST - 1; ++s) request(s);
+  int rd = 0;
+  for (int s = 0; s < nst; ++s) {
+    // stage s has landed (this wave's share: at most the NST - 2 stages behind it in flight; everybody's: the barrier), and
+    // everybody is done with the slot of stage s - 1, which is requested anew
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NST - 2) * LQ) : "memory");
+    bare_barrier();
+    request(s + NST - 1);
+    const f32x4* st = smem + (rd * LF + kh * 2 * SF) * 64 + lane;
+    rd = rd + 1 < NST ? rd + 1 : 0;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if (s * 64 + kh * 32 + h * 16 >= a.K) break;                   // uniform
+      f32x4 w[RW], xv[RT];
+#pragma unroll
+      for (int i = 0; i < RW; ++i) w[i] = st[(h * SF + rg * RW + i) * 64];
+#pragma unroll
+      for (int j = 0; j < RT; ++j) xv[j] = st[(h * SF + FN + j) * 64];
+#pragma unroll
+      for (int i = 0; i < RW; ++i)
+#pragma unroll
+        for (int j = 0; j < RT; ++j) acc[i][j] = mfma_f32(w[i], xv[j], acc[i][j]);
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                   // the requests past the end, too: the ring becomes the waves' sums
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < RW; ++i)
+#pragma unroll
+    for (int j = 0; j < RT; ++j) smem[((kh * 4 + rg) * RW * RT + i * RT + j) * 64 + lane] = acc[i][j];
+  __syncthreads();
+  f32_store<2, FN * RT, RT>(a, plan, grouped, y, n0, t0, t1, smem);
+}
+
+// FN: row tiles of a workgroup (1: f32_thin)
+template <int FN>
+__global__ __launch_bounds__(FW* WAVE, 2) void linear_f32_kernel(F32Linear a, MoePlan plan, int grouped) {
+  extern __shared__ __align__(16) f32x4 f32_smem[];
+  const int n0 = blockIdx.x * FN * 16;
   int t0 = blockIdx.y * FB, t1 = a.T;
   const float* W = a.W + (size_t)blockIdx.z * a.N * a.K;
   const float* x = a.x + blockIdx.z * a.hx;
@@ -35,57 +225,54 @@ __global__ __launch_bounds__(256) void linear_f32_kernel(F32Linear a, MoePlan pl
     t0 = tile.y;
     t1 = tile.y + tile.z;
   }
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  float acc[4][4] = {};
-  // loader: thread -> row threadIdx / 4, four k at (threadIdx % 4) * 4
-  const int lr = threadIdx.x >> 2, lk = (threadIdx.x & 3) * 4;
-  int xrow = t0 + lr < t1 ? t0 + lr : t1 - 1;
-  if (grouped && a.gather) xrow = plan.perm[xrow] / a.top;
-  const int wrow = n0 + lr < a.N ? n0 + lr : a.N - 1;
-  for (int k0 = 0; k0 < a.K; k0 += FK) {
-    const f32x4 xv = *reinterpret_cast<const f32x4*>(x + xrow * a.ldx + k0 + lk);
-    const f32x4 wv = *reinterpret_cast<const f32x4*>(W + (size_t)wrow * a.K + k0 + lk);
-    __syncthreads();
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      xs[lk + e][lr] = xv[e];
-      ws[lk + e][lr] = wv[e];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < FK; ++k) {
-      const f32x4 xf = *reinterpret_cast<const f32x4*>(&xs[k][ty * 4]), wf = *reinterpret_cast<const f32x4*>(&ws[k][tx * 4]);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(xf[i], wf[j], acc[i][j]);
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    int t = t0 + ty * 4 + i;
-    if (t >= t1) continue;
-    if (grouped && a.scatter) t = plan.perm[t];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = n0 + tx * 4 + j;
-      if (n >= a.N) continue;
-      float v = acc[i][j] * a.alpha;
-      if (a.act == MLORA_ACT_RELU2) {
-        v = fmaxf(v, 0.f);
-        v = v * v;
-      }
-      float* p = y + t * a.ldy + n;
-      *p = a.accumulate ? *p + v : v;
-    }
-  }
+  t1 = t1 < t0 + FB ? t1 : t0 + FB;
+  const int rt = __builtin_amdgcn_readfirstlane((t1 - t0 + 15) >> 4);
+  auto block = [&](auto RT) {
+    if constexpr (FN == 1) f32_thin<decltype(RT)::value>(a, plan, grouped, x, W, y, n0, t0, t1, f32_smem);
+    else f32_wide<FN, decltype(RT)::value>(a, plan, grouped, x, W, y, n0, t0, t1, f32_smem);
+  };
+  if (rt == 1) block(std::integral_constant<int, 1>());
+  else if (rt == 2) block(std::integral_constant<int, 2>());
+  else if (rt == 3) block(std::integral_constant<int, 3>());
+  else block(std::integral_constant<int, 4>());
 }
 
-int launch(const char* who, const F32Linear& a, const MoePlan& plan, int grouped, int row_blocks, int heads, void* stream) {
-  MLORA_CHECK(a.K % FK == 0 && a.ldx % 4 == 0 && a.hx % 4 == 0 && row_blocks <= 65535 && heads <= 65535, MLORA_ERR_UNSUPPORTED,
-              "%s: need K %% 16 == 0 and rows aligned to 16 bytes (T=%d K=%d N=%d)", who, a.T, a.K, a.N);
-  hipLaunchKernelGGL(linear_f32_kernel, dim3(ceil_div(a.N, FB), row_blocks, heads), dim3(256), 0, (hipStream_t)stream, a, plan, grouped);
+int f32_n_cu() {
+  static const int n_cu = [] {
+    int dev = 0, cu = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cu <= 0) cu = 256;
+    return cu;
+  }();
+  return n_cu;
+}
+
+template <int FN>
+int launch_f32(const char* who, const F32Linear& a, const MoePlan& plan, int grouped, int row_blocks, int heads, hipStream_t stream) {
+  constexpr size_t lds = FN == 1 ? FW * 4 * 1024 : (FN == 4 ? 4 : 3) * 4 * (FN + 4) * 1024;
+  static const hipError_t configured =               // the attribute is per kernel, set once per process, by one thread
+      hipFuncSetAttribute((const void*)linear_f32_kernel<FN>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (configured != hipSuccess) return mlora_set_error(MLORA_ERR_LAUNCH, "%s: cannot reserve %zu bytes of LDS: %s", who, lds, hipGetErrorString(configured));
+  hipLaunchKernelGGL((linear_f32_kernel<FN>), dim3(ceil_div(a.N, FN * 16), row_blocks, heads), dim3(FW * WAVE), lds, stream, a, plan, grouped);
   return mlora_launch_status(who);
+}
+
+int launch(const char* who, F32Linear a, const MoePlan& plan, int grouped, int row_blocks, int heads, void* stream) {
+  MLORA_CHECK(a.K % 16 == 0 && a.ldx % 4 == 0 && a.hx % 4 == 0 && row_blocks <= 65535 && heads <= 65535, MLORA_ERR_UNSUPPORTED,
+              "%s: need K %% 16 == 0 and rows aligned to 16 bytes (T=%d K=%d N=%d)", who, a.T, a.K, a.N);
+  a.vec = a.ldy % 4 == 0 && a.hy % 4 == 0 && ((uintptr_t)a.y & 15) == 0;
+  // Rounds of the compute units times what a workgroup takes, in us at K = 2048 as measured for 1, 2 and 4 token tiles: 16 rows
+  // 11, 13, 23; 64 rows 20, 25, 46; 128 rows 34, 45, 80.  So 16 rows serve a grid that does not fill the chip (32 x 7680 x 2048:
+  // 45 against 96 and 173 us), 128 rows one that fills it several times over (4096 x 2048 x 11264: 3443, 1961, 1715 us), 64 rows
+  // what lies between (299 x 7680 x 2048: 193, 165, 290 us).
+  const int entries = grouped ? a.T / row_blocks : a.T, rt = entries >= FB ? FB / 16 : entries > 16 ? ceil_div(entries, 16) : 1;
+  auto cost = [&](int tiles, double once, double per_tile) {
+    const long blocks = (long)ceil_div(a.N, tiles * 16) * row_blocks * heads;
+    return (double)((blocks + f32_n_cu() - 1) / f32_n_cu()) * (once + per_tile * rt);
+  };
+  const double c1 = cost(1, 8, 3.8), c4 = cost(4, 12, 9), c8 = cost(8, 20, 15);
+  if (c1 <= c4 && c1 <= c8) return launch_f32<1>(who, a, plan, grouped, row_blocks, heads, (hipStream_t)stream);
+  if (c4 <= c8) return launch_f32<4>(who, a, plan, grouped, row_blocks, heads, (hipStream_t)stream);
+  return launch_f32<8>(who, a, plan, grouped, row_blocks, heads, (hipStream_t)stream);
 }
 
 }  // namespace

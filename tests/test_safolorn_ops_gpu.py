@@ -377,3 +377,18 @@ def test_fp32_linear(ops, T, K, N):
     a0 = f64(acc)
     ops.linear(x, W, out=acc, accumulate=True)
     assert err(acc, a0 + want) < 1e-6
+
+
+@pytest.mark.parametrize("T,K,N", [(1, 16, 1), (16, 48, 31), (17, 208, 4100), (63, 2064, 70), (65, 80, 2050), (64, 16, 16400), (130, 48, 33000), (200, 112, 33001)])
+def test_fp32_linear_forms(ops, T, K, N):
+    """16, 64 and 128 rows per workgroup, ragged tokens, rows and K, stored 16 bytes at a time or by element.  Every product and every
+    sum rounds once: at most K + 2 roundings of 2^-24 on what is added up."""
+    rng = np.random.default_rng(K)
+    x, W = (torch.from_numpy(rng.normal(size=s)).float().to(DEV) for s in ((T, K), (N, K)))
+    want, room = x.double() @ W.double().T, x.abs().double() @ W.abs().double().T
+    y = ops.linear(x, W)
+    assert bool(((y.double() - want).abs() <= (K + 2) * 2.0 ** -24 * room).all())
+    y0 = torch.from_numpy(rng.normal(size=(T, N))).float().to(DEV)
+    y1 = ops.linear(x, W, out=y0.clone(), accumulate=True)
+    torch.cuda.synchronize()
+    assert torch.equal(y1, y0 + y)
