@@ -866,70 +866,187 @@ __global__ __launch_bounds__(LO_WAVES* WAVE, 2) void latent_out_kernel(LatentAtt
 
 #else   // fp32
 
-constexpr int LA_KEYS = 256;
-constexpr int LA_DPT = 4;      // output dims per thread
-// One workgroup per (token, head, 1024 output dims): scores of 256 keys at a time, one key per thread, online softmax.
-__global__ __launch_bounds__(256) void latent_attn_f32_kernel(LatentAttn a) {
-  extern __shared__ __align__(16) float fsm[];    // query row
-  __shared__ float ps[LA_KEYS], red[4];
-  __shared__ int pgs[LA_KEYS / PAGE];
-  const int t = blockIdx.x, h = blockIdx.y, d0 = blockIdx.z * 256 * LA_DPT;
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));   // 16 bytes at any element
+constexpr int LA_QBLOCKS = 48;  // query blocks that LDS takes
+
+// A workgroup takes one token, 16 heads (the columns of the matrix-core tiles: the heads of a key/value head) and NRB blocks of
+// the output (blockIdx.z); a wave takes every NW-th page, all in IEEE fp32 (v_mfma_f32_16x16x4_f32):
+//   S^T = K . Q^T       lane (token, g) holds 4 consecutive dims of its key, element e of the four g is one product
+//   O^T += V^T . P^T    lane (dims 4 r .. 4 r + 3, g) holds those of tokens 4 g + e: element i belongs to the row tile of the dims 4 r + i
+// so that every load is 16 contiguous bytes per lane and no operand changes lanes.  The waves' states (m, l, O) meet in LDS, added in the
+// order of the waves.  A page is 272 products of 32 cycles at rank 512 + 64: bound by the matrix cores while there are
+// workgroups enough, by the page's latency below that.  At rank 512 + 64 and 16 heads, 299 tokens at context 150: 75 us, one token at context 2048:
+// 134 us.  Every head by itself on the vector ALUs, each reading its keys twice: 649 and 705 us.
+template <int NRB, int NW>
+__global__ __launch_bounds__(NW * WAVE, NW == 8 ? 2 : 4) void latent_attn_f32_kernel(LatentAttn a) {
+  constexpr int NS = NRB / 2, CD = NRB * 32, LD = CD + 4;            // spans of 64 dims; columns of a chunk, padded
+  extern __shared__ __align__(16) float fsm[];                       // queries [block][half][lane][4], later the sums [16][LD]
+  __shared__ float sm[NW][16], sl[NW][16];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
+  const int t = blockIdx.x, b0 = blockIdx.z * NRB, qd = a.NB * 32, rd = a.RB * 32;
+  const int kvh = blockIdx.y / a.gt, hw = (blockIdx.y - kvh * a.gt) * 16, h0 = kvh * a.gs + hw, hn = a.gs - hw;
   int seq;
-  const int ctx = latent_ctx(a, t, seq), qd = a.NB * 32, rd = a.RB * 32;
-  const int32_t* bt = a.block_table + (size_t)seq * a.max_blocks;
-  for (int d = threadIdx.x; d < qd; d += 256) fsm[d] = a.q[((size_t)t * a.H + h) * qd + d];
-  const int kvh = h / a.gs;                       // one key/value head unless tied
-  const float slope = a.slopes ? a.slopes[h] : 0.f;
-  float m = a.sink ? a.sink[h] : -INFINITY, l = a.sink ? 1.f : 0.f, o[LA_DPT] = {};
-  for (int j0 = 0; j0 < ctx; j0 += LA_KEYS) {
-    __syncthreads();
-    if (threadIdx.x < LA_KEYS / PAGE) {
-      const int pg = j0 / PAGE + threadIdx.x;
-      const int page = pg * PAGE < ctx ? bt[pg] : -1;
-      pgs[threadIdx.x] = page >= 0 && page < a.n_pages ? page * a.G + kvh : -1;
+  const int ctx = latent_ctx(a, t, seq), npages = (ctx + PAGE - 1) / PAGE;
+  const int32_t* __restrict__ bt = a.block_table + (size_t)seq * a.max_blocks;
+  const float* __restrict__ q = a.q + ((size_t)t * a.H + h0) * qd;
+  const bool q_lds = a.NB <= LA_QBLOCKS;
+  if (q_lds) {
+    for (int i = threadIdx.x; i < a.NB * 128; i += NW * WAVE) {
+      const int c = i & 15, d = (i >> 7) * 32 + ((i >> 4) & 3) * 8 + ((i >> 6) & 1) * 4;
+      *reinterpret_cast<f32x4*>(fsm + i * 4) = c < hn ? *reinterpret_cast<const f32x4u*>(q + (size_t)c * qd + d) : f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    __syncthreads();
-    const int j = j0 + threadIdx.x, page = pgs[threadIdx.x / PAGE];
-    float s = -INFINITY;
-    if (j < ctx && page >= 0) {
-      const float* kp = a.cache + (size_t)page * a.NB * 512 + (j % PAGE) * 8;
-      float acc = 0.f;
-      for (int b = 0; b < a.NB * 4; ++b)
+  }
+  __syncthreads();
+  const int head = r16 < hn ? r16 : 0;                               // (columns past the heads: computed, not stored)
+  const float slope = a.slopes ? a.slopes[h0 + head] : 0.f;
+  const float* qg = q + (size_t)head * qd + g * 8;
+  float m = -INFINITY, l = 0.f;
+  f32x4 O[NS][4];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) acc = fmaf(kp[(size_t)b * 128 + e], fsm[b * 8 + e], acc);
-      s = acc * a.scale;
-      if (a.key_scale) s *= a.key_scale[(size_t)page * PAGE + j % PAGE];
-      if (a.slopes) s = fmaf(-slope, (float)(ctx - 1 - j), s);
-    }
-    float mx = wave_max(s);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
-    __syncthreads();
-    const float m_new = fmaxf(m, fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
-    const float alpha = m == -INFINITY ? 0.f : expf(m - m_new);
-    const float p = s == -INFINITY ? 0.f : expf(s - m_new);
-    ps[threadIdx.x] = p;
-    const float sum = wave_sum(p);
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = sum;
-    __syncthreads();
-    l = l * alpha + ((red[0] + red[1]) + (red[2] + red[3]));
-    m = m_new;
+  for (int s = 0; s < NS; ++s)
 #pragma unroll
-    for (int u = 0; u < LA_DPT; ++u) {
-      const int d = d0 + u * 256 + threadIdx.x;
-      o[u] *= alpha;
-      if (d >= rd) continue;
-      for (int k = 0; k < LA_KEYS && j0 + k < ctx; ++k) {
-        const int pg = pgs[k / PAGE];
-        if (pg >= 0) o[u] = fmaf(ps[k], a.cache[latent_offset(pg, a.NB, k % PAGE, d)], o[u]);
+    for (int i = 0; i < 4; ++i) O[s][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto mfma4 = [](const f32x4& x, const f32x4& y, f32x4 c) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], y[e], c, 0, 0, 0);
+    return c;
+  };
+  for (int pg = wave; pg < npages; pg += NW) {
+    const int id = bt[pg];
+    const bool ok = id >= 0 && id < a.n_pages;                       // a page outside the cache: every key of it is masked
+    const int page = (ok ? id : 0) * a.G + kvh;
+    const float* kp = a.cache + (size_t)page * a.NB * 512;
+    f32x4 st = f32x4{0.f, 0.f, 0.f, 0.f}, st1 = st;                  // S[token 4 g + r][head r16], two chains
+    auto scores = [&](int b, auto N) {                               // N blocks of 32 dims, all requested first
+      constexpr int n = decltype(N)::value;
+      f32x4 k[n][2];
+#pragma unroll
+      for (int u = 0; u < n; ++u)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) k[u][h] = *reinterpret_cast<const f32x4u*>(kp + (b + u) * 512 + g * 128 + r16 * 8 + 4 * h);
+#pragma unroll
+      for (int u = 0; u < n; ++u) {
+        f32x4 q0, q1;
+        if (q_lds) {                                                 // uniform
+          q0 = *reinterpret_cast<const f32x4*>(fsm + ((b + u) * 128 + lane) * 4);
+          q1 = *reinterpret_cast<const f32x4*>(fsm + ((b + u) * 128 + 64 + lane) * 4);
+        } else {
+          q0 = *reinterpret_cast<const f32x4u*>(qg + (b + u) * 32);
+          q1 = *reinterpret_cast<const f32x4u*>(qg + (b + u) * 32 + 4);
+        }
+        st = mfma4(k[u][0], q0, st);
+        st1 = mfma4(k[u][1], q1, st1);
       }
+    };
+    int b = 0;
+    constexpr int UB = NW == 8 ? 6 : 3;
+    for (; b + UB <= a.NB; b += UB) scores(b, std::integral_constant<int, UB>());
+    for (; b < a.NB; ++b) scores(b, std::integral_constant<int, 1>());
+    st += st1;
+    f32x4 ksc = f32x4{1.f, 1.f, 1.f, 1.f};
+    if (a.key_scale) ksc = *reinterpret_cast<const f32x4u*>(a.key_scale + (size_t)page * PAGE + 4 * g);
+    float pm = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int j = pg * PAGE + 4 * g + r;
+      float sc = st[r] * a.scale;
+      if (a.key_scale) sc *= ksc[r];
+      if (a.slopes) sc = fmaf(-slope, (float)(ctx - 1 - j), sc);
+      st[r] = !ok || j >= ctx ? -INFINITY : sc;
+      pm = fmaxf(pm, st[r]);
+    }
+    pm = fmaxf(pm, __shfl_xor(pm, 16, WAVE));
+    pm = fmaxf(pm, __shfl_xor(pm, 32, WAVE));
+    const float m_new = fmaxf(m, pm);
+    if (__any(m_new > m)) {                                          // uniform
+      const float alpha = m == -INFINITY ? 0.f : expf(m - m_new);
+      l *= alpha;
+#pragma unroll
+      for (int s = 0; s < NS; ++s)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) O[s][i] *= alpha;
+      m = m_new;
+    }
+    f32x4 p;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      p[r] = st[r] == -INFINITY ? 0.f : expf(st[r] - m);
+      l += p[r];
+    }
+    const bool whole = ok && (pg + 1) * PAGE <= ctx;                 // slots without a key may hold anything: taken as zero
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      int vb = b0 + 2 * s + (r16 >> 3);                              // (blocks past the output's: computed, not stored)
+      vb = vb < a.RB ? vb : a.RB - 1;
+      const float* vp = kp + vb * 512 + ((r16 >> 1) & 3) * 128 + 4 * g * 8 + (r16 & 1) * 4;
+      f32x4 v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        v[e] = *reinterpret_cast<const f32x4u*>(vp + e * 8);
+        if (!whole && (!ok || pg * PAGE + 4 * g + e >= ctx)) v[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) O[s][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e][i], p[e], O[s][i], 0, 0, 0);
     }
   }
-#pragma unroll
-  for (int u = 0; u < LA_DPT; ++u) {
-    const int d = d0 + u * 256 + threadIdx.x;
-    if (d < rd) a.out[((size_t)t * a.H + h) * rd + d] = l > 0.f ? o[u] / l : 0.f;
+  l += __shfl_xor(l, 16, WAVE);
+  l += __shfl_xor(l, 32, WAVE);
+  if (g == 0) {
+    sm[wave][r16] = m;
+    sl[wave][r16] = l;
   }
+  __syncthreads();                                                   // (and everybody is done with the queries)
+  float M = a.sink ? a.sink[h0 + head] : -INFINITY;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) M = fmaxf(M, sm[w][r16]);
+  float L = a.sink ? expf(a.sink[h0 + head] - M) : 0.f;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) L += sm[w][r16] == -INFINITY ? 0.f : sl[w][r16] * expf(sm[w][r16] - M);
+  const float f = m == -INFINITY ? 0.f : expf(m - M);
+  for (int w = 0; w < NW; ++w) {
+    if (wave == w) {
+#pragma unroll
+      for (int s = 0; s < NS; ++s)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {                                // dims 64 s + 4 (4 g + j) .. + 3 of head r16
+          f32x4* o = reinterpret_cast<f32x4*>(fsm + r16 * LD + s * 64 + 16 * g + 4 * j);
+          const f32x4 v = f32x4{O[s][0][j], O[s][1][j], O[s][2][j], O[s][3][j]} * f;
+          *o = w ? *o + v : v;
+        }
+    }
+    __syncthreads();
+  }
+  if (wave == 0 && g == 0) sl[0][r16] = L;
+  __syncthreads();
+  for (int i = threadIdx.x; i < 16 * (CD / 4); i += NW * WAVE) {
+    const int c = i / (CD / 4), d = (i - c * (CD / 4)) * 4;
+    if (c >= hn || b0 * 32 + d >= rd) continue;
+    const f32x4 v = *reinterpret_cast<const f32x4*>(fsm + c * LD + d);
+    const float den = sl[0][c];
+    *reinterpret_cast<f32x4u*>(a.out + ((size_t)t * a.H + h0 + c) * rd + b0 * 32 + d) = den > 0.f ? v / den : f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+}
+
+template <int NRB, int NW>
+int launch_latent_f32(const LatentAttn& a, int tiles, hipStream_t s) {
+  const size_t q = (size_t)(a.NB <= LA_QBLOCKS ? a.NB : 0) * 2048, o = (size_t)16 * (NRB * 32 + 4) * sizeof(float);
+  static const hipError_t configured =               // the attribute is per kernel, set once per process, by one thread
+      hipFuncSetAttribute((const void*)latent_attn_f32_kernel<NRB, NW>, hipFuncAttributeMaxDynamicSharedMemorySize, LA_QBLOCKS * 2048);
+  if (configured != hipSuccess) return mlora_set_error(MLORA_ERR_LAUNCH, "latent_attn: cannot reserve LDS: %s", hipGetErrorString(configured));
+  hipLaunchKernelGGL((latent_attn_f32_kernel<NRB, NW>), dim3(a.T, tiles, ceil_div(a.RB, NRB)), dim3(NW * WAVE), q > o ? q : o, s, a);
+  return MLORA_OK;
+}
+
+// tiles: of 16 heads.  Few workgroups: more of them (with narrower outputs, the scores computed by each) and more waves on the pages.
+int launch_latent_f32(LatentAttn a, hipStream_t s) {
+  if (!a.key_scale) a.G = 1, a.gs = a.H, a.gt = ceil_div(a.H, 16);
+  const int tiles = a.G * a.gt;
+  if ((long)a.T * tiles < 256) return launch_latent_f32<4, 16>(a, tiles, s);
+  if (a.RB <= 4) return launch_latent_f32<4, 8>(a, tiles, s);
+  if (a.RB <= 8) return launch_latent_f32<8, 8>(a, tiles, s);
+  return launch_latent_f32<16, 8>(a, tiles, s);
 }
 #endif
 
@@ -1148,7 +1265,7 @@ static int latent_attn_impl(void* out, const void* q, const void* cache, const i
 #ifdef MLORA_ELT_F32
   (void)o; (void)workspace; (void)workspace_bytes;
   MLORA_CHECK(splits == 1 && a.NB * 128 <= 48 * 1024, MLORA_ERR_UNSUPPORTED, "latent_attn: splits=%d R=%d not served in fp32", splits, R);
-  hipLaunchKernelGGL(latent_attn_f32_kernel, dim3(T, H, ceil_div(a.RB * 32, 256 * LA_DPT)), dim3(256), a.NB * 128, s, a);
+  if (const int e = launch_latent_f32(a, s)) return e;
 #else
   if (splits > 1) {
     MLORA_CHECK(workspace && workspace_bytes >= mlora_latent_attn_workspace_bytes(T, H, R, splits), MLORA_ERR_WORKSPACE,
@@ -1337,7 +1454,7 @@ extern "C" int mlora_tied_attn(void* out, int out_layout, const void* q, const v
 #ifdef MLORA_ELT_F32
   (void)workspace; (void)workspace_bytes;
   MLORA_CHECK(splits == 1, MLORA_ERR_UNSUPPORTED, "tied_attn: splits=%d not served in fp32", splits);
-  hipLaunchKernelGGL(latent_attn_f32_kernel, dim3(T, H, ceil_div(a.RB * 32, 256 * LA_DPT)), dim3(256), a.NB * 128, s, a);
+  if (const int e = launch_latent_f32(a, s)) return e;
 #else
   if (splits > 1) {
     MLORA_CHECK(workspace && workspace_bytes >= mlora_latent_attn_workspace_bytes(T, H, D, splits), MLORA_ERR_WORKSPACE,

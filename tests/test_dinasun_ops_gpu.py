@@ -523,3 +523,27 @@ def test_linear_groups(D, ops, T, K, rows, ext):
         assert torch.equal(Wp.rows(i * rows, rows).unpack(), W[i * rows:(i + 1) * rows])
     assert y2.shape[0] == (1 if T > 64 else 8 if K >= 2048 else max(K // 256, 1))
     assert err(y2.sum(0), f64(xs[4]) @ f64(W[4 * rows:]).T) < 2e-6
+
+
+@pytest.mark.parametrize("T,ctx", [(1, 1), (3, 130), (70, 40), (300, 17)])
+@pytest.mark.parametrize("H,G,dim", [(4, 4, 24), (40, 2, 40), (18, 1, 200), (2, 1, 500)])
+def test_fp32_attention_of_few_and_many_tokens(D, T, ctx, H, G, dim):
+    """All output widths, heads that do not fill a tile of 16, workgroups of 8 and of 16 waves; what lies in slots without a key must
+    not count.  Scores are of order 1 (scale 1 / sqrt(dim)): their sums of dim products, of order sqrt(dim), round to about
+    2^-24 sqrt(dim / 8) sqrt(dim), times the scale 5e-7 at 500 dims, which is the relative error of a weight."""
+    dt, scale = torch.float32, dim ** -0.5
+    vals, pages, scales, bt, rng = tied_case(D, dt, [ctx + 5], H, G, dim)
+    put_values(D, vals, pages, scales, bt, H, G, dim, 1e-5)
+    pos = [ctx + 4 if t % 2 else (t * 7) % (ctx + 5) for t in range(T)]
+    spare = torch.ones(pages.shape[0], dtype=torch.bool, device=DEV)
+    spare[bt[1][bt[1] >= 0].long()] = False
+    pages[spare] = float("nan")
+    last = int(bt[1][(ctx + 4) // 16])
+    pages[last, :, :, :, (ctx + 4) % 16 + 1:] = float("nan")
+    q = rng.normal(size=(T, H, dim))
+    slopes = R.slopes(H).astype(np.float32)
+    out = torch.empty((T, H * D.pad32(dim)), dtype=dt, device=DEV)
+    D.tied_attn(put_q(D, q, dt), pages, scales, bt, i32([1] * T), i32(pos), torch.from_numpy(slopes).to(DEV), scale, G, dim, ctx + 5, out)
+    torch.cuda.synchronize()
+    got, want = out.view(T, H, -1)[..., :dim], tied_want(vals, q.astype(np.float32).astype(np.float64), [0] * T, pos, slopes, scale, 1e-5)
+    assert err(got, want) < tol(dt)
