@@ -158,7 +158,7 @@ def linear_sum(x, W, split=True):
     T, K = x.shape
     N = W.shape[0]
     L = lib_of(W.dtype)
-    ks = L.mlora_gemv_ksplit(T, K, N)
+    ks = ops._size(W.dtype, "mlora_gemv_ksplit", T, K, N)
     y = torch.empty((T, N), dtype=torch.float32, device=x.device)
     part = torch.empty((ks - 1) * T * N, dtype=torch.float32, device=x.device) if ks > 1 else None
     check(L.mlora_linear_ksplit_store(y.data_ptr(), _ptr(part), ks, x.data.data_ptr(), W.data.data_ptr(), T, K, N, _stream()), W.dtype)
@@ -230,7 +230,7 @@ def gate_up_clipglu(x, W, W_il, scale, limit, alpha, out):
         if T <= 64:
             check(L.mlora_gemv_frag_clipglu(out.data.data_ptr(), x.data.data_ptr(), W_il.data.data_ptr(), *args), x.dtype)
             return out
-        if L.mlora_gemm_frag_preferred(T, K, I2):
+        if ops._size(x.dtype, "mlora_gemm_frag_preferred", T, K, I2):
             check(L.mlora_linear_frag_clipglu(out.data.data_ptr(), x.data.data_ptr(), W.data.data_ptr(), *args), x.dtype)
             return out
     return clipglu_mul(ops.linear(x, W), scale, limit, alpha, out)
@@ -257,7 +257,7 @@ def gate_up_silu(x, W, W_il, out):
         if T <= 64:
             check(L.mlora_gemv_frag_silu(out.data.data_ptr(), x.data.data_ptr(), W_il.data.data_ptr(), T, K, I2 // 2, _stream()), x.dtype)
             return out
-        if L.mlora_gemm_frag_preferred(T, K, I2):
+        if ops._size(x.dtype, "mlora_gemm_frag_preferred", T, K, I2):
             check(L.mlora_linear_frag_silu(out.data.data_ptr(), x.data.data_ptr(), W.data.data_ptr(), T, K, I2 // 2, None, 0, None, 0, _stream()),
                   x.dtype)
             return out
@@ -341,8 +341,8 @@ def tied_attn(q, pages, key_scale, block_table, tok_seq, tok_pos, slopes, scale,
     n_seq, max_blocks = block_table.shape
     L = lib_of(q.dtype)
     if splits is None:
-        splits = L.mlora_tied_attn_splits(T, H, G, max_ctx)
-    nb = L.mlora_latent_attn_workspace_bytes(T, H, dim, splits)
+        splits = ops._size(q.dtype, "mlora_tied_attn_splits", T, H, G, max_ctx)
+    nb = ops._size(q.dtype, "mlora_latent_attn_workspace_bytes", T, H, dim, splits)
     ws = torch.empty(nb // 4, dtype=torch.float32, device=q.device) if nb else None
     frag = isinstance(out, FragActivation)
     check(L.mlora_tied_attn(out.data.data_ptr() if frag else _dev(out, q.dtype), FRAG if frag else ROWMAJOR, _dev(q), _dev(pages, q.dtype),
@@ -433,7 +433,7 @@ def latent_prefill(plan, q, q_rot, pages, uk, uv, sink, scale, R, dim, rot, vdim
 
 def latent_attn_splits(T, H, max_ctx, dtype) -> int:
     """Shares of the context that attention over contexts up to max_ctx is cut into."""
-    return lib_of(dtype).mlora_latent_attn_splits(T, H, max_ctx)
+    return ops._size(dtype, "mlora_latent_attn_splits", T, H, max_ctx)
 
 
 def latent_attn_out(q, pages, block_table, tok_seq, tok_pos, sink, scale, R, rot, splits, uv, vp, out):
@@ -442,7 +442,7 @@ def latent_attn_out(q, pages, block_table, tok_seq, tok_pos, sink, scale, R, rot
     T, H, _ = q.shape
     n_seq, max_blocks = block_table.shape
     L = lib_of(q.dtype)
-    nb = L.mlora_latent_attn_workspace_bytes(T, H, R, splits)
+    nb = ops._size(q.dtype, "mlora_latent_attn_workspace_bytes", T, H, R, splits)
     ws = torch.empty(nb // 4, dtype=torch.float32, device=q.device)
     frag = isinstance(out, FragActivation)
     check(L.mlora_latent_attn_out(out.data.data_ptr() if frag else _dev(out, q.dtype), FRAG if frag else ROWMAJOR, H * vp, _wptr(uv), vp, _dev(q),
@@ -459,9 +459,9 @@ def latent_attn(q, pages, block_table, tok_seq, tok_pos, sink, scale, R, rot, ma
     n_seq, max_blocks = block_table.shape
     L = lib_of(q.dtype)
     if splits is None:
-        splits = L.mlora_latent_attn_splits(T, H, max_ctx)
+        splits = ops._size(q.dtype, "mlora_latent_attn_splits", T, H, max_ctx)
     out = torch.empty((T, H, pad32(R)), dtype=q.dtype, device=q.device) if out is None else out
-    nb = L.mlora_latent_attn_workspace_bytes(T, H, R, splits)
+    nb = ops._size(q.dtype, "mlora_latent_attn_workspace_bytes", T, H, R, splits)
     ws = torch.empty(nb // 4, dtype=torch.float32, device=q.device) if nb else None
     check(L.mlora_latent_attn(_dev(out), _dev(q), _dev(pages, q.dtype), _dev(block_table, torch.int32), max_blocks, _dev(tok_seq, torch.int32),
                               _dev(tok_pos, torch.int32), _ptr(sink), scale, T, H, R, rot, pages.shape[0], n_seq, splits, _ptr(ws), nb, _stream()),

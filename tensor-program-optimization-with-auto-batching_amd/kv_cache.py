@@ -99,14 +99,11 @@ class PageTable:
         if device_meta is not None:
             tok_seq, tok_pos, ctx = device_meta
         elif decode:
-            tok_seq = torch.from_numpy(rows).to(self.device)
-            tok_pos = torch.from_numpy(base).to(self.device)
-            ctx = torch.from_numpy(base + 1).to(self.device)
+            tok_seq, tok_pos, ctx = torch.from_numpy(np.stack([rows, base, base + 1])).to(self.device)      # (one copy)
         else:
             ts = np.repeat(rows, append_lens).astype(np.int32)
             tp = np.concatenate([b + np.arange(n, dtype=np.int32) for b, n in zip(base, append_lens)]).astype(np.int32)
-            tok_seq = torch.from_numpy(ts).to(self.device)
-            tok_pos = torch.from_numpy(tp).to(self.device)
+            tok_seq, tok_pos = torch.from_numpy(np.stack([ts, tp])).to(self.device)
             ctx = None
         self._cur = (list(seq_ids), list(append_lens), decode, tok_seq, tok_pos, ctx)
 
@@ -202,15 +199,23 @@ class PagedLatentCache(PageTable):
         columns)."""
         if self._cur is None:
             raise RuntimeError("latent_attention outside begin_forward/end_forward")
-        seq_ids, append_lens, decode, tok_seq, tok_pos, _ = self._cur
+        seq_ids, append_lens, _, tok_seq, tok_pos, _ = self._cur
         ctx = [self.lens[s] + n for s, n in zip(seq_ids, append_lens)]
-        plan = None
-        if not decode and att.prompt_form_pays(list(zip(append_lens, ctx))):
-            if self._plan is None or self._plan[0] is not self._cur:         # one plan per pass serves all its layers
-                self._plan = (self._cur, PrefillPlan([(self.pages_of(s), n, c) for s, n, c in zip(seq_ids, append_lens, ctx)], self.device))
-            plan = self._plan[1]
         return att.attend(qkv, self.pages[layer], self.block_table, tok_seq, tok_pos, *self.rope[layer], max_ctx=max(ctx),
-                          store=self.owner[layer] == layer, plan=plan, out=out)
+                          store=self.owner[layer] == layer, plan=self.attention_plan(att), out=out)
+
+    def attention_plan(self, att):
+        """The pass's plan for the prompt form where `att` takes that (one serves all layers), else None.  Making it waits for the
+        stream: a model asks for it ahead of its first layer, while little is queued."""
+        seq_ids, append_lens, decode = self._cur[:3]
+        if decode:
+            return None
+        ctx = [self.lens[s] + n for s, n in zip(seq_ids, append_lens)]
+        if not att.prompt_form_pays(list(zip(append_lens, ctx))):
+            return None
+        if self._plan is None or self._plan[0] is not self._cur:
+            self._plan = (self._cur, PrefillPlan([(self.pages_of(s), n, c) for s, n, c in zip(seq_ids, append_lens, ctx)], self.device))
+        return self._plan[1]
 
 
 class PagedStateCache(PageTable):
@@ -262,21 +267,34 @@ class PagedStateCache(PageTable):
 
     def time_mix(self, run, mixes, mixer):
         """The recurrence of a layer run on the five mixes of the pass (mixer: time_mix.TimeMix)."""
-        m, plan, heads = self._pass(), None, mixer.spec.heads
-        if m["host"] is not None and mixer.prompt_form:
-            if heads not in m["ranges"]:
-                m["ranges"][heads] = TimeMixPlan(m["host"], heads, self.device)
-            plan = m["ranges"][heads]
-        return mixer.run(mixes, self.entries[run][0], m["segs"], self._cur[3], self._cur[4], plan)
+        m = self._pass()
+        return mixer.run(mixes, self.entries[run][0], m["segs"], self._cur[3], self._cur[4], self.time_mix_plan(mixer))
+
+    def time_mix_plan(self, mixer):
+        """The pass's ranges where `mixer` takes the prompt form, else None (made ahead of the first layer, as an attention's)."""
+        m, heads = self._pass(), mixer.spec.heads
+        if m["host"] is None or not mixer.prompt_form:
+            return None
+        if heads not in m["ranges"]:
+            m["ranges"][heads] = TimeMixPlan(m["host"], heads, self.device)
+        return m["ranges"][heads]
+
+    def attention_plan(self, att):
+        """The pass's plan where `att` takes the prompt form, else None.  Making it waits for the stream: a model asks for it ahead
+        of its first layer, while little is queued."""
+        m = self._pass()
+        seq_ids, append_lens, decode = self._cur[:3]
+        seqs = [(n, self.lens[s] + n) for s, n in zip(seq_ids, append_lens)]
+        if decode or not att.prompt_form_pays(seqs):
+            return None
+        if m["plan"] is None:
+            m["plan"] = PrefillPlan([(self.pages_of(s), n, c) for s, (n, c) in zip(seq_ids, seqs)], self.device)
+        return m["plan"]
 
     def tied_attention(self, run, y, att):
         """The attention of a layer run behind its input projection y (att: tied_attention.TiedAttention)."""
-        m = self._pass()
-        seq_ids, append_lens, decode, tok_seq, tok_pos, _ = self._cur
-        seqs = [(n, self.lens[s] + n) for s, n in zip(seq_ids, append_lens)]
-        plan = None
-        if not decode and att.prompt_form_pays(seqs):
-            if m["plan"] is None:
-                m["plan"] = PrefillPlan([(self.pages_of(s), n, c) for s, (n, c) in zip(seq_ids, seqs)], self.device)
-            plan = m["plan"]
-        return att.attend(y, *self.entries[run], self.block_table, tok_seq, tok_pos, max_ctx=max(c for _, c in seqs), plan=plan)
+        if self._cur is None:
+            raise RuntimeError("outside begin_forward/end_forward")
+        seq_ids, append_lens, _, tok_seq, tok_pos, _ = self._cur
+        max_ctx = max(self.lens[s] + n for s, n in zip(seq_ids, append_lens))
+        return att.attend(y, *self.entries[run], self.block_table, tok_seq, tok_pos, max_ctx=max_ctx, plan=self.attention_plan(att))

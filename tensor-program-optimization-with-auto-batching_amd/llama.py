@@ -245,7 +245,7 @@ class LlamaForCausalLM(CausalLM):
 
     def _workspace(self, T, K, r):
         # three slices: projections that share an input (q, k, v) keep their shrink results side by side
-        need = 3 * (ops.lib().mlora_gather_mm_workspace_bytes(T, K, r) // 4) + 4
+        need = 3 * (ops._size(torch.float16, "mlora_gather_mm_workspace_bytes", T, K, r) // 4) + 4
         if self._ws is None or self._ws.numel() < need:
             self._ws = torch.empty(need, dtype=torch.float32, device=self.device)
         return self._ws
@@ -488,7 +488,7 @@ class LlamaForCausalLM(CausalLM):
         adapter types of the pass."""
         if T > 64 or not any(self.lora_types[t].tables.get((l, proj)) is not None for t in tids):
             return 0
-        return ops.lib().mlora_gemv_shrink_rows(K, 1, 1)
+        return ops._size(torch.float16, "mlora_gemv_shrink_rows", K, 1, 1)
 
     @staticmethod
     def _linear_acc(x, W, resid, ks_ws, riding_rows=0):

@@ -5,11 +5,15 @@ enqueues on torch's current stream.  None of them has a CPU path.
 """
 from __future__ import annotations
 
+import functools
+import struct
+
 import torch
 
 from . import _lib
 from ._lib import F16, F32, ROWMAJOR, FRAG, STORE, ACCUMULATE, lib
 
+_BUCKET = struct.Struct("@PPiif4x")          # mlora_lora_bucket
 _LIB_OF = {torch.float16: "float16", torch.bfloat16: "bfloat16", torch.float32: "float32"}
 
 
@@ -23,7 +27,14 @@ def check(code: int, dtype: torch.dtype = torch.float16) -> None:
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """The current stream of the current device, without the object around it (6 us less per call)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+
+
+@functools.lru_cache(maxsize=4096)
+def _size(dtype, fn, *args):
+    """A sizing or shape-rule function of the library (they depend on their integer arguments alone)."""
+    return getattr(lib_of(dtype), fn)(*args)
 
 
 def _dev(t: torch.Tensor, dtype=None, name="tensor") -> int:
@@ -49,7 +60,7 @@ class FragActivation:
 
     def __init__(self, T: int, K: int, device, data: torch.Tensor = None, dtype: torch.dtype = torch.float16):
         self.T, self.K = T, K
-        n = lib_of(dtype if data is None else data.dtype).mlora_frag_activation_elems(T, K)
+        n = _size(dtype if data is None else data.dtype, "mlora_frag_activation_elems", T, K)
         self.data = torch.empty(n, dtype=dtype, device=device) if data is None else data
         if self.data.numel() < n:
             raise ValueError("FragActivation: buffer too small")
@@ -99,7 +110,7 @@ def _x_arg(x, name="x"):
 
 
 def gather_mm_workspace(T: int, K: int, r: int, device) -> torch.Tensor:
-    n = lib().mlora_gather_mm_workspace_bytes(T, K, r)
+    n = _size(torch.float16, "mlora_gather_mm_workspace_bytes", T, K, r)
     return torch.empty(max(n, 16) // 4, dtype=torch.float32, device=device)
 
 
@@ -149,31 +160,28 @@ def gather_mm_static(y, x, A, B, tok_adapter, scaling: float):
 def gather_mm_multi(y, x, buckets, tok_bucket, tok_adapter, workspace=None):
     """Adapters of several ranks in one batch: buckets = [(A [n_ad,r,K], B [n_ad,N,r], scaling) | None, ...]; token t uses
     adapter tok_adapter[t] of bucket tok_bucket[t] (-1 = none).  y is updated in place."""
-    import ctypes
-    from ._lib import LoraBucket
     xptr, xlay, T, K = _x_arg(x)
     N = y.shape[1]
     if y.shape[0] != T or tok_bucket.shape != (T,) or tok_adapter.shape != (T,):
         raise ValueError("gather_mm_multi: inconsistent shapes")
-    arr = (LoraBucket * len(buckets))()
+    arr = b""
     rmax = 8
     for i, bk in enumerate(buckets):
         if bk is None:                      # the bucket's adapters do not target this projection
-            arr[i].A = arr[i].B = None
+            arr += _BUCKET.pack(0, 0, 0, 0, 0.0)
             continue
         A, B, scaling = bk
         n_ad, r, K2 = A.shape
         if K2 != K or B.shape != (n_ad, N, r):
             raise ValueError(f"gather_mm_multi: bucket {i} has A{tuple(A.shape)} B{tuple(B.shape)} for K={K} N={N}")
-        arr[i].A, arr[i].B = _dev(A, torch.float16, "A"), _dev(B, torch.float16, "B")
-        arr[i].r, arr[i].n_ad, arr[i].scaling = r, n_ad, float(scaling)
+        arr += _BUCKET.pack(_dev(A, torch.float16, "A"), _dev(B, torch.float16, "B"), r, n_ad, float(scaling))
         rmax = max(rmax, r)
     if workspace is None:
         workspace = gather_mm_workspace(T, K, rmax, x.device)
     if not y.is_cuda or y.stride(1) != 1:
         raise ValueError("gather_mm_multi: y must be a GPU tensor with unit inner stride")
     ldy = y.stride(0) if T > 1 else max(N, y.stride(0))
-    check(lib().mlora_gather_mm_multi(y.data_ptr(), _dt(y), ldy, xptr, xlay, ctypes.cast(arr, ctypes.c_void_p), len(buckets),
+    check(lib().mlora_gather_mm_multi(y.data_ptr(), _dt(y), ldy, xptr, xlay, arr, len(buckets),
                                       _dev(tok_bucket, torch.int32, "tok_bucket"), _dev(tok_adapter, torch.int32, "tok_adapter"),
                                       T, K, N, _dev(workspace, torch.float32, "workspace"), workspace.numel() * 4, _stream()))
     return y
@@ -183,8 +191,6 @@ def gather_mm_multi_proj(y, x, proj_buckets, col_offsets, n_cols, tok_bucket, to
     """gather_mm_multi for several projections that read the same x and own disjoint column ranges of y (q, k, v in the
     fused qkv row; gate and up): proj_buckets[p] is the bucket list of projection p (as for gather_mm_multi, all of the
     same length), whose delta goes to y[:, col_offsets[p] : col_offsets[p] + n_cols[p]].  One launch at decode sizes."""
-    import ctypes
-    from ._lib import LoraBucket
     xptr, xlay, T, K = _x_arg(x)
     n_proj = len(proj_buckets)
     n_buckets = len(proj_buckets[0])
@@ -193,21 +199,19 @@ def gather_mm_multi_proj(y, x, proj_buckets, col_offsets, n_cols, tok_bucket, to
         raise ValueError("gather_mm_multi_proj: inconsistent shapes")
     if T == 0:
         return y
-    arr = (LoraBucket * (n_proj * n_buckets))()
+    arr = b""
     rmax = 8
     for p, buckets in enumerate(proj_buckets):
         for i, bk in enumerate(buckets):
-            e = arr[p * n_buckets + i]
             if bk is None:                      # the bucket's adapters do not target this projection
-                e.A = e.B = None
+                arr += _BUCKET.pack(0, 0, 0, 0, 0.0)
                 continue
             A, B, scaling = bk
             n_ad, r, K2 = A.shape
             if K2 != K or B.shape != (n_ad, n_cols[p], r):
                 raise ValueError(f"gather_mm_multi_proj: projection {p} bucket {i} has A{tuple(A.shape)} B{tuple(B.shape)} "
                                  f"for K={K} N={n_cols[p]}")
-            e.A, e.B = _dev(A, torch.float16, "A"), _dev(B, torch.float16, "B")
-            e.r, e.n_ad, e.scaling = r, n_ad, float(scaling)
+            arr += _BUCKET.pack(_dev(A, torch.float16, "A"), _dev(B, torch.float16, "B"), r, n_ad, float(scaling))
             rmax = max(rmax, r)
     if workspace is None:
         one = gather_mm_workspace(T, K, rmax, x.device).numel()
@@ -215,10 +219,8 @@ def gather_mm_multi_proj(y, x, proj_buckets, col_offsets, n_cols, tok_bucket, to
     if not y.is_cuda or y.stride(1) != 1:
         raise ValueError("gather_mm_multi_proj: y must be a GPU tensor with unit inner stride")
     ldy = y.stride(0) if T > 1 else max(y.shape[1], y.stride(0))
-    co = (ctypes.c_int32 * n_proj)(*[int(c) for c in col_offsets])
-    nc = (ctypes.c_int32 * n_proj)(*[int(c) for c in n_cols])
-    check(lib().mlora_gather_mm_multi_proj(y.data_ptr(), _dt(y), ldy, xptr, xlay, ctypes.cast(arr, ctypes.c_void_p), n_buckets, n_proj,
-                                           ctypes.cast(co, ctypes.c_void_p), ctypes.cast(nc, ctypes.c_void_p),
+    co, nc = (struct.pack(f"{n_proj}i", *(int(c) for c in v)) for v in (col_offsets, n_cols))
+    check(lib().mlora_gather_mm_multi_proj(y.data_ptr(), _dt(y), ldy, xptr, xlay, arr, n_buckets, n_proj, co, nc,
                                            _dev(tok_bucket, torch.int32, "tok_bucket"), _dev(tok_adapter, torch.int32, "tok_adapter"),
                                            T, K, _dev(workspace, torch.float32, "workspace"), workspace.numel() * 4, _stream()))
     return y
@@ -375,7 +377,7 @@ def _linear_frag(x, W, out, out_dtype, accumulate):
 
 def gemm_frag_preferred(T: int, K: int, N: int) -> bool:
     """Whether a [T, K] x [N, K]^T product of this size runs best with its activations in fragment order."""
-    return bool(lib().mlora_gemm_frag_preferred(T, K, N))
+    return bool(_size(torch.float16, "mlora_gemm_frag_preferred", T, K, N))
 
 
 def lora_block_adapters(tok_adapter: torch.Tensor, n_ad: int):
@@ -507,8 +509,8 @@ def linear_acc_ksplit(x: FragActivation, W: PackedWeight, resid: torch.Tensor, w
     if K2 != K or resid.shape != (T, N) or resid.dtype != torch.float32:
         raise ValueError(f"linear_acc_ksplit: x{x.shape} W{W.shape} resid{tuple(resid.shape)}")
     L = lib_of(W.dtype)
-    ks = L.mlora_gemv_ksplit(T, K, N + riding_rows) if ws is not None else 1
-    if ks > 1 and ws.numel() * 4 < L.mlora_gemv_ksplit_bytes(T, N, ks):
+    ks = _size(W.dtype, "mlora_gemv_ksplit", T, K, N + riding_rows) if ws is not None else 1
+    if ks > 1 and ws.numel() * 4 < _size(W.dtype, "mlora_gemv_ksplit_bytes", T, N, ks):
         ks = 1
     check(L.mlora_gemv_frag_acc_ksplit(_dev(resid, torch.float32), None, _dev(ws, torch.float32) if ks > 1 else None, ks,
                                        x.data.data_ptr(), W.data.data_ptr(), T, K, N, 0, None, None, 0, None, 0, 0, _stream()), W.dtype)

@@ -165,6 +165,8 @@ class SafolornForCausalLM(CausalLM):
         split = T <= 256 or bool(kv._cur[2])          # short passes and decode steps split K of the narrow output projections
         frag = self.dtype != torch.float32
         parts = branch = None
+        for L in self.layers if T else ():                    # what the host makes for the pass
+            kv.attention_plan(L["att"])
         for l, L in enumerate(self.layers):
             att, dense, moe = L["att"], L["dense"], L["moe"]
             n, n_row = self._norm(x, parts, branch, row=moe is not None)

@@ -76,7 +76,7 @@ class TimeMix:
         if self.dtype == torch.float32:
             rows = torch.empty((len(MIXES), T, width_p), dtype=self.dtype, device=device)
             return Mixes(list(rows), rows)
-        n = ops.lib_of(self.dtype).mlora_frag_activation_elems(T, width_p)
+        n = ops._size(self.dtype, "mlora_frag_activation_elems", T, width_p)
         data = torch.empty(len(MIXES) * n, dtype=self.dtype, device=device)
         return Mixes([ops.FragActivation(T, width_p, device, data[i * n:(i + 1) * n]) for i in range(len(MIXES))], data)
 
