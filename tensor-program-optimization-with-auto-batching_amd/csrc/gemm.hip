@@ -723,23 +723,25 @@ int launch_gemm_pp(void* y, const elt* x, int ldx, int x_tt, const elt* Wp, int 
 // Four (three) stages, of which three (two) are in flight per compute unit - across the barrier of a stage, which is
 // the bare instruction (bare_barrier): behind __syncthreads() the compiler first waits for every request in flight,
 // the ring ran as if it had one stage and the launch pulled 2 to 3.4 TB/s of weights whatever its depth.
-// What bounds the kernel now is what the second-level caches hand to the compute units: at 256 tokens the counters
-// show 417 MB of requests per 100 MB matrix (each weight fragment for two token blocks, the token block once per
-// row block), 70 % of them hits, delivered at 8 to 10 TB/s over the chip - every tiling that gives all compute units
-// a workgroup has to take in about that much.
+// What bounds the kernel is LDS: per stage of 256 x 96 the waves read 112 KiB of fragments and the loads bring 44 KiB, at 128
+// bytes a cycle, beside 768 cycles of products per SIMD; so the reads go out between the products (3 to 9 % of a launch over reads
+// ahead of them: gate/up at 137 tokens 61.7 -> 56.6 us).  It is neither the second-level caches (a compute unit can take in 130 GB/s
+// of hits, the kernel asks for 45) nor the depth of the ring (a ring of seven weight stages beside three of tokens was 2 to 5 %
+// slower).
 // grid = (weight-row blocks, K slices, token blocks).
 // With K slices, slice 0 produces the result proper (store or accumulate) and slice s > 0 stores its fp32 partial
 // sums to part[s - 1][T][ld_part] - for the two narrow accumulating linears of a layer, whose partials the next
 // RMSNorm of the row adds in slice order.
 // ---------------------------------------------------------------------------------------------
 constexpr int MID_KS = 2;                      // 32-k steps per stage
+constexpr int mid_stages(int FT) { return FT == 16 ? 3 : 4; }
 
 // GX: the rows are groups of gx_rows (a multiple of 16 FN) that read activations of their own, gx_stride elements apart.
 template <int OUT, int FT, int FN, bool GX = false>
 __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_mid_kernel(void* __restrict__ yv, float* __restrict__ part, int ld_part,
                                                                     const elt* __restrict__ xf, int x_tt, const elt* __restrict__ Wp,
                                                                     int T, int K, int N, int gx_rows = 0, long gx_stride = 0) {
-  constexpr int MID_STAGES = FT == 16 ? 3 : 4;
+  constexpr int MID_STAGES = mid_stages(FT);
   constexpr int SF = FN + FT;                  // fragments of one 32-k step: weights, then tokens
   constexpr int LF = MID_KS * SF;              // fragments per stage
   constexpr int LQ = (LF + PP_WAVES - 1) / PP_WAVES;   // ... of which a wave fetches LQ (fragment f = wave + 8 q: fragment f % SF of k-step f / SF)
@@ -750,8 +752,6 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_mid_kernel(void* __res
   constexpr int VM = (MID_STAGES - 2) * LQ;    // a wave's loads that may still be in flight when the next stage is read
   constexpr int VM1 = (MID_STAGES - 2) * (LQ - 1);   // ... for the waves with one fragment fewer
   static_assert(FT % 4 == 0 && FN % 2 == 0 && WNF <= 4, "the tile divides over the waves");
-  static_assert(VM == 5 || VM == 6 || VM == 8, "wait_next has an instruction for each of these");
-  static_assert(LREM == 0 || VM1 == 5 || VM1 == 6, "wait_next has an instruction for each of these");
   extern __shared__ __align__(16) elt smem[];  // [MID_STAGES][STAGE_ELEMS]; the output staging reuses it after the K loop
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int KB = K / 32;
@@ -835,24 +835,41 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_mid_kernel(void* __res
   // stage multiplied next has landed; with everybody's wait and fragment reads behind the barrier, the slot of the
   // stage just read is refilled
   auto wait_next = [&]() {
-    if (LREM != 0 && wave >= LREM) {             // uniform
-      if constexpr (VM1 == 5) asm volatile("s_waitcnt vmcnt(5) lgkmcnt(0)" ::: "memory");
-      else asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)" ::: "memory");
-      return;
-    }
-    if constexpr (VM == 5) asm volatile("s_waitcnt vmcnt(5) lgkmcnt(0)" ::: "memory");
-    else if constexpr (VM == 6) asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
+    if (LREM != 0 && wave >= LREM) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(VM1) : "memory");       // uniform
+    else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(VM) : "memory");
   };
-  auto stage = [&](auto U) {
+  // A stage: the fragment reads of its successor go out between its products.  All at once ahead of them, the reads of eight
+  // waves (8 - 16 KiB each, 128 bytes a cycle) hold up the first product by as long as the products take.
+  auto stage = [&](auto U, auto WHOLE) {
     constexpr int u = decltype(U)::value;
     wait_next();
     bare_barrier();
     issue();
-    read_frags(std::integral_constant<int, 1 - u>());
-    __builtin_amdgcn_sched_barrier(0);
-    multiply(U);
-    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (decltype(WHOLE)::value) {
+      constexpr int NP = MID_KS * WNF * WTF, NR = MID_KS * (WNF + WTF), SPAN = NP * 3 / 4;
+      const elt* st = smem + rd * STAGE_ELEMS + lane * 8;
+      rd = rd + 1 == MID_STAGES ? 0 : rd + 1;
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int p = 0; p < NP; ++p) {
+        const int ks = p / (WNF * WTF), i = p / WTF % WNF, j = p % WTF;
+        acc[i][j] = mfma_16x16x32(a[u][ks][i], b[u][ks][j], acc[i][j]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int r = p * NR / SPAN; r < (p + 1) * NR / SPAN && r < NR; ++r) {
+          const int rs = r / (WNF + WTF), f = r % (WNF + WTF);
+          if (f < WTF) b[1 - u][rs][f] = ld8(st + (rs * SF + FN + wt * WTF + f) * 512);
+          else a[1 - u][rs][f - WTF] = ld8(st + (rs * SF + wn * WNF + f - WTF) * 512);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      done_ks += MID_KS;
+    } else {
+      read_frags(std::integral_constant<int, 1 - u>());
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(U);
+      __builtin_amdgcn_sched_barrier(0);
+    }
   };
 #pragma unroll
   for (int i = 0; i < MID_STAGES - 1; ++i) issue();
@@ -861,11 +878,13 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_mid_kernel(void* __res
   issue();
   read_frags(std::integral_constant<int, 0>());
   int g = 0;
-  for (; g + 1 < nst; g += 2) {
-    stage(std::integral_constant<int, 0>());
-    stage(std::integral_constant<int, 1>());
+  const int whole = nks / MID_KS;              // stages of two steps; an odd slice ends in one of a single step
+  for (; g + 1 < whole; g += 2) {
+    stage(std::integral_constant<int, 0>(), std::true_type());
+    stage(std::integral_constant<int, 1>(), std::true_type());
   }
-  if (g < nst) stage(std::integral_constant<int, 0>());
+  if (g < nst) stage(std::integral_constant<int, 0>(), std::false_type());
+  if (g + 1 < nst) stage(std::integral_constant<int, 1>(), std::false_type());
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");   // nothing is in flight into the LDS that the epilogue reuses
   __syncthreads();
 
@@ -938,42 +957,45 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_mid_kernel(void* __res
   }
 }
 
-// Block shape and K slices of the mid-size kernel for a shape: 128-token blocks when 256-token ones would leave most
-// compute units without a workgroup, and 64 weight rows per block instead of 128 when that still leaves half of them
-// idle (up to 128 tokens: 170 instead of 192 us for the four linears of a 4096 / 11008 layer; with two token blocks
-// the narrow form loses, so it is not taken there); 96 rows for the launches without K slices where that fills more
-// units in the same number of rounds.
+// Block shape (16 ft tokens x 16 fn weight rows) and K slices of the mid-size kernel for a shape: the one that finishes first by
+// two estimates, in units of 31 ns per 64-k stage.  A workgroup takes ft + 1.6 fn + 1 per stage - its operands through LDS, the
+// products, the barrier (measured on 4096 x 12288: 0.46 us at 8 / 4, 0.63 at 8 / 8, 0.73 at 12 / 6, 0.92 at 16 / 8) - times the
+// rounds that the compute units need for all workgroups.  All of them together take in their fragments, 0.0012 each, and those that
+// miss the second-level caches (weights once, tokens once per XCD) 0.02 each.  The two overlap in part: root of the sum of squares.
+// Measured where the choice matters, in us: 137 tokens, q/k/v 33.9 at 8 / 6, 36.0 at 12 / 4, 48 at 16 / 6; gate/up (22016 rows)
+// 53.1 at 12 / 6, 60.8 at 16 / 6, 77.8 at 8 / 6; 300 tokens, q/k/v 49.8 at 12 / 6, 52.8 at 16 / 6, 71.5 at 8 / 8; o of 100 tokens in four
+// slices 14.0 at 8 / 4, 17.1 at 8 / 8; 512 tokens x 4096 x 4096 29.6 at 8 / 4, 38.2 at 8 / 6.
 struct MidShape {
   int ft, fn, ksplit;
 };
 MidShape gemm_mid_shape(int T, int K, int N, int ksplit_max) {
   const int by_k = (K / 32) / 16 < 1 ? 1 : (K / 32) / 16;   // at least 16 k-steps per slice
   const int ks_cap = ksplit_max < by_k ? ksplit_max : by_k;
-  MidShape m;
-  const int cols8 = ceil_div(N, 128);
-  m.ft = (T <= 128 || (long)cols8 * ceil_div(T, 256) * ksplit_max <= 128) ? 8 : 16;
-  const int tb = ceil_div(T, m.ft * 16);
-  m.fn = (long)cols8 * tb * ks_cap <= 128 ? 4 : 8;
-  if (ks_cap == 1 && m.fn == 8) {
-    // 96 rows per block where that takes no more rounds of the compute units than 128: more units busy, fewer bytes
-    // per workgroup (q/k/v at 256 tokens: 256 workgroups instead of 192, 43.9 -> 41.2 us; gate/up 230 instead of 172,
-    // 69.0 -> 63.3 us)
-    int n_cu = gemm_n_cu();
-    if (n_cu <= 0) n_cu = 256;
-    const int w8 = cols8 * tb, w6 = ceil_div(N, 96) * tb;
-    if (ceil_div(w6, n_cu) * (m.ft + 6) < ceil_div(w8, n_cu) * (m.ft + 8)) m.fn = 6;
-  }
-  const int cols = ceil_div(N, m.fn * 16);
-  int ks = 256 / (cols * tb);
-  if (ks > ks_cap) ks = ks_cap;
-  m.ksplit = ks < 1 ? 1 : ks;
-  return m;
+  int n_cu = gemm_n_cu();
+  if (n_cu <= 0) n_cu = 256;
+  MidShape best = {8, 4, 1};
+  double least = 0;
+  for (int ft = 8; ft <= 16; ft += 4)
+    for (int fn = 4; fn <= 8; fn += 2) {
+      const long rows = ceil_div(N, fn * 16), tb = ceil_div(T, ft * 16);
+      long ks = n_cu / (rows * tb);
+      ks = ks > ks_cap ? ks_cap : ks < 1 ? 1 : ks;
+      const double rounds = (double)((rows * tb * ks + n_cu - 1) / n_cu), unit = ft + 1.6 * fn + 1;
+      const double mine = rounds * unit / ks, tiles = ceil_div(T, 16);
+      const double all = 0.0012 * rows * (tiles + tb * fn) + 0.02 * (ceil_div(N, 16) + 8 * tiles);
+      const double cost = mine * mine + all * all;
+      if (least == 0 || cost < least) {
+        least = cost;
+        best = MidShape{ft, fn, (int)ks};
+      }
+    }
+  return best;
 }
 
 template <int OUT, int FT, int FN, bool GX = false>
 int launch_gemm_mid_shape(void* y, float* part, int ld_part, int ksplit, const elt* xf, int x_tt, const elt* Wp, int T, int K, int N,
                           hipStream_t s, int gx_rows = 0, long gx_stride = 0) {
-  constexpr size_t lds = (size_t)(FT == 16 ? 3 : 4) * MID_KS * (FN + FT) * 512 * sizeof(elt);
+  constexpr size_t lds = (size_t)mid_stages(FT) * MID_KS * (FN + FT) * 512 * sizeof(elt);
   static_assert(lds >= (size_t)PP_WAVES * PP_OUT_ELEMS * sizeof(elt), "the output staging fits the ring");
   static const hipError_t configured =               // the attribute is per kernel, set once per process, by one thread
       hipFuncSetAttribute((const void*)gemm_mid_kernel<OUT, FT, FN, GX>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -991,6 +1013,11 @@ int launch_gemm_mid(void* y, float* part, int ld_part, const MidShape& m, const 
     if (m.fn == 4) return launch_gemm_mid_shape<OUT, 8, 4>(y, part, ld_part, m.ksplit, xf, x_tt, Wp, T, K, N, s);
     if (m.fn == 6) return launch_gemm_mid_shape<OUT, 8, 6>(y, part, ld_part, m.ksplit, xf, x_tt, Wp, T, K, N, s);
     return launch_gemm_mid_shape<OUT, 8, 8>(y, part, ld_part, m.ksplit, xf, x_tt, Wp, T, K, N, s);
+  }
+  if (m.ft == 12) {
+    if (m.fn == 4) return launch_gemm_mid_shape<OUT, 12, 4>(y, part, ld_part, m.ksplit, xf, x_tt, Wp, T, K, N, s);
+    if (m.fn == 6) return launch_gemm_mid_shape<OUT, 12, 6>(y, part, ld_part, m.ksplit, xf, x_tt, Wp, T, K, N, s);
+    return launch_gemm_mid_shape<OUT, 12, 8>(y, part, ld_part, m.ksplit, xf, x_tt, Wp, T, K, N, s);
   }
   if (m.fn == 4) return launch_gemm_mid_shape<OUT, 16, 4>(y, part, ld_part, m.ksplit, xf, x_tt, Wp, T, K, N, s);
   if (m.fn == 6) return launch_gemm_mid_shape<OUT, 16, 6>(y, part, ld_part, m.ksplit, xf, x_tt, Wp, T, K, N, s);

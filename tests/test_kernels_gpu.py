@@ -1319,3 +1319,25 @@ def test_empty_batches(ops, synth):
     assert ops.embed(W, torch.empty((0,), dtype=torch.int32, device=DEV)).shape == (0, K)
     assert ops.argmax(torch.empty((0, 100), dtype=torch.float32, device=DEV)).shape == (0,)
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("T", [129, 176, 192, 193, 300])
+@pytest.mark.parametrize("K,N", [(32, 22016), (96, 12280), (1056, 4096), (160, 32000), (2080, 2048)])
+def test_mid_size_linear_block_shapes(ops, T, K, N):
+    """Token blocks of 128, 192 and 256 with 64 to 128 rows, odd numbers of k-steps, ragged edges: the bits of the row-major kernel (every
+    output adds its k-steps in the same order); with K slices, their sum."""
+    g = torch.Generator(device=DEV).manual_seed(T + K + N)
+    x = torch.randn((T, K), generator=g, device=DEV).half()
+    W = ops.PackedWeight((torch.randn((N, K), generator=g, device=DEV) * 0.05).half())
+    f = ops.FragActivation.pack(x)
+    assert torch.equal(ops.linear(f, W), ops.linear(x, W, kernel="gemm"))
+    r0 = torch.randn((T, N), generator=g, device=DEV)
+    r = r0.clone()
+    parts = ops.linear_acc_ksplit(f, W, r, torch.empty(3 * T * N, device=DEV))
+    if parts is not None:
+        for q in range(parts.ks - 1):
+            r += parts.part[q * T * N:(q + 1) * T * N].view(T, N)
+    want = r0.double() + x.double() @ W.unpack().double().T
+    room = r0.abs().double() + x.abs().double() @ W.unpack().abs().double().T
+    torch.cuda.synchronize()
+    assert bool(((r.double() - want).abs() <= (K + 4) * 2.0 ** -24 * room).all())
