@@ -283,7 +283,7 @@ class TimeMixPlan:
     """Ranges of a pass for `time_mix_prompt`: segs, per sequence (slot, first token, tokens, position of the first); tokens: of a
     range (chosen by the size of the pass)."""
 
-    def __init__(self, segs, heads, device, tokens=None):
+    def __init__(self, segs, heads, device, tokens=None, wait=True):
         if tokens is None:                                           # about four workgroups per compute unit
             tokens = min(max(1 << max(sum(n for _, _, n, _ in segs) * heads // 1024, 1).bit_length() - 1, 64), 256)
         ranges, seqs, self.n_states = [], [], 0
@@ -297,7 +297,8 @@ class TimeMixPlan:
             if parts > 1:
                 self.n_states += parts
         self.n_ranges, self.n_seqs = len(ranges), len(seqs)
-        both = torch.tensor([x for t in (*ranges, *seqs) for x in t], dtype=torch.int32).to(device)
+        both = torch.tensor([x for t in (*ranges, *seqs) for x in t], dtype=torch.int32)
+        both = both.to(device) if wait else ops.upload(both, device)
         self.ranges, self.seqs = both[: 8 * len(ranges)], both[8 * len(ranges):]
 
 
@@ -394,9 +395,9 @@ def latent_prep(q, q_off, pages, qkv, off_rot, off_c, off_kr, gain, c_norm, eps,
 
 class PrefillPlan:
     """Contexts and query tiles of a pass for `latent_prefill`: per sequence (cache pages of its whole context, tokens that
-    the pass appends, context length after it), in pass order."""
+    the pass appends, context length after it), in pass order.  wait=False: the copy is only queued, on the current stream."""
 
-    def __init__(self, seqs, device):
+    def __init__(self, seqs, device, wait=True):
         L = lib_of(torch.bfloat16)
         n = L.mlora_latent_prefill_tile_tokens()
         phys, tiles, t0 = [], [], 0
@@ -408,7 +409,8 @@ class PrefillPlan:
             t0 += new
         tiles.sort(key=lambda t: -(t[1] + t[3]))                     # the longest key ranges start first
         self.T, self.pages, self.n_tiles = t0, len(phys), len(tiles)
-        both = torch.tensor([x for t in tiles for x in t] + phys, dtype=torch.int32).to(device)
+        both = torch.tensor([x for t in tiles for x in t] + phys, dtype=torch.int32)
+        both = both.to(device) if wait else ops.upload(both, device)
         self.tiles, self.phys = both[: 4 * len(tiles)], both[4 * len(tiles):]
 
 

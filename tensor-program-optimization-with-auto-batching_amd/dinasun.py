@@ -143,7 +143,7 @@ class DinasunForCausalLM(CausalLM):
 
     # ------------------------------------------------------------------ forward
     def embed(self, input_ids: torch.Tensor) -> LoopHidden:
-        ids = input_ids.reshape(-1).to(self.device, torch.int32).contiguous()
+        ids = ops.upload(input_ids.reshape(-1), self.device, torch.int32).contiguous()
         entry = half = None
         if self.loop_in is not None:
             Hp = self.width_p
@@ -167,10 +167,6 @@ class DinasunForCausalLM(CausalLM):
         c, ids, entry = self.config, hidden.ids, hidden.entry
         T, Hp = hidden.shape
         split = T <= 256 or bool(kv._cur[2])          # short passes and decode steps split K of the narrow output projections
-        if T:
-            for l, _ in self.runs:                                # what the host makes for the pass
-                mixer = self.layers[l]["mixer"]
-                (kv.time_mix_plan if isinstance(mixer, TimeMix) else kv.attention_plan)(mixer)
         plans = self.routing.plans(ids) if T else {}
         stream = D.ResidualStream(hidden.x, self.dtype, c.residual_mult)
         for run, (l, enters) in enumerate(self.runs):

@@ -51,6 +51,7 @@ class PageTable:
         self.block_table = torch.from_numpy(self.table_h.copy()).to(self.device)
         self._dirty = False
         self._cur = None
+        self._staged = None     # (stream, event) of arrays queued last
 
     # ------------------------------------------------------------------ protocol
     def add_sequence(self, sid):
@@ -90,8 +91,10 @@ class PageTable:
                     raise RuntimeError("paged KV cache out of pages")
                 self.table_h[row, j] = self.free.pop(0)
                 self._dirty = True
+        self._join()
+        staged = self._dirty or device_meta is None
         if self._dirty:
-            self.block_table.copy_(torch.from_numpy(self.table_h), non_blocking=False)
+            self.block_table.copy_(ops.upload(torch.from_numpy(self.table_h), self.device))
             self._dirty = False
         decode = all(n == 1 for n in append_lens)
         rows = np.asarray([self.slot[s] for s in seq_ids], dtype=np.int32)
@@ -99,13 +102,29 @@ class PageTable:
         if device_meta is not None:
             tok_seq, tok_pos, ctx = device_meta
         elif decode:
-            tok_seq, tok_pos, ctx = torch.from_numpy(np.stack([rows, base, base + 1])).to(self.device)      # (one copy)
+            tok_seq, tok_pos, ctx = ops.upload(torch.from_numpy(np.stack([rows, base, base + 1])), self.device)
         else:
             ts = np.repeat(rows, append_lens).astype(np.int32)
             tp = np.concatenate([b + np.arange(n, dtype=np.int32) for b, n in zip(base, append_lens)]).astype(np.int32)
-            tok_seq, tok_pos = torch.from_numpy(np.stack([ts, tp])).to(self.device)
+            tok_seq, tok_pos = ops.upload(torch.from_numpy(np.stack([ts, tp])), self.device)
             ctx = None
+        if staged:
+            self._stage()
         self._cur = (list(seq_ids), list(append_lens), decode, tok_seq, tok_pos, ctx)
+
+    def _stage(self):
+        """Host-made arrays have been queued on the current stream (not waited for): another stream's work has to."""
+        if self.device.type == "cuda" and not torch.cuda.is_current_stream_capturing():
+            s = torch.cuda.current_stream(self.device)
+            self._staged = (s.cuda_stream, s.record_event())
+
+    def _join(self):
+        """Work queued from here on sees the arrays that were staged, on whichever stream (a capture begins behind a wait for the
+        whole device; no event from outside it may enter)."""
+        if self._staged is not None:
+            s = torch._C._cuda_getCurrentRawStream(self._staged[1].device.index)
+            if s != self._staged[0] and not torch.cuda.is_current_stream_capturing():
+                torch.cuda.current_stream(self.device).wait_event(self._staged[1])
 
     def end_forward(self):
         seq_ids, append_lens = self._cur[0], self._cur[1]
@@ -145,6 +164,7 @@ class PagedKVCache(PageTable):
         ops.paged_attn_decode - the call then returns (attention output, head shares of the o projection's shrink)."""
         if self._cur is None:
             raise RuntimeError("attention_with_fused_qkv outside begin_forward/end_forward")
+        self._join()
         _, append_lens, decode, tok_seq, tok_pos, ctx = self._cur
         T = sum(append_lens)
         qkv = qkv.view(T, n_q_heads + 2 * self.Hkv, self.D)
@@ -199,14 +219,14 @@ class PagedLatentCache(PageTable):
         columns)."""
         if self._cur is None:
             raise RuntimeError("latent_attention outside begin_forward/end_forward")
+        self._join()
         seq_ids, append_lens, _, tok_seq, tok_pos, _ = self._cur
         ctx = [self.lens[s] + n for s, n in zip(seq_ids, append_lens)]
         return att.attend(qkv, self.pages[layer], self.block_table, tok_seq, tok_pos, *self.rope[layer], max_ctx=max(ctx),
                           store=self.owner[layer] == layer, plan=self.attention_plan(att), out=out)
 
     def attention_plan(self, att):
-        """The pass's plan for the prompt form where `att` takes that (one serves all layers), else None.  Making it waits for the
-        stream: a model asks for it ahead of its first layer, while little is queued."""
+        """The pass's plan for the prompt form where `att` takes that (one serves all layers), else None."""
         seq_ids, append_lens, decode = self._cur[:3]
         if decode:
             return None
@@ -214,7 +234,8 @@ class PagedLatentCache(PageTable):
         if not att.prompt_form_pays(list(zip(append_lens, ctx))):
             return None
         if self._plan is None or self._plan[0] is not self._cur:
-            self._plan = (self._cur, PrefillPlan([(self.pages_of(s), n, c) for s, n, c in zip(seq_ids, append_lens, ctx)], self.device))
+            self._plan = (self._cur, PrefillPlan([(self.pages_of(s), n, c) for s, n, c in zip(seq_ids, append_lens, ctx)], self.device, wait=False))
+            self._stage()
         return self._plan[1]
 
 
@@ -249,6 +270,7 @@ class PagedStateCache(PageTable):
         {slot, first token, tokens, position}} - both None in a decode step - and the plans of the prompt forms, once taken."""
         if self._cur is None:
             raise RuntimeError("outside begin_forward/end_forward")
+        self._join()
         if self._meta is None or self._meta[0] is not self._cur:
             seq_ids, lens, decode = self._cur[:3]
             m = {"last": None, "segs": None, "plan": None, "ranges": {}, "host": None}
@@ -256,7 +278,8 @@ class PagedStateCache(PageTable):
                 ends = np.cumsum(lens)
                 m["host"] = segs = [(self.slot[s], int(e) - n, n, self.lens[s]) for s, n, e in zip(seq_ids, lens, ends)]
                 both = np.concatenate([np.asarray(segs, dtype=np.int32).reshape(-1), np.repeat(ends - 1, lens).astype(np.int32)])
-                both = torch.from_numpy(both).to(self.device)
+                both = ops.upload(torch.from_numpy(both), self.device)
+                self._stage()
                 m["segs"], m["last"] = both[: 4 * len(segs)].view(-1, 4), both[4 * len(segs):]
             self._meta = (self._cur, m)
         return self._meta[1]
@@ -271,24 +294,25 @@ class PagedStateCache(PageTable):
         return mixer.run(mixes, self.entries[run][0], m["segs"], self._cur[3], self._cur[4], self.time_mix_plan(mixer))
 
     def time_mix_plan(self, mixer):
-        """The pass's ranges where `mixer` takes the prompt form, else None (made ahead of the first layer, as an attention's)."""
+        """The pass's ranges where `mixer` takes the prompt form, else None."""
         m, heads = self._pass(), mixer.spec.heads
         if m["host"] is None or not mixer.prompt_form:
             return None
         if heads not in m["ranges"]:
-            m["ranges"][heads] = TimeMixPlan(m["host"], heads, self.device)
+            m["ranges"][heads] = TimeMixPlan(m["host"], heads, self.device, wait=False)
+            self._stage()
         return m["ranges"][heads]
 
     def attention_plan(self, att):
-        """The pass's plan where `att` takes the prompt form, else None.  Making it waits for the stream: a model asks for it ahead
-        of its first layer, while little is queued."""
+        """The pass's plan where `att` takes the prompt form, else None."""
         m = self._pass()
         seq_ids, append_lens, decode = self._cur[:3]
         seqs = [(n, self.lens[s] + n) for s, n in zip(seq_ids, append_lens)]
         if decode or not att.prompt_form_pays(seqs):
             return None
         if m["plan"] is None:
-            m["plan"] = PrefillPlan([(self.pages_of(s), n, c) for s, (n, c) in zip(seq_ids, seqs)], self.device)
+            m["plan"] = PrefillPlan([(self.pages_of(s), n, c) for s, (n, c) in zip(seq_ids, seqs)], self.device, wait=False)
+            self._stage()
         return m["plan"]
 
     def tied_attention(self, run, y, att):

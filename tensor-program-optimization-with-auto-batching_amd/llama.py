@@ -240,7 +240,7 @@ class LlamaForCausalLM(CausalLM):
     # ------------------------------------------------------------------ forward
     def embed(self, input_ids: torch.Tensor) -> torch.Tensor:
         """input_ids [T] or [b, s] int32 -> hidden [T, H] fp32 (the residual stream)."""
-        ids = input_ids.reshape(-1).to(self.device, torch.int32).contiguous()
+        ids = ops.upload(input_ids.reshape(-1), self.device, torch.int32).contiguous()
         return ops.embed(self.embed_tokens, ids, out_dtype=torch.float32)
 
     def _workspace(self, T, K, r):
@@ -511,7 +511,7 @@ class LlamaForCausalLM(CausalLM):
                 if p.size != w.size or (p.size and (p.min() < 0 or p.max() >= T)):
                     raise ValueError("sids / wids mismatch")
                 full[p] = w
-            out[tid] = full if host else torch.from_numpy(full).to(self.device)
+            out[tid] = full if host else ops.upload(torch.from_numpy(full), self.device)
         return out
 
     def prefill_a(self, tid, h, kv, wids):

@@ -5,6 +5,8 @@ from __future__ import annotations
 import numpy as np
 import torch
 
+from . import ops
+
 
 class CausalLM:
     dtypes = ("float16",)     # element types the model runs in
@@ -20,7 +22,7 @@ class CausalLM:
 
     def _last_rows(self, kv):
         lens = kv._cur[1]
-        return torch.from_numpy(np.cumsum(lens).astype(np.int64) - 1).to(self.device)
+        return ops.upload(torch.from_numpy(np.cumsum(lens).astype(np.int64) - 1), self.device)
 
     def prefill_no_adapter(self, h, kv):
         return self.forward(h, kv, None, self._last_rows(kv)), kv

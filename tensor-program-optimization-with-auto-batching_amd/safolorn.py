@@ -138,7 +138,7 @@ class SafolornForCausalLM(CausalLM):
 
     # ------------------------------------------------------------------ forward
     def embed(self, input_ids: torch.Tensor) -> TokenHidden:
-        ids = input_ids.reshape(-1).to(self.device, torch.int32).contiguous()
+        ids = ops.upload(input_ids.reshape(-1), self.device, torch.int32).contiguous()
         return TokenHidden(ops.embed(self.embed_tokens, ids, out_dtype=torch.float32), ids)
 
     def _norm(self, x, parts=None, branch=None, gain=1.0, row=False):
@@ -165,8 +165,6 @@ class SafolornForCausalLM(CausalLM):
         split = T <= 256 or bool(kv._cur[2])          # short passes and decode steps split K of the narrow output projections
         frag = self.dtype != torch.float32
         parts = branch = None
-        for L in self.layers if T else ():                    # what the host makes for the pass
-            kv.attention_plan(L["att"])
         for l, L in enumerate(self.layers):
             att, dense, moe = L["att"], L["dense"], L["moe"]
             n, n_row = self._norm(x, parts, branch, row=moe is not None)

@@ -1341,3 +1341,29 @@ def test_mid_size_linear_block_shapes(ops, T, K, N):
     room = r0.abs().double() + x.abs().double() @ W.unpack().abs().double().T
     torch.cuda.synchronize()
     assert bool(((r.double() - want).abs() <= (K + 4) * 2.0 ** -24 * room).all())
+
+
+@pytest.mark.parametrize("decode", [False, True])
+def test_staged_arrays_reach_another_stream(decode):
+    """begin_forward does not wait for its copies: work on another stream than the one they were queued on has to."""
+    kvm = load_pkg("kv_cache")
+    lens = [1, 1, 1] if decode else [5, 33, 1]
+    cache = kvm.PagedKVCache(1, 16, 2, 64, max_seqs=4, max_blocks=4, rope_theta=10000.0, max_pos=64, device=DEV)
+    for s in range(3):
+        cache.add_sequence(s)
+    busy = torch.randn(4096, 4096, device=DEV)
+    torch.cuda.synchronize()
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.cuda.stream(first):
+        for _ in range(20):                                # the copies queue behind milliseconds of work
+            busy = busy @ busy * 1e-3
+        cache.begin_forward([2, 0, 1], lens)
+    with torch.cuda.stream(second):
+        cache._join()
+        got = [t.clone() for t in (cache.block_table, *cache._cur[3:5])]
+    second.synchronize()
+    assert np.array_equal(got[0].cpu().numpy(), cache.table_h)
+    assert got[1].tolist() == [s for s, n in zip([2, 0, 1], lens) for _ in range(n)]
+    assert got[2].tolist() == [i for n in lens for i in range(n)]
+    torch.cuda.synchronize()
+    cache.end_forward()
