@@ -509,18 +509,41 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
   f32x4 acc[8][WTF];
   eltx8 a[2][8], b[2][WTF];
   int rd = 0;                                  // ring slot of the stage whose fragments are read next
-  auto read_frags = [&](auto U) {
+  // The token fragments of a wave: four in a row; of a plan's tile every fourth, so that the places a tile does have - often few of
+  // its 256 - spread over all waves, and the first `have` of them are worked on (uniform; fragments and products of the others are
+  // left out, their accumulators never stored).
+  auto tfrag = [&](int j) { return GROUPED ? wt + 4 * j : wt * WTF + j; };
+  auto fragments_of = [&](int L) {
+    if constexpr (!GROUPED) return WTF;
+    int n0, tile;
+    block_of(L < nb ? L : blockIdx.x, n0, tile);
+    const int places = gr.plan.tiles[tile].z - wt * 16;
+    return __builtin_amdgcn_readfirstlane(places <= 0 ? 0 : (places + 63) / 64);
+  };
+  auto read_frags = [&](auto U, int have) {
     constexpr int u = decltype(U)::value;
     const elt* st = smem + rd * PP_STAGE_ELEMS + lane * 8;
 #pragma unroll
-    for (int j = 0; j < WTF; ++j) b[u][j] = ld8(st + (PP_F + wt * WTF + j) * 512);
+    for (int j = 0; j < WTF; ++j)
+      b[u][j] = ld8(st + (PP_F + tfrag(j)) * 512);
+    {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) a[u][i] = ld8(st + (wn * 8 + i) * 512);
+      for (int i = 0; i < 8; ++i) a[u][i] = ld8(st + (wn * 8 + i) * 512);
+    }
     rd = (rd + 1) & (PP_STAGES - 1);
   };
   // half (uniform): -1 all eight row tiles, 0 / 1 the first / last four (a LoRA stage of the gate / up projection)
-  auto multiply = [&](auto U, int half) {
+  auto multiply = [&](auto U, int half, int have) {
     constexpr int u = decltype(U)::value;
+    if constexpr (GROUPED) {
+#pragma unroll
+      for (int j = 0; j < WTF; ++j)
+        if (j < have) {                        // uniform
+#pragma unroll
+          for (int i = 0; i < 8; ++i) acc[i][j] = mfma_16x16x32(a[u][i], b[u][j], acc[i][j]);
+        }
+      return;
+    }
     if (half != 1) {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
@@ -538,14 +561,14 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
   // everybody's: the barrier).  The wait also covers this wave's fragment reads of the stage about to be multiplied,
   // so after the barrier nobody reads that ring slot any more and it is refilled; then the reads of the successor go
   // out, then the MFMAs.
-  auto stage = [&](auto U, auto PLAIN, int half) {
+  auto stage = [&](auto U, auto PLAIN, int half, int have, int have_next) {
     constexpr int u = decltype(U)::value;
     asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
     __syncthreads();
     issue(PLAIN);
-    read_frags(std::integral_constant<int, 1 - u>());
+    read_frags(std::integral_constant<int, 1 - u>(), have_next);
     __builtin_amdgcn_sched_barrier(0);
-    multiply(U, half);
+    multiply(U, half, have);
     __builtin_amdgcn_sched_barrier(0);
   };
 
@@ -556,7 +579,8 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
   asm volatile("s_waitcnt vmcnt(8)" ::: "memory");     // the first stage of this wave has landed
   __syncthreads();
   issue(std::false_type());
-  read_frags(std::integral_constant<int, 0>());
+  int have_next = fragments_of(blockIdx.x);
+  read_frags(std::integral_constant<int, 0>(), have_next);
   elt* ostage = smem + PP_STAGES * PP_STAGE_ELEMS + wave * PP_OUT_ELEMS;
   const int r16 = lane & 15, g = lane >> 4;
   for (int L = blockIdx.x; L < nb; L += G) {
@@ -572,6 +596,8 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
       t0 = __builtin_amdgcn_readfirstlane(tile.y);
       tend = t0 + __builtin_amdgcn_readfirstlane(tile.z);
     }
+    const int have = have_next;
+    have_next = fragments_of(L + G);
     int nst = KB;                                      // KB and E are even (checked by the launcher): the register sets alternate
     if constexpr (LORA) {
       int slot;
@@ -583,14 +609,14 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
       if constexpr (SILU && LORA) {
         // one copy of the pair; a pair of LoRA stages belongs to one projection and multiplies that half of the tiles only
         const int half = kb < KB ? -1 : (has_gate && kb - KB < EP ? 0 : 1);   // uniform
-        stage(std::integral_constant<int, 0>(), std::false_type(), half);
-        stage(std::integral_constant<int, 1>(), std::false_type(), half);
+        stage(std::integral_constant<int, 0>(), std::false_type(), half, WTF, WTF);
+        stage(std::integral_constant<int, 1>(), std::false_type(), half, WTF, WTF);
       } else if (LORA && load_kb + 2 < KB) {             // uniform: the two stages fetched next are ordinary k-steps inside their block
-        stage(std::integral_constant<int, 0>(), std::true_type(), -1);
-        stage(std::integral_constant<int, 1>(), std::true_type(), -1);
+        stage(std::integral_constant<int, 0>(), std::true_type(), -1, WTF, WTF);
+        stage(std::integral_constant<int, 1>(), std::true_type(), -1, WTF, WTF);
       } else {
-        stage(std::integral_constant<int, 0>(), std::false_type(), -1);
-        stage(std::integral_constant<int, 1>(), std::false_type(), -1);
+        stage(std::integral_constant<int, 0>(), std::false_type(), -1, have, have);
+        stage(std::integral_constant<int, 1>(), std::false_type(), -1, have, kb + 2 < nst ? have : have_next);
       }
     }
     if constexpr (SILU) {
@@ -599,7 +625,7 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
       // are 512 contiguous bytes
 #pragma unroll
       for (int j = 0; j < WTF; ++j) {
-        const int t = t0 + (wt * WTF + j) * 16 + r16;
+        const int t = t0 + tfrag(j) * 16 + r16;
         if ((t >> 4) >= x_tt || (GROUPED && t >= tend)) continue;   // the token tile does not exist (the place is another expert's)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -617,7 +643,7 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
       // four channels of a token = one 8-byte piece of the output fragment
 #pragma unroll
       for (int j = 0; j < WTF; ++j) {
-        const int t = t0 + (wt * WTF + j) * 16 + r16;
+        const int t = t0 + tfrag(j) * 16 + r16;
         if (t >= tend) continue;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
@@ -649,7 +675,7 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
           for (int q = 0; q < 2; ++q) {
             const int c = q * 64 + lane;           // 16-byte chunk: token row c / 8, columns (c % 8) * 8 ..
             const int tr = c >> 3, cc = (c & 7) * 8;
-            const int t = t0 + (wt * WTF + j) * 16 + tr;
+            const int t = t0 + tfrag(j) * 16 + tr;
             int row = t;
             if constexpr (GROUPED) row = gr.plan.perm[t < tend ? t : tend - 1];
             const int n = n0 + (wn * 8 + h * 4) * 16 + cc;
@@ -671,7 +697,7 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
     } else {
 #pragma unroll
       for (int j = 0; j < WTF; ++j) {
-        const int t = t0 + (wt * WTF + j) * 16 + r16;
+        const int t = t0 + tfrag(j) * 16 + r16;
         if (t >= T) continue;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
