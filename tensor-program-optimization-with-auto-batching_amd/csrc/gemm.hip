@@ -1138,9 +1138,22 @@ extern "C" int mlora_linear_packed(void* y, int y_dtype, int mode, const void* x
 
 extern "C" int mlora_gemv_frag(void* y, int y_dtype, int mode, const void* xf, const void* Wp, int T, int K, int N, void* stream);
 
-// 256 x 256 output blocks: enough of them to give every compute unit one, and whole pairs of 32-k steps
+// 256 x 256 output blocks: enough of them to give every compute unit one, and whole pairs of 32-k steps (the forms with an
+// epilogue of their own - a gated product, LoRA deltas - exist from there on)
 extern "C" int mlora_gemm_frag_preferred(int T, int K, int N) {
   return T > 64 && K > 0 && K % 64 == 0 && N > 0 && (long)ceil_div(T, PP_F * 16) * ceil_div(N, PP_F * 16) >= 256;
+}
+
+// The plain linear: the persistent kernel or the mid-size one, whose smaller blocks cost 2 to 16 % where the rounds of 256 blocks are
+// full and save up to a third where they are not.  Measured, persistent / mid-size, bf16, us: one round of 160 blocks (2500 x 4096 x
+// 4096) 94 / 88, 176 (1000 x 11264 x 2048) 50 / 53, 192 (2000 x 6144 x 2048) 51 / 52, 224 (3500 x 4096 x 4096) 103 / 111, 256 105 / 115;
+// 264 (1500 x 11264 x 2048) 91 / 71, 288 (1500 x 12288 x 4096) 180 / 140, 336 (1792) 187 / 171, 344 (1000 x 22016 x 4096) 178 / 174,
+// 384 (1900 x 12288 x 4096) 192 / 181, 440 (2500 x 11264 x 2048) 105 / 120; from 512 on 0.98 to 1.16 as long.  From 345 to 400 blocks the
+// two differ by 0 to 6 % and a pass's other products of that size are fused with their epilogue: the persistent kernel stays.  Up to 128
+// tokens half of its work is padding: 128256 x 4096, 128 tokens 263 / 212, 200 tokens 272 / 280.
+static bool persistent_pays(int T, int K, int N) {
+  const long nb = (long)ceil_div(T, PP_F * 16) * ceil_div(N, PP_F * 16);
+  return K % 64 == 0 && T > 128 && nb >= 176 && (nb <= 256 || nb >= 345);
 }
 
 extern "C" int mlora_linear_frag(void* y, int y_dtype, int mode, const void* xf, const void* Wp, int T, int K, int N,
@@ -1154,7 +1167,7 @@ extern "C" int mlora_linear_frag(void* y, int y_dtype, int mode, const void* xf,
   const elt* W = (const elt*)Wp;
   const int tt = mlora_frag_tiles(T);
   int e;
-  if (mlora_gemm_frag_preferred(T, K, N)) {
+  if (persistent_pays(T, K, N)) {
     if (mode == MLORA_ACCUMULATE) e = launch_gemm_pp<OUT_ACC_F32>(y, x, 0, tt, W, T, K, N, s);
     else if (y_dtype == MLORA_F32) e = launch_gemm_pp<OUT_F32>(y, x, 0, tt, W, T, K, N, s);
     else e = launch_gemm_pp<OUT_F16>(y, x, 0, tt, W, T, K, N, s);

@@ -1343,6 +1343,20 @@ def test_mid_size_linear_block_shapes(ops, T, K, N):
     assert bool(((r.double() - want).abs() <= (K + 4) * 2.0 ** -24 * room).all())
 
 
+@pytest.mark.parametrize("T,N", [(128, 176), (129, 175), (129, 176), (256, 256), (200, 257), (255, 344), (256, 345), (1100, 37), (2310, 36), (1281, 71),
+                                 (4001, 23)])
+def test_linear_by_number_of_blocks(ops, T, N):
+    """Both sides of every line between the mid-size and the persistent kernel (N in blocks of 256 rows, the last one ragged), and blocks
+    whose number is no multiple of 8 or of a band: the bits of the row-major kernel."""
+    K, N = 128, N * 256 - 24
+    g = torch.Generator(device=DEV).manual_seed(T + N)
+    x = torch.randn((T, K), generator=g, device=DEV).half()
+    W = ops.PackedWeight((torch.randn((N, K), generator=g, device=DEV) * 0.05).half())
+    f = ops.FragActivation.pack(x)
+    assert torch.equal(ops.linear(f, W), ops.linear(x, W, kernel="gemm"))
+    assert torch.equal(ops.linear(f, W, out_dtype=torch.float32), ops.linear(x, W, out_dtype=torch.float32, kernel="gemm"))
+
+
 @pytest.mark.parametrize("decode", [False, True])
 def test_staged_arrays_reach_another_stream(decode):
     """begin_forward does not wait for its copies: work on another stream than the one they were queued on has to."""
