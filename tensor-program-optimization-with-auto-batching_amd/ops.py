@@ -34,10 +34,12 @@ def _stream() -> int:
 def upload(t: torch.Tensor, device, dtype=None) -> torch.Tensor:
     """A host tensor's copy on `device`, queued on the current stream; the host does not wait.  The values go through pinned memory
     of torch's pool, which keeps it until the copy has run.  (A copy from pageable memory waits for all that the stream holds: four
-    of them left the GPU idle for 100 to 400 us of an eager pass.)  A capture refuses the copy as it did: its replays would read
-    memory given back."""
+    of them left the GPU idle for 100 to 400 us of an eager pass.)  Above 64 KiB the host waits as it did: the copy engine that
+    takes those makes the next release of device memory, as a capture begins with, 3 ms longer.  A capture refuses the copy as it
+    did: its replays would read memory given back."""
     dtype = dtype or t.dtype
-    if t.is_cuda or not t.numel() or torch.device(device).type != "cuda" or torch.cuda.is_current_stream_capturing():
+    if (t.is_cuda or not 0 < t.numel() * dtype.itemsize <= 65536 or torch.device(device).type != "cuda"
+            or torch.cuda.is_current_stream_capturing()):
         return t.to(device, dtype)
     return torch.empty(t.shape, dtype=dtype, pin_memory=True).copy_(t).to(device, non_blocking=True)
 
