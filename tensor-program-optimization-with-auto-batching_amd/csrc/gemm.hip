@@ -1074,16 +1074,15 @@ int launch_gemm_lds(void* y, const elt* x, int ldx, const elt* Wp, int T, int K,
   return MLORA_OK;
 }
 
-// Block shape by problem size: 256 x 256 (wave 128 x 128) when there are enough blocks to fill the chip, else
-// 256 tokens x 64 columns (wave 64 x 64, several workgroups per CU) so that a few hundred tokens still spread
-// over all CUs.
+// Block shape by problem size: 256 x 256 on the persistent kernel when more than half of the compute units get a block (2500 x 4096 x
+// 4096, 160 blocks: 102 us against 136 on blocks of 256 x 64; 700 x 12288 x 4096, 144 blocks: 101, 138; up to 128 blocks 103, 94), else 256
+// tokens x 64 columns (wave 64 x 64, several workgroups per CU) so that a few hundred tokens still spread over all CUs.
 template <int OUT>
 int launch_gemm_lds_auto(void* y, const elt* x, int ldx, const elt* Wp, int T, int K, int N, hipStream_t s) {
-  if ((long)ceil_div(T, 256) * ceil_div(N, 256) >= 256) {
-    // x rows must be 16-byte aligned for the direct-to-LDS loads (ldx % 8 == 0 is checked; the base may be a slice)
-    if (((uintptr_t)x & 15) == 0 && K % 64 == 0) return launch_gemm_pp<OUT>(y, x, ldx, 0, Wp, T, K, N, s);
-    return launch_gemm_lds<OUT, 16, 16, 8, 8>(y, x, ldx, Wp, T, K, N, s);
-  }
+  const long nb = (long)ceil_div(T, 256) * ceil_div(N, 256);
+  // x rows must be 16-byte aligned for the direct-to-LDS loads (ldx % 8 == 0 is checked; the base may be a slice)
+  if (nb > 128 && ((uintptr_t)x & 15) == 0 && K % 64 == 0) return launch_gemm_pp<OUT>(y, x, ldx, 0, Wp, T, K, N, s);
+  if (nb >= 256) return launch_gemm_lds<OUT, 16, 16, 8, 8>(y, x, ldx, Wp, T, K, N, s);
   return launch_gemm_lds<OUT, 16, 4, 4, 4>(y, x, ldx, Wp, T, K, N, s);
 }
 

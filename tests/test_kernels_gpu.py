@@ -1357,6 +1357,19 @@ def test_linear_by_number_of_blocks(ops, T, N):
     assert torch.equal(ops.linear(f, W, out_dtype=torch.float32), ops.linear(x, W, out_dtype=torch.float32, kernel="gemm"))
 
 
+@pytest.mark.parametrize("T,N,K,shift", [(200, 128, 128, 0), (200, 129, 128, 0), (1300, 22, 64, 8), (1300, 22, 128, 4), (400, 70, 96, 0), (256, 255, 192, 0)])
+def test_row_major_linear_by_number_of_blocks(ops, T, N, K, shift):
+    """Row-major tokens on both sides of 128 blocks (N in blocks of 256 rows, the last one ragged), rows of a wider tensor, bases that are
+    not aligned to 16 bytes and odd pairs of k-steps: fp32 results within the rounding of K additions."""
+    N = N * 256 - 24
+    g = torch.Generator(device=DEV).manual_seed(T + N + shift)
+    x = torch.randn((T, K + 16), generator=g, device=DEV).half()[:, shift:shift + K]
+    W = ops.PackedWeight((torch.randn((N, K), generator=g, device=DEV) * 0.05).half())
+    y = ops.linear(x, W, out_dtype=torch.float32)
+    w = W.unpack().double()
+    assert bool(((y.double() - x.double() @ w.T).abs() <= (K + 2) * 2.0 ** -24 * (x.abs().double() @ w.abs().T)).all())
+
+
 @pytest.mark.parametrize("decode", [False, True])
 def test_staged_arrays_reach_another_stream(decode):
     """begin_forward does not wait for its copies: work on another stream than the one they were queued on has to."""
