@@ -3,6 +3,8 @@ import ctypes
 import json
 import os
 import re
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -119,6 +121,22 @@ def test_decoder_argument_validation():
     lp = lambda pages=4, dim=64, elems=1 << 30, sc=16: b.mlora_latent_prefill(16, 0, 64, 16, 64, 16, 16, 16, pages, 16, 1, 16, 16, None, 0.1, 8, 2, 64, dim, 16,
                                                                               64, 8, sc, elems, None)
     assert lp(pages=5) == -2 and lp(dim=256) == -2 and lp(elems=8) == -3 and lp(sc=None) == -1
+
+
+def test_experts_without_tiles():
+    """A plan of no tiles is nothing to do, a negative number is refused, in every library (in a process of its own: what a library gets
+    wrong here may be fatal)."""
+    load_pkg("build").ensure("bfloat16"), load_pkg("build").ensure("float32")
+    code = """
+import sys
+sys.path[:0] = [".", "tests"]
+from conftest import load_pkg
+for dt, rows in (("bfloat16", 16), ("float32", 64)):
+    call = lambda tiles: load_pkg("_lib").lib(dt).mlora_moe_linear(16, 16, 16, 16, 16, 16, rows, tiles, 64, 4, 64, 64, 2, 0, 1, 1.0, 16, 1 << 20, None)
+    assert call(0) == 0 and call(-1) < 0, dt
+"""
+    p = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=300)
+    assert p.returncode == 0, (p.returncode, p.stderr)
 
 
 # ------------------------------------------------------------------ the oracle by what the equations fix
