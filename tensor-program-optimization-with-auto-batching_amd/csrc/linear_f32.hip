@@ -10,6 +10,7 @@ namespace {
 
 constexpr int FB = 64;       // tokens of a block
 constexpr int FW = 8;        // waves of a workgroup
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));   // 16 bytes at any element
 
 struct F32Linear {
   float* y;
@@ -21,7 +22,6 @@ struct F32Linear {
   float alpha;
   int accumulate, act;       // act: MLORA_ACT_*
   int gather, scatter, top;  // expert tiles (blockIdx.y = tile): gather: x row = entry / top; scatter: y row = entry
-  int vec;                   // rows of y can be stored 16 bytes at a time
 };
 
 // The fp32 16 x 16 x 4 product takes one element per lane: a lane holds 4 consecutive k of its row, element e of the four
@@ -54,8 +54,8 @@ __device__ __forceinline__ void f32_store(const F32Linear& a, const MoePlan& pla
         v[r] *= v[r];
       }
     }
-    if (a.vec && n + 4 <= a.N) {
-      f32x4* q = reinterpret_cast<f32x4*>(p);
+    if (n + 4 <= a.N) {
+      f32x4u* q = reinterpret_cast<f32x4u*>(p);
       *q = a.accumulate ? *q + v : v;
     } else {
 #pragma unroll
@@ -95,12 +95,12 @@ __device__ __forceinline__ void f32_thin(const F32Linear& a, const MoePlan& plan
   auto load = [&](auto S, int p) {
     constexpr int s = decltype(S)::value;
     const int k = (p < steps ? p : 0) * 32, k1 = k + 16 < a.K ? k + 16 : k;     // past the end: valid addresses, not multiplied
-    wf[s][0] = *reinterpret_cast<const f32x4*>(wp + k);
-    wf[s][1] = *reinterpret_cast<const f32x4*>(wp + k1);
+    wf[s][0] = *reinterpret_cast<const f32x4u*>(wp + k);
+    wf[s][1] = *reinterpret_cast<const f32x4u*>(wp + k1);
 #pragma unroll
     for (int j = 0; j < RT; ++j) {
-      xf[s][j][0] = *reinterpret_cast<const f32x4*>(xp[j] + k);
-      xf[s][j][1] = *reinterpret_cast<const f32x4*>(xp[j] + k1);
+      xf[s][j][0] = *reinterpret_cast<const f32x4u*>(xp[j] + k);
+      xf[s][j][1] = *reinterpret_cast<const f32x4u*>(xp[j] + k1);
     }
   };
   auto turn = [&](auto S, int p) {
@@ -129,13 +129,16 @@ __device__ __forceinline__ void f32_thin(const F32Linear& a, const MoePlan& plan
   f32_store<FW, RT, RT>(a, plan, grouped, y, n0, t0, t1, red);
 }
 
+constexpr int wide_stages(int FN) { return FN == 4 ? 4 : 3; }
+
 // FN * 16 weight rows by up to 64 tokens: four waves share the rows (FN / 4 tiles each, all tokens), twice, for the two halves
 // of every 64 k.  Both operands go from global memory straight into an LDS ring (fragments of 16 rows x 16 k as the lanes read
 // them) that is NST - 1 stages of 64 k ahead, one bare barrier per stage.  Bound by the matrix cores (157 TFLOP/s nominal).
-template <int FN, int RT>
+// DIRECT: operands are 16-byte aligned; others go through registers.
+template <int FN, int RT, bool DIRECT>
 __device__ __forceinline__ void f32_wide(const F32Linear& a, const MoePlan& plan, int grouped, const float* __restrict__ x, const float* __restrict__ W,
                                          float* __restrict__ y, int n0, int t0, int t1, f32x4* smem) {
-  constexpr int NST = FN == 4 ? 4 : 3, RW = FN / 4, SF = FN + RT, LF = 4 * SF, LQ = (LF + FW - 1) / FW;   // fragments: of 16 k, of a stage, per loading wave
+  constexpr int NST = wide_stages(FN), RW = FN / 4, SF = FN + RT, LF = 4 * SF, LQ = (LF + FW - 1) / FW;   // fragments: of 16 k, of a stage, per loading wave
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
   // fragment f = wave + 8 q of a stage: 16 k number f / SF, there weight tile or (behind those) token tile f % SF
   const float* src[LQ];
@@ -162,9 +165,12 @@ __device__ __forceinline__ void f32_wide(const F32Linear& a, const MoePlan& plan
   auto request = [&](int s) {
 #pragma unroll
     for (int q = 0; q < LQ; ++q) {
-      const int k = s * 64 + fk[q];               // past the end: a valid address, not multiplied
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[q] + (k < a.K ? k : 0)),
-                                       (__attribute__((address_space(3))) void*)(smem + (slot * LF + fd[q]) * 64), 16, 0, 0);
+      const float* p = src[q] + (s * 64 + fk[q] < a.K ? s * 64 + fk[q] : 0);      // past the end: a valid address, not multiplied
+      f32x4* d = smem + (slot * LF + fd[q]) * 64;
+      if constexpr (DIRECT)
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)p, (__attribute__((address_space(3))) void*)d, 16, 0, 0);
+      else
+        d[lane] = *reinterpret_cast<const f32x4u*>(p);
     }
     slot = slot + 1 < NST ? slot + 1 : 0;
   };
@@ -210,7 +216,7 @@ __device__ __forceinline__ void f32_wide(const F32Linear& a, const MoePlan& plan
 }
 
 // FN: row tiles of a workgroup (1: f32_thin)
-template <int FN>
+template <int FN, bool DIRECT>
 __global__ __launch_bounds__(FW* WAVE, 2) void linear_f32_kernel(F32Linear a, MoePlan plan, int grouped) {
   extern __shared__ __align__(16) f32x4 f32_smem[];
   const int n0 = blockIdx.x * FN * 16;
@@ -229,7 +235,7 @@ __global__ __launch_bounds__(FW* WAVE, 2) void linear_f32_kernel(F32Linear a, Mo
   const int rt = __builtin_amdgcn_readfirstlane((t1 - t0 + 15) >> 4);
   auto block = [&](auto RT) {
     if constexpr (FN == 1) f32_thin<decltype(RT)::value>(a, plan, grouped, x, W, y, n0, t0, t1, f32_smem);
-    else f32_wide<FN, decltype(RT)::value>(a, plan, grouped, x, W, y, n0, t0, t1, f32_smem);
+    else f32_wide<FN, decltype(RT)::value, DIRECT>(a, plan, grouped, x, W, y, n0, t0, t1, f32_smem);
   };
   if (rt == 1) block(std::integral_constant<int, 1>());
   else if (rt == 2) block(std::integral_constant<int, 2>());
@@ -246,20 +252,19 @@ int f32_n_cu() {
   return n_cu;
 }
 
-template <int FN>
+template <int FN, bool DIRECT = true>
 int launch_f32(const char* who, const F32Linear& a, const MoePlan& plan, int grouped, int row_blocks, int heads, hipStream_t stream) {
-  constexpr size_t lds = FN == 1 ? FW * 4 * 1024 : (FN == 4 ? 4 : 3) * 4 * (FN + 4) * 1024;
+  constexpr size_t lds = FN == 1 ? FW * 4 * 1024 : wide_stages(FN) * 4 * (FN + 4) * 1024;
   static const hipError_t configured =               // the attribute is per kernel, set once per process, by one thread
-      hipFuncSetAttribute((const void*)linear_f32_kernel<FN>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      hipFuncSetAttribute((const void*)linear_f32_kernel<FN, DIRECT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (configured != hipSuccess) return mlora_set_error(MLORA_ERR_LAUNCH, "%s: cannot reserve %zu bytes of LDS: %s", who, lds, hipGetErrorString(configured));
-  hipLaunchKernelGGL((linear_f32_kernel<FN>), dim3(ceil_div(a.N, FN * 16), row_blocks, heads), dim3(FW * WAVE), lds, stream, a, plan, grouped);
+  hipLaunchKernelGGL((linear_f32_kernel<FN, DIRECT>), dim3(ceil_div(a.N, FN * 16), row_blocks, heads), dim3(FW * WAVE), lds, stream, a, plan, grouped);
   return mlora_launch_status(who);
 }
 
 int launch(const char* who, F32Linear a, const MoePlan& plan, int grouped, int row_blocks, int heads, void* stream) {
   MLORA_CHECK(a.K % 16 == 0 && a.ldx % 4 == 0 && a.hx % 4 == 0 && row_blocks <= 65535 && heads <= 65535, MLORA_ERR_UNSUPPORTED,
               "%s: need K %% 16 == 0 and rows aligned to 16 bytes (T=%d K=%d N=%d)", who, a.T, a.K, a.N);
-  a.vec = a.ldy % 4 == 0 && a.hy % 4 == 0 && ((uintptr_t)a.y & 15) == 0;
   // Rounds of the compute units times what a workgroup takes, in us at K = 2048 as measured for 1, 2 and 4 token tiles: 16 rows
   // 11, 13, 23; 64 rows 20, 25, 46; 128 rows 34, 45, 80.  So 16 rows serve a grid that does not fill the chip (32 x 7680 x 2048:
   // 45 against 96 and 173 us), 128 rows one that fills it several times over (4096 x 2048 x 11264: 3443, 1961, 1715 us), 64 rows
@@ -270,9 +275,11 @@ int launch(const char* who, F32Linear a, const MoePlan& plan, int grouped, int r
     return (double)((blocks + f32_n_cu() - 1) / f32_n_cu()) * (once + per_tile * rt);
   };
   const double c1 = cost(1, 8, 3.8), c4 = cost(4, 12, 9), c8 = cost(8, 20, 15);
-  if (c1 <= c4 && c1 <= c8) return launch_f32<1>(who, a, plan, grouped, row_blocks, heads, (hipStream_t)stream);
-  if (c4 <= c8) return launch_f32<4>(who, a, plan, grouped, row_blocks, heads, (hipStream_t)stream);
-  return launch_f32<8>(who, a, plan, grouped, row_blocks, heads, (hipStream_t)stream);
+  const bool direct = (((uintptr_t)a.x | (uintptr_t)a.W) & 15) == 0;           // x may begin at any column of a wider tensor
+  const hipStream_t s = (hipStream_t)stream;
+  if (c1 <= c4 && c1 <= c8) return launch_f32<1>(who, a, plan, grouped, row_blocks, heads, s);
+  if (c4 <= c8) return direct ? launch_f32<4>(who, a, plan, grouped, row_blocks, heads, s) : launch_f32<4, false>(who, a, plan, grouped, row_blocks, heads, s);
+  return direct ? launch_f32<8>(who, a, plan, grouped, row_blocks, heads, s) : launch_f32<8, false>(who, a, plan, grouped, row_blocks, heads, s);
 }
 
 }  // namespace

@@ -392,3 +392,20 @@ def test_fp32_linear_forms(ops, T, K, N):
     y1 = ops.linear(x, W, out=y0.clone(), accumulate=True)
     torch.cuda.synchronize()
     assert torch.equal(y1, y0 + y)
+
+
+@pytest.mark.parametrize("T,K,N", [(63, 208, 39), (130, 208, 2051), (200, 272, 8200), (300, 144, 33001)])
+def test_fp32_linear_at_any_element(ops, T, K, N):
+    """Operands that begin at any element give the bits of aligned ones, with 16, 64 and 128 rows per workgroup; the rows of y
+    likewise.  Rounding as in test_fp32_linear_forms."""
+    rng = np.random.default_rng(K + N)
+    x, W, y0 = (torch.from_numpy(rng.normal(size=s)).float().to(DEV) for s in ((T, K), (N, K), (T, N)))
+    y = ops.linear(x, W)
+    assert bool(((y.double() - x.double() @ W.double().T).abs() <= (K + 2) * 2.0 ** -24 * (x.abs().double() @ W.abs().double().T)).all())
+    at = lambda t, i: torch.cat([t.new_zeros(i), t.reshape(-1), t.new_zeros(4 - i)])[i:i + t.numel()].view(t.shape)
+    for i, j, k in ((1, 0, 2), (0, 2, 0), (3, 1, 1)):
+        wide = torch.cat([x.new_zeros(T, i), x, x.new_zeros(T, 8 - i)], 1)[:, i:i + K]      # columns of a wider tensor
+        out = at(y0, k)
+        ops.linear(wide, at(W, j), out=out, accumulate=True)
+        torch.cuda.synchronize()
+        assert torch.equal(out, y0 + y), (i, j, k)
