@@ -27,7 +27,7 @@ struct F32Linear {
 // The fp32 16 x 16 x 4 product takes one element per lane: a lane holds 4 consecutive k of its row, element e of the four
 // k-groups of 16 lanes is one MFMA (any order of k serves, as long as both operands have the same).
 //
-// At T x K x N = 299 x 2048 x 2048: 49 us (51 TFLOP/s), 1 x 2048 x 11264: 23 us (3.9 TB/s), 4096 x 2048 x 11264: 1715 us
+// At T x K x N = 299 x 2048 x 2048: 46 us (55 TFLOP/s), 1 x 2048 x 11264: 24 us (3.8 TB/s), 4096 x 2048 x 11264: 1715 us
 // (110 TFLOP/s).  The vector ALUs (64 x 64 blocks, both operands staged through LDS behind two barriers per 16 k): 122, 139,
 // 2415 us.
 
@@ -134,7 +134,8 @@ constexpr int wide_stages(int FN) { return FN == 4 ? 4 : 3; }
 // FN * 16 weight rows by up to 64 tokens: four waves share the rows (FN / 4 tiles each, all tokens), twice, for the two halves
 // of every 64 k.  Both operands go from global memory straight into an LDS ring (fragments of 16 rows x 16 k as the lanes read
 // them) that is NST - 1 stages of 64 k ahead, one bare barrier per stage.  Bound by the matrix cores (157 TFLOP/s nominal).
-// DIRECT: operands are 16-byte aligned; others go through registers.
+// With 64 rows a K of fewer than NST stages lies in LDS whole, in no more than it needs: up to four workgroups on a compute unit, where
+// each waits for its one or two stages.  DIRECT: operands are 16-byte aligned; others go through registers.
 template <int FN, int RT, bool DIRECT>
 __device__ __forceinline__ void f32_wide(const F32Linear& a, const MoePlan& plan, int grouped, const float* __restrict__ x, const float* __restrict__ W,
                                          float* __restrict__ y, int n0, int t0, int t1, f32x4* smem) {
@@ -180,15 +181,18 @@ __device__ __forceinline__ void f32_wide(const F32Linear& a, const MoePlan& plan
   for (int i = 0; i < RW; ++i)
 #pragma unroll
     for (int j = 0; j < RT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const bool whole = FN == 4 && nst < NST;        // uniform
 #pragma unroll
-  for (int s = 0; s < NST - 1; ++s) request(s);
+  for (int s = 0; s < NST - 1; ++s)
+    if (s < nst || !whole) request(s);
   int rd = 0;
   for (int s = 0; s < nst; ++s) {
     // stage s has landed (this wave's share: at most the NST - 2 stages behind it in flight; everybody's: the barrier), and
     // everybody is done with the slot of stage s - 1, which is requested anew
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NST - 2) * LQ) : "memory");
+    if (whole) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NST - 2) * LQ) : "memory");
     bare_barrier();
-    request(s + NST - 1);
+    if (!whole) request(s + NST - 1);
     const f32x4* st = smem + (rd * LF + kh * 2 * SF) * 64 + lane;
     rd = rd + 1 < NST ? rd + 1 : 0;
 #pragma unroll
@@ -252,11 +256,20 @@ int f32_n_cu() {
   return n_cu;
 }
 
+// LDS of a workgroup: the waves' sums (16 rows), the ring, or all of a K of fewer stages (which the sums fit as well)
+template <int FN>
+constexpr size_t f32_lds(int K) {
+  constexpr int NST = wide_stages(FN);
+  const int stages = (K + 63) / 64;
+  return FN == 1 ? FW * 4 * 1024 : (FN == 4 && stages < NST ? stages : NST) * 4 * (FN + 4) * 1024;
+}
+
 template <int FN, bool DIRECT = true>
 int launch_f32(const char* who, const F32Linear& a, const MoePlan& plan, int grouped, int row_blocks, int heads, hipStream_t stream) {
-  constexpr size_t lds = FN == 1 ? FW * 4 * 1024 : wide_stages(FN) * 4 * (FN + 4) * 1024;
+  constexpr int most = (int)f32_lds<FN>(1 << 20);
   static const hipError_t configured =               // the attribute is per kernel, set once per process, by one thread
-      hipFuncSetAttribute((const void*)linear_f32_kernel<FN, DIRECT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      hipFuncSetAttribute((const void*)linear_f32_kernel<FN, DIRECT>, hipFuncAttributeMaxDynamicSharedMemorySize, most);
+  const size_t lds = f32_lds<FN>(a.K);
   if (configured != hipSuccess) return mlora_set_error(MLORA_ERR_LAUNCH, "%s: cannot reserve %zu bytes of LDS: %s", who, lds, hipGetErrorString(configured));
   hipLaunchKernelGGL((linear_f32_kernel<FN, DIRECT>), dim3(ceil_div(a.N, FN * 16), row_blocks, heads), dim3(FW * WAVE), lds, stream, a, plan, grouped);
   return mlora_launch_status(who);
@@ -265,16 +278,22 @@ int launch_f32(const char* who, const F32Linear& a, const MoePlan& plan, int gro
 int launch(const char* who, F32Linear a, const MoePlan& plan, int grouped, int row_blocks, int heads, void* stream) {
   MLORA_CHECK(a.K % 16 == 0 && a.ldx % 4 == 0 && a.hx % 4 == 0 && row_blocks <= 65535 && heads <= 65535, MLORA_ERR_UNSUPPORTED,
               "%s: need K %% 16 == 0 and rows aligned to 16 bytes (T=%d K=%d N=%d)", who, a.T, a.K, a.N);
-  // Rounds of the compute units times what a workgroup takes, in us at K = 2048 as measured for 1, 2 and 4 token tiles: 16 rows
-  // 11, 13, 23; 64 rows 20, 25, 46; 128 rows 34, 45, 80.  So 16 rows serve a grid that does not fill the chip (32 x 7680 x 2048:
-  // 45 against 96 and 173 us), 128 rows one that fills it several times over (4096 x 2048 x 11264: 3443, 1961, 1715 us), 64 rows
-  // what lies between (299 x 7680 x 2048: 193, 165, 290 us).
+  // The form that finishes first, in us by what was measured with 1, 2 and 4 token tiles: rounds of the compute units times what a workgroup
+  // multiplies (at K = 2048: 64 rows 15, 24, 41; 128 rows 30, 45, 75) and what it waits for (3.2 and 4; where K lies in LDS whole, several
+  // wait at once); 16 rows per workgroup take 10, 13.5 and 20, and at least 24 ns per k of the first 256, one stage of every wave.  So 16 rows
+  // serve a grid that does not fill the chip (32 x 7680 x 2048: 45 against 96 and 173 us), 128 rows one that fills it several times over
+  // (4096 x 2048 x 11264: 3443, 1961, 1715 us), 64 rows what lies between (299 x 7680 x 2048: 193, 165, 290 us) and every K up to 128
+  // (4000 x 64 x 4096: 128, 34, 37 us; 467 x 64 x 9975 15, with one workgroup per compute unit 36).
   const int entries = grouped ? a.T / row_blocks : a.T, rt = entries >= FB ? FB / 16 : entries > 16 ? ceil_div(entries, 16) : 1;
-  auto cost = [&](int tiles, double once, double per_tile) {
-    const long blocks = (long)ceil_div(a.N, tiles * 16) * row_blocks * heads;
-    return (double)((blocks + f32_n_cu() - 1) / f32_n_cu()) * (once + per_tile * rt);
+  auto rounds = [&](int tiles, int at_once) {
+    const long blocks = (long)ceil_div(a.N, tiles * 16) * row_blocks * heads, slots = (long)f32_n_cu() * at_once;
+    return (double)((blocks + slots - 1) / slots);
   };
-  const double c1 = cost(1, 8, 3.8), c4 = cost(4, 12, 9), c8 = cost(8, 20, 15);
+  const double k = a.K / 2048.0;
+  const int thin_k = a.K < 256 ? a.K : 256, at_once = (int)((160 << 10) / f32_lds<4>(a.K));        // (of at most four: 32 waves)
+  const double c1 = rounds(1, 1) * fmax(0.024 * thin_k, 2.5 + (4 + 3.5 * rt) * k);
+  const double c4 = rounds(4, 1) * (7 + 8.5 * rt) * k + rounds(4, at_once < 4 ? at_once : 4) * 3.2;
+  const double c8 = rounds(8, 1) * ((15 + 15 * rt) * k + 4);
   const bool direct = (((uintptr_t)a.x | (uintptr_t)a.W) & 15) == 0;           // x may begin at any column of a wider tensor
   const hipStream_t s = (hipStream_t)stream;
   if (c1 <= c4 && c1 <= c8) return launch_f32<1>(who, a, plan, grouped, row_blocks, heads, s);

@@ -394,10 +394,10 @@ def test_fp32_linear_forms(ops, T, K, N):
     assert torch.equal(y1, y0 + y)
 
 
-@pytest.mark.parametrize("T,K,N", [(63, 208, 39), (130, 208, 2051), (200, 272, 8200), (300, 144, 33001)])
+@pytest.mark.parametrize("T,K,N", [(63, 208, 39), (65, 16, 2050), (130, 128, 4101), (65, 192, 4109), (130, 208, 2051), (65, 272, 8200), (190, 144, 8198)])
 def test_fp32_linear_at_any_element(ops, T, K, N):
-    """Operands that begin at any element give the bits of aligned ones, with 16, 64 and 128 rows per workgroup; the rows of y
-    likewise.  Rounding as in test_fp32_linear_forms."""
+    """Operands that begin at any element give the bits of aligned ones, with 16, 64 and 128 rows per workgroup, a K that lies in LDS whole and
+    one that does not; the rows of y likewise.  Rounding as in test_fp32_linear_forms."""
     rng = np.random.default_rng(K + N)
     x, W, y0 = (torch.from_numpy(rng.normal(size=s)).float().to(DEV) for s in ((T, K), (N, K), (T, N)))
     y = ops.linear(x, W)
