@@ -878,7 +878,7 @@ constexpr int LA_QBLOCKS = 48;  // query blocks that LDS takes
 // workgroups enough, by the page's latency below that.  At rank 512 + 64 and 16 heads, 299 tokens at context 150: 75 us, one token at context 2048:
 // 134 us.  Every head by itself on the vector ALUs, each reading its keys twice: 649 and 705 us.
 template <int NRB, int NW>
-__global__ __launch_bounds__(NW * WAVE, NW == 8 ? 2 : 4) void latent_attn_f32_kernel(LatentAttn a) {
+__global__ __launch_bounds__(NW * WAVE, NW == 8 && NRB > 2 ? 2 : 4) void latent_attn_f32_kernel(LatentAttn a) {
   constexpr int NS = NRB / 2, CD = NRB * 32, LD = CD + 4;            // spans of 64 dims; columns of a chunk, padded
   extern __shared__ __align__(16) float fsm[];                       // queries [block][half][lane][4], later the sums [16][LD]
   __shared__ float sm[NW][16], sl[NW][16];
@@ -939,7 +939,7 @@ __global__ __launch_bounds__(NW * WAVE, NW == 8 ? 2 : 4) void latent_attn_f32_ke
       }
     };
     int b = 0;
-    constexpr int UB = NW == 8 ? 6 : 3;
+    constexpr int UB = NW == 8 && NRB > 2 ? 6 : 3;
     for (; b + UB <= a.NB; b += UB) scores(b, std::integral_constant<int, UB>());
     for (; b < a.NB; ++b) scores(b, std::integral_constant<int, 1>());
     st += st1;
@@ -1039,12 +1039,22 @@ int launch_latent_f32(const LatentAttn& a, int tiles, hipStream_t s) {
   return MLORA_OK;
 }
 
-// tiles: of 16 heads.  Few workgroups: more of them (with narrower outputs, the scores computed by each) and more waves on the pages.
+// tiles: of 16 heads.  The fewer workgroups there are, the more waves share a context; few tiles also split the output in blocks of 128 dims
+// (the scores computed by each).  Four waves where a compute unit has workgroups for more: its waves then wait less for each other at the
+// end, which is what a short context costs.  16 / 8 / 4 waves, us: 20 tokens, 32 heads of 192 dims on 8 20.0 / 15.0 / 9.3 (320 workgroups);
+// 100 tokens at context 100, 32 heads of 64 dims on 32 112 / 77 / 32, with the output's two blocks instead of four 39 / 24; 300 at 300 400 / 295 / 144
+// and 152 / 106; 64 tokens at context 1500, 2 heads of 256 dims on 2 (256 workgroups) 67 / 72 / 104.
 int launch_latent_f32(LatentAttn a, hipStream_t s) {
   if (!a.key_scale) a.G = 1, a.gs = a.H, a.gt = ceil_div(a.H, 16);
   const int tiles = a.G * a.gt;
-  if ((long)a.T * tiles < 256) return launch_latent_f32<4, 16>(a, tiles, s);
-  if (a.RB <= 4) return launch_latent_f32<4, 8>(a, tiles, s);
+  const bool few = (long)a.T * tiles < 256;
+  if (few || a.RB <= 4) {
+    const long groups = (long)a.T * tiles * ceil_div(a.RB, 4);
+    const bool narrow = !few && a.RB <= 2;
+    if (groups >= 320) return narrow ? launch_latent_f32<2, 4>(a, tiles, s) : launch_latent_f32<4, 4>(a, tiles, s);
+    if (few && groups <= 256) return launch_latent_f32<4, 16>(a, tiles, s);
+    return narrow ? launch_latent_f32<2, 8>(a, tiles, s) : launch_latent_f32<4, 8>(a, tiles, s);
+  }
   if (a.RB <= 8) return launch_latent_f32<8, 8>(a, tiles, s);
   return launch_latent_f32<16, 8>(a, tiles, s);
 }

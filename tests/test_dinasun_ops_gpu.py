@@ -547,3 +547,19 @@ def test_fp32_attention_of_few_and_many_tokens(D, T, ctx, H, G, dim):
     torch.cuda.synchronize()
     got, want = out.view(T, H, -1)[..., :dim], tied_want(vals, q.astype(np.float32).astype(np.float64), [0] * T, pos, slopes, scale, 1e-5)
     assert err(got, want) < tol(dt)
+
+
+@pytest.mark.parametrize("T,n,H,G,dim", [(100, 40, 12, 4, 64), (70, 40, 4, 4, 40), (300, 20, 2, 1, 100), (110, 130, 6, 3, 128), (330, 17, 1, 1, 120), (90, 35, 2, 1, 500)])
+def test_fp32_attention_by_number_of_workgroups(D, T, n, H, G, dim):
+    """One to sixteen heads of a key/value head on four and on eight waves, outputs of 64 and 128 dims and in parts."""
+    dt, scale = torch.float32, dim ** -0.5
+    vals, pages, scales, bt, rng = tied_case(D, dt, [n], H, G, dim)
+    put_values(D, vals, pages, scales, bt, H, G, dim, 1e-5)
+    pos = [(t * 7) % n for t in range(T)]
+    q = rng.normal(size=(T, H, dim))
+    slopes = R.slopes(H).astype(np.float32)
+    out = torch.empty((T, H * D.pad32(dim)), dtype=dt, device=DEV)
+    D.tied_attn(put_q(D, q, dt), pages, scales, bt, i32([1] * T), i32(pos), torch.from_numpy(slopes).to(DEV), scale, G, dim, n, out)
+    torch.cuda.synchronize()
+    got, want = out.view(T, H, -1)[..., :dim], tied_want(vals, q.astype(np.float32).astype(np.float64), [0] * T, pos, slopes, scale, 1e-5)
+    assert err(got, want) < tol(dt)

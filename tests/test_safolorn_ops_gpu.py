@@ -409,3 +409,22 @@ def test_fp32_linear_at_any_element(ops, T, K, N):
         ops.linear(wide, at(W, j), out=out, accumulate=True)
         torch.cuda.synchronize()
         assert torch.equal(out, y0 + y), (i, j, k)
+
+
+@pytest.mark.parametrize("T,n,H,rank,rot", [(300, 60, 3, 200, 40), (290, 50, 16, 512, 64), (260, 33, 2, 100, 24), (330, 33, 2, 100, 24), (301, 40, 2, 64, 16),
+                                            (260, 40, 2, 60, 16), (100, 40, 17, 512, 64), (70, 40, 2, 512, 16), (2, 70, 18, 1600, 64), (70, 20, 1, 1560, 32),
+                                            (270, 18, 1, 1560, 32)])
+@pytest.mark.parametrize("sunk", [True, False])
+def test_fp32_latent_attention_of_prompts(D, T, n, H, rank, rot, sunk):
+    """Four, eight and sixteen waves, outputs of 64 to 512 dims and in parts, queries that do not fit LDS, a second tile of heads."""
+    dt = torch.float32
+    lat, pages, bt, rng = latent_case(D, dt, [n], H, rank, rot, seed=T)
+    pos = rng.integers(0, n, T)
+    q = torch.from_numpy(rng.normal(size=(T, H, rank + rot))).to(torch.bfloat16).double().numpy()
+    sink = rng.normal(2.0, 1.0, H).astype(np.float32) if sunk else None
+    scale = 3.0 * (rank + rot) ** -0.5
+    got = D.latent_attn(put_queries(D, q, rank, rot, dt), pages, bt, torch.ones(T, dtype=torch.int32, device=DEV),
+                        torch.from_numpy(pos.astype(np.int32)).to(DEV), torch.from_numpy(sink).to(DEV) if sunk else None, scale, rank, rot, max_ctx=n)
+    torch.cuda.synchronize()
+    assert err(got[..., :rank], attn_want(lat, q, [0] * T, pos, sink, scale, rank)) < tol(dt)
+    assert float(got[..., rank:].abs().sum()) == 0
