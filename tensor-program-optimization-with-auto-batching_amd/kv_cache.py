@@ -51,7 +51,8 @@ class PageTable:
         self.block_table = torch.from_numpy(self.table_h.copy()).to(self.device)
         self._dirty = False
         self._cur = None
-        self._staged = None     # (stream, event) of arrays queued last
+        self._staged = None     # (raw stream, event) of arrays queued last
+        self._users = {}        # raw stream -> (stream, event behind the last pass's work or None): streams whose work reads the arrays
 
     # ------------------------------------------------------------------ protocol
     def add_sequence(self, sid):
@@ -91,7 +92,7 @@ class PageTable:
                     raise RuntimeError("paged KV cache out of pages")
                 self.table_h[row, j] = self.free.pop(0)
                 self._dirty = True
-        self._join()
+        self._enter()
         staged = self._dirty or device_meta is None
         if self._dirty:
             self.block_table.copy_(ops.upload(torch.from_numpy(self.table_h), self.device))
@@ -112,25 +113,59 @@ class PageTable:
             self._stage()
         self._cur = (list(seq_ids), list(append_lens), decode, tok_seq, tok_pos, ctx)
 
+    # Host-made arrays are queued on the stream that is current, not waited for, and the next pass overwrites the block table.  So a
+    # stream that goes on with a pass waits for its arrays, and the stream that begins the next one waits for all that the last was
+    # queued on.  No event from outside may enter a capture: one begins behind a wait for the whole device, or on a stream that its
+    # caller has ordered.
+    def _raw_stream(self):
+        return torch._C._cuda_getCurrentRawStream(self.block_table.device.index)
+
+    def _enter(self):
+        """A pass begins on the current stream."""
+        if self.device.type != "cuda" or torch.cuda.is_current_stream_capturing():
+            return
+        raw = self._raw_stream()
+        stream = self._users[raw][0] if raw in self._users else torch.cuda.current_stream(self.device)
+        for r, (other, behind) in self._users.items():
+            if r != raw:
+                stream.wait_stream(other) if behind is None else stream.wait_event(behind)
+        self._users = {raw: (stream, None)}
+
     def _stage(self):
-        """Host-made arrays have been queued on the current stream (not waited for): another stream's work has to."""
+        """Arrays of the pass have been queued on the current stream."""
         if self.device.type == "cuda" and not torch.cuda.is_current_stream_capturing():
-            s = torch.cuda.current_stream(self.device)
-            self._staged = (s.cuda_stream, s.record_event())
+            raw = self._raw_stream()
+            if raw not in self._users:
+                self._users[raw] = (torch.cuda.current_stream(self.device), None)
+            self._staged = (raw, self._users[raw][0].record_event())
 
     def _join(self):
-        """Work queued from here on sees the arrays that were staged, on whichever stream (a capture begins behind a wait for the
-        whole device; no event from outside it may enter)."""
-        if self._staged is not None:
-            s = torch._C._cuda_getCurrentRawStream(self._staged[1].device.index)
-            if s != self._staged[0] and not torch.cuda.is_current_stream_capturing():
-                torch.cuda.current_stream(self.device).wait_event(self._staged[1])
+        """The pass goes on on the current stream."""
+        if self.device.type != "cuda":
+            return
+        raw = self._raw_stream()
+        elsewhere = self._staged is not None and raw != self._staged[0]
+        if (raw in self._users and not elsewhere) or torch.cuda.is_current_stream_capturing():
+            return
+        stream = torch.cuda.current_stream(self.device)
+        self._users[raw] = (stream, None)
+        if elsewhere:
+            stream.wait_event(self._staged[1])
+            for t in self._pass_arrays():          # their memory may be given out again, to the stream they were made on
+                t.record_stream(stream)
+
+    def _pass_arrays(self):
+        """Arrays that were made for the current pass."""
+        return [t for t in self._cur[3:] if t is not None]
 
     def end_forward(self):
         seq_ids, append_lens = self._cur[0], self._cur[1]
         for sid, n in zip(seq_ids, append_lens):
             self.lens[sid] += n
         self._cur = None
+        for raw, (stream, _) in self._users.items():         # (the default stream outlives every pass: no event before one is waited for)
+            if raw and not torch.cuda.is_current_stream_capturing():
+                self._users[raw] = (stream, stream.record_event())
 
     # ------------------------------------------------------------------ helpers
     def pages_of(self, sid):
@@ -225,6 +260,10 @@ class PagedLatentCache(PageTable):
         return att.attend(qkv, self.pages[layer], self.block_table, tok_seq, tok_pos, *self.rope[layer], max_ctx=max(ctx),
                           store=self.owner[layer] == layer, plan=self.attention_plan(att), out=out)
 
+    def _pass_arrays(self):
+        plan = self._plan[1] if self._plan is not None and self._plan[0] is self._cur else None
+        return super()._pass_arrays() + ([plan.tiles, plan.phys] if plan is not None else [])
+
     def attention_plan(self, att):
         """The pass's plan for the prompt form where `att` takes that (one serves all layers), else None."""
         seq_ids, append_lens, decode = self._cur[:3]
@@ -283,6 +322,14 @@ class PagedStateCache(PageTable):
                 m["segs"], m["last"] = both[: 4 * len(segs)].view(-1, 4), both[4 * len(segs):]
             self._meta = (self._cur, m)
         return self._meta[1]
+
+    def _pass_arrays(self):
+        out, m = super()._pass_arrays(), self._meta[1] if self._meta is not None and self._meta[0] is self._cur else {}
+        if m.get("segs") is not None:
+            out += [m["segs"], m["last"]]
+        if m.get("plan") is not None:
+            out += [m["plan"].tiles, m["plan"].phys]
+        return out + [a for r in m.get("ranges", {}).values() for a in (r.ranges, r.seqs)]
 
     def token_meta(self):
         """(sequence, position, last token of its sequence in the pass) per token."""

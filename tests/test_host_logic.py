@@ -220,3 +220,74 @@ def test_text_prompt_path_with_a_stub_tokenizer():
     assert g2.eos_token_id == 3
     g2.set_exec_vars(None, "cpu", None, _StubTokenizer(), None, None, eos_token_id=11)
     assert g2.eos_token_id == 11
+
+
+class FakeStreams:
+    """Stands in for torch's streams: `log` holds what was asked of them, in order."""
+
+    def __init__(self, monkeypatch, ops):
+        self.log, self.now, self.streams = [], 0, {}
+        fake = self
+
+        class Stream:
+            def __init__(self, raw):
+                self.cuda_stream = raw
+
+            def record_event(self):
+                fake.log.append(("record", self.cuda_stream))
+                event = type("Event", (), {})()
+                event.stamp, event.device = (self.cuda_stream, len(fake.log)), torch.device("cuda", 0)
+                return event
+
+            def wait_event(self, event):
+                fake.log.append(("wait", self.cuda_stream, *event.stamp))
+
+            def wait_stream(self, other):
+                fake.log.append(("wait", self.cuda_stream, other.cuda_stream, len(fake.log)))
+
+        def upload(t, device, dtype=None):
+            fake.log.append(("upload", fake.now))
+            return t.clone()
+
+        monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: fake.streams.setdefault(fake.now, Stream(fake.now)))
+        monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: fake.now, raising=False)
+        monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+        monkeypatch.setattr(torch.Tensor, "record_stream", lambda t, s: fake.log.append(("keep", s.cuda_stream, t.data_ptr())))
+        monkeypatch.setattr(ops, "upload", upload)
+
+    def at(self, stream):
+        """The entries behind the last call, and `stream` is current from here on."""
+        out, self.log[:], self.now = list(self.log), [], stream
+        return out
+
+
+def test_passes_on_several_streams_are_ordered(monkeypatch):
+    """A stream that goes on with a pass waits for its arrays and keeps their memory; the stream that begins the next pass waits for all that
+    the last was queued on before it overwrites the table.  On one stream nothing waits."""
+    kvm = load_pkg("kv_cache")
+    kv = kvm.PagedStateCache([], 32, 8, max_seqs=2, max_blocks=2, max_pos=32, dtype=torch.float32, device="cpu")
+    fake = FakeStreams(monkeypatch, kvm.ops)
+    kv.device = torch.device("cuda")
+    for s in "ab":
+        kv.add_sequence(s)
+    for _ in range(2):                                    # the default stream alone
+        kv.begin_forward("ab", [3, 2])
+        kv.token_meta()
+        kv.end_forward()
+    assert {e[0] for e in fake.at(0)} <= {"upload", "record"}
+    kv.begin_forward("ab", [2, 2])                        # begun on 0, goes on on 7 and 9
+    begun = fake.at(7)
+    last = [i for i, e in enumerate(begun) if e[0] == "record"][-1] + 1
+    seq, pos, ends = kv.token_meta()
+    log = fake.at(9)
+    assert log[0] == ("wait", 7, 0, last) and {e[2] for e in log if e[:2] == ("keep", 7)} == {seq.data_ptr(), pos.data_ptr()}
+    kv.token_meta()
+    log = fake.at(0)
+    assert log[0][:3] == ("wait", 9, 7) and {e[2] for e in log if e[:2] == ("keep", 9)} >= {seq.data_ptr(), pos.data_ptr(), ends.data_ptr()}
+    kv.end_forward()
+    ended = fake.at(5)
+    kv.begin_forward("ab", [16, 1])                       # a new page, on 5
+    log = fake.at(5)
+    waits, first_upload = [e for e in log if e[0] == "wait"], [e[0] for e in log].index("upload")
+    assert {e[2] for e in waits} == {0, 7, 9} and all(e[1] == 5 for e in waits) and [e[0] for e in log[:3]] == ["wait"] * 3 and first_upload == 3
+    assert {("record", 7), ("record", 9)} <= set(ended)   # behind the whole pass

@@ -1394,3 +1394,39 @@ def test_staged_arrays_reach_another_stream(decode):
     assert got[2].tolist() == [i for n in lens for i in range(n)]
     torch.cuda.synchronize()
     cache.end_forward()
+
+
+@pytest.mark.parametrize("decode", [False, True])
+def test_pass_on_another_stream_and_its_successor(ops, decode):
+    """A pass begun on one stream, its attention behind milliseconds of work on another, and the next pass begun on the first: it takes over
+    a sequence's row of the block table, and its arrays have the size of those still to be read.  The results are those of one stream."""
+    kvm = load_pkg("kv_cache")
+    lens, Hq, Hkv, D = ([1, 1, 1], 8, 2, 64) if decode else ([20, 33, 16], 8, 2, 64)
+    g = torch.Generator(device=DEV).manual_seed(1)
+    qkv = [torch.randn((sum(lens), Hq + 2 * Hkv, D), generator=g, device=DEV).half() for _ in range(3)]
+    busy = torch.randn(4096, 4096, device=DEV)
+
+    def passes(streams):
+        cache = kvm.PagedKVCache(1, 24, Hkv, D, max_seqs=3, max_blocks=7, rope_theta=10000.0, max_pos=112, device=DEV)
+        out = []
+        for s in range(3):
+            cache.add_sequence(s)
+        torch.cuda.synchronize()
+        for i, x in enumerate(qkv):
+            with torch.cuda.stream(streams[0]):
+                cache.begin_forward([0 if i < 2 else 3, 1, 2], lens)
+            with torch.cuda.stream(streams[1]):
+                b = busy
+                for _ in range(20 if streams[0] != streams[1] else 0):
+                    b = b @ busy * 1e-3
+                out.append(cache.attention_with_fused_qkv(0, x.clone(), Hq))
+                cache.end_forward()
+            if i == 1:
+                cache.free_sequence(0)                     # its pages and its row go to another
+                cache.add_sequence(3)
+        torch.cuda.synchronize()
+        return out
+
+    one = torch.cuda.Stream()
+    for a, b in zip(passes((one, one)), passes((one, torch.cuda.Stream()))):
+        assert torch.equal(a, b)
