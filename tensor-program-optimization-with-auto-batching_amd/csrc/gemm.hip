@@ -344,14 +344,21 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
   // on 22016 rows.  Row-major x, 64 bytes of 16 rows per fragment, keeps one band (4: 3000 x 12288 x 4096 305 -> 323 us).  Over a
   // plan a band of 3 tiles has most of an expert's tiles together (32 experts of 5504 x 4096, 8000 tokens of 4: 1660 us in one
   // band, 1585 with 3 or 4, 1592 with 8; 4000 tokens 912, 892, 902, 910).
-  const int band = GROUPED ? 3 : x_tt > 0 ? 4 : gy;
+  constexpr unsigned BAND = GROUPED ? 3 : 4;
   auto block_of = [&](int L, int& n0, int& t0) {
-    const int xcd = L & 7, more = nb & 7;
-    const int idx = xcd * (nb >> 3) + (xcd < more ? xcd : more) + (L >> 3);
-    const int first = idx / (band * gx) * band, r = idx - first * gx;
-    const int h = gy - first < band ? gy - first : band;
-    n0 = r / h * BN;
-    t0 = first + r % h;
+    const unsigned xcd = L & 7, more = nb & 7;
+    const unsigned idx = xcd * (nb >> 3) + (xcd < more ? xcd : more) + (L >> 3);
+    unsigned first = 0, r = idx, h = gy, row;
+    if (GROUPED || x_tt > 0) {
+      first = idx / (BAND * gx) * BAND;        // the only division by a number that is not a constant: they take longer than a k-step
+      r -= first * gx;
+      h = gy - first < BAND ? gy - first : BAND;
+      row = h == 4 ? r / 4 : h == 3 ? r / 3 : h == 2 ? r / 2 : r;
+    } else {
+      row = r / h;
+    }
+    n0 = row * BN;
+    t0 = first + r - row * h;
     if constexpr (GROUPED) t0 = __builtin_amdgcn_readfirstlane(t0);      // a tile of the plan
     else t0 *= PP_F * 16;
   };
@@ -521,35 +528,26 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
   eltx8 a[2][8], b[2][WTF];
   int rd = 0;                                  // ring slot of the stage whose fragments are read next
   // The token fragments of a wave: four in a row; of a plan's tile every fourth, so that the places a tile does have - often few of
-  // its 256 - spread over all waves, and the first `have` of them are worked on (uniform; fragments and products of the others are
-  // left out, their accumulators never stored).
+  // its 256 - spread over all waves, and the first `have` of them are multiplied (uniform; the others are fetched and read like them, but
+  // their accumulators never stored).
   auto tfrag = [&](int j) { return GROUPED ? wt + 4 * j : wt * WTF + j; };
-  auto fragments_of = [&](int L) {
-    if constexpr (!GROUPED) return WTF;
-    int n0, tile;
-    block_of(L < nb ? L : blockIdx.x, n0, tile);
-    const int places = gr.plan.tiles[tile].z - wt * 16;
-    return __builtin_amdgcn_readfirstlane(places <= 0 ? 0 : (places + 63) / 64);
-  };
-  auto read_frags = [&](auto U, int have) {
+  auto read_frags = [&](auto U) {
     constexpr int u = decltype(U)::value;
     const elt* st = smem + rd * PP_STAGE_ELEMS + lane * 8;
 #pragma unroll
-    for (int j = 0; j < WTF; ++j)
-      b[u][j] = ld8(st + (PP_F + tfrag(j)) * 512);
-    {
+    for (int j = 0; j < WTF; ++j) b[u][j] = ld8(st + (PP_F + tfrag(j)) * 512);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) a[u][i] = ld8(st + (wn * 8 + i) * 512);
-    }
+    for (int i = 0; i < 8; ++i) a[u][i] = ld8(st + (wn * 8 + i) * 512);
     rd = (rd + 1) & (PP_STAGES - 1);
   };
   // half (uniform): -1 all eight row tiles, 0 / 1 the first / last four (a LoRA stage of the gate / up projection)
   auto multiply = [&](auto U, int half, int have) {
     constexpr int u = decltype(U)::value;
     if constexpr (GROUPED) {
+      asm volatile("" : "+s"(have));           // compared where it is used, in scalar registers
 #pragma unroll
       for (int j = 0; j < WTF; ++j)
-        if (j < have) {                        // uniform
+        if (__builtin_expect(j < have, 1)) {   // uniform; the products of a full tile follow each other without a jump
 #pragma unroll
           for (int i = 0; i < 8; ++i) acc[i][j] = mfma_16x16x32(a[u][i], b[u][j], acc[i][j]);
         }
@@ -572,12 +570,13 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
   // everybody's: the barrier).  The wait also covers this wave's fragment reads of the stage about to be multiplied,
   // so after the barrier nobody reads that ring slot any more and it is refilled; then the reads of the successor go
   // out, then the MFMAs.
-  auto stage = [&](auto U, auto PLAIN, int half, int have, int have_next) {
+  auto stage = [&](auto U, auto PLAIN, int half, int have) {
     constexpr int u = decltype(U)::value;
     asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
+    if constexpr (GROUPED) __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0) in the compiler's own terms: else it waits again ahead of the products
     __syncthreads();
     issue(PLAIN);
-    read_frags(std::integral_constant<int, 1 - u>(), have_next);
+    read_frags(std::integral_constant<int, 1 - u>());
     __builtin_amdgcn_sched_barrier(0);
     multiply(U, half, have);
     __builtin_amdgcn_sched_barrier(0);
@@ -590,8 +589,7 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
   asm volatile("s_waitcnt vmcnt(8)" ::: "memory");     // the first stage of this wave has landed
   __syncthreads();
   issue(std::false_type());
-  int have_next = fragments_of(blockIdx.x);
-  read_frags(std::integral_constant<int, 0>(), have_next);
+  read_frags(std::integral_constant<int, 0>());
   elt* ostage = smem + PP_STAGES * PP_STAGE_ELEMS + wave * PP_OUT_ELEMS;
   const int r16 = lane & 15, g = lane >> 4;
   for (int L = blockIdx.x; L < nb; L += G) {
@@ -601,14 +599,13 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
       for (int j = 0; j < WTF; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     int n0, t0;
     block_of(L, n0, t0);
-    int tend = T;
+    int tend = T, have = WTF;
     if constexpr (GROUPED) {
       const int4 tile = gr.plan.tiles[t0];
       t0 = __builtin_amdgcn_readfirstlane(tile.y);
       tend = t0 + __builtin_amdgcn_readfirstlane(tile.z);
+      have = tend - t0 <= wt * 16 ? 0 : (tend - t0 - wt * 16 + 63) / 64;
     }
-    const int have = have_next;
-    have_next = fragments_of(L + G);
     int nst = KB;                                      // KB and E are even (checked by the launcher): the register sets alternate
     if constexpr (LORA) {
       int slot;
@@ -620,14 +617,14 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
       if constexpr (SILU && LORA) {
         // one copy of the pair; a pair of LoRA stages belongs to one projection and multiplies that half of the tiles only
         const int half = kb < KB ? -1 : (has_gate && kb - KB < EP ? 0 : 1);   // uniform
-        stage(std::integral_constant<int, 0>(), std::false_type(), half, WTF, WTF);
-        stage(std::integral_constant<int, 1>(), std::false_type(), half, WTF, WTF);
+        stage(std::integral_constant<int, 0>(), std::false_type(), half, WTF);
+        stage(std::integral_constant<int, 1>(), std::false_type(), half, WTF);
       } else if (LORA && load_kb + 2 < KB) {             // uniform: the two stages fetched next are ordinary k-steps inside their block
-        stage(std::integral_constant<int, 0>(), std::true_type(), -1, WTF, WTF);
-        stage(std::integral_constant<int, 1>(), std::true_type(), -1, WTF, WTF);
+        stage(std::integral_constant<int, 0>(), std::true_type(), -1, WTF);
+        stage(std::integral_constant<int, 1>(), std::true_type(), -1, WTF);
       } else {
-        stage(std::integral_constant<int, 0>(), std::false_type(), -1, have, have);
-        stage(std::integral_constant<int, 1>(), std::false_type(), -1, have, kb + 2 < nst ? have : have_next);
+        stage(std::integral_constant<int, 0>(), std::false_type(), -1, have);
+        stage(std::integral_constant<int, 1>(), std::false_type(), -1, have);
       }
     }
     if constexpr (SILU) {

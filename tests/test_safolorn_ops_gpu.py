@@ -428,3 +428,28 @@ def test_fp32_latent_attention_of_prompts(D, T, n, H, rank, rot, sunk):
     torch.cuda.synchronize()
     assert err(got[..., :rank], attn_want(lat, q, [0] * T, pos, sink, scale, rank)) < tol(dt)
     assert float(got[..., rank:].abs().sum()) == 0
+
+
+@pytest.mark.parametrize("glu", [False, True])
+@pytest.mark.parametrize("counts", [[300], [257, 0, 64], [1, 16, 17, 64, 65, 255, 256], [511, 0, 0, 240, 241], [128] * 10, [700, 1, 1, 900, 33, 48, 49],
+                                    [256, 512, 768]])
+def test_experts_over_ragged_tiles(D, counts, glu):
+    """Tiles of 256 places with few, some and all of their fragments, one to nine of them (bands of three, whole and cut), in each of the three
+    epilogues.  The hidden values round once to bf16 (2^-9; gate and up beforehand as well: |silu| and |silu'| are at most |g| and 1.1), the
+    results once more; the fp32 sums are far below that."""
+    dt, E, K, ff, N, T = torch.bfloat16, len(counts), 128, 320, 288, sum(counts)
+    rng = np.random.default_rng(T)
+    pick = rng.permutation(np.repeat(np.arange(E), counts))
+    plan = D.MoePlan(torch.from_numpy(pick.astype(np.int32)).to(DEV).view(T, 1), E, dt)
+    assert plan.tile_rows == 256
+    x, up, down = rnd(rng, T, K, dt=dt), rnd(rng, E, ff * (2 if glu else 1), K, std=K ** -0.5, dt=dt), rnd(rng, E, N, ff, std=ff ** -0.5, dt=dt)
+    mid = D.moe_linear(x, D.weight(up.view(-1, K)), plan, ff, K, D.MOE_UP, D.ACT_GLU if glu else D.ACT_RELU2)
+    got = f64(D.moe_linear(mid, D.weight(down.view(-1, ff)), plan, N, ff, D.MOE_DOWN))
+    torch.cuda.synchronize()
+    for e in range(E):
+        rows = pick == e
+        v = f64(x)[rows] @ f64(up)[e].T
+        g, u = v[:, :ff], v[:, -ff:]
+        h, room = (g / (1 + np.exp(-g)) * u, 2 * np.abs(g * u)) if glu else (np.maximum(g, 0) ** 2,) * 2
+        want = h @ f64(down)[e].T
+        assert (np.abs(got[rows] - want) <= 2.0 ** -8 * (room @ np.abs(f64(down)[e]).T + np.abs(want)) + 1e-6).all(), e
