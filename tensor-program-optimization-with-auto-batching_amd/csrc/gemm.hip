@@ -1071,15 +1071,17 @@ int launch_gemm_lds(void* y, const elt* x, int ldx, const elt* Wp, int T, int K,
   return MLORA_OK;
 }
 
-// Block shape by problem size: 256 x 256 on the persistent kernel when more than half of the compute units get a block (2500 x 4096 x
-// 4096, 160 blocks: 102 us against 136 on blocks of 256 x 64; 700 x 12288 x 4096, 144 blocks: 101, 138; up to 128 blocks 103, 94), else 256
-// tokens x 64 columns (wave 64 x 64, several workgroups per CU) so that a few hundred tokens still spread over all CUs.
+// Block shape by problem size.  256 tokens x 64 columns (wave 64 x 64) spread a few hundred tokens over all compute units, two blocks on
+// each; a second round doubles their time, and from there on the persistent kernel is faster, up to half a round of whose blocks would be
+// empty: 2500 tokens x 4096 x 4096 (640 small blocks) 102 us against 136, 700 x 4096 x 12288 (576) 101, 138, 3226 x 1024 x 2504 (520) 35, 42; 2425 x 512 x
+// 3248 (510) 23, 20.  Not for a K that its blocks' ends outweigh: 281 x 64 x 23664 12.1, 9.2, 876 x 128 x 9648 13.6, 11.8, 1410 x 256 x 6520 15.9, 16.6.
 template <int OUT>
 int launch_gemm_lds_auto(void* y, const elt* x, int ldx, const elt* Wp, int T, int K, int N, hipStream_t s) {
-  const long nb = (long)ceil_div(T, 256) * ceil_div(N, 256);
+  const long nb = (long)ceil_div(T, 256) * ceil_div(N, 256), cu = gemm_n_cu() > 0 ? gemm_n_cu() : 256;
+  const bool large = nb >= cu, second = (long)ceil_div(T, 256) * ceil_div(N, 64) > 2 * cu && K >= 256;
   // x rows must be 16-byte aligned for the direct-to-LDS loads (ldx % 8 == 0 is checked; the base may be a slice)
-  if (nb > 128 && ((uintptr_t)x & 15) == 0 && K % 64 == 0) return launch_gemm_pp<OUT>(y, x, ldx, 0, Wp, T, K, N, s);
-  if (nb >= 256) return launch_gemm_lds<OUT, 16, 16, 8, 8>(y, x, ldx, Wp, T, K, N, s);
+  if ((large || second) && ((uintptr_t)x & 15) == 0 && K % 64 == 0) return launch_gemm_pp<OUT>(y, x, ldx, 0, Wp, T, K, N, s);
+  if (large) return launch_gemm_lds<OUT, 16, 16, 8, 8>(y, x, ldx, Wp, T, K, N, s);
   return launch_gemm_lds<OUT, 16, 4, 4, 4>(y, x, ldx, Wp, T, K, N, s);
 }
 
@@ -1140,16 +1142,19 @@ extern "C" int mlora_gemm_frag_preferred(int T, int K, int N) {
   return T > 64 && K > 0 && K % 64 == 0 && N > 0 && (long)ceil_div(T, PP_F * 16) * ceil_div(N, PP_F * 16) >= 256;
 }
 
-// The plain linear: the persistent kernel or the mid-size one, whose smaller blocks cost 2 to 16 % where the rounds of 256 blocks are
-// full and save up to a third where they are not.  Measured, persistent / mid-size, bf16, us: one round of 160 blocks (2500 x 4096 x
-// 4096) 94 / 88, 176 (1000 x 11264 x 2048) 50 / 53, 192 (2000 x 6144 x 2048) 51 / 52, 224 (3500 x 4096 x 4096) 103 / 111, 256 105 / 115;
-// 264 (1500 x 11264 x 2048) 91 / 71, 288 (1500 x 12288 x 4096) 180 / 140, 336 (1792) 187 / 171, 344 (1000 x 22016 x 4096) 178 / 174,
-// 384 (1900 x 12288 x 4096) 192 / 181, 440 (2500 x 11264 x 2048) 105 / 120; from 512 on 0.98 to 1.16 as long.  From 345 to 400 blocks the
-// two differ by 0 to 6 % and a pass's other products of that size are fused with their epilogue: the persistent kernel stays.  Up to 128
-// tokens half of its work is padding: 128256 x 4096, 128 tokens 263 / 212, 200 tokens 272 / 280.
+// The plain linear: the persistent kernel or the mid-size one.  The first takes whole rounds of one 256 x 256 block per compute unit: padding
+// and empty units cost as much as products.  So in one round it needs five eighths of the chip in products, and the second round a number of
+// blocks; small K, where a block's end weighs more, fewer of them.  Measured, persistent / mid-size, us.  One round, by T N / 2^16: 105 (264 x
+// 4096 x 26032) 111 / 101, 144 (557 x 2048 x 16968) 59 / 56, 156 (2500 x 4096 x 4096) 94 / 88, 164 (646 x 8192 x 16672) 214 / 228, 180 (673 x 512 x 17568)
+// 22 / 25, 198 (601 x 4096 x 21584) 115 / 129, 256 105 / 115.  More blocks, K from 2048 on: 264 (3034 x 2048 x 5464) 100 / 85, 280 (3540 x 8192 x 4976)
+// 370 / 303, 336 (1792 x 4096 x 12288) 187 / 171, 348 (719 x 2048 x 29496) 113 / 107, 385 (2784 x 4096 x 8856) 210 / 221, 400 (1963 x 2048 x 12776) 114 / 130; below: 276
+// (1306 x 512 x 11536) 35 / 33, 300 (1379 x 256 x 12664) 23 / 27, 324 (2909 x 512 x 6744) 36 / 40, 342 (4602 x 1024 x 4712) 59 / 62.  Up to 128 tokens half of its work
+// is padding: 128256 x 4096, 128 tokens 263 / 212.
 static bool persistent_pays(int T, int K, int N) {
-  const long nb = (long)ceil_div(T, PP_F * 16) * ceil_div(N, PP_F * 16);
-  return K % 64 == 0 && T > 128 && nb >= 176 && (nb <= 256 || nb >= 345);
+  const long cu = gemm_n_cu() > 0 ? gemm_n_cu() : 256, nb = (long)ceil_div(T, PP_F * 16) * ceil_div(N, PP_F * 16);
+  if (K % 64 || T <= 128) return false;
+  if (nb <= cu) return (long)T * N >= cu * 5 / 8 * (PP_F * 16 * PP_F * 16);
+  return nb > cu * (K >= 2048 ? 43 : 36) / 32;
 }
 
 extern "C" int mlora_linear_frag(void* y, int y_dtype, int mode, const void* xf, const void* Wp, int T, int K, int N,

@@ -1430,3 +1430,29 @@ def test_pass_on_another_stream_and_its_successor(ops, decode):
     one = torch.cuda.Stream()
     for a, b in zip(passes((one, one)), passes((one, torch.cuda.Stream()))):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("T,N,K", [(250, 42000, 64), (250, 41900, 64), (256, 288 * 256, 128), (256, 289 * 256, 128), (256, 343 * 256, 2048),
+                                   (130, 344 * 256, 2112), (130, 345 * 256, 2048)])
+def test_linear_around_a_round_of_blocks(ops, T, N, K):
+    """Both sides of the lines between the mid-size and the persistent kernel that depend on what a round multiplies and on K: the bits of the
+    row-major kernel."""
+    g = torch.Generator(device=DEV).manual_seed(T + N)
+    x = torch.randn((T, K), generator=g, device=DEV).half()
+    W = ops.PackedWeight((torch.randn((N, K), generator=g, device=DEV) * 0.05).half())
+    f = ops.FragActivation.pack(x)
+    want = ops.linear(x, W, kernel="gemm")
+    assert torch.equal(ops.linear(f, W), want)
+    w = W.unpack()[-300:].double()
+    assert bool(((want[:, -300:].double() - x.double() @ w.T).abs() <= ((K + 2) * 2.0 ** -24 + 2.0 ** -11) * (x.abs().double() @ w.abs().T)).all())
+
+
+@pytest.mark.parametrize("T,N,K", [(2425, 3264, 512), (2425, 3268, 512), (300, 16448, 192), (300, 16448, 256), (1300, 6560, 192), (1300, 5600, 320)])
+def test_row_major_linear_around_a_round_of_blocks(ops, T, N, K):
+    """512 and 522 blocks of 256 x 64, K on both sides of 256: fp32 results within the rounding of K additions."""
+    g = torch.Generator(device=DEV).manual_seed(T + N)
+    x = torch.randn((T, K), generator=g, device=DEV).half()
+    W = ops.PackedWeight((torch.randn((N, K), generator=g, device=DEV) * 0.05).half())
+    y = ops.linear(x, W, out_dtype=torch.float32)
+    w = W.unpack().double()
+    assert bool(((y.double() - x.double() @ w.T).abs() <= (K + 2) * 2.0 ** -24 * (x.abs().double() @ w.abs().T)).all())
