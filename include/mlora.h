@@ -514,7 +514,7 @@ int mlora_rmsnorm_ksplit(void* y, int y_layout, float* resid, const float* part,
  * Scratch buffers are caller-owned (sizes in elements):
  *   resid f32 [T*H]; xn, attn: mlora_frag_activation_elems(T, H | Hq*D) f16; qkv f16 [T*(Hq+2Hkv)*D];
  *   gate_up f16 [T*2I]; act: mlora_frag_activation_elems(T, I) f16; logits f32 [T*V];
- *   lora_ws: 5 slots of max(mlora_gather_mm_workspace_bytes(T, max(H, I, Hq*D), r), 4 * T * n_ad * r) bytes;
+ *   lora_ws: 5 slots of max(mlora_gather_mm_workspace_bytes(T, K, r) for K = H, I and Hq*D, 4 * T * n_ad * r) bytes;
  *     with lora_dense, (3 * kq + 2) slots for kq = mlora_gemv_split_kq(T, H, (Hq+2Hkv)*D, 3 * n_ad * r) (at most 14).
  * ------------------------------------------------------------------------------------------- */
 typedef struct mlora_lora_proj {

@@ -182,9 +182,10 @@ extern "C" int mlora_decode_step(const mlora_decode_plan* p, void* stream) {
   void* ws_qkv = ws;
   void* ws_o = ws + (size_t)3 * kq * slot;
   void* ws_down = ws + (size_t)(3 * kq + 1) * slot;
+  const size_t down_bytes = lora ? p->lora_ws_bytes - (size_t)(3 * kq + 1) * slot : 0;   // (a smaller K may take more than the largest)
   auto delta = [&](void* y, int y_dtype, int ldy, const void* x, const mlora_lora_proj& lp, int K, int N) -> int {
     if (!lora || !lp.A) return MLORA_OK;
-    return mlora_gather_mm(y, y_dtype, ldy, x, MLORA_FRAG, lp.A, lp.B, p->tok_adapter, sc, T, K, N, r, n_ad, ws_down, slot, stream);
+    return mlora_gather_mm(y, y_dtype, ldy, x, MLORA_FRAG, lp.A, lp.B, p->tok_adapter, sc, T, K, N, r, n_ad, ws_down, down_bytes, stream);
   };
   // K split of the two narrow accumulating GEMVs: the slices' partials are summed by the RMSNorm that reads the
   // residual next.  N_total counts the appended adapter rows of the dense shrink.

@@ -134,7 +134,7 @@ class NativeDecodeSession:
         r = lt.r if lt is not None else 0
         # five slots (q, k, v, o, down); the dense q/k/v shrink may come as up to four K-range blocks of three slots
         # (a slot also holds the o shrink's head shares, [heads, T, r] fp32)
-        ws_bytes = 14 * max(_lib.lib().mlora_gather_mm_workspace_bytes(T, max(H, I, s.q_size), max(r, 8)),
+        ws_bytes = 14 * max(*(_lib.lib().mlora_gather_mm_workspace_bytes(T, K, max(r, 8)) for K in (H, I, s.q_size)),
                             4 * T * (lt.n_adapters if lt is not None else 0) * max(r, 8), 4 * s.num_attention_heads * T * max(r, 8))
         self.buf["lora_ws"] = torch.empty(ws_bytes // 4, dtype=f32, device=dev)
         # partials of the K-split o_proj / down_proj GEMVs (up to 3 slices of [T, H + appended adapter rows])

@@ -266,3 +266,18 @@ def test_native_step_over_the_padded_union_of_adapter_types(ranks, dense):
     else:
         for a, b in ((out["dense"][1].float(), out["native"][1].float()), (out["dense"][2], out["native"][2])):
             assert (a - b).abs().max().item() <= 2e-3 * b.abs().max().item()
+
+
+def test_native_step_where_the_largest_k_needs_the_least_scratch():
+    """Hidden size 4096 takes eight K slices, intermediate size 4608 five: every adapted projection finds room for its own, with separate
+    shrink units and no dense tables; tokens and keys of the per-operator path."""
+    synth, llama = load_pkg("synth"), load_pkg("llama")
+    wl = synth.config3(num_layers=1, batch=5, prompt_len=20)
+    wl.shape.intermediate_size = 4608
+    wl.lora = synth.LoraSpec(r=64, alpha=32, n_adapters=3, targets=("q_proj", "k_proj", "v_proj", "o_proj", "gate_proj", "up_proj", "down_proj"))
+    ids = np.array([0, 2, -1, 1, 0], dtype=np.int32)
+    model = llama.LlamaForCausalLM.from_synthetic(wl.seed, wl.shape, [wl.lora], DEV)
+    prompts = synth.prompts(wl)
+    a, ka, _ = _run(model, wl, prompts, ids, "py", 3, synth)
+    b, kb, _ = _run(model, wl, prompts, ids, "native", 3, synth)
+    assert np.array_equal(a, b) and torch.equal(ka, kb)
