@@ -5,6 +5,7 @@ enqueues on torch's current stream.  None of them has a CPU path.
 """
 from __future__ import annotations
 
+import ctypes
 import functools
 import struct
 
@@ -29,6 +30,11 @@ def check(code: int, dtype: torch.dtype = torch.float16) -> None:
 def _stream() -> int:
     """The current stream of the current device, without the object around it (6 us less per call)."""
     return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+
+
+def _bucket(A, B, r, n_ad, scaling) -> bytes:
+    """A mlora_lora_bucket (a scaling beyond fp32 is infinite, which struct alone refuses)."""
+    return _BUCKET.pack(A, B, r, n_ad, ctypes.c_float(scaling).value)
 
 
 def upload(t: torch.Tensor, device, dtype=None) -> torch.Tensor:
@@ -181,13 +187,13 @@ def gather_mm_multi(y, x, buckets, tok_bucket, tok_adapter, workspace=None):
     rmax = 8
     for i, bk in enumerate(buckets):
         if bk is None:                      # the bucket's adapters do not target this projection
-            arr += _BUCKET.pack(0, 0, 0, 0, 0.0)
+            arr += _bucket(0, 0, 0, 0, 0.0)
             continue
         A, B, scaling = bk
         n_ad, r, K2 = A.shape
         if K2 != K or B.shape != (n_ad, N, r):
             raise ValueError(f"gather_mm_multi: bucket {i} has A{tuple(A.shape)} B{tuple(B.shape)} for K={K} N={N}")
-        arr += _BUCKET.pack(_dev(A, torch.float16, "A"), _dev(B, torch.float16, "B"), r, n_ad, float(scaling))
+        arr += _bucket(_dev(A, torch.float16, "A"), _dev(B, torch.float16, "B"), r, n_ad, scaling)
         rmax = max(rmax, r)
     if workspace is None:
         workspace = gather_mm_workspace(T, K, rmax, x.device)
@@ -217,14 +223,14 @@ def gather_mm_multi_proj(y, x, proj_buckets, col_offsets, n_cols, tok_bucket, to
     for p, buckets in enumerate(proj_buckets):
         for i, bk in enumerate(buckets):
             if bk is None:                      # the bucket's adapters do not target this projection
-                arr += _BUCKET.pack(0, 0, 0, 0, 0.0)
+                arr += _bucket(0, 0, 0, 0, 0.0)
                 continue
             A, B, scaling = bk
             n_ad, r, K2 = A.shape
             if K2 != K or B.shape != (n_ad, n_cols[p], r):
                 raise ValueError(f"gather_mm_multi_proj: projection {p} bucket {i} has A{tuple(A.shape)} B{tuple(B.shape)} "
                                  f"for K={K} N={n_cols[p]}")
-            arr += _BUCKET.pack(_dev(A, torch.float16, "A"), _dev(B, torch.float16, "B"), r, n_ad, float(scaling))
+            arr += _bucket(_dev(A, torch.float16, "A"), _dev(B, torch.float16, "B"), r, n_ad, scaling)
             rmax = max(rmax, r)
     if workspace is None:
         one = gather_mm_workspace(T, K, rmax, x.device).numel()

@@ -291,3 +291,12 @@ def test_passes_on_several_streams_are_ordered(monkeypatch):
     waits, first_upload = [e for e in log if e[0] == "wait"], [e[0] for e in log].index("upload")
     assert {e[2] for e in waits} == {0, 7, 9} and all(e[1] == 5 for e in waits) and [e[0] for e in log[:3]] == ["wait"] * 3 and first_upload == 3
     assert {("record", 7), ("record", 9)} <= set(ended)   # behind the whole pass
+
+
+@pytest.mark.parametrize("scaling", [0.5, np.float32(0.3), 1e39, -1e300, float("inf"), 7])
+def test_adapter_buckets_as_the_library_reads_them(scaling):
+    import ctypes
+    bucket = load_pkg("_lib").LoraBucket
+    got = bucket.from_buffer_copy(load_pkg("ops")._bucket(1 << 40, 24, 16, 3, scaling))
+    want = bucket(1 << 40, 24, 16, 3, float(scaling))
+    assert bytes(got) == bytes(want) and got.scaling == ctypes.c_float(float(scaling)).value
