@@ -34,7 +34,7 @@ def _stream() -> int:
 
 def _bucket(A, B, r, n_ad, scaling) -> bytes:
     """A mlora_lora_bucket (a scaling beyond fp32 is infinite, which struct alone refuses)."""
-    return _BUCKET.pack(A, B, r, n_ad, ctypes.c_float(scaling).value)
+    return _BUCKET.pack(A, B, r, n_ad, ctypes.c_float(float(scaling)).value)
 
 
 def upload(t: torch.Tensor, device, dtype=None) -> torch.Tensor:

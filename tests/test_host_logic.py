@@ -293,7 +293,7 @@ def test_passes_on_several_streams_are_ordered(monkeypatch):
     assert {("record", 7), ("record", 9)} <= set(ended)   # behind the whole pass
 
 
-@pytest.mark.parametrize("scaling", [0.5, np.float32(0.3), 1e39, -1e300, float("inf"), 7])
+@pytest.mark.parametrize("scaling", [0.5, np.float32(0.3), torch.tensor(0.25), 1e39, -1e300, float("inf"), 7])
 def test_adapter_buckets_as_the_library_reads_them(scaling):
     import ctypes
     bucket = load_pkg("_lib").LoraBucket
