@@ -453,3 +453,30 @@ def test_experts_over_ragged_tiles(D, counts, glu):
         h, room = (g / (1 + np.exp(-g)) * u, 2 * np.abs(g * u)) if glu else (np.maximum(g, 0) ** 2,) * 2
         want = h @ f64(down)[e].T
         assert (np.abs(got[rows] - want) <= 2.0 ** -8 * (room @ np.abs(f64(down)[e]).T + np.abs(want)) + 1e-6).all(), e
+
+
+@pytest.mark.parametrize("counts", [[300, 1, 65, 130], [16, 17, 0, 33], [64, 128, 64]])
+@pytest.mark.parametrize("K,N", [(272, 72), (128, 4100), (272, 8200), (208, 12290)])
+def test_fp32_experts_over_ragged_tiles(D, counts, K, N):
+    """One to four token tiles of 16 per workgroup, rows gathered from tokens and scattered to entries, with 16, 64 and 128 weight rows, a K
+    that lies in LDS whole and one that does not; K + 3 roundings of 2^-24 on what is added up, twice that for the square."""
+    dt, E, top = torch.float32, len(counts), 2
+    rng = np.random.default_rng(K + N)
+    pick = rng.permutation(np.repeat(np.arange(E), np.array(counts) * top)).astype(np.int32)
+    T = sum(counts)
+    plan = D.MoePlan(torch.from_numpy(pick).to(DEV).view(T, top), E, dt)
+    torch.cuda.synchronize()
+    perm = plan.perm[: int(plan.n_tiles[1])].long()
+    places = (perm >= 0).nonzero().view(-1)
+    entry = perm[places]
+    x, rows, W = (torch.from_numpy(rng.normal(size=s).astype(np.float32)).to(DEV) for s in ((T, K), (plan.places, K), (E, N, K)))
+    up = D.moe_linear(x, W.view(-1, K), plan, N, K, D.MOE_UP, D.ACT_RELU2)
+    down = D.moe_linear(rows, W.view(-1, K), plan, N, K, D.MOE_DOWN)
+    eps = (K + 3) * 2.0 ** -24
+    for e in range(E):
+        at = places[torch.from_numpy(pick).to(DEV)[entry] == e]
+        src, w = x[perm[at] // top].double(), W[e].double()
+        v, room = src @ w.T, src.abs() @ w.abs().T
+        assert bool(((up[at].double() - v.clamp(min=0) ** 2).abs() <= 2 * eps * room ** 2).all()), e
+        v, room = rows[at].double() @ w.T, rows[at].double().abs() @ w.abs().T
+        assert bool(((down[perm[at]].double() - v).abs() <= eps * room).all()), e
