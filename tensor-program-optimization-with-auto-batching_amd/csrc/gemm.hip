@@ -270,8 +270,8 @@ __global__ __launch_bounds__(256) void gemm_lds_kernel(void* __restrict__ yv, co
 //   * Fragment registers are double-buffered: the LDS reads of stage g + 1 are issued right before the MFMAs of stage
 //     g and complete under them.
 //   * fp16 results cross a small LDS buffer so that a store instruction writes whole 128-byte lines of a token row.
-// Blocks are numbered so that an XCD (workgroup id mod 8) works through a contiguous range of weight-row blocks, all
-// token blocks of one weight block next to each other: every XCD streams its own share of W through its L2 once.
+// Blocks are numbered so that an XCD (workgroup id mod 8) works through a contiguous range of them, in bands of a few token
+// blocks that share their weights and tokens in its L2 (block_of).
 // ---------------------------------------------------------------------------------------------
 constexpr int PP_WAVES = 8;
 constexpr int PP_STAGES = 4;
@@ -336,14 +336,16 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
     if ((int)blockIdx.x >= nb) return;         // fewer blocks than workgroups: nothing was requested yet
   }
 
-  // Block number -> (weight-row block, token block).  Each XCD takes an eighth of the blocks, in their order: bands of `band`
+  // Block number -> (weight-row block, token block).  Each XCD takes an eighth of the blocks, in their order: bands of BAND
   // token blocks, within a band all token blocks of a weight-row block before those of the next.  So the 32 blocks that an XCD
   // multiplies at a time are some token blocks times some weight-row blocks and share both in its L2, where all token blocks of
   // one weight-row block shared only that.  Bands of 4 against one band, fragment-ordered x: 4001 tokens x 22016 x 4096 653 -> 614 us,
   // 8192 tokens 1301 -> 1150, 8192 tokens x 4096 x 11008 611 -> 552, 2500 x 12288 x 4096 190 -> 189; 8 is within 1 %, 2 to 3 % slower
   // on 22016 rows.  Row-major x, 64 bytes of 16 rows per fragment, keeps one band (4: 3000 x 12288 x 4096 305 -> 323 us).  Over a
-  // plan a band of 3 tiles has most of an expert's tiles together (32 experts of 5504 x 4096, 8000 tokens of 4: 1660 us in one
-  // band, 1585 with 3 or 4, 1592 with 8; 4000 tokens 912, 892, 902, 910).
+  // plan a band of 3 tiles has most of an expert's tiles together (32 experts of 5504 x 4096, uniform plans alone, 8000 tokens of 4: 1660 us
+  // in one band, 1585 with 3 or 4, 1592 with 8; 4000 tokens 912, 892, 902, 910).  In whole passes, where runs
+  // differ by 0.2 to 0.4 %, one band, 4 and 8 take as long as 3 and 1.3 %, -0.1 %, 0.4 % (Dinasun over 4001 tokens), 0.6 %, 0.5 %, 0.2 %
+  // (Safolorn over 3683) more.
   constexpr unsigned BAND = GROUPED ? 3 : 4;
   auto block_of = [&](int L, int& n0, int& t0) {
     const unsigned xcd = L & 7, more = nb & 7;
@@ -748,10 +750,10 @@ int launch_gemm_pp(void* y, const elt* x, int ldx, int x_tt, const elt* Wp, int 
 }
 
 // ---------------------------------------------------------------------------------------------
-// Token blocks between the decode GEMV and the persistent kernel above (65 to a few hundred tokens: a decode step of
-// many sequences, a short prefill).  The weights are read once and the matrix cores and the operand loads weigh about
-// the same, so the block is as tall as the token block allows and narrow enough to give every compute unit a
-// workgroup: FT x FN fragments (128 or 256 tokens x 128, 96 or 64 weight rows), eight waves, both operands in fragment
+// Products between the decode GEMV and the persistent kernel above (from 65 tokens on: a decode step of many sequences, a
+// short prefill, and what does not fill whole rounds of the kernel above).  The matrix cores, LDS and the operand loads
+// weigh about the same, so the block is chosen by size (gemm_mid_shape): FT x FN fragments (128, 192 or 256 tokens x 128, 96 or
+// 64 weight rows), eight waves, both operands in fragment
 // order and copied from global memory straight into an LDS ring.  A stage of the ring is TWO 32-k steps: with the
 // few MFMAs a wave has per 32-k step here (4 to 16), a barrier and a wait per step cost more than the step itself.
 // Four (three) stages, of which three (two) are in flight per compute unit - across the barrier of a stage, which is
@@ -998,7 +1000,8 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_mid_kernel(void* __res
 // miss the second-level caches (weights once, tokens once per XCD) 0.02 each.  The two overlap in part: root of the sum of squares.
 // Measured where the choice matters, in us: 137 tokens, q/k/v 33.9 at 8 / 6, 36.0 at 12 / 4, 48 at 16 / 6; gate/up (22016 rows)
 // 53.1 at 12 / 6, 60.8 at 16 / 6, 77.8 at 8 / 6; 300 tokens, q/k/v 49.8 at 12 / 6, 52.8 at 16 / 6, 71.5 at 8 / 8; o of 100 tokens in four
-// slices 14.0 at 8 / 4, 17.1 at 8 / 8; 512 tokens x 4096 x 4096 29.6 at 8 / 4, 38.2 at 8 / 6.
+// slices 14.0 at 8 / 4, 17.1 at 8 / 8; 512 tokens x 4096 x 4096 29.6 at 8 / 4, 38.2 at 8 / 6.  Over 180 sizes of 100 to 520 blocks of 256 x 256
+// the choice takes 1 % longer than the best of the nine on average, 10 % at most.
 struct MidShape {
   int ft, fn, ksplit;
 };
