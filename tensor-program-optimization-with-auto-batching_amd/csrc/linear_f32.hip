@@ -129,17 +129,15 @@ __device__ __forceinline__ void f32_thin(const F32Linear& a, const MoePlan& plan
   f32_store<FW, RT, RT>(a, plan, grouped, y, n0, t0, t1, red);
 }
 
-constexpr int wide_stages(int FN) { return FN == 4 ? 4 : 3; }
-
 // FN * 16 weight rows by up to 64 tokens: four waves share the rows (FN / 4 tiles each, all tokens), twice, for the two halves
 // of every 64 k.  Both operands go from global memory straight into an LDS ring (fragments of 16 rows x 16 k as the lanes read
-// them) that is NST - 1 stages of 64 k ahead, one bare barrier per stage.  Bound by the matrix cores (157 TFLOP/s nominal).
-// With 64 rows a K of fewer than NST stages lies in LDS whole, in no more than it needs: up to four workgroups on a compute unit, where
-// each waits for its one or two stages.  DIRECT: operands are 16-byte aligned; others go through registers.
-template <int FN, int RT, bool DIRECT>
+// them) that is NST - 1 stages of 64 k ahead, one bare barrier per stage.  Bound by the matrix cores (157 TFLOP/s nominal) or, for few
+// tokens, by what a workgroup takes in.  NST: a deep ring where a workgroup has a compute unit to itself, one of two stages where two
+// share it and their waits overlap.  DIRECT: operands are 16-byte aligned; others go through registers.
+template <int FN, int RT, int NST, bool DIRECT>
 __device__ __forceinline__ void f32_wide(const F32Linear& a, const MoePlan& plan, int grouped, const float* __restrict__ x, const float* __restrict__ W,
                                          float* __restrict__ y, int n0, int t0, int t1, f32x4* smem) {
-  constexpr int NST = wide_stages(FN), RW = FN / 4, SF = FN + RT, LF = 4 * SF, LQ = (LF + FW - 1) / FW;   // fragments: of 16 k, of a stage, per loading wave
+  constexpr int RW = FN / 4, SF = FN + RT, LF = 4 * SF, LQ = (LF + FW - 1) / FW;   // fragments: of 16 k, of a stage, per loading wave
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
   // fragment f = wave + 8 q of a stage: 16 k number f / SF, there weight tile or (behind those) token tile f % SF
   const float* src[LQ];
@@ -181,18 +179,15 @@ __device__ __forceinline__ void f32_wide(const F32Linear& a, const MoePlan& plan
   for (int i = 0; i < RW; ++i)
 #pragma unroll
     for (int j = 0; j < RT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const bool whole = FN == 4 && nst < NST;        // uniform
 #pragma unroll
-  for (int s = 0; s < NST - 1; ++s)
-    if (s < nst || !whole) request(s);
+  for (int s = 0; s < NST - 1; ++s) request(s);
   int rd = 0;
   for (int s = 0; s < nst; ++s) {
     // stage s has landed (this wave's share: at most the NST - 2 stages behind it in flight; everybody's: the barrier), and
     // everybody is done with the slot of stage s - 1, which is requested anew
-    if (whole) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NST - 2) * LQ) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NST - 2) * LQ) : "memory");
     bare_barrier();
-    if (!whole) request(s + NST - 1);
+    if (NST > 2 || s + 1 < nst) request(s + NST - 1);       // (the wait counts the requests past the end of a deeper ring)
     const f32x4* st = smem + (rd * LF + kh * 2 * SF) * 64 + lane;
     rd = rd + 1 < NST ? rd + 1 : 0;
 #pragma unroll
@@ -220,7 +215,7 @@ __device__ __forceinline__ void f32_wide(const F32Linear& a, const MoePlan& plan
 }
 
 // FN: row tiles of a workgroup (1: f32_thin)
-template <int FN, bool DIRECT>
+template <int FN, int NST, bool DIRECT>
 __global__ __launch_bounds__(FW* WAVE, 2) void linear_f32_kernel(F32Linear a, MoePlan plan, int grouped) {
   extern __shared__ __align__(16) f32x4 f32_smem[];
   const int n0 = blockIdx.x * FN * 16;
@@ -239,7 +234,7 @@ __global__ __launch_bounds__(FW* WAVE, 2) void linear_f32_kernel(F32Linear a, Mo
   const int rt = __builtin_amdgcn_readfirstlane((t1 - t0 + 15) >> 4);
   auto block = [&](auto RT) {
     if constexpr (FN == 1) f32_thin<decltype(RT)::value>(a, plan, grouped, x, W, y, n0, t0, t1, f32_smem);
-    else f32_wide<FN, decltype(RT)::value, DIRECT>(a, plan, grouped, x, W, y, n0, t0, t1, f32_smem);
+    else f32_wide<FN, decltype(RT)::value, NST, DIRECT>(a, plan, grouped, x, W, y, n0, t0, t1, f32_smem);
   };
   if (rt == 1) block(std::integral_constant<int, 1>());
   else if (rt == 2) block(std::integral_constant<int, 2>());
@@ -256,49 +251,46 @@ int f32_n_cu() {
   return n_cu;
 }
 
-// LDS of a workgroup: the waves' sums (16 rows), the ring, or all of a K of fewer stages (which the sums fit as well)
-template <int FN>
-constexpr size_t f32_lds(int K) {
-  constexpr int NST = wide_stages(FN);
-  const int stages = (K + 63) / 64;
-  return FN == 1 ? FW * 4 * 1024 : (FN == 4 && stages < NST ? stages : NST) * 4 * (FN + 4) * 1024;
-}
-
-template <int FN, bool DIRECT = true>
+template <int FN, int NST = 0, bool DIRECT = true>
 int launch_f32(const char* who, const F32Linear& a, const MoePlan& plan, int grouped, int row_blocks, int heads, hipStream_t stream) {
-  constexpr int most = (int)f32_lds<FN>(1 << 20);
+  constexpr size_t stage = 4 * (FN + 4) * 1024, most = FN == 1 ? FW * 4 * 1024 : NST * stage;      // the waves' sums, or the ring (which these fit)
+  const size_t lds = NST == 2 && a.K <= 64 ? stage : most;
   static const hipError_t configured =               // the attribute is per kernel, set once per process, by one thread
-      hipFuncSetAttribute((const void*)linear_f32_kernel<FN, DIRECT>, hipFuncAttributeMaxDynamicSharedMemorySize, most);
-  const size_t lds = f32_lds<FN>(a.K);
+      hipFuncSetAttribute((const void*)linear_f32_kernel<FN, NST, DIRECT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)most);
   if (configured != hipSuccess) return mlora_set_error(MLORA_ERR_LAUNCH, "%s: cannot reserve %zu bytes of LDS: %s", who, lds, hipGetErrorString(configured));
-  hipLaunchKernelGGL((linear_f32_kernel<FN, DIRECT>), dim3(ceil_div(a.N, FN * 16), row_blocks, heads), dim3(FW * WAVE), lds, stream, a, plan, grouped);
+  hipLaunchKernelGGL((linear_f32_kernel<FN, NST, DIRECT>), dim3(ceil_div(a.N, FN * 16), row_blocks, heads), dim3(FW * WAVE), lds, stream, a, plan, grouped);
   return mlora_launch_status(who);
 }
 
 int launch(const char* who, F32Linear a, const MoePlan& plan, int grouped, int row_blocks, int heads, void* stream) {
   MLORA_CHECK(a.K % 16 == 0 && a.ldx % 4 == 0 && a.hx % 4 == 0 && row_blocks <= 65535 && heads <= 65535, MLORA_ERR_UNSUPPORTED,
               "%s: need K %% 16 == 0 and rows aligned to 16 bytes (T=%d K=%d N=%d)", who, a.T, a.K, a.N);
-  // The form that finishes first, in us by what was measured with 1, 2 and 4 token tiles: rounds of the compute units times what a workgroup
-  // multiplies (at K = 2048: 64 rows 15, 24, 41; 128 rows 30, 45, 75) and what it waits for (3.2 and 4; where K lies in LDS whole, several
-  // wait at once); 16 rows per workgroup take 10, 13.5 and 20, and at least 24 ns per k of the first 256, one stage of every wave.  So 16 rows
-  // serve a grid that does not fill the chip (32 x 7680 x 2048: 45 against 96 and 173 us), 128 rows one that fills it several times over
-  // (4096 x 2048 x 11264: 3443, 1961, 1715 us), 64 rows what lies between (299 x 7680 x 2048: 193, 165, 290 us) and every K up to 128
-  // (4000 x 64 x 4096: 128, 34, 37 us; 467 x 64 x 9975 15, with one workgroup per compute unit 36).
-  const int entries = grouped ? a.T / row_blocks : a.T, rt = entries >= FB ? FB / 16 : entries > 16 ? ceil_div(entries, 16) : 1;
-  auto rounds = [&](int tiles, int at_once) {
-    const long blocks = (long)ceil_div(a.N, tiles * 16) * row_blocks * heads, slots = (long)f32_n_cu() * at_once;
-    return (double)((blocks + slots - 1) / slots);
-  };
-  const double k = a.K / 2048.0;
-  const int thin_k = a.K < 256 ? a.K : 256, at_once = (int)((160 << 10) / f32_lds<4>(a.K));        // (of at most four: 32 waves)
-  const double c1 = rounds(1, 1) * fmax(0.024 * thin_k, 2.5 + (4 + 3.5 * rt) * k);
-  const double c4 = rounds(4, 1) * (7 + 8.5 * rt) * k + rounds(4, at_once < 4 ? at_once : 4) * 3.2;
-  const double c8 = rounds(8, 1) * ((15 + 15 * rt) * k + 4);
+  // The form that finishes first, in us, m token tiles of 16 and k times 2048 k: rounds of the compute units times what a workgroup takes.
+  // 16 rows: 2.2 + (2.8 + 3.1 m) k, and at least 24 ns per k of the first 256, one stage of every wave.  64 rows, ring of four: (15 + 4.6 m) k
+  // + 2.8; ring of two: (35 + 5.7 m) k two together, (24.5 + 2.4 m) k alone in the last round, and 1.4 of waiting, which four share where K is
+  // one stage.  128 rows: (30 + 8 m) k or, from two tiles on, (14 + 15.5 m) k, and 3.  Against the best form, over 814 sizes of 1 to 4000 tokens with
+  // weights from memory: 1 % on average, 34 % at most.  Tokens x K x rows, 16 rows / 64 with four stages / 64 with two / 128, us: 1 x 2048 x 2000 9 / 21 / 36 / 37, 1 x 2048 x 12300 27 / 25 / 39 / 40,
+  // 24 x 2048 x 12300 54 / 31 / 44 / 49, 64 x 2048 x 2000 24 / 48 / 49 / 89, 4000 x 64 x 4096 128 / 81 / 33 / 37, 4000 x 256 x 4096 411 / 131 / 94 / 111, 1500 x 2048 x 2048
+  // 237 / 132 / 122 / 157; on the vector ALUs 4000 x 64 x 4096 40, 4000 x 256 x 4096 121.  128 rows are for one token block and many rows
+  // (8 x 4096 x 32000 101 us, with 64 rows 123; 64 x 4096 x 32000 165, 176).  Over a plan: its tiles as far as the
+  // host can tell, half of the experts' last ones.
+  const int full = a.T / FB, experts = row_blocks - full, tiles = !grouped ? row_blocks : full + experts / 2 > experts ? full + experts / 2 : experts;
+  const double m = (double)(grouped ? a.T / tiles : a.T < FB ? a.T : FB) / 16, k = a.K / 2048.0;
+  const long cu = f32_n_cu(), col = (long)tiles * heads, n1 = ceil_div(a.N, 16) * col, n4 = ceil_div(a.N, 64) * col, n8 = ceil_div(a.N, 128) * col;
+  auto rounds = [](long blocks, long slots) { return (double)((blocks + slots - 1) / slots); };
+  const double r1 = m > 0.5 || n1 < cu ? rounds(n1, cu) : (double)n1 / cu;       // (few tokens: the next workgroups start as units are free)
+  const double c1 = r1 * fmax(0.024 * (a.K < 256 ? a.K : 256), 2.2 + (2.8 + 3.1 * m) * k);
+  const double c4 = rounds(n4, cu) * ((15 + 4.6 * m) * k + 2.8);
+  const int alone = n4 % (2 * cu) > 0 && n4 % (2 * cu) <= cu ? 1 : 0;
+  const double c2 = ((rounds(n4, 2 * cu) - alone) * (35 + 5.7 * m) + alone * (24.5 + 2.4 * m)) * k + rounds(n4, (a.K <= 64 ? 4 : 2) * cu) * 1.4;
+  const double c8 = rounds(n8, cu) * (fmax(30 + 8 * m, 14 + 15.5 * m) * k + 3);
   const bool direct = (((uintptr_t)a.x | (uintptr_t)a.W) & 15) == 0;           // x may begin at any column of a wider tensor
   const hipStream_t s = (hipStream_t)stream;
-  if (c1 <= c4 && c1 <= c8) return launch_f32<1>(who, a, plan, grouped, row_blocks, heads, s);
-  if (c4 <= c8) return direct ? launch_f32<4>(who, a, plan, grouped, row_blocks, heads, s) : launch_f32<4, false>(who, a, plan, grouped, row_blocks, heads, s);
-  return direct ? launch_f32<8>(who, a, plan, grouped, row_blocks, heads, s) : launch_f32<8, false>(who, a, plan, grouped, row_blocks, heads, s);
+  if (c1 <= c4 && c1 <= c2 && (col > 1 || c1 <= c8)) return launch_f32<1>(who, a, plan, grouped, row_blocks, heads, s);
+  if (!direct) return launch_f32<4, 2, false>(who, a, plan, grouped, row_blocks, heads, s);
+  if (col == 1 && c8 < c4 && c8 < c2) return launch_f32<8, 3>(who, a, plan, grouped, row_blocks, heads, s);
+  if (c4 < c2) return launch_f32<4, 4>(who, a, plan, grouped, row_blocks, heads, s);
+  return launch_f32<4, 2>(who, a, plan, grouped, row_blocks, heads, s);
 }
 
 }  // namespace

@@ -394,10 +394,10 @@ def test_fp32_linear_forms(ops, T, K, N):
     assert torch.equal(y1, y0 + y)
 
 
-@pytest.mark.parametrize("T,K,N", [(63, 208, 39), (65, 16, 2050), (130, 128, 4101), (65, 192, 4109), (130, 208, 2051), (65, 272, 8200), (190, 144, 8198)])
+@pytest.mark.parametrize("T,K,N", [(63, 2064, 70), (65, 16, 2050), (63, 208, 39), (130, 128, 4101), (65, 272, 8200), (20, 1040, 8201), (4, 1040, 32001)])
 def test_fp32_linear_at_any_element(ops, T, K, N):
-    """Operands that begin at any element give the bits of aligned ones, with 16, 64 and 128 rows per workgroup, a K that lies in LDS whole and
-    one that does not; the rows of y likewise.  Rounding as in test_fp32_linear_forms."""
+    """Operands that begin at any element give the bits of aligned ones, with 16, 64 (rings of two and of four stages, a K of one stage and of
+    more) and 128 rows per workgroup; the rows of y likewise.  Rounding as in test_fp32_linear_forms."""
     rng = np.random.default_rng(K + N)
     x, W, y0 = (torch.from_numpy(rng.normal(size=s)).float().to(DEV) for s in ((T, K), (N, K), (T, N)))
     y = ops.linear(x, W)
@@ -458,8 +458,8 @@ def test_experts_over_ragged_tiles(D, counts, glu):
 @pytest.mark.parametrize("counts", [[300, 1, 65, 130], [16, 17, 0, 33], [64, 128, 64]])
 @pytest.mark.parametrize("K,N", [(272, 72), (128, 4100), (272, 8200), (208, 12290)])
 def test_fp32_experts_over_ragged_tiles(D, counts, K, N):
-    """One to four token tiles of 16 per workgroup, rows gathered from tokens and scattered to entries, with 16, 64 and 128 weight rows, a K
-    that lies in LDS whole and one that does not; K + 3 roundings of 2^-24 on what is added up, twice that for the square."""
+    """One to four token tiles of 16 per workgroup, rows gathered from tokens and scattered to entries, with 16 and 64 weight rows, ragged
+    ones and a ragged K; K + 3 roundings of 2^-24 on what is added up, twice that for the square."""
     dt, E, top = torch.float32, len(counts), 2
     rng = np.random.default_rng(K + N)
     pick = rng.permutation(np.repeat(np.arange(E), np.array(counts) * top)).astype(np.int32)
