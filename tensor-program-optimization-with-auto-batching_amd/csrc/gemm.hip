@@ -997,11 +997,13 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_mid_kernel(void* __res
 // two estimates, in units of 31 ns per 64-k stage.  A workgroup takes ft + 1.6 fn + 1 per stage - its operands through LDS, the
 // products, the barrier (measured on 4096 x 12288: 0.46 us at 8 / 4, 0.63 at 8 / 8, 0.73 at 12 / 6, 0.92 at 16 / 8) - times the
 // rounds that the compute units need for all workgroups.  All of them together take in their fragments, 0.0012 each, and those that
-// miss the second-level caches (weights once, tokens once per XCD) 0.02 each.  The two overlap in part: root of the sum of squares.
+// miss the second-level caches: weights once, 0.02 each, tokens, 0.0107 each, once per row block or XCD where they are too many to stay
+// in the memory-side cache (4568 tokens x 9984 x 400: seven row blocks of 64 99 us, five of 96 80).  The two overlap in part: root of the sum of
+// squares.
 // Measured where the choice matters, in us: 137 tokens, q/k/v 33.9 at 8 / 6, 36.0 at 12 / 4, 48 at 16 / 6; gate/up (22016 rows)
 // 53.1 at 12 / 6, 60.8 at 16 / 6, 77.8 at 8 / 6; 300 tokens, q/k/v 49.8 at 12 / 6, 52.8 at 16 / 6, 71.5 at 8 / 8; o of 100 tokens in four
-// slices 14.0 at 8 / 4, 17.1 at 8 / 8; 512 tokens x 4096 x 4096 29.6 at 8 / 4, 38.2 at 8 / 6.  Over 180 sizes of 100 to 520 blocks of 256 x 256
-// the choice takes 1 % longer than the best of the nine on average, 10 % at most.
+// slices 14.0 at 8 / 4, 17.1 at 8 / 8; 512 tokens x 4096 x 4096 29.6 at 8 / 4, 38.2 at 8 / 6.  Over 240 sizes the choice takes 1 % longer than the
+// best of the nine on average, 10 % at most without and 29 % with K slices.
 struct MidShape {
   int ft, fn, ksplit;
 };
@@ -1019,7 +1021,8 @@ MidShape gemm_mid_shape(int T, int K, int N, int ksplit_max) {
       ks = ks > ks_cap ? ks_cap : ks < 1 ? 1 : ks;
       const double rounds = (double)((rows * tb * ks + n_cu - 1) / n_cu), unit = ft + 1.6 * fn + 1;
       const double mine = rounds * unit / ks, tiles = ceil_div(T, 16);
-      const double all = 0.0012 * rows * (tiles + tb * fn) + 0.02 * (ceil_div(N, 16) + 8 * tiles);
+      const int copies = (long)T * K * 2 > 16 << 20 && rows < 8 ? (int)rows : 8;       // of the tokens: one per XCD that has a row block
+      const double all = 0.0012 * rows * (tiles + tb * fn) + 0.02 * ceil_div(N, 16) + 0.0107 * copies * tiles;
       const double cost = mine * mine + all * all;
       if (least == 0 || cost < least) {
         least = cost;

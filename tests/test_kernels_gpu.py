@@ -1456,3 +1456,17 @@ def test_row_major_linear_around_a_round_of_blocks(ops, T, N, K):
     y = ops.linear(x, W, out_dtype=torch.float32)
     w = W.unpack().double()
     assert bool(((y.double() - x.double() @ w.T).abs() <= (K + 2) * 2.0 ** -24 * (x.abs().double() @ w.abs().T)).all())
+
+
+@pytest.mark.parametrize("T,N,K", [(4568, 400, 1824), (4568, 400, 1856), (3000, 456, 2816), (2800, 504, 3008), (2700, 520, 3136)])
+def test_mid_size_linear_of_many_tokens_and_few_rows(ops, T, N, K):
+    """Tokens on both sides of 16 MiB, where a row block's own copy of them counts: the bits of the row-major kernel."""
+    g = torch.Generator(device=DEV).manual_seed(T + N)
+    x = torch.randn((T, K), generator=g, device=DEV).half()
+    W = ops.PackedWeight((torch.randn((N, K), generator=g, device=DEV) * 0.05).half())
+    f = ops.FragActivation.pack(x)
+    assert torch.equal(ops.linear(f, W), ops.linear(x, W, kernel="gemm"))
+    y0 = torch.randn((T, N), generator=g, device=DEV)
+    y = ops.linear(f, W, out=y0.clone(), accumulate=True)
+    w = W.unpack().double()
+    assert bool(((y.double() - y0.double() - x.double() @ w.T).abs() <= (K + 2) * 2.0 ** -24 * (y0.abs().double() + x.abs().double() @ w.abs().T)).all())
