@@ -154,6 +154,11 @@ class PageTable:
             for t in self._pass_arrays():          # their memory may be given out again, to the stream they were made on
                 t.record_stream(stream)
 
+    def __getstate__(self):
+        """A copy, or a pickle, is made behind all that the passes have queued and knows no streams (which neither takes)."""
+        self._enter()
+        return {**self.__dict__, "_staged": None, "_users": {}}
+
     def _pass_arrays(self):
         """Arrays that were made for the current pass."""
         return [t for t in self._cur[3:] if t is not None]

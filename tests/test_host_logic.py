@@ -293,6 +293,31 @@ def test_passes_on_several_streams_are_ordered(monkeypatch):
     assert {("record", 7), ("record", 9)} <= set(ended)   # behind the whole pass
 
 
+def test_caches_can_be_copied_and_pickled(monkeypatch):
+    """Behind their passes, one of which went on on another stream; the copy goes on by itself."""
+    import copy
+    import pickle
+    kvm = load_pkg("kv_cache")
+    kv = kvm.PagedStateCache([], 32, 8, max_seqs=2, max_blocks=2, max_pos=32, dtype=torch.float32, device="cpu")
+    fake = FakeStreams(monkeypatch, kvm.ops)
+    kv.device = torch.device("cuda")
+    kv.add_sequence("a")
+    for make in (copy.deepcopy, lambda c: pickle.loads(pickle.dumps(c))):
+        fake.at(3)
+        kv.begin_forward("a", [3])
+        fake.at(7)
+        kv.token_meta()
+        kv.end_forward()
+        fake.at(5)
+        kv._staged = (3, torch.cuda.Event())              # a real one: neither copy nor pickle takes it
+        other = make(kv)
+        assert {e[:3] for e in fake.at(5)} >= {("wait", 5, 3), ("wait", 5, 7)}
+        assert other.lens == kv.lens and torch.equal(other.block_table, kv.block_table)
+        other.begin_forward("a", [1])
+        other.end_forward()
+        assert other.lens["a"] == kv.lens["a"] + 1
+
+
 @pytest.mark.parametrize("scaling", [0.5, np.float32(0.3), torch.tensor(0.25), 1e39, -1e300, float("inf"), 7])
 def test_adapter_buckets_as_the_library_reads_them(scaling):
     import ctypes
