@@ -875,10 +875,10 @@ constexpr int LA_QBLOCKS = 48;  // query blocks that LDS takes
 //   O^T += V^T . P^T    lane (dims 4 r .. 4 r + 3, g) holds those of tokens 4 g + e: element i belongs to the row tile of the dims 4 r + i
 // so that every load is 16 contiguous bytes per lane and no operand changes lanes.  The waves' states (m, l, O) meet in LDS, added in the
 // order of the waves.  A page is 272 products of 32 cycles at rank 512 + 64: bound by the matrix cores while there are
-// workgroups enough, by the page's latency below that.  At rank 512 + 64 and 16 heads, 299 tokens at context 150: 75 us, one token at context 2048:
-// 134 us.  Every head by itself on the vector ALUs, each reading its keys twice: 649 and 705 us.
+// workgroups enough, by the page's latency below that.  At rank 512 + 64 and 16 heads, 299 tokens at context 150: 67 us, one token at context 2048:
+// 134 us.  Every head by itself on the vector ALUs, each reading its keys twice: 348 and 701 us.
 template <int NRB, int NW>
-__global__ __launch_bounds__(NW * WAVE, NW == 8 && NRB > 2 ? 2 : 4) void latent_attn_f32_kernel(LatentAttn a) {
+__global__ __launch_bounds__(NW * WAVE, NRB > 4 || (NW == 8 && NRB > 2) ? 2 : 4) void latent_attn_f32_kernel(LatentAttn a) {
   constexpr int NS = NRB / 2, CD = NRB * 32, LD = CD + 4;            // spans of 64 dims; columns of a chunk, padded
   extern __shared__ __align__(16) float fsm[];                       // queries [block][half][lane][4], later the sums [16][LD]
   __shared__ float sm[NW][16], sl[NW][16];
@@ -1005,7 +1005,11 @@ __global__ __launch_bounds__(NW * WAVE, NW == 8 && NRB > 2 ? 2 : 4) void latent_
 #pragma unroll
   for (int w = 0; w < NW; ++w) L += sm[w][r16] == -INFINITY ? 0.f : sl[w][r16] * expf(sm[w][r16] - M);
   const float f = m == -INFINITY ? 0.f : expf(m - M);
+  // Only waves that had a page (the first in any case): 77 tokens at context 16, 8 heads of 32 dims 10.0 -> 6.7 us with 16 waves.
+  const int nw = npages < NW ? npages : NW;
+#pragma unroll
   for (int w = 0; w < NW; ++w) {
+    if (w && w >= nw) break;
     if (wave == w) {
 #pragma unroll
       for (int s = 0; s < NS; ++s)
@@ -1040,23 +1044,28 @@ int launch_latent_f32(const LatentAttn& a, int tiles, hipStream_t s) {
 }
 
 // tiles: of 16 heads.  The fewer workgroups there are, the more waves share a context; few tiles also split the output in blocks of 128 dims
-// (the scores computed by each).  Four waves where a compute unit has workgroups for more: its waves then wait less for each other at the
-// end, which is what a short context costs.  16 / 8 / 4 waves, us: 20 tokens, 32 heads of 192 dims on 8 20.0 / 15.0 / 9.3 (320 workgroups);
-// 100 tokens at context 100, 32 heads of 64 dims on 32 112 / 77 / 32, with the output's two blocks instead of four 39 / 24; 300 at 300 400 / 295 / 144
-// and 152 / 106; 64 tokens at context 1500, 2 heads of 256 dims on 2 (256 workgroups) 67 / 72 / 104.
+// (the scores computed by each), as long as these are one round of the compute units.  Four waves where a compute unit has workgroups for more:
+// its waves then wait less for each other, and another workgroup's work covers the meeting at the end.  Every token at the end of its context, vector
+// ALUs / 16 / 8 / 4 waves, us: 64 tokens at 1500, 2 heads of 256 dims on 2 260 / 63 / 66 / 85; one at 2048, 16 heads of 512 + 64 dims 701 / 136 / 143 / 217;
+// 100 at 100, 32 heads of 64 on 32 44 / 98 / 87 / 43, with the output's two blocks instead of four 32; 300 at 300 516 / 527 / 405 / 225 and 158.
+// Outputs of more than 128 dims, vector ALUs / blocks of 128 with 16 waves / of 256 with eight / of 256 with four: 112 at 1600, 2 heads of 192 on 2
+// (224 tiles) 277 / 107 / 76 / 100; 20 at 20, 32 of 192 on 8 10.4 / 14.0 / 9.3 / 9.3; 76 at 742, 16 of 512 + 64 561 / 110 / 66 / 83; 300 at 300, 16 of
+// 192 on 16 (4800 tiles) 340 / 644 / 386 / 246.  Of 512 with eight / with four waves, 1 to 20 heads: 275 tiles at context 16 29 / 21,
+// 320 of a prompt of 340 52 / 63, 412 at 650 151 / 145, 612 at 15 45 / 38, 822 at 296 171 / 146; from 385 tiles on four waves take 0.84 as long on average.
 int launch_latent_f32(LatentAttn a, hipStream_t s) {
   if (!a.key_scale) a.G = 1, a.gs = a.H, a.gt = ceil_div(a.H, 16);
   const int tiles = a.G * a.gt;
-  const bool few = (long)a.T * tiles < 256;
-  if (few || a.RB <= 4) {
-    const long groups = (long)a.T * tiles * ceil_div(a.RB, 4);
-    const bool narrow = !few && a.RB <= 2;
-    if (groups >= 320) return narrow ? launch_latent_f32<2, 4>(a, tiles, s) : launch_latent_f32<4, 4>(a, tiles, s);
-    if (few && groups <= 256) return launch_latent_f32<4, 16>(a, tiles, s);
-    return narrow ? launch_latent_f32<2, 8>(a, tiles, s) : launch_latent_f32<4, 8>(a, tiles, s);
+  const long rows = (long)a.T * tiles;
+  auto groups = [&](int blocks) { return rows * ceil_div(a.RB, blocks); };
+  if (a.RB > 4 && groups(4) > 256) {
+    if (groups(8) <= 256) return launch_latent_f32<8, 8>(a, tiles, s);
+    if (a.RB <= 8) return launch_latent_f32<8, 4>(a, tiles, s);
+    if (rows < 256) return launch_latent_f32<4, 4>(a, tiles, s);
+    return rows <= 384 ? launch_latent_f32<16, 8>(a, tiles, s) : launch_latent_f32<16, 4>(a, tiles, s);
   }
-  if (a.RB <= 8) return launch_latent_f32<8, 8>(a, tiles, s);
-  return launch_latent_f32<16, 8>(a, tiles, s);
+  if (rows < 256) return launch_latent_f32<4, 16>(a, tiles, s);
+  if (rows < 320) return a.RB <= 2 ? launch_latent_f32<2, 8>(a, tiles, s) : launch_latent_f32<4, 8>(a, tiles, s);
+  return a.RB <= 2 ? launch_latent_f32<2, 4>(a, tiles, s) : launch_latent_f32<4, 4>(a, tiles, s);
 }
 #endif
 

@@ -549,7 +549,8 @@ def test_fp32_attention_of_few_and_many_tokens(D, T, ctx, H, G, dim):
     assert err(got, want) < tol(dt)
 
 
-@pytest.mark.parametrize("T,n,H,G,dim", [(100, 40, 12, 4, 64), (70, 40, 4, 4, 40), (300, 20, 2, 1, 100), (110, 130, 6, 3, 128), (330, 17, 1, 1, 120), (90, 35, 2, 1, 500)])
+@pytest.mark.parametrize("T,n,H,G,dim", [(100, 40, 12, 4, 64), (70, 40, 4, 4, 40), (300, 20, 2, 1, 100), (110, 130, 6, 3, 128), (330, 17, 1, 1, 120), (90, 35, 2, 1, 500), (60, 30, 6, 3, 250),
+                                            (90, 40, 6, 3, 200), (40, 16, 4, 4, 64)])
 def test_fp32_attention_by_number_of_workgroups(D, T, n, H, G, dim):
     """One to sixteen heads of a key/value head on four and on eight waves, outputs of 64 and 128 dims and in parts."""
     dt, scale = torch.float32, dim ** -0.5

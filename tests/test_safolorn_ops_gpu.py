@@ -413,7 +413,8 @@ def test_fp32_linear_at_any_element(ops, T, K, N):
 
 @pytest.mark.parametrize("T,n,H,rank,rot", [(300, 60, 3, 200, 40), (290, 50, 16, 512, 64), (260, 33, 2, 100, 24), (330, 33, 2, 100, 24), (301, 40, 2, 64, 16),
                                             (260, 40, 2, 60, 16), (100, 40, 17, 512, 64), (70, 40, 2, 512, 16), (2, 70, 18, 1600, 64), (70, 20, 1, 1560, 32),
-                                            (270, 18, 1, 1560, 32)])
+                                            (270, 18, 1, 1560, 32), (200, 20, 3, 200, 40), (257, 18, 5, 250, 16), (5, 17, 3, 96, 16),
+                                            (200, 20, 17, 512, 32), (450, 18, 1, 1560, 32)])
 @pytest.mark.parametrize("sunk", [True, False])
 def test_fp32_latent_attention_of_prompts(D, T, n, H, rank, rot, sunk):
     """Four, eight and sixteen waves, outputs of 64 to 512 dims and in parts, queries that do not fit LDS, a second tile of heads."""
