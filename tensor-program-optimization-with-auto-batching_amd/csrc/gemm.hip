@@ -1149,18 +1149,20 @@ extern "C" int mlora_gemm_frag_preferred(int T, int K, int N) {
 }
 
 // The plain linear: the persistent kernel or the mid-size one.  The first takes whole rounds of one 256 x 256 block per compute unit: padding
-// and empty units cost as much as products.  So in one round it needs five eighths of the chip in products, and the second round a number of
-// blocks; small K, where a block's end weighs more, fewer of them.  Measured, persistent / mid-size, us.  One round, by T N / 2^16: 105 (264 x
-// 4096 x 26032) 111 / 101, 144 (557 x 2048 x 16968) 59 / 56, 156 (2500 x 4096 x 4096) 94 / 88, 164 (646 x 8192 x 16672) 214 / 228, 180 (673 x 512 x 17568)
-// 22 / 25, 198 (601 x 4096 x 21584) 115 / 129, 256 105 / 115.  More blocks, K from 2048 on: 264 (3034 x 2048 x 5464) 100 / 85, 280 (3540 x 8192 x 4976)
-// 370 / 303, 336 (1792 x 4096 x 12288) 187 / 171, 348 (719 x 2048 x 29496) 113 / 107, 385 (2784 x 4096 x 8856) 210 / 221, 400 (1963 x 2048 x 12776) 114 / 130; below: 276
-// (1306 x 512 x 11536) 35 / 33, 300 (1379 x 256 x 12664) 23 / 27, 324 (2909 x 512 x 6744) 36 / 40, 342 (4602 x 1024 x 4712) 59 / 62.  Up to 128 tokens half of its work
-// is padding: 128256 x 4096, 128 tokens 263 / 212.
+// and empty units cost as much as products.  So what is asked is T N / 2^16, the blocks' worth of products: about five eighths of the chip in
+// one round, and above that what pays for the second round; less of it for small K, where the mid-size kernel's block ends weigh more.
+// Measured, persistent / mid-size, us.  One round, K from 2048 on: 105 (264 x 4096 x 26032) 111 / 101, 144 (557 x 2048 x 16968) 59 / 56, 156 (2500 x 4096
+// x 4096) 94 / 88, 163 (1079 x 7744 x 9928) 202 / 184, 198 (601 x 4096 x 21584) 115 / 129, 256 105 / 115; below: 140 (4723 x 1152 x 1944) 35 / 34, 154
+// (879 x 192 x 11488) 13 / 14, 159 (493 x 384 x 21192) 17.5 / 21, 180 (673 x 512 x 17568) 22 / 25.  Two, K from 1280 on: 253 (3034 x 2048 x 5464) 100 / 85, 267 (557 x 4288 x
+// 31432) 222 / 186, 289 (831 x 2688 x 22768) 144 / 130, 309 (1657 x 1408 x 12224) 83 / 67, 324 (719 x 2048 x 29496) 113 / 107, 336 (1792 x 4096 x
+// 12288) 187 / 171, 376 (2784 x 4096 x 8856) 210 / 221, 382 (1963 x 2048 x 12776) 114 / 130; below: 199 (520 x 640 x 25064) 44 / 35, 272 (655 x 832 x 27208)
+// 56 / 50, 299 (2909 x 512 x 6744) 36 / 40, 331 (4602 x 1024 x 4712) 55 / 59.  Over 240 sizes of 140 to 460 blocks the choice takes 0.6 % longer than the
+// better one on average, 10 % at most.  Up to 128 tokens half of its work is padding: 128256 x 4096, 128 tokens 263 / 212.
 static bool persistent_pays(int T, int K, int N) {
   const long cu = gemm_n_cu() > 0 ? gemm_n_cu() : 256, nb = (long)ceil_div(T, PP_F * 16) * ceil_div(N, PP_F * 16);
   if (K % 64 || T <= 128) return false;
-  if (nb <= cu) return (long)T * N >= cu * 5 / 8 * (PP_F * 16 * PP_F * 16);
-  return nb > cu * (K >= 2048 ? 43 : 36) / 32;
+  const long least = cu * (nb <= cu ? (K >= 2048 ? 21 : 19) : K >= 1280 ? 43 : 35) / 32;
+  return (long)T * N >= least * (PP_F * 16 * PP_F * 16);
 }
 
 extern "C" int mlora_linear_frag(void* y, int y_dtype, int mode, const void* xf, const void* Wp, int T, int K, int N,

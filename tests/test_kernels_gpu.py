@@ -1433,7 +1433,8 @@ def test_pass_on_another_stream_and_its_successor(ops, decode):
 
 
 @pytest.mark.parametrize("T,N,K", [(250, 42000, 64), (250, 41900, 64), (256, 288 * 256, 128), (256, 289 * 256, 128), (256, 343 * 256, 2048),
-                                   (130, 344 * 256, 2112), (130, 345 * 256, 2048)])
+                                   (130, 344 * 256, 2112), (130, 345 * 256, 2048), (256, 151 * 256, 192), (256, 152 * 256, 192), (256, 167 * 256, 2048), (256, 168 * 256, 2048),
+                                   (641, 28500, 192), (641, 28700, 192), (256, 343 * 256, 1280), (256, 344 * 256, 1280)])
 def test_linear_around_a_round_of_blocks(ops, T, N, K):
     """Both sides of the lines between the mid-size and the persistent kernel that depend on what a round multiplies and on K: the bits of the
     row-major kernel."""
