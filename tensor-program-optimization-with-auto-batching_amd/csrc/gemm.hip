@@ -997,9 +997,10 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_mid_kernel(void* __res
 // two estimates, in units of 31 ns per 64-k stage.  A workgroup takes ft + 1.6 fn + 1 per stage - its operands through LDS, the
 // products, the barrier (measured on 4096 x 12288: 0.46 us at 8 / 4, 0.63 at 8 / 8, 0.73 at 12 / 6, 0.92 at 16 / 8) - times the
 // rounds that the compute units need for all workgroups.  All of them together take in their fragments, 0.0012 each, and those that
-// miss the second-level caches: weights once, 0.02 each, tokens, 0.0107 each, once per row block or XCD where they are too many to stay
-// in the memory-side cache (4568 tokens x 9984 x 400: seven row blocks of 64 99 us, five of 96 80).  The two overlap in part: root of the sum of
-// squares.
+// miss the second-level caches: weights once, 0.02 each, tokens, 0.0107 each, once per XCD, or once per row block where these are fewer and the
+// tokens more than 16 MiB (4568 tokens x 9984 x 400: seven row blocks of 64 99 us, five of 96 80).  The limit is a fit: over 200 sizes of 400 to
+// 8192 tokens and 64 to 1040 rows the choice takes 0.6 % longer than the best of the nine on average and 14 % at most, with 32 MiB 0.8 and 17 %, without
+// it 1.4 and 29 %.  The two overlap in part: root of the sum of squares.
 // Measured where the choice matters, in us: 137 tokens, q/k/v 33.9 at 8 / 6, 36.0 at 12 / 4, 48 at 16 / 6; gate/up (22016 rows)
 // 53.1 at 12 / 6, 60.8 at 16 / 6, 77.8 at 8 / 6; 300 tokens, q/k/v 49.8 at 12 / 6, 52.8 at 16 / 6, 71.5 at 8 / 8; o of 100 tokens in four
 // slices 14.0 at 8 / 4, 17.1 at 8 / 8; 512 tokens x 4096 x 4096 29.6 at 8 / 4, 38.2 at 8 / 6.  Over 240 sizes the choice takes 1 % longer than the
