@@ -267,8 +267,12 @@ __global__ __launch_bounds__(256) void gemm_lds_kernel(void* __restrict__ yv, co
 //     cache lines, which costs the load path a third of its speed.
 //   * The ring runs on across block boundaries: while the last stages of a block are multiplied and its results are
 //     stored, the first stages of the workgroup's next block are already in flight.
-//   * Fragment registers are double-buffered: the LDS reads of stage g + 1 are issued right before the MFMAs of stage
-//     g and complete under them.
+//   * The two waves of a SIMD take turns: half a stage apart, one multiplies (32 products, 512 cycles) while the other reads its
+//     fragments from LDS, requests its share of a later stage and waits; a bare barrier, twice per stage, swaps them.  With all eight
+//     waves in step behind one barrier per stage, reads of the next stage ahead of the products of this one, the matrix cores
+//     were busy half of the time (0.52 of the cycles at 2.17 GHz, 4096 tokens x 12288 x 4096; now 0.72 at 1.85 GHz, where the
+//     power limit begins).  bf16, then and now, us: 4096 x 12288 x 4096 319 -> 287, 4096 x 4096 x 4096 103 -> 94,
+//     4096 x 22016 x 4096 614 -> 517, 8192 x 8192 x 8192 845 -> 696 (1.58 PFLOP/s).
 //   * fp16 results cross a small LDS buffer so that a store instruction writes whole 128-byte lines of a token row.
 // Blocks are numbered so that an XCD (workgroup id mod 8) works through a contiguous range of them, in bands of a few token
 // blocks that share their weights and tokens in its L2 (block_of).
@@ -366,17 +370,20 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
   };
   // the LoRA part of a block: projection slot and adapter (-1: none), everything uniform
   auto lora_of = [&](int n0, int t0, int& slot) -> int {
+    // (through the constant cache: a vector load would wait behind everything that is on its way to LDS)
+    const auto adapter_of = [&](int t0) { return ((const __attribute__((address_space(4))) int32_t*)lo.blk_adapter)[__builtin_amdgcn_readfirstlane(t0) / (PP_F * 16)]; };
     if constexpr (SILU) {
       slot = 0;
-      return lo.blk_adapter[t0 / (PP_F * 16)];
+      return adapter_of(t0);
     }
     slot = -1;
 #pragma unroll
     for (int i = 0; i < 3; ++i)
       if (i < lo.n_proj && n0 >= lo.n_begin[i] && n0 < lo.n_begin[i] + lo.n_rows[i]) slot = i;
     if (slot < 0) return -1;
-    return lo.blk_adapter[t0 / (PP_F * 16)];
+    return adapter_of(t0);
   };
+  auto pick = [](int i, auto a, auto b, auto c) { return i == 0 ? a : i == 1 ? b : c; };   // by value: `lo` is never indexed by a variable
   const int EP = LORA ? 2 * (lo.r / 32) : 0;    // extra k-steps per projection of a block with a delta: hi halves, then lo halves
   const bool has_gate = SILU && LORA && lo.B[0] != nullptr;
   const int E = SILU ? EP * ((lo.B[0] != nullptr) + (lo.B[1] != nullptr)) : EP;
@@ -409,15 +416,10 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
         l_n0 = n0;
         l_t0 = t0;
       } else if (a >= 0) {
-        const elt* Bt = lo.B[0];
-        const elt* vh = lo.vh[0];
-        const elt* vl = lo.vl[0];
-        int nbeg = lo.n_begin[0], nrows = lo.n_rows[0];
-#pragma unroll
-        for (int i = 1; i < 3; ++i)
-          if (i == slot) {                     // uniform select: the struct is never indexed dynamically
-            Bt = lo.B[i]; vh = lo.vh[i]; vl = lo.vl[i]; nbeg = lo.n_begin[i]; nrows = lo.n_rows[i];
-          }
+        const elt* Bt = pick(slot, lo.B[0], lo.B[1], lo.B[2]);
+        const elt* vh = pick(slot, lo.vh[0], lo.vh[1], lo.vh[2]);
+        const elt* vl = pick(slot, lo.vl[0], lo.vl[1], lo.vl[2]);
+        const int nbeg = pick(slot, lo.n_begin[0], lo.n_begin[1], lo.n_begin[2]), nrows = pick(slot, lo.n_rows[0], lo.n_rows[1], lo.n_rows[2]);
         if (wave < NW / 2) {
           l_src = Bt + ((size_t)a * nrows + (n0 - nbeg)) * lo.r;
           l_lo = 0;
@@ -527,60 +529,57 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
   // ---- compute role: rows wn * 128 .., tokens wt * 64 ..
   const int wn = wave & 1, wt = wave >> 1;
   f32x4 acc[8][WTF];
-  eltx8 a[2][8], b[2][WTF];
+  eltx8 a[8], b[WTF];
   int rd = 0;                                  // ring slot of the stage whose fragments are read next
   // The token fragments of a wave: four in a row; of a plan's tile every fourth, so that the places a tile does have - often few of
   // its 256 - spread over all waves, and the first `have` of them are multiplied (uniform; the others are fetched and read like them, but
   // their accumulators never stored).
   auto tfrag = [&](int j) { return GROUPED ? wt + 4 * j : wt * WTF + j; };
-  auto read_frags = [&](auto U) {
-    constexpr int u = decltype(U)::value;
+  // First half of a stage: this wave's fragments from LDS into registers, its share of the stage three ahead on its way into the slot
+  // that all waves have done with, and the wait for its share of the next stage (at most the two stages after that still in flight).
+  auto fetch = [&](auto PLAIN) {
     const elt* st = smem + rd * PP_STAGE_ELEMS + lane * 8;
 #pragma unroll
-    for (int j = 0; j < WTF; ++j) b[u][j] = ld8(st + (PP_F + tfrag(j)) * 512);
+    for (int j = 0; j < WTF; ++j) b[j] = ld8(st + (PP_F + tfrag(j)) * 512);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) a[u][i] = ld8(st + (wn * 8 + i) * 512);
+    for (int i = 0; i < 8; ++i) a[i] = ld8(st + (wn * 8 + i) * 512);
     rd = (rd + 1) & (PP_STAGES - 1);
+    issue(PLAIN);
+    asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    bare_barrier();
+    __builtin_amdgcn_sched_barrier(0);
   };
-  // half (uniform): -1 all eight row tiles, 0 / 1 the first / last four (a LoRA stage of the gate / up projection)
-  auto multiply = [&](auto U, int half, int have) {
-    constexpr int u = decltype(U)::value;
+  // Second half: the products.  half (uniform): -1 all eight row tiles, 0 / 1 the first / last four (a LoRA stage of the gate / up
+  // projection).  The barrier at its end lets the other group begin: ahead of the last four or eight products, to cover its latency, it
+  // has both groups multiply at once and costs 10 % (4096 x 12288 x 4096 287 -> 314 us).
+  auto multiply = [&](int half, int have) {
+    __builtin_amdgcn_s_setprio(1);
     if constexpr (GROUPED) {
       asm volatile("" : "+s"(have));           // compared where it is used, in scalar registers
 #pragma unroll
       for (int j = 0; j < WTF; ++j)
         if (__builtin_expect(j < have, 1)) {   // uniform; the products of a full tile follow each other without a jump
 #pragma unroll
-          for (int i = 0; i < 8; ++i) acc[i][j] = mfma_16x16x32(a[u][i], b[u][j], acc[i][j]);
+          for (int i = 0; i < 8; ++i) acc[i][j] = mfma_16x16x32(a[i], b[j], acc[i][j]);
         }
-      return;
+    } else {
+      if (half != 1) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int j = 0; j < WTF; ++j) acc[i][j] = mfma_16x16x32(a[i], b[j], acc[i][j]);
+      }
+      if (half != 0) {
+#pragma unroll
+        for (int i = 4; i < 8; ++i)
+#pragma unroll
+          for (int j = 0; j < WTF; ++j) acc[i][j] = mfma_16x16x32(a[i], b[j], acc[i][j]);
+      }
     }
-    if (half != 1) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < WTF; ++j) acc[i][j] = mfma_16x16x32(a[u][i], b[u][j], acc[i][j]);
-    }
-    if (half != 0) {
-#pragma unroll
-      for (int i = 4; i < 8; ++i)
-#pragma unroll
-        for (int j = 0; j < WTF; ++j) acc[i][j] = mfma_16x16x32(a[u][i], b[u][j], acc[i][j]);
-    }
-  };
-  // One stage: its successor must be in LDS (this wave's share: at most the two stages issued after it still in flight;
-  // everybody's: the barrier).  The wait also covers this wave's fragment reads of the stage about to be multiplied,
-  // so after the barrier nobody reads that ring slot any more and it is refilled; then the reads of the successor go
-  // out, then the MFMAs.
-  auto stage = [&](auto U, auto PLAIN, int half, int have) {
-    constexpr int u = decltype(U)::value;
-    asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
-    if constexpr (GROUPED) __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0) in the compiler's own terms: else it waits again ahead of the products
-    __syncthreads();
-    issue(PLAIN);
-    read_frags(std::integral_constant<int, 1 - u>());
+    __builtin_amdgcn_s_setprio(0);
     __builtin_amdgcn_sched_barrier(0);
-    multiply(U, half, have);
+    bare_barrier();
     __builtin_amdgcn_sched_barrier(0);
   };
 
@@ -589,9 +588,8 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
   issue(std::false_type());
   issue(std::false_type());
   asm volatile("s_waitcnt vmcnt(8)" ::: "memory");     // the first stage of this wave has landed
-  __syncthreads();
-  issue(std::false_type());
-  read_frags(std::integral_constant<int, 0>());
+  bare_barrier();
+  if (wave >= NW / 2) bare_barrier();                  // the second group: half a stage behind the first
   elt* ostage = smem + PP_STAGES * PP_STAGE_ELEMS + wave * PP_OUT_ELEMS;
   const int r16 = lane & 15, g = lane >> 4;
   for (int L = blockIdx.x; L < nb; L += G) {
@@ -608,26 +606,24 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
       tend = t0 + __builtin_amdgcn_readfirstlane(tile.z);
       have = tend - t0 <= wt * 16 ? 0 : (tend - t0 - wt * 16 + 63) / 64;
     }
-    int nst = KB;                                      // KB and E are even (checked by the launcher): the register sets alternate
+    int nst = KB;
     if constexpr (LORA) {
       int slot;
       if (lora_of(n0, t0, slot) >= 0) nst += E;
       nst = __builtin_amdgcn_readfirstlane(nst);
     }
-    for (int kb = 0; kb < nst; kb += 2) {
-      // (the plain GEMM keeps one copy of the pair: with two, the compiler's register allocation of this loop falls apart)
-      if constexpr (SILU && LORA) {
-        // one copy of the pair; a pair of LoRA stages belongs to one projection and multiplies that half of the tiles only
-        const int half = kb < KB ? -1 : (has_gate && kb - KB < EP ? 0 : 1);   // uniform
-        stage(std::integral_constant<int, 0>(), std::false_type(), half, WTF);
-        stage(std::integral_constant<int, 1>(), std::false_type(), half, WTF);
-      } else if (LORA && load_kb + 2 < KB) {             // uniform: the two stages fetched next are ordinary k-steps inside their block
-        stage(std::integral_constant<int, 0>(), std::true_type(), -1, WTF);
-        stage(std::integral_constant<int, 1>(), std::true_type(), -1, WTF);
-      } else {
-        stage(std::integral_constant<int, 0>(), std::false_type(), -1, have);
-        stage(std::integral_constant<int, 1>(), std::false_type(), -1, have);
-      }
+    // While ordinary k-steps of one block are fetched and multiplied nothing is tested; the last stages of a block and those of a
+    // delta take the general form.
+    int kb = KB - 1 - load_kb;
+    kb = kb < 0 ? 0 : kb < KB ? kb : KB;
+    for (int left = kb; left > 0; --left) {
+      fetch(std::true_type());
+      multiply(-1, have);
+    }
+    for (; kb < nst; ++kb) {
+      const int half = !(SILU && LORA) || kb < KB ? -1 : (has_gate && kb - KB < EP ? 0 : 1);   // uniform
+      fetch(std::false_type());
+      multiply(half, have);
     }
     if constexpr (SILU) {
       // acc[i] and acc[4 + i] are the gate and the up half of channels n0 + wn * 64 + i * 16 + 4 g .. + 3 for token r16 of
@@ -709,21 +705,24 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
       for (int j = 0; j < WTF; ++j) {
         const int t = t0 + tfrag(j) * 16 + r16;
         if (t >= T) continue;
+        const int n = n0 + wn * 128 + g * 4;           // of the first row tile; N is a multiple of 4 (checked)
+        float* p = (float*)yv + (size_t)t * N + n;
+        if constexpr (OUT == OUT_ACC_F32) {
+          // the eight values of a token are requested together: stored one by one they would be read one by one, a memory round each
+          f32x4 old[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const int n = n0 + (wn * 8 + i) * 16 + g * 4;
-          if (n >= N) continue;
-          const size_t o = (size_t)t * N + n;
-          if constexpr (OUT == OUT_F32) {
-            *reinterpret_cast<f32x4*>((float*)yv + o) = acc[i][j];
-          } else {
-            f32x4* p = reinterpret_cast<f32x4*>((float*)yv + o);
-            *p = *p + acc[i][j];
-          }
+          for (int i = 0; i < 8; ++i)
+            if (n + i * 16 < N) old[i] = *reinterpret_cast<const f32x4*>(p + i * 16);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) acc[i][j] = old[i] + acc[i][j];
         }
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          if (n + i * 16 < N) *reinterpret_cast<f32x4*>(p + i * 16) = acc[i][j];
       }
     }
   }
+  if (wave < NW / 2) bare_barrier();
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the loads issued past the last block must not outlive the workgroup's LDS
 }
 

@@ -1471,3 +1471,20 @@ def test_mid_size_linear_of_many_tokens_and_few_rows(ops, T, N, K):
     y = ops.linear(f, W, out=y0.clone(), accumulate=True)
     w = W.unpack().double()
     assert bool(((y.double() - y0.double() - x.double() @ w.T).abs() <= (K + 2) * 2.0 ** -24 * (y0.abs().double() + x.abs().double() @ w.abs().T)).all())
+
+
+@pytest.mark.parametrize("K", [64, 128, 192, 256, 320])
+def test_persistent_blocks_shorter_than_the_ring(ops, K):
+    """Two and three blocks of a workgroup one after another, of fewer, as many and more k-steps than are in flight ahead: the bits of
+    the kernel without LDS, for the three ways a result is stored."""
+    T, N = 2310, 64 * 256 - 24
+    g = torch.Generator(device=DEV).manual_seed(K)
+    x = torch.randn((T, K), generator=g, device=DEV).half()
+    W = (torch.randn((N, K), generator=g, device=DEV) * 0.05).half()
+    f, P = ops.FragActivation.pack(x), ops.PackedWeight(W)
+    assert torch.equal(ops.linear(f, P), ops.linear(x, W, kernel="gemm"))
+    assert torch.equal(ops.linear(f, P, out_dtype=torch.float32), ops.linear(x, W, out_dtype=torch.float32, kernel="gemm"))
+    r, q = (torch.ones((T, N), device=DEV) for _ in range(2))
+    ops.linear(f, P, out=r, accumulate=True)
+    ops.linear(x, W, out=q, accumulate=True, kernel="gemm")
+    assert torch.equal(r, q)
