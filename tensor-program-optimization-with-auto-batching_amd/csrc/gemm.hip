@@ -589,7 +589,6 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
   issue(std::false_type());
   asm volatile("s_waitcnt vmcnt(8)" ::: "memory");     // the first stage of this wave has landed
   bare_barrier();
-  if (wave >= NW / 2) bare_barrier();                  // the second group: half a stage behind the first
   elt* ostage = smem + PP_STAGES * PP_STAGE_ELEMS + wave * PP_OUT_ELEMS;
   const int r16 = lane & 15, g = lane >> 4;
   for (int L = blockIdx.x; L < nb; L += G) {
@@ -616,6 +615,7 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
     // delta take the general form.
     int kb = KB - 1 - load_kb;
     kb = kb < 0 ? 0 : kb < KB ? kb : KB;
+    if (wave >= NW / 2) bare_barrier();        // the second group: half a stage behind the first
     for (int left = kb; left > 0; --left) {
       fetch(std::true_type());
       multiply(-1, have);
@@ -625,6 +625,9 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
       fetch(std::false_type());
       multiply(half, have);
     }
+    // Both groups store together; half a stage apart each waited for the other's memory rounds: 4096 x 12288 x 4096 in bf16, three rounds
+    // of blocks, with a gated product 290 -> 285 us, added to fp32 341 -> 338, 4096 x 4096 x 4096 added to fp32 110 -> 108.
+    if (wave < NW / 2) bare_barrier();
     if constexpr (SILU) {
       // acc[i] and acc[4 + i] are the gate and the up half of channels n0 + wn * 64 + i * 16 + 4 g .. + 3 for token r16 of
       // token fragment j: four products = one 8-byte piece of the output fragment; the pieces of a store instruction
@@ -722,7 +725,6 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
       }
     }
   }
-  if (wave < NW / 2) bare_barrier();
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the loads issued past the last block must not outlive the workgroup's LDS
 }
 
