@@ -1488,3 +1488,14 @@ def test_persistent_blocks_shorter_than_the_ring(ops, K):
     ops.linear(f, P, out=r, accumulate=True)
     ops.linear(x, W, out=q, accumulate=True, kernel="gemm")
     assert torch.equal(r, q)
+
+
+def test_silu_product_over_every_gate(ops):
+    """silu(g) u with u = 1 for every finite fp16 g: within half a place of the fp16 result and what the hardware's exponential and reciprocal
+    add, which is the exponent's rounding (25 * 1.5 * 2^-24 * ln 2 where the result is not zero) and four roundings: 2^-19 together."""
+    g = torch.arange(65536, device=DEV, dtype=torch.int32).to(torch.int16).view(torch.float16)
+    g = g[torch.isfinite(g)].view(1, -1)
+    gu = torch.cat([g, torch.ones_like(g)], 1).contiguous()
+    got, x = ops.silu_mul(gu).double(), g.double()
+    want = x / (1.0 + torch.exp(-x))
+    assert bool(((got - want).abs() <= (2.0 ** -11 + 2.0 ** -19) * want.abs() + 2.0 ** -25).all())
