@@ -307,6 +307,8 @@ struct PPGroup {
 };
 // With OUT_SILU the group's up stage ends in a gated product: an expert's weights are its gate rows, then its up rows.
 
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+
 __device__ __forceinline__ unsigned long long uniform64(unsigned long long v) {
   const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v), hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
   return ((unsigned long long)hi << 32) | lo;
@@ -383,6 +385,7 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
     if (slot < 0) return -1;
     return adapter_of(t0);
   };
+  auto tile_of = [&](int i) { return ((const __attribute__((address_space(4))) i32x4*)gr.plan.tiles)[i]; };   // i uniform: through the constant cache, a vector load would wait behind everything on its way to LDS
   auto pick = [](int i, auto a, auto b, auto c) { return i == 0 ? a : i == 1 ? b : c; };   // by value: `lo` is never indexed by a variable
   const int EP = LORA ? 2 * (lo.r / 32) : 0;    // extra k-steps per projection of a block with a delta: hi halves, then lo halves
   const bool has_gate = SILU && LORA && lo.B[0] != nullptr;
@@ -402,10 +405,12 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
     block_of(L < nb ? L : blockIdx.x, n0, t0); // past the last block: valid addresses, the data is never multiplied
     load_nst = KB;
     const elt* Wb = Wp;
+    int last_tt = x_tt - 1;                    // tiles past it: a valid fragment, results dropped (of a plan's tile its own last one, at hand already)
     if constexpr (GROUPED) {
-      const int4 tile = gr.plan.tiles[t0];
+      const i32x4 tile = tile_of(t0);
       Wb = Wp + __builtin_amdgcn_readfirstlane(tile.x) * gr.w_elems;
       t0 = __builtin_amdgcn_readfirstlane(tile.y);
+      last_tt = (t0 + __builtin_amdgcn_readfirstlane(tile.z) - 1) / 16;
     }
     if constexpr (LORA) {
       int slot;
@@ -454,7 +459,7 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
 #pragma unroll
       for (int q = 0; q < LQ; ++q) {
         int tt = t0 / 16 + (wave - NW / 2) * LQ + q;
-        tt = tt < x_tt ? tt : x_tt - 1;
+        tt = tt < last_tt ? tt : last_tt;
         src[q] = x + (size_t)tt * 512 + lane * 8;
       }
       step = x_tt * 512;
@@ -527,7 +532,8 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
   };
 
   // ---- compute role: rows wn * 128 .., tokens wt * 64 ..
-  const int wn = wave & 1, wt = wave >> 1;
+  // (a group has 128 of the weight rows, a SIMD's two waves the two halves)
+  const int wn = wave / (NW / 2), wt = wave & 3;
   f32x4 acc[8][WTF];
   eltx8 a[8], b[WTF];
   int rd = 0;                                  // ring slot of the stage whose fragments are read next
@@ -600,10 +606,10 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
     block_of(L, n0, t0);
     int tend = T, have = WTF;
     if constexpr (GROUPED) {
-      const int4 tile = gr.plan.tiles[t0];
+      const i32x4 tile = tile_of(t0);
       t0 = __builtin_amdgcn_readfirstlane(tile.y);
       tend = t0 + __builtin_amdgcn_readfirstlane(tile.z);
-      have = tend - t0 <= wt * 16 ? 0 : (tend - t0 - wt * 16 + 63) / 64;
+      have = tend - t0 <= wt * 16 || (SILU ? n0 + wn * 64 >= I : n0 + wn * 128 >= N) ? 0 : (tend - t0 - wt * 16 + 63) / 64;
     }
     int nst = KB;
     if constexpr (LORA) {
@@ -669,6 +675,14 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
       }
     } else if constexpr (OUT == OUT_F16) {
       // 16 tokens x 64 columns at a time through the wave's staging buffer: D[n][t] fragments in, token rows out
+      int rows[WTF][2];                                // requested together
+#pragma unroll
+      for (int j = 0; j < WTF; ++j)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          rows[j][q] = t0 + tfrag(j) * 16 + q * 8 + (lane >> 3);
+          if constexpr (GROUPED) rows[j][q] = gr.plan.perm[rows[j][q] < tend ? rows[j][q] : tend - 1];
+        }
 #pragma unroll
       for (int j = 0; j < WTF; ++j) {
 #pragma unroll
@@ -685,8 +699,7 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
             const int c = q * 64 + lane;           // 16-byte chunk: token row c / 8, columns (c % 8) * 8 ..
             const int tr = c >> 3, cc = (c & 7) * 8;
             const int t = t0 + tfrag(j) * 16 + tr;
-            int row = t;
-            if constexpr (GROUPED) row = gr.plan.perm[t < tend ? t : tend - 1];
+            const int row = rows[j][q];
             const int n = n0 + (wn * 8 + h * 4) * 16 + cc;
             const eltx4 lo = *reinterpret_cast<const eltx4*>(ostage + tr * PP_OUT_LD + cc);
             const eltx4 hi = *reinterpret_cast<const eltx4*>(ostage + tr * PP_OUT_LD + cc + 4);

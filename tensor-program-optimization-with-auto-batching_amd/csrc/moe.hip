@@ -110,8 +110,10 @@ __global__ __launch_bounds__(PL_THREADS) void moe_plan_kernel(int32_t* __restric
   }
   __syncthreads();
   for (int e = threadIdx.x; e < E; e += PL_THREADS) {
-    const int c = count[e];
-    for (int i = 0, k = 0; i < c; i += tile_rows, ++k) tiles[tile0[e] + k] = make_int4(e, first[e] + i, c - i < tile_rows ? c - i : tile_rows, 0);
+    // As many tiles as whole ones would make, but of about the same size: the tiles of a pass are dealt out in rounds, which last as long as
+    // their largest tile (345 entries as 176 + 169 instead of 256 + 89).
+    const int c = count[e], nt = (c + tile_rows - 1) / tile_rows, rows = nt > 0 ? ((c + nt - 1) / nt + 15) & ~15 : tile_rows;
+    for (int i = 0, k = 0; i < c; i += rows, ++k) tiles[tile0[e] + k] = make_int4(e, first[e] + i, c - i < rows ? c - i : rows, 0);
     for (int i = c; i & 15; ++i) perm[first[e] + i] = -1;
     count[e] = 0;
   }
