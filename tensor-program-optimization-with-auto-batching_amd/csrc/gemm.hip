@@ -1164,20 +1164,21 @@ extern "C" int mlora_gemm_frag_preferred(int T, int K, int N) {
 }
 
 // The plain linear: the persistent kernel or the mid-size one.  The first takes whole rounds of one 256 x 256 block per compute unit: padding
-// and empty units cost as much as products.  So what is asked is T N / 2^16, the blocks' worth of products: about five eighths of the chip in
-// one round, and above that what pays for the second round; less of it for small K, where the mid-size kernel's block ends weigh more.
-// Measured, persistent / mid-size, us.  One round, K from 2048 on: 105 (264 x 4096 x 26032) 111 / 101, 144 (557 x 2048 x 16968) 59 / 56, 156 (2500 x 4096
-// x 4096) 94 / 88, 163 (1079 x 7744 x 9928) 202 / 184, 198 (601 x 4096 x 21584) 115 / 129, 256 105 / 115; below: 140 (4723 x 1152 x 1944) 35 / 34, 154
-// (879 x 192 x 11488) 13 / 14, 159 (493 x 384 x 21192) 17.5 / 21, 180 (673 x 512 x 17568) 22 / 25.  Two, K from 1280 on: 253 (3034 x 2048 x 5464) 100 / 85, 267 (557 x 4288 x
-// 31432) 222 / 186, 289 (831 x 2688 x 22768) 144 / 130, 309 (1657 x 1408 x 12224) 83 / 67, 324 (719 x 2048 x 29496) 113 / 107, 336 (1792 x 4096 x
-// 12288) 187 / 171, 376 (2784 x 4096 x 8856) 210 / 221, 382 (1963 x 2048 x 12776) 114 / 130; below: 199 (520 x 640 x 25064) 44 / 35, 272 (655 x 832 x 27208)
-// 56 / 50, 299 (2909 x 512 x 6744) 36 / 40, 331 (4602 x 1024 x 4712) 55 / 59.  Over 240 sizes of 140 to 460 blocks the choice takes 0.6 % longer than the
-// better one on average, 10 % at most.  Up to 128 tokens half of its work is padding: 128256 x 4096, 128 tokens 263 / 212.
+// and empty units cost as much as products.  So what is asked is T N / 2^16, the blocks' worth of products.  In one round more than half of
+// the chip: up to there the mid-size kernel has a round of its own largest blocks, of half that size.  Above one round what pays for the second;
+// less of it for small K, where the mid-size kernel's block ends weigh more.
+// Measured, persistent / mid-size, us.  One round: 113 (1843 x 2304 x 4032) 46 / 37, 120 (640 x 4096 x 12288) 77 / 72, 126 (1500 x 1024 x 5504) 26 / 29,
+// 128 (2048 x 4096 x 4096) 77 / 63, 129 (1500 x 2048 x 5632) 41 / 47, 134 (400 x 4096 x 22016) 81 / 107, 141 (3000 x 2048 x 3072) 45 / 45, 144 (768 x 4096 x 12288)
+// 78 / 86, 156 (2500 x 4096 x 4096) 78 / 93, 172 (512 x 4096 x 22016) 82 / 112.  Two, K from 1280 on: 190 (548 x 3264 x 22704) 122 / 105, 258 (3000 x 2048 x 5632)
+// 82 / 76, 258 (768 x 4096 x 22016) 152 / 152, 281 (1500 x 4096 x 12288) 155 / 147, 302 (900 x 4096 x 22016) 161 / 183, 394 (900 x 4096 x 28672) 173 / 231; below:
+// 235 (3123 x 1024 x 4928) 46 / 43, 252 (3000 x 1024 x 5504) 48 / 54, 274 (815 x 384 x 22032) 26 / 35, 290 (643 x 320 x 29560) 24 / 32.  Over 142 sizes of
+// 90 to 420 blocks the choice takes 0.5 % longer than the better one on average, 21 % at most (448 x 5504 x 37128 216 / 261).  Up to 128 tokens half of
+// its work is padding.
 static bool persistent_pays(int T, int K, int N) {
   const long cu = gemm_n_cu() > 0 ? gemm_n_cu() : 256, nb = (long)ceil_div(T, PP_F * 16) * ceil_div(N, PP_F * 16);
   if (K % 64 || T <= 128) return false;
-  const long least = cu * (nb <= cu ? (K >= 2048 ? 21 : 19) : K >= 1280 ? 43 : 35) / 32;
-  return (long)T * N >= least * (PP_F * 16 * PP_F * 16);
+  const long block = PP_F * 16 * PP_F * 16;
+  return nb <= cu ? (long)T * N * 2 > cu * block : (long)T * N * 32 >= cu * (K >= 1280 ? 36 : 31) * block;
 }
 
 extern "C" int mlora_linear_frag(void* y, int y_dtype, int mode, const void* xf, const void* Wp, int T, int K, int N,

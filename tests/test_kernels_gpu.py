@@ -1499,3 +1499,13 @@ def test_silu_product_over_every_gate(ops):
     got, x = ops.silu_mul(gu).double(), g.double()
     want = x / (1.0 + torch.exp(-x))
     assert bool(((got - want).abs() <= (2.0 ** -11 + 2.0 ** -19) * want.abs() + 2.0 ** -25).all())
+
+
+@pytest.mark.parametrize("T,N,K", [(256, 128 * 256, 192), (256, 128 * 256 + 8, 192), (256, 128 * 256, 2048), (256, 128 * 256 + 8, 2048), (641, 25352, 192),
+                                   (641, 25360, 192), (256, 287 * 256, 1280), (256, 288 * 256, 1280)])
+def test_linear_around_half_a_round_and_the_second_one(ops, T, N, K):
+    """Both sides of half a round of blocks, and of what pays for a second round: the bits of the kernel without LDS."""
+    g = torch.Generator(device=DEV).manual_seed(T + N)
+    x = torch.randn((T, K), generator=g, device=DEV).half()
+    W = ops.PackedWeight((torch.randn((N, K), generator=g, device=DEV) * 0.05).half())
+    assert torch.equal(ops.linear(ops.FragActivation.pack(x), W), ops.linear(x, W.unpack(), kernel="gemm"))
