@@ -171,7 +171,8 @@ __device__ __forceinline__ eltx4 moe_out(f32x4 s, const MoeLinear& a) {
 }
 
 // Tiles of 16 entries (a decode step: a few tokens per expert): the weights are what is read.  A workgroup takes 16 NT rows
-// of one expert, its waves split K, the partial tiles meet in LDS in wave order.
+// of one expert, its waves split K, the partial tiles meet in LDS in wave order.  Besides its weights a workgroup reads the tile's tokens,
+// 16 K elements at most against 16 NT K: NT = 2 while a tile has few tokens, NT = 4 when they weigh (moe_gemv_wide).
 constexpr int MG_WAVES = 8;
 // GLU: the weights are gate rows, then up rows (a.N of each); a workgroup takes NT / 2 tiles of both and stores their product.
 template <int NT, int PIPE, bool GLU = false>
@@ -323,6 +324,22 @@ extern "C" int mlora_moe_combine(float* x, const float* part, int n_part, const 
 }
 
 #ifndef MLORA_ELT_F32
+// Four row tiles per workgroup of the 16-entry tiles, or two.  us, two / four, by entries per expert: up with a gated product, 64 experts of 1408 x
+// 2048, 2 entries 107 / 104, 6 127 / 123, 12 142 / 129, 16 161 / 144, 32 experts of 2752 x 4096, 6 245 / 251, 10 253 / 261, 12 266 / 258, 16 321 / 306;
+// down, 2048 x 1408, 4 63 / 64, 8 72 / 69, 12 83 / 71, 16 93 / 77, 4096 x 2752, 8 130 / 129, 12 147 / 134, 16 169 / 147; up without a gate,
+// 1408 x 2048, whose 1408 workgroups fill the last round badly, 4 61 / 70, 12 69 / 74, 16 80 / 81, 2752 x 4096, 8 131 / 132, 12 143 / 137, 16 166 / 160.
+static bool moe_gemv_wide(int T, int K, int N, int top, int max_tiles, int act) {
+  static const int n_cu = [] {
+    int dev = 0, cu = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cu <= 0) cu = 256;
+    return cu;
+  }();
+  const bool gated = act == MLORA_ACT_GLU;
+  const long n = (long)T * top, E = max_tiles - n / 16 > 0 ? max_tiles - n / 16 : 1;      // (what the number of tiles was made of)
+  const bool many = ceil_div(N, gated ? 32 : 64) * E >= 8L * n_cu;
+  return (many && K <= 2048 && (gated || n >= 8 * E)) || ((many || K >= 4096) && n >= 11 * E);
+}
+
 extern "C" int mlora_moe_linear(void* y, const void* x, const void* W, const int32_t* perm, const int32_t* tiles, const int32_t* n_tiles,
                                 int tile_rows, int max_tiles, int places, int T, int K, int N, int top, int stage, int act, float alpha,
                                 void* workspace, size_t workspace_elems, void* stream) {
@@ -352,8 +369,15 @@ extern "C" int mlora_moe_linear(void* y, const void* x, const void* W, const int
   MoeLinear a;
   a.y = (elt*)y; a.x = (const elt*)x; a.W = (const elt*)W; a.w_elems = (size_t)N * K * (act == MLORA_ACT_GLU ? 2 : 1);
   a.K = K; a.N = N; a.top = top; a.up = stage == MLORA_MOE_UP; a.act = act; a.alpha = alpha;
-  if (act == MLORA_ACT_GLU) hipLaunchKernelGGL((moe_gemv_kernel<2, 4, true>), dim3(N / 16, max_tiles), dim3(MG_WAVES * WAVE), 0, s, a, p);
-  else hipLaunchKernelGGL((moe_gemv_kernel<2, 4>), dim3(ceil_div(N, 32), max_tiles), dim3(MG_WAVES * WAVE), 0, s, a, p);
+  const dim3 block(MG_WAVES * WAVE);
+  const bool wide = moe_gemv_wide(T, K, N, top, max_tiles, act);
+  if (act == MLORA_ACT_GLU) {
+    if (wide) hipLaunchKernelGGL((moe_gemv_kernel<4, 2, true>), dim3(ceil_div(N, 32), max_tiles), block, 0, s, a, p);
+    else hipLaunchKernelGGL((moe_gemv_kernel<2, 4, true>), dim3(N / 16, max_tiles), block, 0, s, a, p);
+  } else {
+    if (wide) hipLaunchKernelGGL((moe_gemv_kernel<4, 2>), dim3(ceil_div(N, 64), max_tiles), block, 0, s, a, p);
+    else hipLaunchKernelGGL((moe_gemv_kernel<2, 4>), dim3(ceil_div(N, 32), max_tiles), block, 0, s, a, p);
+  }
   return mlora_launch_status("moe_linear");
 }
 #endif

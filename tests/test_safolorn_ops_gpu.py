@@ -481,3 +481,27 @@ def test_fp32_experts_over_ragged_tiles(D, counts, K, N):
         assert bool(((up[at].double() - v.clamp(min=0) ** 2).abs() <= 2 * eps * room ** 2).all()), e
         v, room = rows[at].double() @ w.T, rows[at].double().abs() @ w.abs().T
         assert bool(((down[perm[at]].double() - v).abs() <= eps * room).all()), e
+
+
+@pytest.mark.parametrize("glu", [False, True])
+@pytest.mark.parametrize("top,ff,N", [(7, 224, 240), (9, 224, 240), (15, 256, 272)])
+def test_experts_of_a_few_entries_with_four_row_tiles(D, glu, top, ff, N):
+    """Tiles of 16 entries on both sides of what takes four row tiles per workgroup (eight entries per expert), rows that are and are not whole
+    blocks of them.  Bounds as for the large tiles."""
+    dt, E, K, T = torch.bfloat16, 512, 96, 512
+    rng = np.random.default_rng(top)
+    pick = np.argsort(rng.random((T, E)), -1)[:, :top].astype(np.int32)
+    plan = D.MoePlan(torch.from_numpy(pick).to(DEV), E, dt)
+    assert plan.tile_rows == 16
+    x, up, down = rnd(rng, T, K, dt=dt), rnd(rng, E, ff * (2 if glu else 1), K, std=K ** -0.5, dt=dt), rnd(rng, E, N, ff, std=ff ** -0.5, dt=dt)
+    mid = D.moe_linear(x, D.weight(up.view(-1, K)), plan, ff, K, D.MOE_UP, D.ACT_GLU if glu else D.ACT_RELU2)
+    got = f64(D.moe_linear(mid, D.weight(down.view(-1, ff)), plan, N, ff, D.MOE_DOWN)).reshape(T, top, N)
+    torch.cuda.synchronize()
+    X, U, Dn = f64(x), f64(up), f64(down)
+    for e in range(E):
+        t, j = np.nonzero(pick == e)
+        v = X[t] @ U[e].T
+        g, u = v[:, :ff], v[:, -ff:]
+        h, room = (g / (1 + np.exp(-g)) * u, 2 * np.abs(g * u)) if glu else (np.maximum(g, 0) ** 2,) * 2
+        want = h @ Dn[e].T
+        assert (np.abs(got[t, j] - want) <= 2.0 ** -8 * (room @ np.abs(Dn[e]).T + np.abs(want)) + 1e-6).all(), e
