@@ -19,6 +19,7 @@ struct F32Linear {
   long ldx, ldy;
   long hx, hy;               // head strides of x and y (blockIdx.z = head; the weights of a head are [N, K] blocks)
   int T, K, N;
+  int tb;                    // tokens of a block (without a plan)
   float alpha;
   int accumulate, act;       // act: MLORA_ACT_*
   int gather, scatter, top;  // expert tiles (blockIdx.y = tile): gather: x row = entry / top; scatter: y row = entry
@@ -27,8 +28,8 @@ struct F32Linear {
 // The fp32 16 x 16 x 4 product takes one element per lane: a lane holds 4 consecutive k of its row, element e of the four
 // k-groups of 16 lanes is one MFMA (any order of k serves, as long as both operands have the same).
 //
-// At T x K x N = 299 x 2048 x 2048: 46 us (55 TFLOP/s), 1 x 2048 x 11264: 24 us (3.8 TB/s), 4096 x 2048 x 11264: 1715 us
-// (110 TFLOP/s).  The vector ALUs (64 x 64 blocks, both operands staged through LDS behind two barriers per 16 k): 122, 139,
+// At T x K x N = 299 x 2048 x 2048: 41 us (61 TFLOP/s), 4 x 2048 x 11264: 19 us (4.9 TB/s), 4096 x 2048 x 11264: 1667 us
+// (113 TFLOP/s).  The vector ALUs (64 x 64 blocks, both operands staged through LDS behind two barriers per 16 k): 122, 139 (one token),
 // 2415 us.
 
 // Adds the sums of the waves that share K, in their order, and stores.  red [KW][tiles][lane]: four rows n of a token; tile = row
@@ -130,8 +131,7 @@ __device__ __forceinline__ void f32_thin(const F32Linear& a, const MoePlan& plan
 }
 
 // FN * 16 weight rows by up to 64 tokens: four waves share the rows (FN / 4 tiles each, all tokens), twice, for the two halves
-// of every 64 k.  Both operands go from global memory straight into an LDS ring (fragments of 16 rows x 16 k as the lanes read
-// them) that is NST - 1 stages of 64 k ahead, one bare barrier per stage.  Bound by the matrix cores (157 TFLOP/s nominal) or, for few
+// of every 64 k.  Both operands go from global memory straight into an LDS ring that is NST - 1 stages of 64 k ahead, one bare barrier per stage.  Bound by the matrix cores (157 TFLOP/s nominal) or, for few
 // tokens, by what a workgroup takes in.  NST: a deep ring where a workgroup has a compute unit to itself, one of two stages where two
 // share it and their waits overlap.  DIRECT: operands are 16-byte aligned; others go through registers.
 template <int FN, int RT, int NST, bool DIRECT>
@@ -139,24 +139,27 @@ __device__ __forceinline__ void f32_wide(const F32Linear& a, const MoePlan& plan
                                          float* __restrict__ y, int n0, int t0, int t1, f32x4* smem) {
   constexpr int RW = FN / 4, SF = FN + RT, LF = 4 * SF, LQ = (LF + FW - 1) / FW;   // fragments: of 16 k, of a stage, per loading wave
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
-  // fragment f = wave + 8 q of a stage: 16 k number f / SF, there weight tile or (behind those) token tile f % SF
+  // request f = wave + 8 q of a stage: four rows of weight tile or (behind those) token tile f / 4, 64 k each: whole lines.  (16 rows of 16 k a
+  // request, as the lanes multiply them, are half lines: 16 x 2048 x 11264 25 -> 18 us, 299 x 5632 x 2048 125 -> 109, 192 entries over 64 experts of 2048 x
+  // 1408 134 -> 121.)  A row's quad c lies in LDS at place c ^ row, so that 16 rows' quads fall on different banks.
   const float* src[LQ];
-  int fk[LQ], fd[LQ];
+  int fd[LQ], fk[LQ];
 #pragma unroll
   for (int q = 0; q < LQ; ++q) {
     int f = wave + FW * q;
     f = f < LF ? f : LF - 1;                      // (twice the same: every wave has LQ requests per stage)
-    fk[q] = f / SF * 16;
     fd[q] = f;
-    f -= f / SF * SF;
+    const int row = (f & 3) * 4 + g;
+    f >>= 2;
+    fk[q] = (r16 ^ row) * 4;
     if (f < FN) {
-      const int n = n0 + f * 16 + r16;
-      src[q] = W + (size_t)(n < a.N ? n : a.N - 1) * a.K + g * 4;
+      const int n = n0 + f * 16 + row;
+      src[q] = W + (size_t)(n < a.N ? n : a.N - 1) * a.K;
     } else {
-      int t = t0 + (f - FN) * 16 + r16;
+      int t = t0 + (f - FN) * 16 + row;
       t = t < t1 ? t : t1 - 1;
       if (grouped && a.gather) t = plan.perm[t] / a.top;
-      src[q] = x + t * a.ldx + g * 4;
+      src[q] = x + t * a.ldx;
     }
   }
   const int nst = (a.K + 63) / 64;
@@ -188,16 +191,17 @@ __device__ __forceinline__ void f32_wide(const F32Linear& a, const MoePlan& plan
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NST - 2) * LQ) : "memory");
     bare_barrier();
     if (NST > 2 || s + 1 < nst) request(s + NST - 1);       // (the wait counts the requests past the end of a deeper ring)
-    const f32x4* st = smem + (rd * LF + kh * 2 * SF) * 64 + lane;
+    const f32x4* st = smem + rd * LF * 64 + r16 * 16;
     rd = rd + 1 < NST ? rd + 1 : 0;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       if (s * 64 + kh * 32 + h * 16 >= a.K) break;                   // uniform
+      const int at = (kh * 8 + h * 4 + g) ^ r16;
       f32x4 w[RW], xv[RT];
 #pragma unroll
-      for (int i = 0; i < RW; ++i) w[i] = st[(h * SF + rg * RW + i) * 64];
+      for (int i = 0; i < RW; ++i) w[i] = st[(rg * RW + i) * 256 + at];
 #pragma unroll
-      for (int j = 0; j < RT; ++j) xv[j] = st[(h * SF + FN + j) * 64];
+      for (int j = 0; j < RT; ++j) xv[j] = st[(FN + j) * 256 + at];
 #pragma unroll
       for (int i = 0; i < RW; ++i)
 #pragma unroll
@@ -219,7 +223,7 @@ template <int FN, int NST, bool DIRECT>
 __global__ __launch_bounds__(FW* WAVE, 2) void linear_f32_kernel(F32Linear a, MoePlan plan, int grouped) {
   extern __shared__ __align__(16) f32x4 f32_smem[];
   const int n0 = blockIdx.x * FN * 16;
-  int t0 = blockIdx.y * FB, t1 = a.T;
+  int t0 = blockIdx.y * a.tb, t1 = a.T;
   const float* W = a.W + (size_t)blockIdx.z * a.N * a.K;
   const float* x = a.x + blockIdx.z * a.hx;
   float* y = a.y + blockIdx.z * a.hy;
@@ -230,7 +234,7 @@ __global__ __launch_bounds__(FW* WAVE, 2) void linear_f32_kernel(F32Linear a, Mo
     t0 = tile.y;
     t1 = tile.y + tile.z;
   }
-  t1 = t1 < t0 + FB ? t1 : t0 + FB;
+  t1 = t1 < t0 + a.tb ? t1 : t0 + a.tb;
   const int rt = __builtin_amdgcn_readfirstlane((t1 - t0 + 15) >> 4);
   auto block = [&](auto RT) {
     if constexpr (FN == 1) f32_thin<decltype(RT)::value>(a, plan, grouped, x, W, y, n0, t0, t1, f32_smem);
@@ -266,29 +270,41 @@ int launch(const char* who, F32Linear a, const MoePlan& plan, int grouped, int r
   MLORA_CHECK(a.K % 16 == 0 && a.ldx % 4 == 0 && a.hx % 4 == 0 && row_blocks <= 65535 && heads <= 65535, MLORA_ERR_UNSUPPORTED,
               "%s: need K %% 16 == 0 and rows aligned to 16 bytes (T=%d K=%d N=%d)", who, a.T, a.K, a.N);
   // The form that finishes first, in us, m token tiles of 16 and k times 2048 k: rounds of the compute units times what a workgroup takes.
-  // 16 rows: 2.2 + (2.8 + 3.1 m) k, and at least 24 ns per k of the first 256, one stage of every wave.  64 rows, ring of four: (15 + 4.6 m) k
-  // + 2.8; ring of two: (35 + 5.7 m) k two together, (24.5 + 2.4 m) k alone in the last round, and 1.4 of waiting, which four share where K is
-  // one stage.  128 rows: (30 + 8 m) k or, from two tiles on, (14 + 15.5 m) k, and 3.  Against the best form, over 814 sizes of 1 to 4000 tokens with
-  // weights from memory: 1 % on average, 34 % at most.  Tokens x K x rows, 16 rows / 64 with four stages / 64 with two / 128, us: 1 x 2048 x 2000 9 / 21 / 36 / 37, 1 x 2048 x 12300 27 / 25 / 39 / 40,
-  // 24 x 2048 x 12300 54 / 31 / 44 / 49, 64 x 2048 x 2000 24 / 48 / 49 / 89, 4000 x 64 x 4096 128 / 81 / 33 / 37, 4000 x 256 x 4096 411 / 131 / 94 / 111, 1500 x 2048 x 2048
-  // 237 / 132 / 122 / 157; on the vector ALUs 4000 x 64 x 4096 40, 4000 x 256 x 4096 121.  128 rows are for one token block and many rows
-  // (8 x 4096 x 32000 101 us, with 64 rows 123; 64 x 4096 x 32000 165, 176).  Over a plan: its tiles as far as the
-  // host can tell, half of the experts' last ones.
+  // 16 rows: 3.65 + (2.7 + 2 m) k, and at least 11 ns per k of the first 256, one stage of every wave; without a plan its token blocks are of 16, 32
+  // or 64, as leaves least.  64 rows, ring of four: (2.7 + 7.9 m) k, at least 12.3 k, and 1.3; ring of two: (8.1 + 15.2 m) k two together,
+  // (1.8 + 8.1 m) k, at least 35 k, alone in the last round, and 0.9 of waiting, which four share where K is one stage.  128 rows: (7.2 +
+  // 15.2 m) k, at least 27.6 k, and 1.7.  Over 170 sizes of 1 to 500 tokens with weights from memory the choice takes 1.2 % longer than the best form
+  // on average, 20 % at most.  Tokens x K x rows, 16 rows in blocks of 16 tokens / 64 tokens / 64 rows with four stages / with two / 128, us: 1 x 2048 x 2048 9 / 9 / 17 / 20 / 29,
+  // 4 x 2048 x 11264 24 / 25 / 19 / 29 / 30, 32 x 2048 x 2048 13 / 17 / 25 / 25 / 43, 299 x 2048 x 128 12 / 22 / 41 / 41 / 74, 299 x 2048 x 2048 97 / 63 / 43 / 44 / 76, 24 x 2048 x 32000
+  // 141 / 108 / 55 / 52 / 48, 299 x 2048 x 11264 495 / 269 / 156 / 154 / 149.  Over a plan: its tiles as far as the host can tell, half of the experts' last ones.
   const int full = a.T / FB, experts = row_blocks - full, tiles = !grouped ? row_blocks : full + experts / 2 > experts ? full + experts / 2 : experts;
   const double m = (double)(grouped ? a.T / tiles : a.T < FB ? a.T : FB) / 16, k = a.K / 2048.0;
-  const long cu = f32_n_cu(), col = (long)tiles * heads, n1 = ceil_div(a.N, 16) * col, n4 = ceil_div(a.N, 64) * col, n8 = ceil_div(a.N, 128) * col;
+  const long cu = f32_n_cu(), col = (long)tiles * heads, n4 = ceil_div(a.N, 64) * col, n8 = ceil_div(a.N, 128) * col;
   auto rounds = [](long blocks, long slots) { return (double)((blocks + slots - 1) / slots); };
-  const double r1 = m > 0.5 || n1 < cu ? rounds(n1, cu) : (double)n1 / cu;       // (few tokens: the next workgroups start as units are free)
-  const double c1 = r1 * fmax(0.024 * (a.K < 256 ? a.K : 256), 2.2 + (2.8 + 3.1 * m) * k);
-  const double c4 = rounds(n4, cu) * ((15 + 4.6 * m) * k + 2.8);
+  auto thin = [&](long col, double m) {
+    const long n1 = ceil_div(a.N, 16) * col;
+    const double r1 = m > 0.5 || n1 < cu ? rounds(n1, cu) : (double)n1 / cu;     // (few tokens: the next workgroups start as units are free)
+    return r1 * fmax(0.011 * (a.K < 256 ? a.K : 256), 3.65 + (2.7 + 2 * m) * k);
+  };
+  a.tb = FB;
+  double c1 = thin(col, m);
+  for (int tb = FB / 2; !grouped && tb >= 16 && tb < a.T && ceil_div(a.T, tb) <= 65535; tb /= 2) {
+    const double c = thin((long)ceil_div(a.T, tb) * heads, tb / 16.0);
+    if (c < c1) {
+      c1 = c;
+      a.tb = tb;
+    }
+  }
+  const double c4 = rounds(n4, cu) * (fmax(12.3, 2.7 + 7.9 * m) * k + 1.3);
   const int alone = n4 % (2 * cu) > 0 && n4 % (2 * cu) <= cu ? 1 : 0;
-  const double c2 = ((rounds(n4, 2 * cu) - alone) * (35 + 5.7 * m) + alone * (24.5 + 2.4 * m)) * k + rounds(n4, (a.K <= 64 ? 4 : 2) * cu) * 1.4;
-  const double c8 = rounds(n8, cu) * (fmax(30 + 8 * m, 14 + 15.5 * m) * k + 3);
+  const double c2 = ((rounds(n4, 2 * cu) - alone) * (8.1 + 15.2 * m) + alone * fmax(35, 1.8 + 8.1 * m)) * k + rounds(n4, (a.K <= 64 ? 4 : 2) * cu) * 0.9;
+  const double c8 = rounds(n8, cu) * (fmax(27.6, 7.2 + 15.2 * m) * k + 1.7);
   const bool direct = (((uintptr_t)a.x | (uintptr_t)a.W) & 15) == 0;           // x may begin at any column of a wider tensor
   const hipStream_t s = (hipStream_t)stream;
-  if (c1 <= c4 && c1 <= c2 && (col > 1 || c1 <= c8)) return launch_f32<1>(who, a, plan, grouped, row_blocks, heads, s);
+  if (c1 <= c4 && c1 <= c2 && c1 <= c8) return launch_f32<1>(who, a, plan, grouped, grouped ? row_blocks : ceil_div(a.T, a.tb), heads, s);
+  a.tb = FB;
   if (!direct) return launch_f32<4, 2, false>(who, a, plan, grouped, row_blocks, heads, s);
-  if (col == 1 && c8 < c4 && c8 < c2) return launch_f32<8, 3>(who, a, plan, grouped, row_blocks, heads, s);
+  if (c8 < c4 && c8 < c2) return launch_f32<8, 3>(who, a, plan, grouped, row_blocks, heads, s);
   if (c4 < c2) return launch_f32<4, 4>(who, a, plan, grouped, row_blocks, heads, s);
   return launch_f32<4, 2>(who, a, plan, grouped, row_blocks, heads, s);
 }

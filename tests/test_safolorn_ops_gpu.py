@@ -505,3 +505,20 @@ def test_experts_of_a_few_entries_with_four_row_tiles(D, glu, top, ff, N):
         h, room = (g / (1 + np.exp(-g)) * u, 2 * np.abs(g * u)) if glu else (np.maximum(g, 0) ** 2,) * 2
         want = h @ Dn[e].T
         assert (np.abs(got[t, j] - want) <= 2.0 ** -8 * (room @ np.abs(Dn[e]).T + np.abs(want)) + 1e-6).all(), e
+
+
+@pytest.mark.parametrize("T,K,N", [(17, 2048, 64), (33, 1040, 100), (100, 2048, 36), (299, 512, 128), (70, 16, 4100), (70, 48, 4100), (130, 80, 8200), (65, 144, 2052),
+                                   (300, 2064, 2052), (299, 208, 20004)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_fp32_linear_token_blocks_and_row_lengths(ops, T, K, N, shift):
+    """Few weight rows in blocks of 16, 32 and 64 tokens, and rows whose last 64 k are not whole on each of the other forms, x beginning at any
+    column of a wider tensor: K additions and products of fp32."""
+    g = torch.Generator(device=DEV).manual_seed(T + K + N)
+    x = torch.randn((T, K + 16), generator=g, device=DEV)[:, shift:shift + K]
+    W = torch.randn((N, K), generator=g, device=DEV) * K ** -0.5
+    want, room = x.double() @ W.double().T, x.double().abs() @ W.double().abs().T
+    y = ops.linear(x, W)
+    acc = torch.ones((T, N), device=DEV)
+    ops.linear(x, W, out=acc, accumulate=True)
+    assert bool(((y.double() - want).abs() <= (K + 2) * 2.0 ** -24 * room).all())
+    assert bool(((acc.double() - 1 - want).abs() <= (K + 3) * 2.0 ** -24 * (room + 1)).all())
