@@ -323,8 +323,9 @@ class LlamaForCausalLM(CausalLM):
             ta = torch.where(has, tok_adapter[tid], ta)
         return {"multi": (tb, ta)}
 
-    def forward(self, hidden: torch.Tensor, kv: PagedKVCache, tok_adapter=None, logits_rows=None) -> torch.Tensor:
-        """hidden [T, H] fp32 (updated in place), tokens in kv.begin_forward order -> logits fp32."""
+    def forward(self, hidden: torch.Tensor, kv: PagedKVCache, tok_adapter=None, logits_rows=None, host_ids=None) -> torch.Tensor:
+        """hidden [T, H] fp32 (updated in place), tokens in kv.begin_forward order -> logits fp32.  host_ids: the ids of
+        tok_adapter on the host as well, where the caller has them."""
         s = self.shape
         tok_adapter = tok_adapter or {}
         # the adapter types of this pass (a batch merged beforehand may name any loaded type)
@@ -347,15 +348,21 @@ class LlamaForCausalLM(CausalLM):
         ks_ws = self._ksplit_ws(T) if dec_frag or (frag and (T <= 256 or is_decode)) else None
         # a prefill-sized pass of one adapter type of rank 32 or 64: where a 256-token block agrees on one adapter its
         # deltas ride in the base GEMM as extra k-steps; `rest` names the tokens that still need the separate call
-        # (a prefill pass only: the choice needs one read-back, which a decode step recorded into a graph cannot make)
+        # (a prefill pass only: where the ids are known on the device only, the choice needs a read-back, which a decode
+        # step recorded into a graph cannot make)
         fuse = None
         if (tok_adapter and "multi" not in tok_adapter and frag and T > 64 and not is_decode
                 and not torch.cuda.is_current_stream_capturing() and ops.gemm_frag_preferred(T, H, H)):
             (tid, ids), = tok_adapter.items()
             lt = self.lora_types[tid]
             if lt.r in (32, 64):
-                blk, rest = ops.lora_block_adapters(ids, lt.n_adapters)
-                fuse = (lt, ids, blk, {tid: rest} if bool((rest >= 0).any()) else None)     # one read-back per pass
+                if host_ids is not None:
+                    # no read-back: the host keeps running ahead (8 x 512 tokens, two layers: 3299 -> 3275 us a pass)
+                    blk, rest = (ops.upload(torch.from_numpy(a), self.device) if a is not None else None for a in block_adapters(host_ids[tid], lt.n_adapters))
+                else:
+                    blk, rest = ops.lora_block_adapters(ids, lt.n_adapters)
+                    rest = rest if bool((rest >= 0).any()) else None
+                fuse = (lt, ids, blk, None if rest is None else {tid: rest})
         o_shares = None
         if tok_adapter and "multi" not in tok_adapter and len(tok_adapter) == 1 and is_decode and T > 64 and frag:
             (tid, ids), = tok_adapter.items()
@@ -518,8 +525,8 @@ class LlamaForCausalLM(CausalLM):
         """Prefill of the sequences announced to kv.begin_forward; wids: one weight id per sequence
         (the reference prefills one sequence per call: wids [1])."""
         lens = kv._cur[1]
-        w = np.repeat(_host_i32(wids), lens)
-        return self.forward(h, kv, self._ids(h.shape[0], {tid: (None, w)}), self._last_rows(kv)), kv
+        ids = self._ids(h.shape[0], {tid: (None, np.repeat(_host_i32(wids), lens))}, host=True)
+        return self.forward(h, kv, {t: ops.upload(torch.from_numpy(a), self.device) for t, a in ids.items()}, self._last_rows(kv), ids), kv
 
     def decode_a(self, tid, h, kv, wids):
         return self.forward(h, kv, self._ids(h.shape[0], {tid: (None, wids)})), kv
@@ -557,6 +564,16 @@ class LlamaForCausalLM(CausalLM):
         s = self.shape
         per_layer = sum(np.prod(linear_dims(s, p)) for p in LINEARS)
         return int(2 * (per_layer * s.num_hidden_layers + s.vocab_size * s.hidden_size))
+
+
+def block_adapters(ids, n_ad):
+    """`ops.lora_block_adapters` of ids [T] on the host; the second array is None where no token is left over."""
+    T = len(ids)
+    ids = np.where((ids >= 0) & (ids < n_ad), ids, -1).astype(np.int32)
+    pad = np.concatenate([ids, np.full(-T % 256, ids[(T - 1) // 256 * 256], np.int32)]).reshape(-1, 256)
+    blk = np.where((pad == pad[:, :1]).all(1), pad[:, 0], -1).astype(np.int32)
+    rest = np.where(np.repeat(blk, 256)[:T] >= 0, -1, ids).astype(np.int32)
+    return blk, rest if (rest >= 0).any() else None
 
 
 def _host_i32(a):

@@ -1509,3 +1509,15 @@ def test_linear_around_half_a_round_and_the_second_one(ops, T, N, K):
     x = torch.randn((T, K), generator=g, device=DEV).half()
     W = ops.PackedWeight((torch.randn((N, K), generator=g, device=DEV) * 0.05).half())
     assert torch.equal(ops.linear(ops.FragActivation.pack(x), W), ops.linear(x, W.unpack(), kernel="gemm"))
+
+
+@pytest.mark.parametrize("T", [65, 256, 257, 700, 1024])
+@pytest.mark.parametrize("pattern", ["one", "halves", "mixed", "none", "out of range"])
+def test_block_adapters_on_the_host(ops, T, pattern):
+    """The adapters of 256-token blocks made on the host are those the kernel makes."""
+    ids = {"one": np.full(T, 3), "halves": np.arange(T) // 300, "mixed": np.random.default_rng(T).integers(-1, 5, T), "none": np.full(T, -1),
+           "out of range": np.where(np.arange(T) < 256, 7, 2)}[pattern].astype(np.int32)
+    blk, rest = load_pkg("llama").block_adapters(ids, 5)
+    want_blk, want_rest = (t.cpu().numpy() for t in ops.lora_block_adapters(torch.from_numpy(ids).to(DEV), 5))
+    assert np.array_equal(blk, want_blk)
+    assert (rest is None and (want_rest < 0).all()) or np.array_equal(rest, want_rest)
