@@ -2,15 +2,10 @@
 // loop without any host work between kernels, so the step can be captured into a graph and replayed.
 #include "common.h"
 
-namespace {
+int mlora_argmax_advance(int32_t* ids, const float* logits, int B, int V, int32_t* pos, int32_t* ctx, void* stream);
+int mlora_embed_rmsnorm(void* y, float* resid, const void* table, const int32_t* ids, int V, const void* w, float eps, int T, int H, void* stream);
 
-__global__ void advance_kernel(int32_t* __restrict__ pos, int32_t* __restrict__ ctx, int T) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < T) {
-    pos[t] += 1;
-    ctx[t] += 1;
-  }
-}
+namespace {
 
 #define STEP(call)                   \
   do {                               \
@@ -122,9 +117,7 @@ int decode_step_wide(const mlora_decode_plan* p, void* stream) {
   }
   STEP(norm(p->norm, pending_ks));
   STEP(mlora_linear_frag(p->logits, MLORA_F32, MLORA_STORE, p->xn, p->lm_head_p, T, H, p->vocab, stream));
-  STEP(mlora_argmax(p->tokens, p->logits, T, p->vocab, stream));
-  hipLaunchKernelGGL(advance_kernel, dim3((T + 63) / 64), dim3(64), 0, (hipStream_t)stream, p->pos, p->ctx, T);
-  return mlora_launch_status("decode_step");
+  return mlora_argmax_advance(p->tokens, p->logits, T, p->vocab, p->pos, p->ctx, stream);
 }
 
 }  // namespace
@@ -219,10 +212,11 @@ extern "C" int mlora_decode_step(const mlora_decode_plan* p, void* stream) {
   };
   const void* pending_B = nullptr;    // down_proj expand and partials of the previous layer
   int pending_ks = 1;
-  STEP(mlora_embed(p->resid, MLORA_F32, p->embed, p->tokens, T, H, p->vocab, stream));
+  if (p->n_layers == 0) STEP(mlora_embed(p->resid, MLORA_F32, p->embed, p->tokens, T, H, p->vocab, stream));
   for (int l = 0; l < p->n_layers; ++l) {
     const mlora_layer& L = p->layers[l];
-    STEP(norm(L.ln1, pending_B, ws_down, I, pending_ks));
+    if (l == 0) STEP(mlora_embed_rmsnorm(p->xn, p->resid, p->embed, p->tokens, p->vocab, L.ln1, p->eps, T, H, stream));
+    else STEP(norm(L.ln1, pending_B, ws_down, I, pending_ks));
     const bool qkv_lora = lora && (L.lora[MLORA_Q].A || L.lora[MLORA_K].A || L.lora[MLORA_V].A);
     const bool o_lora = lora && L.lora[MLORA_O].A;
     const bool o_via_ride = o_lora && o_ride;   // the attention launch writes the o shrink's head shares, riders of the o GEMV expand them
@@ -278,7 +272,5 @@ extern "C" int mlora_decode_step(const mlora_decode_plan* p, void* stream) {
   }
   STEP(norm(p->norm, pending_B, ws_down, I, pending_ks));
   STEP(mlora_gemv_frag(p->logits, MLORA_F32, MLORA_STORE, p->xn, p->lm_head_p, T, H, p->vocab, stream));
-  STEP(mlora_argmax(p->tokens, p->logits, T, p->vocab, stream));
-  hipLaunchKernelGGL(advance_kernel, dim3(1), dim3(64), 0, (hipStream_t)stream, p->pos, p->ctx, T);
-  return mlora_launch_status("decode_step");
+  return mlora_argmax_advance(p->tokens, p->logits, T, p->vocab, p->pos, p->ctx, stream);
 }

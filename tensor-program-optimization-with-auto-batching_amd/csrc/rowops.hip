@@ -251,8 +251,59 @@ __device__ __forceinline__ void amax_merge(float& v, int& i, float ov, int oi) {
   }
 }
 
+// The embedding of a row and its RMSNorm into fragment order: embed_kernel<float> and rmsnorm_kernel<float, VPT> in one launch, the same
+// sums in the same order (a decode step's first two launches; a launch is 2 to 3 us of a step, 100 us of four requests in two layers of 1024).
+template <int VPT>
+__global__ __launch_bounds__(NORM_THREADS) void embed_rmsnorm_kernel(elt* __restrict__ y, float* __restrict__ resid, const elt* __restrict__ table,
+                                                                     const int32_t* __restrict__ ids, int V, const elt* __restrict__ w, float eps, int H,
+                                                                     int frag_tt) {
+  __shared__ float lds[NORM_THREADS / WAVE];
+  const int row = blockIdx.x;
+  const int id = ids[row];
+  const bool ok = id >= 0 && id < V;
+  float v[VPT][8];
+  eltx8 wv[VPT];
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    const int c = (i * NORM_THREADS + threadIdx.x) * 8;
+    if (c < H) {
+      wv[i] = ld8(w + c);
+      eltx8 t = eltx8{0, 0, 0, 0, 0, 0, 0, 0};
+      if (ok) t = ld8(table + (size_t)id * H + c);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[i][e] = (float)t[e];
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    const int c = (i * NORM_THREADS + threadIdx.x) * 8;
+    if (c < H) {
+      float* o = resid + (size_t)row * H + c;
+      *reinterpret_cast<f32x4*>(o) = f32x4{v[i][0], v[i][1], v[i][2], v[i][3]};
+      *reinterpret_cast<f32x4*>(o + 4) = f32x4{v[i][4], v[i][5], v[i][6], v[i][7]};
+#pragma unroll
+      for (int e = 0; e < 8; ++e) ss = fmaf(v[i][e], v[i][e], ss);
+    }
+  }
+  ss = block_sum<NORM_THREADS>(ss, lds);
+  const float inv = rsqrtf(ss / (float)H + eps);
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    const int c = (i * NORM_THREADS + threadIdx.x) * 8;
+    if (c < H) {
+      eltx8 o;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] = (elt)(v[i][e] * inv * (float)wv[i][e]);
+      st8(y + frag_offset(row, c, frag_tt), o);
+    }
+  }
+}
+
 constexpr int AMAX_THREADS = 1024;   // one row per workgroup: many threads, few requests each
-__global__ __launch_bounds__(AMAX_THREADS) void argmax_kernel(int32_t* __restrict__ ids, const float* __restrict__ logits, int V) {
+// pos, ctx (or null): counters of the rows, which go on by one
+__global__ __launch_bounds__(AMAX_THREADS) void argmax_kernel(int32_t* __restrict__ ids, const float* __restrict__ logits, int V,
+                                                              int32_t* __restrict__ pos, int32_t* __restrict__ ctx) {
   __shared__ float lv[AMAX_THREADS / WAVE];
   __shared__ int li[AMAX_THREADS / WAVE];
   const int row = blockIdx.x;
@@ -292,9 +343,22 @@ __global__ __launch_bounds__(AMAX_THREADS) void argmax_kernel(int32_t* __restric
     li[wave] = bi;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < AMAX_THREADS / WAVE; ++w) amax_merge(bv, bi, lv[w], li[w]);
+  if (wave > 0) return;
+  constexpr int NW = AMAX_THREADS / WAVE;
+  bv = lv[lane % NW];
+  bi = li[lane % NW];
+#pragma unroll
+  for (int o = NW / 2; o > 0; o >>= 1) {
+    const float ov = __shfl_xor(bv, o, WAVE);
+    const int oi = __shfl_xor(bi, o, WAVE);
+    amax_merge(bv, bi, ov, oi);
+  }
+  if (lane == 0) {
     ids[row] = bi == 0x7fffffff ? 0 : bi;
+    if (pos) {
+      pos[row] += 1;
+      ctx[row] += 1;
+    }
   }
 }
 
@@ -524,10 +588,30 @@ extern "C" int mlora_embed(void* out, int out_dtype, const void* table, const in
   return mlora_launch_status("embed");
 }
 
-extern "C" int mlora_argmax(int32_t* ids, const float* logits, int B, int V, void* stream) {
+// argmax of the rows; pos and ctx (or null): counters that go on by one with it
+int mlora_argmax_advance(int32_t* ids, const float* logits, int B, int V, int32_t* pos, int32_t* ctx, void* stream) {
   MLORA_CHECK(ids && logits, MLORA_ERR_INVALID, "argmax: null pointer");
   MLORA_CHECK(B >= 0 && V > 0, MLORA_ERR_INVALID, "argmax: bad shape B=%d V=%d", B, V);
   if (B == 0) return MLORA_OK;
-  hipLaunchKernelGGL(argmax_kernel, dim3(B), dim3(AMAX_THREADS), 0, (hipStream_t)stream, ids, logits, V);
+  hipLaunchKernelGGL(argmax_kernel, dim3(B), dim3(AMAX_THREADS), 0, (hipStream_t)stream, ids, logits, V, pos, ctx);
   return mlora_launch_status("argmax");
+}
+
+extern "C" int mlora_argmax(int32_t* ids, const float* logits, int B, int V, void* stream) {
+  return mlora_argmax_advance(ids, logits, B, V, nullptr, nullptr, stream);
+}
+
+// resid [T, H] = embedding of ids, y = its RMSNorm in fragment order, at most 64 rows
+int mlora_embed_rmsnorm(void* y, float* resid, const void* table, const int32_t* ids, int V, const void* w, float eps, int T, int H, void* stream) {
+  MLORA_CHECK(y && resid && table && ids && w, MLORA_ERR_INVALID, "embed_rmsnorm: null pointer");
+  MLORA_CHECK(T > 0 && T <= 64 && H > 0 && H % 32 == 0 && H <= 16384 && V > 0, MLORA_ERR_UNSUPPORTED, "embed_rmsnorm: T=%d H=%d V=%d", T, H, V);
+  const int vpt = ceil_div(H, NORM_THREADS * 8);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(T), dim3(NORM_THREADS), 0, (hipStream_t)stream, (elt*)y, resid, (const elt*)table, ids, V, (const elt*)w, eps, H,
+                       mlora_frag_tiles(T));
+  };
+  if (vpt <= 1) launch(embed_rmsnorm_kernel<1>);
+  else if (vpt <= 2) launch(embed_rmsnorm_kernel<2>);
+  else launch(embed_rmsnorm_kernel<4>);
+  return mlora_launch_status("embed_rmsnorm");
 }

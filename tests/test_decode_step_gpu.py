@@ -281,3 +281,25 @@ def test_native_step_where_the_largest_k_needs_the_least_scratch():
     a, ka, _ = _run(model, wl, prompts, ids, "py", 3, synth)
     b, kb, _ = _run(model, wl, prompts, ids, "native", 3, synth)
     assert np.array_equal(a, b) and torch.equal(ka, kb)
+
+
+@pytest.mark.parametrize("hidden,requests,vocab", [(32, 3, 96), (992, 17, 1004), (4096, 64, 300), (4128, 5, 1024), (8224, 2, 4100)])
+def test_native_step_begins_and_ends_as_its_operators(hidden, requests, vocab):
+    """Embedding and first norm in one launch with one, two and three of eight columns a thread, argmax with the counters: tokens and the whole
+    cache of four steps are the per-operator path's, bit for bit."""
+    synth, llama, dsm, ops = (load_pkg(n) for n in ("synth", "llama", "decode_session", "ops"))
+    shape = synth.LlamaShape(hidden_size=hidden, intermediate_size=64, num_attention_heads=2, num_key_value_heads=2, num_hidden_layers=1, head_dim=64,
+                             vocab_size=vocab)
+    model = llama.LlamaForCausalLM.from_synthetic(7, shape, [], DEV)
+    first = np.random.default_rng(hidden).integers(0, vocab, requests).astype(np.int32)
+    got = []
+    for native in (False, True):
+        kv = model.create_paged_kv_cache(requests, requests * 32, 16, 16, free_pages=list(range(requests * 2)), max_seq_len=32)
+        for s in range(requests):
+            kv.add_sequence(s)
+        seqs = list(range(requests))
+        s = dsm.NativeDecodeSession(model, kv, seqs, np.full(requests, -1, np.int32), first) if native else dsm.DecodeSession(model, kv, seqs, {}, first)
+        got.append(([s.step().cpu().numpy().copy() for _ in range(4)], kv.k.clone(), kv.v.clone()))
+    for a, b in zip(*[g[0] for g in got]):
+        assert np.array_equal(a, b)
+    assert torch.equal(got[0][1], got[1][1]) and torch.equal(got[0][2], got[1][2])
