@@ -544,7 +544,7 @@ void launch_gemv(void* y, int out, const elt* x, int ldx, const elt* W, int T, i
 // Rows per workgroup.  Every workgroup reads the whole token block, so its L2 traffic is T / (16 NT) of the weight
 // traffic and the time of a launch follows the most loaded compute unit: wide matrices (>= 768 tiles) take four tiles
 // per wave, which keeps one or two equal workgroups on every unit; narrow ones one tile (or, with a partials buffer,
-// four tiles and a K split - see mlora_gemv_ksplit).
+// a K split of one, two or four tiles - see mlora_gemv_ksplit and gemv_split_tiles).
 // compute units of the current device (0 if it cannot be asked), read once
 int gemv_n_cu() {
   static const int n_cu = [] {
@@ -553,6 +553,15 @@ int gemv_n_cu() {
     return cu;
   }();
   return n_cu;
+}
+
+// Row tiles per workgroup of a K split: as many as give every compute unit one workgroup, and fewer where four would
+// leave units idle (a launch is as long as one workgroup's share of the weight: the idle units could halve it).
+int gemv_split_tiles(int tiles, int ksplit) {
+  const int n_cu = gemv_n_cu();
+  if (tiles * ksplit <= n_cu) return 1;
+  if (ceil_div(tiles, 2) * ksplit <= n_cu) return 2;
+  return 4;
 }
 
 template <bool PACKED, bool XFRAG, bool SHRINK = false>
@@ -566,6 +575,19 @@ int gemv_dispatch(void* y, int y_dtype, int mode, const void* x, int ldx, const 
   const elt* Wp = (const elt*)W;
   const int tiles = ceil_div(N, 16);
   if constexpr (PACKED && XFRAG) {
+    const int nt = ksplit > 1 && T <= 64 ? gemv_split_tiles(tiles, ksplit) : 4;
+    if (nt == 1) {
+      if (T <= 16) launch_gemv<1, 1, PACKED, XFRAG, SHRINK, 4>(y, out, xp, ldx, Wp, T, K, N, s, sb, n_main, y2, ksplit, part, dr, rblocks);
+      else if (T <= 32) launch_gemv<1, 2, PACKED, XFRAG, SHRINK, 4>(y, out, xp, ldx, Wp, T, K, N, s, sb, n_main, y2, ksplit, part, dr, rblocks);
+      else launch_gemv<1, 4, PACKED, XFRAG, SHRINK, 4>(y, out, xp, ldx, Wp, T, K, N, s, sb, n_main, y2, ksplit, part, dr, rblocks);
+      return mlora_launch_status("gemv");
+    }
+    if (nt == 2) {
+      if (T <= 16) launch_gemv<2, 1, PACKED, XFRAG, SHRINK, 4>(y, out, xp, ldx, Wp, T, K, N, s, sb, n_main, y2, ksplit, part, dr, rblocks);
+      else if (T <= 32) launch_gemv<2, 2, PACKED, XFRAG, SHRINK, 4>(y, out, xp, ldx, Wp, T, K, N, s, sb, n_main, y2, ksplit, part, dr, rblocks);
+      else launch_gemv<2, 4, PACKED, XFRAG, SHRINK, 2>(y, out, xp, ldx, Wp, T, K, N, s, sb, n_main, y2, ksplit, part, dr, rblocks);
+      return mlora_launch_status("gemv");
+    }
     if (T <= 32 && (ksplit > 1 || tiles >= 768)) {
       // three tiles per workgroup where that gives every compute unit exactly one workgroup's worth or less (768 tiles on
       // 256 units: with four tiles a quarter of the units would stay idle and the others set the time); same bits
@@ -684,7 +706,7 @@ extern "C" int mlora_gemv_frag_lora(void* y, int y_dtype, int mode, const void* 
 #endif
 
 // A narrow weight (fewer than 512 row tiles) gives too few workgroups for four tiles each; splitting K over up to four
-// workgroups restores one equal workgroup per compute unit.  At least 24 k-steps per slice keep every wave's pipeline full.
+// workgroups restores one equal workgroup per compute unit (with fewer tiles each where even that leaves units idle).  At least 24 k-steps per slice keep every wave's pipeline full.
 int mlora_gemm_mid_ksplit(int T, int K, int N, int ks_max);
 int mlora_gemm_mid_acc(float* resid, float* part, int ld_part, int ks, const void* xf, const void* Wp, int T, int K, int N, void* stream);
 

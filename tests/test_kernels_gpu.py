@@ -1102,6 +1102,36 @@ def test_gemv_ksplit_partials_summed_by_rmsnorm(ops, synth, T, K, N, ks_expected
     assert torch.equal(r2, r1)
 
 
+@pytest.mark.parametrize("T", [1, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("N,ks", [(16, 4), (1012, 4), (1040, 4), (2048, 4), (2068, 4), (1376, 3), (1364, 2), (4096, 2), (4112, 2)])
+def test_gemv_ksplit_tiles_of_a_workgroup(ops, synth, T, N, ks):
+    """A narrow weight takes one or two row tiles per workgroup, a wide one four.  The order in which a row's products
+    are summed is the same: rows of a narrow matrix have the bits that they have as the first rows of a wide one."""
+    L = load_pkg("_lib")
+    K, wide = 1056, 8224
+    x = synth.normal(31, f"kt.x.{T}", (T, K), 1.0, torch.float16, DEV)
+    W = synth.normal(31, "kt.W", (wide, K), 0.02, torch.float16, DEV)
+    r0 = synth.normal(31, f"kt.r.{T}", (T, wide), 1.0, torch.float32, DEV)
+    xf = ops.FragActivation.pack(x)
+    st = torch.cuda.current_stream().cuda_stream
+    res = []
+    for n in (N, wide):
+        Wp = ops.PackedWeight(W[:n].contiguous())
+        r = torch.full((T + 1, n), float("nan"), dtype=torch.float32, device=DEV)          # a row of NaN behind the result and the parts
+        r[:T] = r0[:, :n]
+        part = torch.full(((ks - 1) * T + 1, n), float("nan"), dtype=torch.float32, device=DEV)
+        L.check(L.lib().mlora_gemv_frag_acc_ksplit(r.data_ptr(), None, part.data_ptr(), ks, xf.data.data_ptr(), Wp.data.data_ptr(), T, K, n, 0,
+                                                   None, None, 0, None, 0, 0, st))
+        torch.cuda.synchronize()
+        assert bool(r[T].isnan().all()) and bool(part[-1].isnan().all())
+        res.append((r[:T, :N], part[:-1, :N]))
+    assert torch.equal(res[0][0], res[1][0]) and torch.equal(res[0][1], res[1][1])
+    got = _np(res[0][0]).astype(np.float64) + _np(res[0][1]).reshape(ks - 1, T, N).astype(np.float64).sum(0)
+    x64, w64 = _np(x).astype(np.float64), _np(W[:N]).astype(np.float64)
+    bound = (K // 32 + 16) * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64).T + np.abs(_np(r0[:, :N])))      # fp32 sums of exact products
+    assert (np.abs(got - (_np(r0[:, :N]).astype(np.float64) + x64 @ w64.T)) <= bound + 1e-30).all()
+
+
 @pytest.mark.parametrize("T,K,r,n_ad", [(32, 4096, 16, 16), (20, 11008, 8, 4), (48, 4096, 16, 16), (64, 2048, 32, 6)])
 def test_gemv_ksplit_with_appended_adapter_rows(ops, synth, T, K, r, n_ad):
     """Dense shrink riding in a K-split GEMV: the appended A rows are split with the matrix and the fused expand +
