@@ -777,7 +777,9 @@ int launch_gemm_pp(void* y, const elt* x, int ldx, int x_tt, const elt* Wp, int 
 // bytes a cycle, beside 768 cycles of products per SIMD; so the reads go out between the products (3 to 9 % of a launch over reads
 // ahead of them: gate/up at 137 tokens 61.7 -> 56.6 us).  It is neither the second-level caches (a compute unit can take in 130 GB/s
 // of hits, the kernel asks for 45) nor the depth of the ring (a ring of seven weight stages beside three of tokens was 2 to 5 %
-// slower).
+// slower).  So a wave whose tokens all lie past T reads and multiplies nothing, which leaves its share of LDS to the others:
+// 137 tokens x 12288 x 4096 32.5 -> 29.0 us, 270 x 22016 x 4096 89.6 -> 80.2, 400 x 22016 80.8 -> 77.3.  (The fragments past T are
+// still loaded: dealing only the others out to the waves, each waiting for a count of its own, took more than it saved, 29.0 -> 32 to 36.)
 // grid = (weight-row blocks, K slices, token blocks).
 // With K slices, slice 0 produces the result proper (store or accumulate) and slice s > 0 stores its fp32 partial
 // sums to part[s - 1][T][ld_part] - for the two narrow accumulating linears of a layer, whose partials the next
@@ -926,15 +928,23 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_mid_kernel(void* __res
   wait_next();
   bare_barrier();
   issue();
-  read_frags(std::integral_constant<int, 0>());
-  int g = 0;
-  const int whole = nks / MID_KS;              // stages of two steps; an odd slice ends in one of a single step
-  for (; g + 1 < whole; g += 2) {
-    stage(std::integral_constant<int, 0>(), std::true_type());
-    stage(std::integral_constant<int, 1>(), std::true_type());
+  if (t0 + wt * WTF * 16 >= T) {               // uniform: no token of this wave exists; it only takes its part in the loads
+    for (int s = 0; s < nst; ++s) {
+      wait_next();
+      bare_barrier();
+      issue();
+    }
+  } else {
+    read_frags(std::integral_constant<int, 0>());
+    int g = 0;
+    const int whole = nks / MID_KS;            // stages of two steps; an odd slice ends in one of a single step
+    for (; g + 1 < whole; g += 2) {
+      stage(std::integral_constant<int, 0>(), std::true_type());
+      stage(std::integral_constant<int, 1>(), std::true_type());
+    }
+    if (g < nst) stage(std::integral_constant<int, 0>(), std::false_type());
+    if (g + 1 < nst) stage(std::integral_constant<int, 1>(), std::false_type());
   }
-  if (g < nst) stage(std::integral_constant<int, 0>(), std::false_type());
-  if (g + 1 < nst) stage(std::integral_constant<int, 1>(), std::false_type());
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");   // nothing is in flight into the LDS that the epilogue reuses
   __syncthreads();
 

@@ -1128,7 +1128,7 @@ def test_gemv_ksplit_tiles_of_a_workgroup(ops, synth, T, N, ks):
     assert torch.equal(res[0][0], res[1][0]) and torch.equal(res[0][1], res[1][1])
     got = _np(res[0][0]).astype(np.float64) + _np(res[0][1]).reshape(ks - 1, T, N).astype(np.float64).sum(0)
     x64, w64 = _np(x).astype(np.float64), _np(W[:N]).astype(np.float64)
-    bound = (K // 32 + 16) * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64).T + np.abs(_np(r0[:, :N])))      # fp32 sums of exact products
+    bound = (K + 16) * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64).T + np.abs(_np(r0[:, :N])))      # fp32 sums of exact products
     assert (np.abs(got - (_np(r0[:, :N]).astype(np.float64) + x64 @ w64.T)) <= bound + 1e-30).all()
 
 
@@ -1487,6 +1487,36 @@ def test_row_major_linear_around_a_round_of_blocks(ops, T, N, K):
     y = ops.linear(x, W, out_dtype=torch.float32)
     w = W.unpack().double()
     assert bool(((y.double() - x.double() @ w.T).abs() <= (K + 2) * 2.0 ** -24 * (x.abs().double() @ w.abs().T)).all())
+
+
+@pytest.mark.parametrize("T", [65, 96, 97, 129, 144, 145, 193, 257, 273, 320, 385])
+@pytest.mark.parametrize("K,N,acc", [(1056, 12288, False), (4128, 1028, True)])
+def test_mid_size_linear_waves_without_tokens(ops, T, K, N, acc):
+    """A block whose last tokens are past T leaves whole waves without tokens: they load and multiply nothing.  One to four
+    waves' worth of tokens in the last block, an odd count of k-steps, with and without K slices; nothing is written past T."""
+    g = torch.Generator(device=DEV).manual_seed(T)
+    x, W = [(torch.randn(n, K, generator=g, device=DEV) * sc).half() for n, sc in ((T, 1.0), (N, 0.02))]
+    xf, Wp = ops.FragActivation.pack(x), ops.PackedWeight(W)
+    ref = x.double() @ W.double().T
+    mag = x.double().abs() @ W.double().abs().T
+    y = torch.full((T + 64, N), float("nan"), dtype=torch.float32 if acc else torch.float16, device=DEV)
+    eps = (K + 4) * 2.0 ** -24                       # fp32 sums of exact products, one rounding each at most
+    if acc:
+        y[:T] = torch.randn(T, N, generator=g, device=DEV)
+        ref, mag = ref + y[:T].double(), mag + y[:T].double().abs()
+        ws = torch.full((3 * T * N,), float("nan"), dtype=torch.float32, device=DEV)
+        parts = ops.linear_acc_ksplit(xf, Wp, y[:T], ws)
+        got = y[:T].double()
+        if parts is not None:
+            got = got + ws[:(parts.ks - 1) * T * N].view(parts.ks - 1, T, N).double().sum(0)
+        bound = eps * mag
+    else:
+        ops.linear(xf, Wp, out=y[:T])
+        got = y[:T].double()
+        bound = eps * mag + 2.0 ** -11 * (ref.abs() + eps * mag) + 2.0 ** -25          # and one rounding to fp16
+    torch.cuda.synchronize()
+    assert bool(y[T:].isnan().all())
+    assert bool(((got - ref).abs() <= bound).all())
 
 
 @pytest.mark.parametrize("T,N,K", [(4568, 400, 1824), (4568, 400, 1856), (3000, 456, 2816), (2800, 504, 3008), (2700, 520, 3136)])
