@@ -108,22 +108,11 @@ __device__ __forceinline__ f32x4 mfma_16x16x32(eltx8 a, eltx8 b, f32x4 c) { retu
 struct GluArgs {
   float scale, limit, alpha;
 };
-// silu(x).  For 16-bit results by the hardware's exponential and reciprocal (1 ulp each; with the rounding of the exponent the value is
-// within 2^-19 wherever it is not rounded to zero), 6 instructions instead of 30: expf and the division took 10 us of a round of the
-// persistent GEMM's gated blocks, 64 products a lane and two waves on each SIMD (bf16, 4096 x 12288 x 4096 285 -> 276 us, 4096 x 12288 x 2048
-// 152 -> 139).  The clipped product keeps them: models with it choose experts by their logits, where a different last place tips
-// near ties.
-__device__ __forceinline__ float silu(float x) {
-#if defined(MLORA_ELT_F32)
-  return x / (1.f + expf(-x));
-#else
-  return x * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(x * -1.44269504088896340736f));
-#endif
-}
 template <int KIND>
 __device__ __forceinline__ float glu(float g, float u, const GluArgs& a) {
   if constexpr (KIND == MLORA_GLU_SILU) {
-    return silu((float)(elt)g) * (float)(elt)u;
+    const float gf = (float)(elt)g;
+    return gf / (1.f + expf(-gf)) * (float)(elt)u;
   } else {
     g = fminf(g * a.scale, a.limit);
     u = fminf(fmaxf(u * a.scale, -a.limit), a.limit);
