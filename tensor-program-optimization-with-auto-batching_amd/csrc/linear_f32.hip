@@ -133,8 +133,11 @@ __device__ __forceinline__ void f32_thin(const F32Linear& a, const MoePlan& plan
 // FN * 16 weight rows by up to 64 tokens: four waves share the rows (FN / 4 tiles each, all tokens), twice, for the two halves
 // of every 64 k.  Both operands go from global memory straight into an LDS ring that is NST - 1 stages of 64 k ahead, one bare barrier per stage.  Bound by the matrix cores (157 TFLOP/s nominal) or, for few
 // tokens, by what a workgroup takes in.  NST: a deep ring where a workgroup has a compute unit to itself, one of two stages where two
-// share it and their waits overlap.  DIRECT: operands are 16-byte aligned; others go through registers.
-template <int FN, int RT, int NST, bool DIRECT>
+// share it and their waits overlap.  DIRECT: operands are 16-byte aligned; others go through registers.  SUMS: of a wave for an output.  Four, by
+// element e, make eight with the two halves of K, as many as f32_thin has: the rounding of a sum does not depend on which form a size takes
+// (4 x 2048 x 11264, error against 64 bits 2.9e-7 here and there, 5.7e-7 with one).  They cost registers, not time (19.7 us both), but where
+// four workgroups share a compute unit: one, for a K of one stage (4000 x 64 x 4096 32 us, with four 39), which f32_thin adds in two chains as well.
+template <int FN, int RT, int NST, bool DIRECT, int SUMS>
 __device__ __forceinline__ void f32_wide(const F32Linear& a, const MoePlan& plan, int grouped, const float* __restrict__ x, const float* __restrict__ W,
                                          float* __restrict__ y, int n0, int t0, int t1, f32x4* smem) {
   constexpr int RW = FN / 4, SF = FN + RT, LF = 4 * SF, LQ = (LF + FW - 1) / FW;   // fragments: of 16 k, of a stage, per loading wave
@@ -177,11 +180,13 @@ __device__ __forceinline__ void f32_wide(const F32Linear& a, const MoePlan& plan
     slot = slot + 1 < NST ? slot + 1 : 0;
   };
   const int rg = wave & 3, kh = wave >> 2;
-  f32x4 acc[RW][RT];
+  f32x4 acc[RW][RT][SUMS];
 #pragma unroll
   for (int i = 0; i < RW; ++i)
 #pragma unroll
-    for (int j = 0; j < RT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < RT; ++j)
+#pragma unroll
+      for (int e = 0; e < SUMS; ++e) acc[i][j][e] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int s = 0; s < NST - 1; ++s) request(s);
   int rd = 0;
@@ -205,7 +210,9 @@ __device__ __forceinline__ void f32_wide(const F32Linear& a, const MoePlan& plan
 #pragma unroll
       for (int i = 0; i < RW; ++i)
 #pragma unroll
-        for (int j = 0; j < RT; ++j) acc[i][j] = mfma_f32(w[i], xv[j], acc[i][j]);
+        for (int j = 0; j < RT; ++j)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[i][j][e % SUMS] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[i][e], xv[j][e], acc[i][j][e % SUMS], 0, 0, 0);
     }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                   // the requests past the end, too: the ring becomes the waves' sums
@@ -213,13 +220,18 @@ __device__ __forceinline__ void f32_wide(const F32Linear& a, const MoePlan& plan
 #pragma unroll
   for (int i = 0; i < RW; ++i)
 #pragma unroll
-    for (int j = 0; j < RT; ++j) smem[((kh * 4 + rg) * RW * RT + i * RT + j) * 64 + lane] = acc[i][j];
+    for (int j = 0; j < RT; ++j) {
+      f32x4 v = acc[i][j][0];
+#pragma unroll
+      for (int e = 1; e < SUMS; ++e) v += acc[i][j][e];
+      smem[((kh * 4 + rg) * RW * RT + i * RT + j) * 64 + lane] = v;
+    }
   __syncthreads();
   f32_store<2, FN * RT, RT>(a, plan, grouped, y, n0, t0, t1, smem);
 }
 
 // FN: row tiles of a workgroup (1: f32_thin)
-template <int FN, int NST, bool DIRECT>
+template <int FN, int NST, bool DIRECT, int SUMS>
 __global__ __launch_bounds__(FW* WAVE, 2) void linear_f32_kernel(F32Linear a, MoePlan plan, int grouped) {
   extern __shared__ __align__(16) f32x4 f32_smem[];
   const int n0 = blockIdx.x * FN * 16;
@@ -238,7 +250,7 @@ __global__ __launch_bounds__(FW* WAVE, 2) void linear_f32_kernel(F32Linear a, Mo
   const int rt = __builtin_amdgcn_readfirstlane((t1 - t0 + 15) >> 4);
   auto block = [&](auto RT) {
     if constexpr (FN == 1) f32_thin<decltype(RT)::value>(a, plan, grouped, x, W, y, n0, t0, t1, f32_smem);
-    else f32_wide<FN, decltype(RT)::value, NST, DIRECT>(a, plan, grouped, x, W, y, n0, t0, t1, f32_smem);
+    else f32_wide<FN, decltype(RT)::value, NST, DIRECT, SUMS>(a, plan, grouped, x, W, y, n0, t0, t1, f32_smem);
   };
   if (rt == 1) block(std::integral_constant<int, 1>());
   else if (rt == 2) block(std::integral_constant<int, 2>());
@@ -255,14 +267,14 @@ int f32_n_cu() {
   return n_cu;
 }
 
-template <int FN, int NST = 0, bool DIRECT = true>
+template <int FN, int NST = 0, bool DIRECT = true, int SUMS = 4>
 int launch_f32(const char* who, const F32Linear& a, const MoePlan& plan, int grouped, int row_blocks, int heads, hipStream_t stream) {
   constexpr size_t stage = 4 * (FN + 4) * 1024, most = FN == 1 ? FW * 4 * 1024 : NST * stage;      // the waves' sums, or the ring (which these fit)
-  const size_t lds = NST == 2 && a.K <= 64 ? stage : most;
+  const size_t lds = SUMS == 1 ? stage : most;    // (a K of one stage)
   static const hipError_t configured =               // the attribute is per kernel, set once per process, by one thread
-      hipFuncSetAttribute((const void*)linear_f32_kernel<FN, NST, DIRECT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)most);
+      hipFuncSetAttribute((const void*)linear_f32_kernel<FN, NST, DIRECT, SUMS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)most);
   if (configured != hipSuccess) return mlora_set_error(MLORA_ERR_LAUNCH, "%s: cannot reserve %zu bytes of LDS: %s", who, lds, hipGetErrorString(configured));
-  hipLaunchKernelGGL((linear_f32_kernel<FN, NST, DIRECT>), dim3(ceil_div(a.N, FN * 16), row_blocks, heads), dim3(FW * WAVE), lds, stream, a, plan, grouped);
+  hipLaunchKernelGGL((linear_f32_kernel<FN, NST, DIRECT, SUMS>), dim3(ceil_div(a.N, FN * 16), row_blocks, heads), dim3(FW * WAVE), lds, stream, a, plan, grouped);
   return mlora_launch_status(who);
 }
 
@@ -303,9 +315,13 @@ int launch(const char* who, F32Linear a, const MoePlan& plan, int grouped, int r
   const hipStream_t s = (hipStream_t)stream;
   if (c1 <= c4 && c1 <= c2 && c1 <= c8) return launch_f32<1>(who, a, plan, grouped, grouped ? row_blocks : ceil_div(a.T, a.tb), heads, s);
   a.tb = FB;
+  const bool c8_least = c8 < c4 && c8 < c2, c4_least = c4 < c2;
+  const bool one_sum = a.K <= 64 && !c8_least && !c4_least;      // (wherever x begins: the same bits)
+  if (!direct && one_sum) return launch_f32<4, 2, false, 1>(who, a, plan, grouped, row_blocks, heads, s);
   if (!direct) return launch_f32<4, 2, false>(who, a, plan, grouped, row_blocks, heads, s);
-  if (c8 < c4 && c8 < c2) return launch_f32<8, 3>(who, a, plan, grouped, row_blocks, heads, s);
-  if (c4 < c2) return launch_f32<4, 4>(who, a, plan, grouped, row_blocks, heads, s);
+  if (c8_least) return launch_f32<8, 3>(who, a, plan, grouped, row_blocks, heads, s);
+  if (c4_least) return launch_f32<4, 4>(who, a, plan, grouped, row_blocks, heads, s);
+  if (one_sum) return launch_f32<4, 2, true, 1>(who, a, plan, grouped, row_blocks, heads, s);
   return launch_f32<4, 2>(who, a, plan, grouped, row_blocks, heads, s);
 }
 

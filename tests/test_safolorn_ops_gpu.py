@@ -522,3 +522,19 @@ def test_fp32_linear_token_blocks_and_row_lengths(ops, T, K, N, shift):
     ops.linear(x, W, out=acc, accumulate=True)
     assert bool(((y.double() - want).abs() <= (K + 2) * 2.0 ** -24 * room).all())
     assert bool(((acc.double() - 1 - want).abs() <= (K + 3) * 2.0 ** -24 * (room + 1)).all())
+
+
+@pytest.mark.parametrize("T,K,N", [(1, 2048, 2048), (4, 2048, 11264), (24, 2048, 5632), (40, 1024, 5632), (16, 5632, 11264), (299, 2048, 2048), (299, 2048, 11264),
+                                   (24, 2048, 32000)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_fp32_linear_adds_in_eight_sums(ops, T, K, N, shift):
+    """The products of an output are added in at least eight chains, whatever the rows per workgroup: beside 1, at any place of K, one product in
+    four is 2^-24 (1 + 2^-10), at most one in an MFMA, and what follows 1 in its chain rounds up to 2^-23 each time.  K / 32 such products in a
+    chain, seven sums of chains, alpha."""
+    n, tiny = torch.arange(N, device=DEV), 2.0 ** -24 * (1 + 2.0 ** -10)
+    W = torch.zeros((N, K // 16, 16), device=DEV)
+    W[:, :, :4] = tiny
+    W.view(N, K)[n, n % (K // 16) * 16 + n // (K // 16) % 4] = 1.0
+    y = ops.linear(torch.ones((T, K + 4), device=DEV)[:, shift:shift + K], W.view(N, K))
+    want = 1.0 + (K // 4 - 1) * tiny
+    assert float((y.double() - want).abs().max()) <= (K // 32 + 8) * 2.0 ** -24 * want
