@@ -278,9 +278,12 @@ int launch_f32(const char* who, const F32Linear& a, const MoePlan& plan, int gro
   return mlora_launch_status(who);
 }
 
-int launch(const char* who, F32Linear a, const MoePlan& plan, int grouped, int row_blocks, int heads, void* stream) {
-  MLORA_CHECK(a.K % 16 == 0 && a.ldx % 4 == 0 && a.hx % 4 == 0 && row_blocks <= 65535 && heads <= 65535, MLORA_ERR_UNSUPPORTED,
-              "%s: need K %% 16 == 0 and rows aligned to 16 bytes (T=%d K=%d N=%d)", who, a.T, a.K, a.N);
+// FN row tiles of 16 and tb tokens of a workgroup's block; a ring of NST stages, SUMS sums of a wave for an output (f32_wide)
+struct F32Form {
+  int fn, tb, nst, sums;
+};
+
+F32Form choose(int T, int K, int N, bool grouped, int row_blocks, int heads) {
   // The form that finishes first, in us, m token tiles of 16 and k times 2048 k: rounds of the compute units times what a workgroup takes.
   // 16 rows: 3.65 + (2.7 + 2 m) k, and at least 11 ns per k of the first 256, one stage of every wave; without a plan its token blocks are of 16, 32
   // or 64, as leaves least.  64 rows, ring of four: (2.7 + 7.9 m) k, at least 12.3 k, and 1.3; ring of two: (8.1 + 15.2 m) k two together,
@@ -289,43 +292,58 @@ int launch(const char* who, F32Linear a, const MoePlan& plan, int grouped, int r
   // on average, 20 % at most.  Tokens x K x rows, 16 rows in blocks of 16 tokens / 64 tokens / 64 rows with four stages / with two / 128, us: 1 x 2048 x 2048 9 / 9 / 17 / 20 / 29,
   // 4 x 2048 x 11264 24 / 25 / 19 / 29 / 30, 32 x 2048 x 2048 13 / 17 / 25 / 25 / 43, 299 x 2048 x 128 12 / 22 / 41 / 41 / 74, 299 x 2048 x 2048 97 / 63 / 43 / 44 / 76, 24 x 2048 x 32000
   // 141 / 108 / 55 / 52 / 48, 299 x 2048 x 11264 495 / 269 / 156 / 154 / 149.  Over a plan: its tiles as far as the host can tell, half of the experts' last ones.
-  const int full = a.T / FB, experts = row_blocks - full, tiles = !grouped ? row_blocks : full + experts / 2 > experts ? full + experts / 2 : experts;
-  const double m = (double)(grouped ? a.T / tiles : a.T < FB ? a.T : FB) / 16, k = a.K / 2048.0;
-  const long cu = f32_n_cu(), col = (long)tiles * heads, n4 = ceil_div(a.N, 64) * col, n8 = ceil_div(a.N, 128) * col;
+  const int full = T / FB, experts = row_blocks - full, tiles = !grouped ? row_blocks : full + experts / 2 > experts ? full + experts / 2 : experts;
+  const double m = (double)(grouped ? T / tiles : T < FB ? T : FB) / 16, k = K / 2048.0;
+  const long cu = f32_n_cu(), col = (long)tiles * heads, n4 = ceil_div(N, 64) * col, n8 = ceil_div(N, 128) * col;
   auto rounds = [](long blocks, long slots) { return (double)((blocks + slots - 1) / slots); };
   auto thin = [&](long col, double m) {
-    const long n1 = ceil_div(a.N, 16) * col;
+    const long n1 = ceil_div(N, 16) * col;
     const double r1 = m > 0.5 || n1 < cu ? rounds(n1, cu) : (double)n1 / cu;     // (few tokens: the next workgroups start as units are free)
-    return r1 * fmax(0.011 * (a.K < 256 ? a.K : 256), 3.65 + (2.7 + 2 * m) * k);
+    return r1 * fmax(0.011 * (K < 256 ? K : 256), 3.65 + (2.7 + 2 * m) * k);
   };
-  a.tb = FB;
+  int tb = FB;
   double c1 = thin(col, m);
-  for (int tb = FB / 2; !grouped && tb >= 16 && tb < a.T && ceil_div(a.T, tb) <= 65535; tb /= 2) {
-    const double c = thin((long)ceil_div(a.T, tb) * heads, tb / 16.0);
+  for (int t = FB / 2; !grouped && t >= 16 && ceil_div(T, t) <= 65535; t /= 2) {
+    if (t >= T) continue;                          // one block either way
+    const double c = thin((long)ceil_div(T, t) * heads, t / 16.0);
     if (c < c1) {
       c1 = c;
-      a.tb = tb;
+      tb = t;
     }
   }
   const double c4 = rounds(n4, cu) * (fmax(12.3, 2.7 + 7.9 * m) * k + 1.3);
   const int alone = n4 % (2 * cu) > 0 && n4 % (2 * cu) <= cu ? 1 : 0;
-  const double c2 = ((rounds(n4, 2 * cu) - alone) * (8.1 + 15.2 * m) + alone * fmax(35, 1.8 + 8.1 * m)) * k + rounds(n4, (a.K <= 64 ? 4 : 2) * cu) * 0.9;
+  const double c2 = ((rounds(n4, 2 * cu) - alone) * (8.1 + 15.2 * m) + alone * fmax(35, 1.8 + 8.1 * m)) * k + rounds(n4, (K <= 64 ? 4 : 2) * cu) * 0.9;
   const double c8 = rounds(n8, cu) * (fmax(27.6, 7.2 + 15.2 * m) * k + 1.7);
+  if (c1 <= c4 && c1 <= c2 && c1 <= c8) return {1, tb, 0, 4};
+  if (c8 < c4 && c8 < c2) return {8, FB, 3, 4};
+  if (c4 < c2) return {4, FB, 4, 4};
+  return {4, FB, 2, K <= 64 ? 1 : 4};
+}
+
+int launch(const char* who, F32Linear a, const MoePlan& plan, int grouped, int row_blocks, int heads, void* stream) {
+  MLORA_CHECK(a.K % 16 == 0 && a.ldx % 4 == 0 && a.hx % 4 == 0 && row_blocks <= 65535 && heads <= 65535, MLORA_ERR_UNSUPPORTED,
+              "%s: need K %% 16 == 0 and rows aligned to 16 bytes (T=%d K=%d N=%d)", who, a.T, a.K, a.N);
+  const F32Form f = choose(a.T, a.K, a.N, grouped, row_blocks, heads);
   const bool direct = (((uintptr_t)a.x | (uintptr_t)a.W) & 15) == 0;           // x may begin at any column of a wider tensor
   const hipStream_t s = (hipStream_t)stream;
-  if (c1 <= c4 && c1 <= c2 && c1 <= c8) return launch_f32<1>(who, a, plan, grouped, grouped ? row_blocks : ceil_div(a.T, a.tb), heads, s);
-  a.tb = FB;
-  const bool c8_least = c8 < c4 && c8 < c2, c4_least = c4 < c2;
-  const bool one_sum = a.K <= 64 && !c8_least && !c4_least;      // (wherever x begins: the same bits)
-  if (!direct && one_sum) return launch_f32<4, 2, false, 1>(who, a, plan, grouped, row_blocks, heads, s);
+  a.tb = f.tb;
+  if (f.fn == 1) return launch_f32<1>(who, a, plan, grouped, grouped ? row_blocks : ceil_div(a.T, a.tb), heads, s);
+  if (!direct && f.sums == 1) return launch_f32<4, 2, false, 1>(who, a, plan, grouped, row_blocks, heads, s);   // (the bits of aligned operands)
   if (!direct) return launch_f32<4, 2, false>(who, a, plan, grouped, row_blocks, heads, s);
-  if (c8_least) return launch_f32<8, 3>(who, a, plan, grouped, row_blocks, heads, s);
-  if (c4_least) return launch_f32<4, 4>(who, a, plan, grouped, row_blocks, heads, s);
-  if (one_sum) return launch_f32<4, 2, true, 1>(who, a, plan, grouped, row_blocks, heads, s);
+  if (f.fn == 8) return launch_f32<8, 3>(who, a, plan, grouped, row_blocks, heads, s);
+  if (f.nst == 4) return launch_f32<4, 4>(who, a, plan, grouped, row_blocks, heads, s);
+  if (f.sums == 1) return launch_f32<4, 2, true, 1>(who, a, plan, grouped, row_blocks, heads, s);
   return launch_f32<4, 2>(who, a, plan, grouped, row_blocks, heads, s);
 }
 
 }  // namespace
+
+// 256 rows + tokens of the blocks that mlora_linear takes for a size
+extern "C" int mlora_linear_block(int T, int K, int N) {
+  const F32Form f = choose(T, K, N, false, ceil_div(T, FB), 1);
+  return f.fn * 16 * 256 + f.tb;
+}
 
 extern "C" int mlora_linear(void* y, int y_dtype, int mode, const void* x, int ldx, const void* W, int T, int K, int N, void* stream) {
   MLORA_CHECK(y && x && W && T >= 0 && K > 0 && N > 0 && ldx >= K, MLORA_ERR_INVALID, "linear: null pointer or bad shape T=%d K=%d N=%d", T, K, N);
