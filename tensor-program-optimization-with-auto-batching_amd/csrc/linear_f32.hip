@@ -284,14 +284,17 @@ struct F32Form {
 };
 
 F32Form choose(int T, int K, int N, bool grouped, int row_blocks, int heads) {
-  // The form that finishes first, in us, m token tiles of 16 and k times 2048 k: rounds of the compute units times what a workgroup takes.
-  // 16 rows: 3.65 + (2.7 + 2 m) k, and at least 11 ns per k of the first 256, one stage of every wave; without a plan its token blocks are of 16, 32
-  // or 64, as leaves least.  64 rows, ring of four: (2.7 + 7.9 m) k, at least 12.3 k, and 1.3; ring of two: (8.1 + 15.2 m) k two together,
-  // (1.8 + 8.1 m) k, at least 35 k, alone in the last round, and 0.9 of waiting, which four share where K is one stage.  128 rows: (7.2 +
-  // 15.2 m) k, at least 27.6 k, and 1.7.  Over 170 sizes of 1 to 500 tokens with weights from memory the choice takes 1.2 % longer than the best form
-  // on average, 20 % at most.  Tokens x K x rows, 16 rows in blocks of 16 tokens / 64 tokens / 64 rows with four stages / with two / 128, us: 1 x 2048 x 2048 9 / 9 / 17 / 20 / 29,
-  // 4 x 2048 x 11264 24 / 25 / 19 / 29 / 30, 32 x 2048 x 2048 13 / 17 / 25 / 25 / 43, 299 x 2048 x 128 12 / 22 / 41 / 41 / 74, 299 x 2048 x 2048 97 / 63 / 43 / 44 / 76, 24 x 2048 x 32000
-  // 141 / 108 / 55 / 52 / 48, 299 x 2048 x 11264 495 / 269 / 156 / 154 / 149.  Over a plan: its tiles as far as the host can tell, half of the experts' last ones.
+  // The form that finishes first, m token tiles of 16 and k times 2048 k: rounds of the compute units times what a workgroup takes, in us but for what a
+  // launch costs in any form.  16 rows: 5.6 + (3 + 2.2 m) k, and at least 6 ns per k of the first 256, one stage of every wave; without a plan its token
+  // blocks are of 16, 32 or 64, as leaves least.  64 rows, ring of four: (2.5 + 10.9 m) k, at least 17.2 k, and 2.2; ring of two: (4.4 + 9.9 m) k two
+  // together, (1.1 + 9.1 m) k, at least 26.5 k, alone in the last round, and 0.94 of waiting, which four share where K is one stage.  128 rows: (5.7 +
+  // 8.9 m) k, at least 19.6 k, and 3.  Fitted to the choices over 882 sizes of 1 to 4096 tokens, K of 16 to 11008, 16 to 36000 rows, heads and experts' plans, weights from
+  // memory: the choice takes 1.1 % longer than the best form on average, 40 % at most (12 entries over 16 experts of 1408 x 2048 31 us instead of 22; 219 x 48 x 224 3.8 instead of 2.9).  Costs fitted to
+  // K from 512 on took 2.5 % longer: 247 x 2864 x 4384 and 500 x 256 x 304 went to 16 rows.  Tokens x K x rows, 16 rows in blocks of 16 tokens / 64
+  // tokens / 64 rows with four stages / with two / 128, us: 1 x 2048 x 2048 9 / 9 / 17 / 20 / 29, 4 x 2048 x 11264 24 / 25 / 19 / 29 / 30, 32 x 2048 x 2048 12 / 17 /
+  // 25 / 25 / 43, 299 x 2048 x 128 12 / 22 / 41 / 41 / 74, 299 x 2048 x 2048 97 / 63 / 43 / 44 / 76, 24 x 2048 x 32000 141 / 108 / 55 / 52 / 48, 299 x 2048 x 11264
+  // 495 / 269 / 156 / 154 / 149, 500 x 256 x 304 20 / 8.9 / 8.3 / 7.8 / 13, 247 x 2864 x 4384 167 / 132 / 114 / 110 / 107.  Over a plan: its tiles as far as the host can tell,
+  // half of the experts' last ones.
   const int full = T / FB, experts = row_blocks - full, tiles = !grouped ? row_blocks : full + experts / 2 > experts ? full + experts / 2 : experts;
   const double m = (double)(grouped ? T / tiles : T < FB ? T : FB) / 16, k = K / 2048.0;
   const long cu = f32_n_cu(), col = (long)tiles * heads, n4 = ceil_div(N, 64) * col, n8 = ceil_div(N, 128) * col;
@@ -299,7 +302,7 @@ F32Form choose(int T, int K, int N, bool grouped, int row_blocks, int heads) {
   auto thin = [&](long col, double m) {
     const long n1 = ceil_div(N, 16) * col;
     const double r1 = m > 0.5 || n1 < cu ? rounds(n1, cu) : (double)n1 / cu;     // (few tokens: the next workgroups start as units are free)
-    return r1 * fmax(0.011 * (K < 256 ? K : 256), 3.65 + (2.7 + 2 * m) * k);
+    return r1 * fmax(0.006 * (K < 256 ? K : 256), 5.6 + (3 + 2.2 * m) * k);
   };
   int tb = FB;
   double c1 = thin(col, m);
@@ -311,10 +314,10 @@ F32Form choose(int T, int K, int N, bool grouped, int row_blocks, int heads) {
       tb = t;
     }
   }
-  const double c4 = rounds(n4, cu) * (fmax(12.3, 2.7 + 7.9 * m) * k + 1.3);
+  const double c4 = rounds(n4, cu) * (fmax(17.2, 2.5 + 10.9 * m) * k + 2.2);
   const int alone = n4 % (2 * cu) > 0 && n4 % (2 * cu) <= cu ? 1 : 0;
-  const double c2 = ((rounds(n4, 2 * cu) - alone) * (8.1 + 15.2 * m) + alone * fmax(35, 1.8 + 8.1 * m)) * k + rounds(n4, (K <= 64 ? 4 : 2) * cu) * 0.9;
-  const double c8 = rounds(n8, cu) * (fmax(27.6, 7.2 + 15.2 * m) * k + 1.7);
+  const double c2 = ((rounds(n4, 2 * cu) - alone) * (4.4 + 9.9 * m) + alone * fmax(26.5, 1.1 + 9.1 * m)) * k + rounds(n4, (K <= 64 ? 4 : 2) * cu) * 0.94;
+  const double c8 = rounds(n8, cu) * (fmax(19.6, 5.7 + 8.9 * m) * k + 3);
   if (c1 <= c4 && c1 <= c2 && c1 <= c8) return {1, tb, 0, 4};
   if (c8 < c4 && c8 < c2) return {8, FB, 3, 4};
   if (c4 < c2) return {4, FB, 4, 4};
@@ -339,10 +342,10 @@ int launch(const char* who, F32Linear a, const MoePlan& plan, int grouped, int r
 
 }  // namespace
 
-// 256 rows + tokens of the blocks that mlora_linear takes for a size
+// how mlora_linear takes a size: weight rows of a workgroup, its tokens and the stages of its ring, a byte each
 extern "C" int mlora_linear_block(int T, int K, int N) {
   const F32Form f = choose(T, K, N, false, ceil_div(T, FB), 1);
-  return f.fn * 16 * 256 + f.tb;
+  return f.fn << 20 | f.tb << 8 | f.nst;
 }
 
 extern "C" int mlora_linear(void* y, int y_dtype, int mode, const void* x, int ldx, const void* W, int T, int K, int N, void* stream) {
