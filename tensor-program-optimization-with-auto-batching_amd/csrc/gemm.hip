@@ -632,7 +632,7 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
       multiply(half, have);
     }
     // Both groups store together; half a stage apart each waited for the other's memory rounds: 4096 x 12288 x 4096 in bf16, three rounds
-    // of blocks, with a gated product 290 -> 285 us, added to fp32 341 -> 338, 4096 x 4096 x 4096 added to fp32 110 -> 108.
+    // of blocks, with a gated product 290 -> 285 us; in fp16 added to fp32 379 -> 351, 4096 x 4096 x 4096 115 -> 112, 2800 x 256 x 9824 56 -> 48.
     if (wave < NW / 2) bare_barrier();
     if constexpr (SILU) {
       // acc[i] and acc[4 + i] are the gate and the up half of channels n0 + wn * 64 + i * 16 + 4 g .. + 3 for token r16 of
@@ -721,20 +721,17 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
       for (int j = 0; j < WTF; ++j) {
         const int t = t0 + tfrag(j) * 16 + r16;
         if (t >= T) continue;
-        const int n = n0 + wn * 128 + g * 4;           // of the first row tile; N is a multiple of 4 (checked)
-        float* p = (float*)yv + (size_t)t * N + n;
-        if constexpr (OUT == OUT_ACC_F32) {
-          // the eight values of a token are requested together: stored one by one they would be read one by one, a memory round each
-          f32x4 old[8];
+        // Added to fp32: each value is read right ahead of its store.  A token's eight requested together leave the compute unit's memory idle while
+        // they are added: fp16, 2800 x 256 x 9824 47.5 -> 51.6 us, 3450 x 512 x 4096 32.1 -> 34.6, 3571 x 2048 x 4096 63.2 -> 65.4, 3219 x 11008 x 4096 235 -> 232;
+        // only rows of 12288 gain by it (2338 x 1408 100.7 -> 102.7, but 4297 x 4096 434 -> 424).
 #pragma unroll
-          for (int i = 0; i < 8; ++i)
-            if (n + i * 16 < N) old[i] = *reinterpret_cast<const f32x4*>(p + i * 16);
-#pragma unroll
-          for (int i = 0; i < 8; ++i) acc[i][j] = old[i] + acc[i][j];
+        for (int i = 0; i < 8; ++i) {
+          const int n = n0 + (wn * 8 + i) * 16 + g * 4;        // N is a multiple of 4 (checked)
+          if (n >= N) continue;
+          f32x4* p = reinterpret_cast<f32x4*>((float*)yv + (size_t)t * N + n);
+          if constexpr (OUT == OUT_ACC_F32) *p = *p + acc[i][j];
+          else *p = acc[i][j];
         }
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-          if (n + i * 16 < N) *reinterpret_cast<f32x4*>(p + i * 16) = acc[i][j];
       }
     }
   }
