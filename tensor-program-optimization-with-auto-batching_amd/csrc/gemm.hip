@@ -1172,20 +1172,23 @@ extern "C" int mlora_gemm_frag_preferred(int T, int K, int N) {
 
 // The plain linear: the persistent kernel or the mid-size one.  The first takes whole rounds of one 256 x 256 block per compute unit: padding
 // and empty units cost as much as products.  So what is asked is T N / 2^16, the blocks' worth of products.  In one round more than half of
-// the chip: up to there the mid-size kernel has a round of its own largest blocks, of half that size.  Above one round what pays for the second;
-// less of it for small K, where the mid-size kernel's block ends weigh more.
+// the chip: up to there the mid-size kernel has a round of its own largest blocks, of half that size.  Above one round what pays for the second:
+// a whole first one and an eighth, less for small K, where the mid-size kernel's block ends weigh more - but not where results are added to fp32, since both
+// kernels' ends then wait for memory.
 // Measured, persistent / mid-size, us.  One round: 113 (1843 x 2304 x 4032) 46 / 37, 120 (640 x 4096 x 12288) 77 / 72, 126 (1500 x 1024 x 5504) 26 / 29,
 // 128 (2048 x 4096 x 4096) 77 / 63, 129 (1500 x 2048 x 5632) 41 / 47, 134 (400 x 4096 x 22016) 81 / 107, 141 (3000 x 2048 x 3072) 45 / 45, 144 (768 x 4096 x 12288)
 // 78 / 86, 156 (2500 x 4096 x 4096) 78 / 93, 172 (512 x 4096 x 22016) 82 / 112.  Two, K from 1280 on: 190 (548 x 3264 x 22704) 122 / 105, 258 (3000 x 2048 x 5632)
 // 82 / 76, 258 (768 x 4096 x 22016) 152 / 152, 281 (1500 x 4096 x 12288) 155 / 147, 302 (900 x 4096 x 22016) 161 / 183, 394 (900 x 4096 x 28672) 173 / 231; below:
-// 235 (3123 x 1024 x 4928) 46 / 43, 252 (3000 x 1024 x 5504) 48 / 54, 274 (815 x 384 x 22032) 26 / 35, 290 (643 x 320 x 29560) 24 / 32.  Over 142 sizes of
-// 90 to 420 blocks the choice takes 0.5 % longer than the better one on average, 21 % at most (448 x 5504 x 37128 216 / 261).  Up to 128 tokens half of
-// its work is padding.
-static bool persistent_pays(int T, int K, int N) {
+// 235 (3123 x 1024 x 4928) 46 / 43, 251 (1515 x 1024 x 10864) 46 / 44, 252 (2549 x 256 x 6504) 21 / 21, 274 (815 x 384 x 22032) 26 / 35, 290 (643 x 320 x 29560)
+// 24 / 32.  Added to: 262 (2281 x 64 x 7520) 39 / 30, 272 (904 x 384 x 19904) 50 / 50, 277 (1268 x 512 x 14296) 55 / 52, 288 (3072 x 2752 x 6136) 134 / 123, 297
+// (3725 x 384 x 5224) 50 / 54, 298 (1451 x 1024 x 13464) 75 / 78, 301 (1492 x 192 x 13216) 44 / 40, 317 (1515 x 2048 x 13720) 115 / 118.  Over 280 sizes of
+// 60 to 560 blocks the choice takes 1.3 % longer than the better one on average, 33 % at most (247 x 256 x 33752, just below half a round, 12 / 17).  Up to
+// 128 tokens half of its work is padding.
+static bool persistent_pays(int T, int K, int N, bool accumulate) {
   const long cu = gemm_n_cu() > 0 ? gemm_n_cu() : 256, nb = (long)ceil_div(T, PP_F * 16) * ceil_div(N, PP_F * 16);
   if (K % 64 || T <= 128) return false;
   const long block = PP_F * 16 * PP_F * 16;
-  return nb <= cu ? (long)T * N * 2 > cu * block : (long)T * N * 32 >= cu * (K >= 1280 ? 36 : 31) * block;
+  return nb <= cu ? (long)T * N * 2 > cu * block : (long)T * N * 32 >= cu * (accumulate ? 37 : K >= 1280 ? 36 : 32) * block;
 }
 
 extern "C" int mlora_linear_frag(void* y, int y_dtype, int mode, const void* xf, const void* Wp, int T, int K, int N,
@@ -1199,7 +1202,7 @@ extern "C" int mlora_linear_frag(void* y, int y_dtype, int mode, const void* xf,
   const elt* W = (const elt*)Wp;
   const int tt = mlora_frag_tiles(T);
   int e;
-  if (persistent_pays(T, K, N)) {
+  if (persistent_pays(T, K, N, mode == MLORA_ACCUMULATE)) {
     if (mode == MLORA_ACCUMULATE) e = launch_gemm_pp<OUT_ACC_F32>(y, x, 0, tt, W, T, K, N, s);
     else if (y_dtype == MLORA_F32) e = launch_gemm_pp<OUT_F32>(y, x, 0, tt, W, T, K, N, s);
     else e = launch_gemm_pp<OUT_F16>(y, x, 0, tt, W, T, K, N, s);

@@ -1570,14 +1570,19 @@ def test_silu_product_over_every_gate(ops, dt):
     assert bool((got[lost] == 0).all()) and not bool(bad.any()), (int(bad.sum()), g[bad][:8], u[bad][:8], got[bad][:8], want[bad][:8])
 
 
-@pytest.mark.parametrize("T,N,K", [(256, 128 * 256, 192), (256, 128 * 256 + 8, 192), (256, 128 * 256, 2048), (256, 128 * 256 + 8, 2048), (641, 25352, 192),
-                                   (641, 25360, 192), (256, 287 * 256, 1280), (256, 288 * 256, 1280)])
+@pytest.mark.parametrize("T,N,K", [(256, 128 * 256, 192), (256, 128 * 256 + 8, 192), (256, 128 * 256, 2048), (256, 128 * 256 + 8, 2048), (641, 26168, 192),
+                                   (641, 26176, 192), (256, 287 * 256, 1280), (256, 288 * 256, 1280), (641, 30256, 192), (641, 30264, 192)])
 def test_linear_around_half_a_round_and_the_second_one(ops, T, N, K):
-    """Both sides of half a round of blocks, and of what pays for a second round: the bits of the kernel without LDS."""
+    """Both sides of half a round of blocks, and of what pays for a second round, stored and added to fp32: the bits of the kernel without LDS."""
     g = torch.Generator(device=DEV).manual_seed(T + N)
     x = torch.randn((T, K), generator=g, device=DEV).half()
     W = ops.PackedWeight((torch.randn((N, K), generator=g, device=DEV) * 0.05).half())
-    assert torch.equal(ops.linear(ops.FragActivation.pack(x), W), ops.linear(x, W.unpack(), kernel="gemm"))
+    f, w = ops.FragActivation.pack(x), W.unpack()
+    assert torch.equal(ops.linear(f, W), ops.linear(x, w, kernel="gemm"))
+    r, q = (torch.ones((T, N), device=DEV) for _ in range(2))
+    ops.linear(f, W, out=r, accumulate=True)
+    ops.linear(x, w, out=q, accumulate=True, kernel="gemm")
+    assert torch.equal(r, q)
 
 
 @pytest.mark.parametrize("T", [65, 256, 257, 700, 1024])
