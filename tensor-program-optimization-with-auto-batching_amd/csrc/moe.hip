@@ -328,6 +328,10 @@ extern "C" int mlora_moe_combine(float* x, const float* part, int n_part, const 
 // 2048, 2 entries 107 / 104, 6 127 / 123, 12 142 / 129, 16 161 / 144, 32 experts of 2752 x 4096, 6 245 / 251, 10 253 / 261, 12 266 / 258, 16 321 / 306;
 // down, 2048 x 1408, 4 63 / 64, 8 72 / 69, 12 83 / 71, 16 93 / 77, 4096 x 2752, 8 130 / 129, 12 147 / 134, 16 169 / 147; up without a gate,
 // 1408 x 2048, whose 1408 workgroups fill the last round badly, 4 61 / 70, 12 69 / 74, 16 80 / 81, 2752 x 4096, 8 131 / 132, 12 143 / 137, 16 166 / 160.
+// Between those widths and around the limits: down, 96 experts of 4096 x 2048, 8 249 / 265, 64 of 2752 x 2048, 12 123 / 127, 13 137 / 128, 128 of 4096 x 1536, 12 330 / 277,
+// 96 of 4096 x 1408, 9 212 / 193; gated, 64 of 2048 x 3584, 12 333 / 308; few workgroups, 8 of 256 x 4096, 14 8.2 / 9.6, 16 of 512 x 5632, 13 30 / 23, 48 of 512 x 4096, 13
+// 47 / 44.  Over 260 sizes of 8 to 128 experts, 512 to 5632 x 256 to 4096, four tiles where this says so take 0.61 to 1.04 of the time of two, and 1.10 in one (48 of 768 x
+// 5632, 16 97 / 107); below 8 workgroups a compute unit they often pay as well (96 of 256 x 512, gated, 14 19 / 13), and the line is drawn where they are never the worse choice.
 static bool moe_gemv_wide(int T, int K, int N, int top, int max_tiles, int act) {
   static const int n_cu = [] {
     int dev = 0, cu = 0;
@@ -336,8 +340,10 @@ static bool moe_gemv_wide(int T, int K, int N, int top, int max_tiles, int act) 
   }();
   const bool gated = act == MLORA_ACT_GLU;
   const long n = (long)T * top, E = max_tiles - n / 16 > 0 ? max_tiles - n / 16 : 1;      // (what the number of tiles was made of)
-  const bool many = ceil_div(N, gated ? 32 : 64) * E >= 8L * n_cu;
-  return (many && K <= 2048 && (gated || n >= 8 * E)) || ((many || K >= 4096) && n >= 11 * E);
+  const long groups = ceil_div(N, gated ? 32 : 64) * E;
+  const bool many = groups >= 8L * n_cu;
+  if (many && (gated ? K <= 2048 : K < 2048 && n >= 8 * E)) return true;
+  return (many || (K >= 4096 && 2 * groups >= n_cu)) && n >= (gated ? 11 : 12) * E;
 }
 
 extern "C" int mlora_moe_linear(void* y, const void* x, const void* W, const int32_t* perm, const int32_t* tiles, const int32_t* n_tiles,
