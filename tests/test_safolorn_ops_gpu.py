@@ -507,6 +507,46 @@ def test_experts_of_a_few_entries_with_four_row_tiles(D, glu, top, ff, N):
         assert (np.abs(got[t, j] - want) <= 2.0 ** -8 * (room @ np.abs(Dn[e]).T + np.abs(want)) + 1e-6).all(), e
 
 
+@pytest.mark.parametrize("E,T,top,K,N,stage", [(128, 64, 4, 1056, 528, "gated"), (128, 64, 2, 2048, 560, "gated"), (128, 300, 4, 1056, 1040, "down"),
+                                               (128, 300, 4, 544, 1072, "up"), (16, 100, 2, 4128, 528, "down"), (16, 100, 2, 4128, 528, "up"),
+                                               (64, 300, 3, 2080, 2064, "gated")])
+def test_experts_with_four_row_tiles_over_many_steps(D, E, T, top, K, N, stage):
+    """Four row tiles per workgroup with two to seventeen steps of 32 k in a wave, not the same number in each, and rows that end in one, two or three of
+    a workgroup's tiles.  fp32 sums of exact products: K + 8 roundings of 2^-24 on what is added up; then one rounding to bf16 (2^-8 of a
+    place's size), of gate and up beforehand as well, |silu| and |silu'| being at most |g| and 1.1."""
+    dt = torch.bfloat16
+    g = torch.Generator(device=DEV).manual_seed(K + N)
+    rand = lambda *sh: torch.randn(*sh, generator=g, device=DEV)
+    pick = torch.argsort(rand(T, E), -1)[:, :top].to(torch.int32).contiguous()
+    plan = D.MoePlan(pick, E, dt)
+    assert plan.tile_rows == 16
+    rows = 2 * N if stage == "gated" else N
+    W = (rand(E, rows, K) * K ** -0.5).to(dt)
+    x = rand(plan.places if stage == "down" else T, K).to(dt)
+    act = {"gated": D.ACT_GLU, "up": D.ACT_RELU2, "down": D.ACT_NONE}[stage]
+    y = D.moe_linear(x, D.weight(W.view(-1, K)), plan, N, K, D.MOE_DOWN if stage == "down" else D.MOE_UP, act)
+    torch.cuda.synchronize()
+    perm, u, eps = plan.perm.long(), 2.0 ** -8, (K + 8) * 2.0 ** -24
+    places = (perm[:int(plan.n_tiles[1])] >= 0).nonzero().view(-1)
+    of = pick.view(-1)[perm[places]]
+    for e in range(E):
+        at = places[of == e]
+        if at.numel() == 0:
+            continue
+        src, w = (x[at] if stage == "down" else x[perm[at] // top]).double(), W[e].double()
+        v, err = src @ w.T, eps * (src.abs() @ w.abs().T)
+        if stage == "gated":
+            v, err = [v[:, :N], v[:, N:]], [err[:, :N] + u * v[:, :N].abs(), err[:, N:] + u * v[:, N:].abs()]
+            want = v[0] * torch.sigmoid(v[0]) * v[1]
+            bound = 1.1 * err[0] * (v[1].abs() + err[1]) + v[0].abs() * err[1]
+        elif stage == "up":
+            want, bound = v.clamp(min=0) ** 2, 2 * v.abs() * err + err ** 2
+        else:
+            want, bound = v, err
+        got = (y[perm[at]] if stage == "down" else y[at]).double()
+        assert bool(((got - want).abs() <= (1 + u) * bound + u * want.abs() + 2.0 ** -30).all()), e
+
+
 @pytest.mark.parametrize("T,K,N", [(17, 2048, 64), (33, 1040, 100), (100, 2048, 36), (299, 512, 128), (70, 16, 4100), (70, 48, 4100), (130, 80, 8200), (65, 144, 2052),
                                    (300, 2064, 2052), (299, 208, 20004)])
 @pytest.mark.parametrize("shift", [0, 1])
