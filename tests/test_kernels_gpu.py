@@ -4,6 +4,7 @@ Tolerance: max relative error 2e-3 against the fp32 oracle on the same fp16-roun
 (relative to max(|ref|, 1e-3 * max|ref|)); integer paths (adapter-index gather, scatter, page-table
 walk, argmax) bit-exact.
 """
+import ctypes
 import math
 
 import numpy as np
@@ -1130,8 +1131,54 @@ def test_gemv_ksplit_tiles_of_a_workgroup(ops, synth, T, N, ks):
     assert torch.equal(res[0][0], res[1][0]) and torch.equal(res[0][1], res[1][1])
     got = _np(res[0][0]).astype(np.float64) + _np(res[0][1]).reshape(ks - 1, T, N).astype(np.float64).sum(0)
     x64, w64 = _np(x).astype(np.float64), _np(W[:N]).astype(np.float64)
-    bound = (K + 16) * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64).T + np.abs(_np(r0[:, :N])))      # fp32 sums of exact products
+    bound = (K + 16) * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64).T + np.abs(_np(r0[:, :N])))      # fp32 sums of exact products: each of the K may round, as may the parts' sums (how an MFMA adds its 32 is not specified)
     assert (np.abs(got - (_np(r0[:, :N]).astype(np.float64) + x64 @ w64.T)) <= bound + 1e-30).all()
+
+
+@pytest.mark.parametrize("T", [5, 32, 64])
+@pytest.mark.parametrize("H,ks", [(512, 4), (1024, 4), (1536, 4), (4096, 3)])
+@pytest.mark.parametrize("r,n_ad", [(8, 3), (16, 5)])
+def test_gemv_ksplit_tiles_with_appended_rows_and_shrink_units(ops, synth, T, H, ks, r, n_ad):
+    """One, two and four row tiles per workgroup with adapter rows appended to the weight (24 and 80, which end inside a workgroup's tiles) and with
+    shrink units in the launch: the appended rows' own block and partial columns are x A^T; with units the result and its partials keep the bits of the
+    launch without them and the shrinks those of an unsplit launch of another width."""
+    L = load_pkg("_lib")
+    lib, K, n_ext = L.lib(), 4096, r * n_ad
+    x = synth.normal(32, f"ka.x.{T}", (T, K), 1.0, torch.float16, DEV)
+    W = synth.normal(32, "ka.W", (4096, K), 0.02, torch.float16, DEV)
+    A = synth.normal(32, f"ka.A.{r}", (n_ad, r, K), 0.02, torch.float16, DEV)
+    r0 = synth.normal(32, f"ka.r.{T}", (T, 4096), 1.0, torch.float32, DEV)
+    ids = synth.randint(32, f"ka.ids.{T}", (T,), n_ad, DEV)
+    ids[1] = -1
+    xf, st = ops.FragActivation.pack(x), torch.cuda.current_stream().cuda_stream
+    Ap = (ctypes.c_void_p * 1)(A.data_ptr())
+
+    def launch(h, k, rows=0, units=False):
+        Wp = ops.PackedWeight(torch.cat([W[:h], A.view(n_ext, K)[:rows]], 0))
+        y, y2, v = r0[:, :h].contiguous(), None, None
+        part = torch.full((max(k - 1, 1) * T, h + rows), float("nan"), device=DEV)
+        if rows:
+            y2 = torch.full((T, rows), float("nan"), device=DEV)
+        if units:
+            v = torch.zeros(lib.mlora_gather_mm_workspace_bytes(T, K, r) // 4, device=DEV)
+        L.check(lib.mlora_gemv_frag_acc_ksplit(y.data_ptr(), y2.data_ptr() if rows else None, part.data_ptr(), k, xf.data.data_ptr(), Wp.data.data_ptr(), T, K, h,
+                                               rows, v.data_ptr() if units else None, Ap if units else None, int(units), ids.data_ptr() if units else None,
+                                               r if units else 0, n_ad if units else 0, st))
+        torch.cuda.synchronize()
+        return y, part.view(-1, T, h + rows), y2, v
+
+    plain, rows, units = launch(H, ks), launch(H, ks, rows=n_ext), launch(H, ks, units=True)
+    assert torch.equal(plain[0], rows[0]) and torch.equal(plain[1], rows[1][:, :, :H])
+    assert torch.equal(plain[0], units[0]) and torch.equal(plain[1], units[1])
+    assert torch.equal(units[3], launch(4096 if H < 4096 else 512, 1, units=True)[3])
+    x64, a64 = x.double(), A.view(n_ext, K).double()
+    got = rows[2].double() + rows[1][:, :, H:].double().sum(0)
+    assert bool(((got - x64 @ a64.T).abs() <= (K + 16) * 2.0 ** -24 * (x64.abs() @ a64.abs().T)).all())       # fp32 sums of exact products
+    shr = units[3][:units[3].numel() // (T * r) * T * r].view(-1, T, r).double().sum(0)
+    for t in range(T):
+        if int(ids[t]) >= 0:
+            a = A[int(ids[t])].double()
+            assert bool(((shr[t] - a @ x64[t]).abs() <= (K + 16) * 2.0 ** -24 * (a.abs() @ x64[t].abs())).all()), t
 
 
 @pytest.mark.parametrize("T,K,r,n_ad", [(32, 4096, 16, 16), (20, 11008, 8, 4), (48, 4096, 16, 16), (64, 2048, 32, 6)])

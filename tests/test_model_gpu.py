@@ -390,7 +390,8 @@ def test_prefill_pass_with_fused_and_separate_lora_blocks(monkeypatch):
     """A prefill pass in which some 256-token blocks agree on one adapter (their deltas ride in the base GEMMs as extra
     k-steps) and others straddle two sequences with different adapters or hold tokens without adapter (the separate
     gather-matmul serves those tokens): the same pass with every delta through the separate call gives the same logits
-    up to where the sum is rounded, and the same greedy tokens wherever the margin decides."""
+    up to where the sum is rounded, and the same greedy tokens wherever the margin decides.  The entry point that knows the ids on the
+    host gives the bits of the pass that has them on the device only, without asking the device."""
     synth, llama, ops = load_pkg("synth"), load_pkg("llama"), load_pkg("ops")
     shape = synth.LlamaShape(hidden_size=1024, intermediate_size=1024, num_attention_heads=8, num_key_value_heads=8,
                              num_hidden_layers=1, head_dim=128, vocab_size=512)
@@ -428,6 +429,17 @@ def test_prefill_pass_with_fused_and_separate_lora_blocks(monkeypatch):
     monkeypatch.setattr(ops, "linear_frag_lora", spy)
     got, kv_f = run()
     assert calls["fused"] >= 3                               # qkv, o and down at least took the fused entry
+    asked = []
+    real_blocks = ops.lora_block_adapters
+    monkeypatch.setattr(ops, "lora_block_adapters", lambda *a: asked.append(a) or real_blocks(*a))
+    kv_h = model.create_paged_kv_cache(B, T + 16 * B, T, 16)
+    for s_ in range(B):
+        kv_h.add_sequence(s_)
+    kv_h.begin_forward(list(range(B)), lens)
+    by_host, _ = model["prefill_a0"](model.embed(tokens), kv_h, seq_ad)
+    kv_h.end_forward()
+    assert not asked and np.array_equal(by_host.float().cpu().numpy(), got)
+    assert torch.equal(kv_h.k, kv_f.k) and torch.equal(kv_h.v, kv_f.v)
     # the same pass with no block taking the extra k-steps: every delta through the separate gather-matmul
     monkeypatch.setattr(ops, "lora_block_adapters",
                         lambda ids, n_ad: (torch.full((-(-ids.numel() // 256),), -1, dtype=torch.int32, device=ids.device), ids.clone()))
