@@ -620,7 +620,7 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_pp_kernel(void* __rest
     // While ordinary k-steps of one block are fetched and multiplied nothing is tested; the last stages of a block and those of a
     // delta take the general form.
     int kb = KB - 1 - load_kb;
-    kb = kb < 0 ? 0 : kb < KB ? kb : KB;
+    kb = kb < 0 ? 0 : kb;
     if (wave >= NW / 2) bare_barrier();        // the second group: half a stage behind the first
     for (int left = kb; left > 0; --left) {
       fetch(std::true_type());
@@ -1164,8 +1164,10 @@ extern "C" int mlora_linear_packed(void* y, int y_dtype, int mode, const void* x
 
 extern "C" int mlora_gemv_frag(void* y, int y_dtype, int mode, const void* xf, const void* Wp, int T, int K, int N, void* stream);
 
-// 256 x 256 output blocks: enough of them to give every compute unit one, and whole pairs of 32-k steps (the forms with an
-// epilogue of their own - a gated product, LoRA deltas - exist from there on)
+// 256 x 256 output blocks: enough of them to give every compute unit one (the forms with an epilogue of their own - a gated product, LoRA deltas -
+// exist from there on).  K in whole 64, here and wherever the persistent kernel is chosen: its ring walks single steps of 32 k, but an odd number of them
+// has been neither tested nor measured.  256 is the number of compute units; the plain linear is taken from half of that on (persistent_pays), these
+// forms have not been measured there.
 extern "C" int mlora_gemm_frag_preferred(int T, int K, int N) {
   return T > 64 && K > 0 && K % 64 == 0 && N > 0 && (long)ceil_div(T, PP_F * 16) * ceil_div(N, PP_F * 16) >= 256;
 }

@@ -140,7 +140,7 @@ __device__ __forceinline__ void f32_thin(const F32Linear& a, const MoePlan& plan
 template <int FN, int RT, int NST, bool DIRECT, int SUMS>
 __device__ __forceinline__ void f32_wide(const F32Linear& a, const MoePlan& plan, int grouped, const float* __restrict__ x, const float* __restrict__ W,
                                          float* __restrict__ y, int n0, int t0, int t1, f32x4* smem) {
-  constexpr int RW = FN / 4, SF = FN + RT, LF = 4 * SF, LQ = (LF + FW - 1) / FW;   // fragments: of 16 k, of a stage, per loading wave
+  constexpr int RW = FN / 4, SF = FN + RT, LF = 4 * SF, LQ = (LF + FW - 1) / FW;   // row tiles of a stage, requests for it (four rows x 64 k), of a wave
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
   // request f = wave + 8 q of a stage: four rows of weight tile or (behind those) token tile f / 4, 64 k each: whole lines.  (16 rows of 16 k a
   // request, as the lanes multiply them, are half lines: 16 x 2048 x 11264 25 -> 18 us, 299 x 5632 x 2048 125 -> 109, 192 entries over 64 experts of 2048 x

@@ -251,6 +251,7 @@ __device__ __forceinline__ void amax_merge(float& v, int& i, float ov, int oi) {
   }
 }
 
+#if !defined(MLORA_ELT_BF16) && !defined(MLORA_ELT_F32)      // the native decode step is fp16
 // The embedding of a row and its RMSNorm into fragment order: embed_kernel<float> and rmsnorm_kernel<float, VPT> in one launch, the same
 // sums in the same order (a decode step's first two launches; a launch is 2 to 3 us of a step, 100 us of four requests in two layers of 1024).
 template <int VPT>
@@ -299,6 +300,7 @@ __global__ __launch_bounds__(NORM_THREADS) void embed_rmsnorm_kernel(elt* __rest
     }
   }
 }
+#endif
 
 constexpr int AMAX_THREADS = 1024;   // one row per workgroup: many threads, few requests each
 // pos, ctx (or null): counters of the rows, which go on by one
@@ -601,6 +603,7 @@ extern "C" int mlora_argmax(int32_t* ids, const float* logits, int B, int V, voi
   return mlora_argmax_advance(ids, logits, B, V, nullptr, nullptr, stream);
 }
 
+#if !defined(MLORA_ELT_BF16) && !defined(MLORA_ELT_F32)
 // resid [T, H] = embedding of ids, y = its RMSNorm in fragment order, at most 64 rows
 int mlora_embed_rmsnorm(void* y, float* resid, const void* table, const int32_t* ids, int V, const void* w, float eps, int T, int H, void* stream) {
   MLORA_CHECK(y && resid && table && ids && w, MLORA_ERR_INVALID, "embed_rmsnorm: null pointer");
@@ -615,3 +618,4 @@ int mlora_embed_rmsnorm(void* y, float* resid, const void* table, const int32_t*
   else launch(embed_rmsnorm_kernel<4>);
   return mlora_launch_status("embed_rmsnorm");
 }
+#endif
