@@ -28,8 +28,8 @@ struct F32Linear {
 // The fp32 16 x 16 x 4 product takes one element per lane: a lane holds 4 consecutive k of its row, element e of the four
 // k-groups of 16 lanes is one MFMA (any order of k serves, as long as both operands have the same).
 //
-// At T x K x N = 299 x 2048 x 2048: 41 us (61 TFLOP/s), 4 x 2048 x 11264: 19 us (4.9 TB/s), 4096 x 2048 x 11264: 1667 us
-// (113 TFLOP/s).  The vector ALUs (64 x 64 blocks, both operands staged through LDS behind two barriers per 16 k): 122, 139 (one token),
+// At T x K x N = 299 x 2048 x 2048: 42 us (60 TFLOP/s), 4 x 2048 x 11264: 20 us (4.6 TB/s), 4096 x 2048 x 11264: 1626 us
+// (116 TFLOP/s).  The vector ALUs (64 x 64 blocks, both operands staged through LDS behind two barriers per 16 k): 122, 139 (one token),
 // 2415 us.
 
 // Adds the sums of the waves that share K, in their order, and stores.  red [KW][tiles][lane]: four rows n of a token; tile = row
@@ -135,7 +135,7 @@ __device__ __forceinline__ void f32_thin(const F32Linear& a, const MoePlan& plan
 // tokens, by what a workgroup takes in.  NST: a deep ring where a workgroup has a compute unit to itself, one of two stages where two
 // share it and their waits overlap.  DIRECT: operands are 16-byte aligned; others go through registers.  SUMS: of a wave for an output.  Four, by
 // element e, make eight with the two halves of K, as many as f32_thin has: the rounding of a sum does not depend on which form a size takes
-// (4 x 2048 x 11264, error against 64 bits 2.9e-7 here and there, 5.7e-7 with one).  They cost registers, not time (19.7 us both), but where
+// (4 x 2048 x 11264, error against 64 bits 2.9e-7 here and there, 5.7e-7 with one).  They cost registers, not time (20.3 us both), but where
 // four workgroups share a compute unit: one, for a K of one stage (4000 x 64 x 4096 32 us, with four 39), which f32_thin adds in two chains as well.
 template <int FN, int RT, int NST, bool DIRECT, int SUMS>
 __device__ __forceinline__ void f32_wide(const F32Linear& a, const MoePlan& plan, int grouped, const float* __restrict__ x, const float* __restrict__ W,
