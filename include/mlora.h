@@ -162,6 +162,12 @@ int mlora_gather_mm_multi_proj(void* y, int y_dtype, int ldy, const void* x, int
                                const int32_t* col_offset, const int32_t* n_cols,
                                const int32_t* tok_bucket, const int32_t* tok_adapter,
                                int T, int K, void* workspace, size_t workspace_bytes, void* stream);
+/* The same for 1..3 projections of one rank, table size and scaling whose tokens come in adapter segments (a prompt, or several behind
+ * each other), any T: on the matrix cores also up to 64 tokens.  Any order of tokens gives right results.  projs [n_proj]; workspace:
+ * n_proj times mlora_gather_mm_workspace_bytes.  Needs K % 32 == 0, n_cols % 16 == 0 and 16-byte aligned rows of y. */
+int mlora_gather_mm_segments(void* y, int y_dtype, int ldy, const void* x, int x_layout, const mlora_lora_bucket* projs, int n_proj,
+                             const int32_t* col_offset, const int32_t* n_cols, const int32_t* tok_adapter, int T, int K,
+                             void* workspace, size_t workspace_bytes, void* stream);
 int mlora_gather_mm_batch(const void* const* sets, int n_sets, int y_dtype, int ldy, int x_layout,
                           const int32_t* tok_adapter, float scaling,
                           int T, int K, int N, int r, int n_ad,

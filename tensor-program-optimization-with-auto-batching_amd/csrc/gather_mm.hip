@@ -1355,8 +1355,12 @@ static int gmm_segments(const SegProjs& pj, int y_dtype, int ldy, const f16* x, 
 }
 
 // the matrix-core kernels need 16-byte aligned rows of y and whole 16-column tiles
+static bool gmm_segments_serve(const void* y, int ldy, int x_layout, int K, int N) {
+  return (x_layout == MLORA_ROWMAJOR || x_layout == MLORA_FRAG) && K % 32 == 0 && N % 16 == 0 && ldy % 8 == 0 && (uintptr_t)y % 16 == 0;
+}
+// what takes them without being told that its tokens come in segments
 static bool gmm_segments_fit(const void* y, int ldy, int x_layout, int T, int K, int N) {
-  return (x_layout == MLORA_ROWMAJOR || x_layout == MLORA_FRAG) && T > 64 && K % 32 == 0 && N % 16 == 0 && ldy % 8 == 0 && (uintptr_t)y % 16 == 0;
+  return T > 64 && gmm_segments_serve(y, ldy, x_layout, K, N);
 }
 
 static int gather_mm_impl(void* y, int y_dtype, int ldy, const void* x, int x_layout, const void* A, const void* B,
@@ -1584,6 +1588,41 @@ extern "C" int mlora_gather_mm_multi_proj(void* y, int y_dtype, int ldy, const v
         return e;
     }
   return MLORA_OK;
+}
+
+// Up to 64 tokens that come in adapter segments - a short prompt or a few - on the matrix cores as well.  The one-launch kernel gives an
+// adapter one group of workgroups that work its tokens off one after the other, and ranks beyond its LDS take two kernels of one wave per
+// (adapter, slice), which read B and x again for every token.  Here a launch takes as long whatever the tokens share, a shrink and an expand of 5 to 8 us.
+// q, k and v of 4096 x 4096, us, before / here: one adapter, rank 8, 16 tokens 22.4 / 12.7; rank 16, 8 tokens 16.6 / 12.4, 41 tokens 61 / 12.5; rank 32, 64
+// tokens 920 / 13.0; rank 64, 24 tokens 496 / 15.9; four adapters, rank 16, 16 tokens 11.2 / 14.3, 64 tokens 28.5 / 12.2 (the caller's rule: llama.py).
+extern "C" int mlora_gather_mm_segments(void* y, int y_dtype, int ldy, const void* x, int x_layout, const mlora_lora_bucket* projs, int n_proj,
+                                        const int32_t* col_offset, const int32_t* n_cols, const int32_t* tok_adapter, int T, int K,
+                                        void* workspace, size_t workspace_bytes, void* stream) {
+  MLORA_CHECK(projs && n_proj >= 1 && n_proj <= SEG_MAX_PROJ, MLORA_ERR_INVALID, "gather_mm_segments: 1..%d projections (n_proj=%d)", SEG_MAX_PROJ, n_proj);
+  MLORA_CHECK(y && x && col_offset && n_cols && tok_adapter, MLORA_ERR_INVALID, "gather_mm_segments: null pointer");
+  MLORA_CHECK(y_dtype == MLORA_F16 || y_dtype == MLORA_F32, MLORA_ERR_INVALID, "gather_mm_segments: bad y_dtype %d", y_dtype);
+  const size_t esz = y_dtype == MLORA_F16 ? 2 : 4;
+  SegProjs pj = {};
+  pj.n = n_proj;
+  for (int p = 0; p < n_proj; ++p) {
+    const mlora_lora_bucket& bk = projs[p];
+    MLORA_CHECK(bk.A && bk.B, MLORA_ERR_INVALID, "gather_mm_segments: projection %d has a null table", p);
+    if (int e = check_lora_shape(T, K, n_cols[p], bk.r, bk.n_ad)) return e;
+    MLORA_CHECK(bk.r == projs[0].r && bk.n_ad == projs[0].n_ad && bk.scaling == projs[0].scaling, MLORA_ERR_UNSUPPORTED,
+                "gather_mm_segments: projections of one rank, table size and scaling (projection %d differs)", p);
+    MLORA_CHECK(col_offset[p] >= 0 && col_offset[p] + n_cols[p] <= ldy, MLORA_ERR_INVALID,
+                "gather_mm_segments: columns %d..%d of projection %d outside a row of %d", col_offset[p], col_offset[p] + n_cols[p], p, ldy);
+    void* yp = (char*)y + (size_t)col_offset[p] * esz;
+    MLORA_CHECK(gmm_segments_serve(yp, ldy, x_layout, K, n_cols[p]), MLORA_ERR_UNSUPPORTED,
+                "gather_mm_segments: need K %% 32 == 0, columns %% 16 == 0 and 16-byte aligned rows (K=%d N=%d ldy=%d)", K, n_cols[p], ldy);
+    pj.A[p] = (const f16*)bk.A; pj.B[p] = (const f16*)bk.B; pj.y[p] = yp; pj.N[p] = n_cols[p];
+  }
+  if (T == 0) return MLORA_OK;
+  MLORA_CHECK(workspace && workspace_bytes >= (size_t)n_proj * mlora_gather_mm_workspace_bytes(T, K, projs[0].r), MLORA_ERR_WORKSPACE,
+              "gather_mm_segments: workspace of %zu bytes given, %zu needed", workspace_bytes,
+              (size_t)n_proj * mlora_gather_mm_workspace_bytes(T, K, projs[0].r));
+  return gmm_segments(pj, y_dtype, ldy, (const f16*)x, x_layout, tok_adapter, projs[0].scaling, T, K, projs[0].r, projs[0].n_ad, (float*)workspace,
+                      BucketFilter{nullptr, 0}, (hipStream_t)stream);
 }
 
 extern "C" int mlora_lora_block_adapters(int32_t* blk_adapter, int32_t* tok_rest, const int32_t* tok_adapter, int T, int n_ad,

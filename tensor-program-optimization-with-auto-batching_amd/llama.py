@@ -250,9 +250,20 @@ class LlamaForCausalLM(CausalLM):
             self._ws = torch.empty(need, dtype=torch.float32, device=self.device)
         return self._ws
 
-    def _lora(self, y, x, l, proj, tok_adapter):
+    def _segments_pay(self, T, n_seq, tok_adapter):
+        """Whether the deltas of a prompt pass of up to 64 tokens go to the matrix cores, where a launch takes as long whatever the tokens
+        share; the one-launch kernel works an adapter's tokens off one after the other.  Three projections of 4096 x 4096, one adapter,
+        us, one launch / matrix cores: rank 8, 8 and 16 tokens 13.1 / 13.0, 22.4 / 12.7; 16, 4 and 8 tokens 11.2 / 12.3, 16.6 / 12.4; 32, 4
+        tokens 17.0 / 12.3; 64, 40 tokens 822 / 14.4; four adapters, rank 16, 16 and 40 tokens 11.2 / 14.3, 20.1 / 13.7; 64, 8 tokens 21.9 / 18.3."""
+        (tid, _), = tok_adapter.items()
+        return T * self.lora_types[tid].r >= 128 * n_seq
+
+    def _lora(self, y, x, l, proj, tok_adapter, segments=False):
         """y += delta for every adapter type that targets (l, proj); tok_adapter: {tid: ids [T] int32}, or the merged
-        form {"multi": (tok_bucket, tok_adapter)} in which a token names its adapter type and weight row."""
+        form {"multi": (tok_bucket, tok_adapter)} in which a token names its adapter type and weight row.  segments: one type, whose
+        deltas go to the matrix cores whatever T is."""
+        if segments:
+            return self._lora_group(y, x, l, ((proj, 0, y.shape[1]),), tok_adapter, True)
         if "multi" in tok_adapter:
             tb, ta = tok_adapter["multi"]
             buckets = []
@@ -273,9 +284,10 @@ class LlamaForCausalLM(CausalLM):
         """Does any loaded adapter type carry tables for one of these projections of layer l?"""
         return any(lt.tables.get((l, p)) is not None for lt in self.lora_types for p in projs)
 
-    def _lora_group(self, y, x, l, projs, tok_adapter):
+    def _lora_group(self, y, x, l, projs, tok_adapter, segments=False):
         """The deltas of projections that read the same x and own column ranges of one fused output row:
-        projs = ((name, first column, columns), ...).  Batches that mix adapter types issue one call for the group."""
+        projs = ((name, first column, columns), ...).  Batches that mix adapter types issue one call for the group.
+        segments: as for `_lora`."""
         if "multi" in tok_adapter:
             tb, ta = tok_adapter["multi"]
             live, offs, cols = [], [], []
@@ -296,6 +308,11 @@ class LlamaForCausalLM(CausalLM):
         lt = self.lora_types[tid]
         live = [(lt.tables.get((l, proj)), c0, n) for proj, c0, n in projs]
         live = [(tab, c0, n) for tab, c0, n in live if tab is not None]
+        if segments:
+            if live:
+                ops.gather_mm_segments(y, x, [tab for tab, _, _ in live], [c0 for _, c0, _ in live], [n for _, _, n in live], ids, lt.scaling,
+                                       self._workspace(x.shape[0], x.shape[1], lt.r))
+            return
         if len(live) >= 2:
             zeros = getattr(self, "_zero_bucket", None)
             if zeros is None or zeros.numel() < ids.numel():
@@ -338,14 +355,18 @@ class LlamaForCausalLM(CausalLM):
         resid = hidden
         # a decode step (one token per sequence, T <= 64) keeps its activations in fragment order
         dec_frag = T <= 64 and kv._cur is not None and kv._cur[2]
-        # so does every larger pass: the operand loads of the matrix-core linears are then plain copies (norm, attention
-        # and SiLU write the order the matrix cores read)
-        frag = dec_frag or (T > 64 and H % 32 == 0 and q_sz % 32 == 0 and I % 32 == 0)
+        # so does every other pass: the operand loads of the matrix-core linears are then plain copies (norm, attention
+        # and SiLU write the order the matrix cores read), and up to 64 tokens the GEMVs read 16 tokens of a k-step as one line, split K
+        # and share a weight fragment among up to 64 of them (41 tokens of the 7B shape, row-major / fragment order, us: q/k/v 48 / 20,
+        # gate/up 92 / 37, down 60 / 19)
+        frag = dec_frag or (T > 0 and H % 32 == 0 and q_sz % 32 == 0 and I % 32 == 0)
         is_decode = kv._cur is not None and bool(kv._cur[2])
         # a decode step (of any number of sequences) and a short prefill split K of the two narrow accumulating linears;
         # the RMSNorm that reads the residual next adds the partial results (the same kernels and slice counts as the
         # native decode step)
         ks_ws = self._ksplit_ws(T) if dec_frag or (frag and (T <= 256 or is_decode)) else None
+        segs = (T <= 64 and frag and not is_decode and kv._cur is not None and len(tok_adapter) == 1 and "multi" not in tok_adapter
+                and self._segments_pay(T, len(kv._cur[0]), tok_adapter))
         # a prefill-sized pass of one adapter type of rank 32 or 64: where a 256-token block agrees on one adapter its
         # deltas ride in the base GEMM as extra k-steps; `rest` names the tokens that still need the separate call
         # (a prefill pass only: where the ids are known on the device only, the choice needs a read-back, which a decode
@@ -377,7 +398,7 @@ class LlamaForCausalLM(CausalLM):
             if qkv is None:
                 qkv = ops.linear(xn, L["qkv"])
                 if tok_adapter:
-                    self._lora_group(qkv, xn, l, qkv_projs, tok_adapter)
+                    self._lora_group(qkv, xn, l, qkv_projs, tok_adapter, segs)
             # a decode step of more than 64 sequences of one adapter type: the o projection's shrink comes off the
             # attention launch in head shares and a launch of expand workgroups adds the deltas behind the base linear
             # (what the native step does for such a batch; same kernels, same order)
@@ -395,10 +416,11 @@ class LlamaForCausalLM(CausalLM):
                 else:
                     parts = self._linear_acc(attn, L["o"], resid, ks_ws, self._riding_rows(l, "o_proj", lora_tids, T, q_sz))
                     if tok_adapter:
-                        self._lora(resid, attn, l, "o_proj", tok_adapter)
+                        self._lora(resid, attn, l, "o_proj", tok_adapter, segs)
             xn = ops.rmsnorm(resid, L["ln2"], s.rms_norm_eps, frag=frag, parts=parts)
-            if dec_frag and I % 32 == 0 and not (tok_adapter and self._targets(l, "gate_proj", "up_proj")):
-                # decode step without an adapter on gate / up: the SiLU product is the epilogue of the GEMV (same bits)
+            if (dec_frag and I % 32 == 0 or T <= 64 and frag and hasattr(self, "_il_cache")) and not (tok_adapter and self._targets(l, "gate_proj", "up_proj")):
+                # decode step (or, where one has made that order of the weights, a short prompt) without an adapter on gate / up: the
+                # SiLU product is the epilogue of the GEMV (same bits)
                 act = ops.gate_up_silu(xn, self.interleaved_gate_up()[l])
             else:
                 gu_projs = (("gate_proj", 0, I), ("up_proj", I, I))
@@ -409,14 +431,14 @@ class LlamaForCausalLM(CausalLM):
                     if gu is None:
                         gu = ops.linear(xn, L["gate_up"])
                         if tok_adapter:
-                            self._lora_group(gu, xn, l, gu_projs, tok_adapter)
+                            self._lora_group(gu, xn, l, gu_projs, tok_adapter, segs)
                     act = ops.silu_mul(gu, frag=frag)
             if fuse and self._fused_linear(fuse, act, L["down"], l, (("down_proj", 0, H),), resid=resid) is not None:
                 parts = None
             else:
                 parts = self._linear_acc(act, L["down"], resid, ks_ws, self._riding_rows(l, "down_proj", lora_tids, T, I))
                 if tok_adapter:
-                    self._lora(resid, act, l, "down_proj", tok_adapter)
+                    self._lora(resid, act, l, "down_proj", tok_adapter, segs)
         if logits_rows is not None:
             if parts is not None:                         # pending K-slice partials of the last down_proj, in slice order
                 pv = parts.part[: (parts.ks - 1) * T * parts.ld].view(parts.ks - 1, T, parts.ld)

@@ -245,6 +245,26 @@ def gather_mm_multi_proj(y, x, proj_buckets, col_offsets, n_cols, tok_bucket, to
     return y
 
 
+def gather_mm_segments(y, x, tables, col_offsets, n_cols, tok_adapter, scaling: float, workspace):
+    """gather_mm for one to three projections ((A, B) in `tables`, of one rank and table size) that read the same x and own column ranges
+    of y, where the tokens come in adapter segments: a prompt, or several behind each other.  On the matrix cores whatever T is."""
+    xptr, xlay, T, K = _x_arg(x)
+    n_ad, r, _ = tables[0][0].shape
+    if y.shape[0] != T or tok_adapter.shape != (T,) or len(col_offsets) != len(tables) or len(n_cols) != len(tables) \
+            or any(A.shape != (n_ad, r, K) or B.shape != (n_ad, n, r) for (A, B), n in zip(tables, n_cols)):
+        raise ValueError("gather_mm_segments: inconsistent shapes")
+    if not y.is_cuda or y.stride(1) != 1:
+        raise ValueError("gather_mm_segments: y must be a GPU tensor with unit inner stride")
+    if T == 0:
+        return y
+    arr = b"".join(_bucket(_dev(A, torch.float16, "A"), _dev(B, torch.float16, "B"), r, n_ad, scaling) for A, B in tables)
+    ldy = y.stride(0) if T > 1 else max(y.shape[1], y.stride(0))
+    co, nc = (struct.pack(f"{len(tables)}i", *v) for v in (col_offsets, n_cols))
+    check(lib().mlora_gather_mm_segments(y.data_ptr(), _dt(y), ldy, xptr, xlay, arr, len(tables), co, nc, _dev(tok_adapter, torch.int32, "tok_adapter"),
+                                         T, K, _dev(workspace, torch.float32, "workspace"), workspace.numel() * 4, _stream()))
+    return y
+
+
 class GatherMMBatch:
     """Several gather-matmul problems of one shape and one token->adapter table, issued as one launch.
     sets: list of (y, x, A, B) as for gather_mm (x row-major); the tensors are kept alive by this object."""

@@ -1642,3 +1642,38 @@ def test_block_adapters_on_the_host(ops, T, pattern):
     want_blk, want_rest = (t.cpu().numpy() for t in ops.lora_block_adapters(torch.from_numpy(ids).to(DEV), 5))
     assert np.array_equal(blk, want_blk)
     assert (rest is None and (want_rest < 0).all()) or np.array_equal(rest, want_rest)
+
+
+@pytest.mark.parametrize("T,segs", [(1, 1), (5, 2), (15, 1), (16, 3), (17, 17), (41, 1), (64, 4), (64, 64)])
+@pytest.mark.parametrize("r", [8, 16, 32, 64])
+@pytest.mark.parametrize("y32", [False, True])
+def test_gather_mm_segments_of_few_tokens(ops, T, segs, r, y32):
+    """Deltas of up to 64 tokens on the matrix cores: whole and partial tiles of one to sixteen adapters, tokens without one, x in both layouts, two
+    projections into column ranges of one row; nothing else of y is touched."""
+    K, cols, n_ad = 1056, (64, 272), 70
+    g = torch.Generator(device=DEV).manual_seed(T * 64 + r)
+    rnd = lambda *shape, std=1.0: torch.randn(shape, generator=g, device=DEV) * std
+    x, tabs = rnd(T, K).half(), [(rnd(n_ad, r, K, std=0.05).half(), rnd(n_ad, n, r, std=0.05).half()) for n in cols]
+    ids = torch.arange(T, device=DEV, dtype=torch.int32) * segs // T * 3 % n_ad
+    if T > 4:
+        ids[3] = -1
+    dt = torch.float32 if y32 else torch.float16
+    y0 = torch.cat([rnd(T, 32), rnd(T, cols[0]), rnd(T, 16), rnd(T, cols[1]), rnd(T, 24)], 1).to(dt)
+    offs = [32, 48 + cols[0]]
+    ws = torch.full((2 * 8 * T * r,), float("nan"), device=DEV)
+    got = [ops.gather_mm_segments(y0.clone(), xx, tabs, offs, cols, ids, 0.5, ws) for xx in (x, ops.FragActivation.pack(x))]
+    torch.cuda.synchronize()
+    want, room = y0.double(), torch.zeros(y0.shape, dtype=torch.float64, device=DEV)
+    live = ids >= 0
+    for (A, B), c, n in zip(tabs, offs, cols):
+        a, b = A[ids.clamp(min=0)].double(), B[ids.clamp(min=0)].double()
+        v, vm = ((t * live[:, None, None]).squeeze(2) for t in (torch.matmul(a, x.double()[:, :, None]), torch.matmul(a.abs(), x.double().abs()[:, :, None])))
+        want[:, c:c + n] += 0.5 * torch.matmul(b, v[:, :, None])[:, :, 0]
+        # v: K products and up to eight ranges of them, each of which may round; its halves: 2^-22 of it (and fp16's smallest step); the r products of them
+        room[:, c:c + n] += 0.5 * torch.matmul(b.abs(), ((K + 16) * 2.0 ** -24 * vm + 2.0 ** -22 * vm + 2.0 ** -24)[:, :, None])[:, :, 0] \
+            + (2 * r + 4) * 2.0 ** -24 * 0.5 * torch.matmul(b.abs(), vm[:, :, None])[:, :, 0]
+    room += (2.0 ** -24 if y32 else 2.0 ** -11) * (want.abs() + room)
+    for y in got:
+        assert bool(((y.double() - want).abs() <= room).all())
+        assert torch.equal(y[~live], y0[~live]) and torch.equal(y[:, :32], y0[:, :32]) and torch.equal(y[:, -24:], y0[:, -24:])
+        assert torch.equal(y[:, 32 + cols[0]:offs[1]], y0[:, 32 + cols[0]:offs[1]])
