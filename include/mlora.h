@@ -579,6 +579,41 @@ typedef struct mlora_decode_plan {
 
 int mlora_decode_step(const mlora_decode_plan* plan, void* stream);
 
+/* A prompt pass (sequences of any length behind each other) enqueued by one call: what decode_step is to a step.  Tokens, caches, block table and
+ * adapters as there; resid f32 [T, hidden] holds the embedded tokens and is left as the residual stream; logits f32 [n_rows, vocab] of the tokens
+ * logits_rows [n_rows] (int64).  tok_adapter: NULL without adapters.  blk_adapter, tok_rest (mlora_lora_block_adapters): the deltas of ranks 32
+ * and 64 as extra k-steps of the GEMMs where a block agrees on an adapter; tok_rest NULL: no token is left over.  segments: the deltas
+ * otherwise go to mlora_gather_mm_segments (any T) instead of mlora_gather_mm.  Needs hidden, inter and n_q_heads * head_dim in whole 32.
+ * ws: mlora_prefill_workspace_bytes(plan) bytes (0 for a plan that is refused), 256-byte aligned.
+ * Replaces: the batched forward of llama_for_causal_lm.py:79-100,121-144 as the host drives it operator by operator. */
+typedef struct mlora_prefill_plan {
+  int n_layers, hidden, inter, n_q_heads, n_kv_heads, head_dim, vocab;
+  float eps;
+  int lora_r, lora_n_ad;
+  float lora_scaling;
+  int segments;
+  const mlora_layer* layers;  /* gate_up_il_p: optional, used up to 64 tokens */
+  const void* norm;
+  const void* lm_head_p;
+  const float* rope_cos;
+  const float* rope_sin;
+  const int32_t* block_table;
+  const int32_t* tok_seq;
+  const int32_t* tok_pos;
+  const int32_t* tok_adapter;
+  const int32_t* blk_adapter;
+  const int32_t* tok_rest;
+  const void* logits_rows;
+  float* resid;
+  float* logits;
+  void* ws;
+  size_t ws_bytes;
+  int max_pos, max_blocks, n_pages, n_seq, T, n_rows;
+} mlora_prefill_plan;
+
+size_t mlora_prefill_workspace_bytes(const mlora_prefill_plan* plan);
+int mlora_prefill(const mlora_prefill_plan* plan, void* stream);
+
 /* act = clipped gated product of [gate | up] = xf . Wp^T: with g = min(scale gate, limit), u = clamp(scale up, +-limit),
  * g sigmoid(alpha g) (u + 1).  The forms of mlora_gemv_frag_silu (interleaved tiles, T <= 64), mlora_linear_frag_silu
  * (persistent GEMM shapes) and mlora_silu_mul. */

@@ -119,6 +119,18 @@ class DecodePlan(C.Structure):
 SIGNATURES["mlora_decode_step"] = (_i, [C.POINTER(DecodePlan), _p])
 
 
+class PrefillPass(C.Structure):
+    _fields_ = [("n_layers", _i), ("hidden", _i), ("inter", _i), ("n_q_heads", _i), ("n_kv_heads", _i), ("head_dim", _i), ("vocab", _i), ("eps", _f),
+                ("lora_r", _i), ("lora_n_ad", _i), ("lora_scaling", _f), ("segments", _i), ("layers", _p), ("norm", _p), ("lm_head_p", _p),
+                ("rope_cos", _p), ("rope_sin", _p), ("block_table", _p), ("tok_seq", _p), ("tok_pos", _p), ("tok_adapter", _p), ("blk_adapter", _p),
+                ("tok_rest", _p), ("logits_rows", _p), ("resid", _p), ("logits", _p), ("ws", _p), ("ws_bytes", _z),
+                ("max_pos", _i), ("max_blocks", _i), ("n_pages", _i), ("n_seq", _i), ("T", _i), ("n_rows", _i)]
+
+
+SIGNATURES["mlora_prefill_workspace_bytes"] = (_z, [C.POINTER(PrefillPass)])
+SIGNATURES["mlora_prefill"] = (_i, [C.POINTER(PrefillPass), _p])
+
+
 class TanhNorm(C.Structure):
     _fields_ = [("w", _p), ("b", _p), ("alpha", _f)]
 

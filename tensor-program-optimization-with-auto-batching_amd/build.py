@@ -15,7 +15,7 @@ from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
-SOURCES = ["api.hip", "gather_mm.hip", "gather_mm_batch.hip", "gemv.hip", "gemm.hip", "rowops.hip", "attention.hip", "decode_step.hip"]
+SOURCES = ["api.hip", "gather_mm.hip", "gather_mm_batch.hip", "gemv.hip", "gemm.hip", "rowops.hip", "attention.hip", "decode_step.hip", "prefill.hip"]
 DECODER_SOURCES = ["stream_ops.hip", "latent_attention.hip", "time_mix.hip", "moe.hip"]
 LIBS = {   # element type -> (library, sources, suffix of the objects, extra flags)
     "float16": (os.path.join(HERE, "libmlora_hip.so"), SOURCES, "", []),

@@ -461,3 +461,45 @@ def test_prefill_pass_with_fused_and_separate_lora_blocks(monkeypatch):
     adapted_rows = seq_ad >= 0
     assert np.abs(none - want)[adapted_rows].max() / std > 5e-2
     assert np.abs(none - want)[~adapted_rows].max() / std <= 1e-2
+
+
+ALL_LINEARS = ("q_proj", "k_proj", "v_proj", "o_proj", "gate_proj", "up_proj", "down_proj")
+
+
+@pytest.mark.parametrize("lens,r,targets", [([1, 2], 8, ("q_proj", "v_proj")), ([5], 16, ("q_proj", "k_proj", "v_proj", "o_proj")), ([41], 64, ALL_LINEARS),
+                                            ([30, 34], 32, ALL_LINEARS), ([9, 1, 55], 16, ALL_LINEARS), ([137], 16, ("o_proj", "down_proj")), ([100, 157], 32, ALL_LINEARS), ([700], 8, ALL_LINEARS),
+                                            ([256 * 64], 32, ALL_LINEARS), ([8000, 8384], 64, ALL_LINEARS), ([40], 0, ()), ([300], 0, ())])
+@pytest.mark.parametrize("decoded", [False, True])
+def test_prompt_pass_in_one_call(lens, r, targets, decoded):
+    """prefill_a0 / prefill_no_adapter queue the pass natively: logits, cache and residual stream have the bits of the per-operator path, with and
+    without the interleaved gate / up weights that a decode session leaves, for ranks and sizes on every path of an adapter's delta."""
+    synth, llama, ops = load_pkg("synth"), load_pkg("llama"), load_pkg("ops")
+    print(f"case prompt pass {lens} r={r}", flush=True)
+    shape = synth.LlamaShape(hidden_size=1024, intermediate_size=1056, num_attention_heads=8, num_key_value_heads=4, num_hidden_layers=2, head_dim=128, vocab_size=520)
+    specs = [synth.LoraSpec(r=r, alpha=2.0 * r, n_adapters=3, targets=targets)] if r else []
+    model = llama.LlamaForCausalLM.from_synthetic(17, shape, specs, DEV)
+    if decoded:
+        model.interleaved_gate_up()
+    B, T = len(lens), sum(lens)
+    wids = np.array([2, -1, 0][:B], np.int32)
+    tokens = synth.randint(3, "one.call", (T,), shape.vocab_size)
+    got = []
+    for native in (True, False):
+        kv = model.create_paged_kv_cache(B, T + 16 * B, T, 16)
+        for s_ in range(B):
+            kv.add_sequence(s_)
+        kv.begin_forward(list(range(B)), lens)
+        h = model.embed(tokens)
+        if native:
+            assert model._native_prefill_serves(h, kv)
+            logits, _ = model["prefill_a0"](h, kv, wids) if r else model["prefill_no_adapter"](h, kv)
+        else:
+            ids = {0: np.repeat(wids, lens)}
+            last = torch.from_numpy(np.cumsum(lens) - 1).to(DEV)
+            logits = model.forward(h, kv, {t: torch.from_numpy(a).to(DEV) for t, a in ids.items()} if r else None, last, ids if r else None)
+        kv.end_forward()
+        got.append((logits, kv.k, kv.v, h))
+    torch.cuda.synchronize()
+    assert bool(torch.isfinite(got[0][0]).all())
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
