@@ -395,89 +395,118 @@ struct LatentExpand {
   int kb_blocks, vb_blocks; // workgroups along x that make keys, then values; one more copies R
 };
 
-// A wave makes 16 LE_ROWS rows (of W_uk or W_uv) x 4 pages; the two halves of a workgroup take the same rows for neighbouring
-// pages, so that a weight fragment crosses from the second-level cache once for both.
-constexpr int LE_ROWS = 4;
-__global__ __launch_bounds__(512, 3) void latent_expand_kernel(LatentExpand a) {
+// A workgroup makes 128 rows (of W_uk or W_uv) x 8 pages, both operands copied from global memory straight into an LDS ring of four 32-k
+// steps; a wave has 4 x 2 tiles, and the two waves of a SIMD take turns at reading fragments and multiplying (as the persistent GEMM: half a
+// step apart, a bare barrier between).  Bound by the second-level caches and, from 3000 tokens on, by the stores.  With fragments straight
+// from the caches into registers, 64 rows x 64 tokens a wave, a launch asked them for one and a half times the bytes with one step in flight.  us, 16
+// heads, rank 512, 128 + 128 dims, then and now: 64 tokens 10.4 -> 8.6, 1000 16.7 -> 10.4, 2000 28.1 -> 15.4, 3700 30.9 -> 22.4; 32 heads, 1000 tokens
+// 21.0 -> 14.1, 4000 52.9 -> 41.4.  256 rows x 16 pages: 18.3, 20.6, 23.0 (16 heads, 1000, 2000, 3700), 22.9, 40.0.
+constexpr int LE_STAGES = 4;
+constexpr int LE_ROWS = 8;         // 16-row tiles of a workgroup, and its pages
+__global__ __launch_bounds__(512, 2) void latent_expand_kernel(LatentExpand a) {
+  constexpr int RT = LE_ROWS, PT = LE_ROWS, F = RT + PT, LQ = F / 8, WN = RT / 2, WT = PT / 4;
+  extern __shared__ __align__(16) elt lsm[];                         // [LE_STAGES][F][512]
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int pg0 = blockIdx.y * 8 + (wave >> 2) * 4, NB = a.RB + a.KR;
-  if (pg0 >= a.pages) return;                                        // no barrier below
-  int page[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    page[j] = a.phys[pg0 + j];
-    if (page[j] >= a.n_pages) page[j] = -1;
-  }
-  const eltx8 zero = eltx8{0, 0, 0, 0, 0, 0, 0, 0};
+  const int pg0 = blockIdx.y * PT, NB = a.RB + a.KR;
+  auto page_of = [&](int p) {                                        // cache page of scratch page p, -1: padding
+    const int q = p < a.pages ? a.phys[p] : -1;
+    return q < a.n_pages ? q : -1;
+  };
   int bx = blockIdx.x;
   if (bx > a.kb_blocks + a.vb_blocks) return;
   if (bx == a.kb_blocks + a.vb_blocks) {
-    for (int i = threadIdx.x & 255; i < 4 * a.KR * 64; i += 256) {
-      const int j = i / (a.KR * 64), o = i - j * (a.KR * 64);
-      const int pj = a.phys[pg0 + j];
-      st8(a.r + ((size_t)(pg0 + j) * a.KR * 64 + o) * 8,
-          pj >= 0 && pj < a.n_pages ? ld8(a.cache + (size_t)pj * NB * 512 + a.RB * 512 + o * 8) : zero);
+    for (int i = threadIdx.x; i < PT * a.KR * 64; i += 512) {
+      const int j = i / (a.KR * 64), o = i - j * (a.KR * 64), pj = page_of(pg0 + j);
+      if (pg0 + j < a.pages)
+        st8(a.r + ((size_t)(pg0 + j) * a.KR * 64 + o) * 8, pj >= 0 ? ld8(a.cache + (size_t)pj * NB * 512 + a.RB * 512 + o * 8) : eltx8{0, 0, 0, 0, 0, 0, 0, 0});
     }
     return;
   }
   const bool val = bx >= a.kb_blocks;                                // uniform
   if (val) bx -= a.kb_blocks;
   const int tiles = val ? a.H * a.VB : a.H * a.KN * 2;
-  const int nt0 = (bx * 4 + (wave & 3)) * LE_ROWS;
-  if (nt0 >= tiles) return;
-  const elt* wp = (val ? a.uv : a.uk) + lane * 8;
-  int wo[LE_ROWS];                                                   // uniform
-  const elt* cp[4];
+  const int nt0 = bx * RT;
+  const elt* src[LQ];
 #pragma unroll
-  for (int i = 0; i < LE_ROWS; ++i) wo[i] = (nt0 + i < tiles ? nt0 + i : tiles - 1) * a.RB * 512;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) cp[i] = a.cache + (size_t)(page[i] >= 0 ? page[i] : 0) * NB * 512 + lane * 8;
-  f32x4 acc[LE_ROWS][4];
-#pragma unroll
-  for (int i = 0; i < LE_ROWS; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  auto products = [&](auto V) {
-    eltx8 w[LE_ROWS], c[4];
-#pragma unroll
-    for (int i = 0; i < LE_ROWS; ++i) w[i] = ld8(wp + wo[i]);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) c[i] = ld8(cp[i]);
-    for (int kb = 1; kb <= a.RB; ++kb) {
-      const int kc = kb < a.RB ? kb : 0;                             // the last prefetch wraps to a valid address and is discarded
-      eltx8 wn[LE_ROWS], cn[4];
-#pragma unroll
-      for (int i = 0; i < LE_ROWS; ++i) wn[i] = ld8(wp + (wo[i] + kc * 512));
-#pragma unroll
-      for (int i = 0; i < 4; ++i) cn[i] = ld8(cp[i] + kc * 512);
-      __builtin_amdgcn_sched_barrier(0);                             // the requests go out ahead of the products
-#pragma unroll
-      for (int i = 0; i < LE_ROWS; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = decltype(V)::value ? mfma_16x16x32(c[j], w[i], acc[i][j]) : mfma_16x16x32(w[i], c[j], acc[i][j]);
-#pragma unroll
-      for (int i = 0; i < LE_ROWS; ++i) w[i] = wn[i];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) c[i] = cn[i];
+  for (int q = 0; q < LQ; ++q) {
+    if (wave < 4) {
+      const int nt = nt0 + wave * LQ + q;
+      src[q] = (val ? a.uv : a.uk) + (size_t)(nt < tiles ? nt : tiles - 1) * a.RB * 512 + lane * 8;      // tiles past the last: a valid fragment, results dropped
+    } else {
+      const int pj = page_of(pg0 + (wave - 4) * LQ + q);
+      src[q] = a.cache + (size_t)(pj >= 0 ? pj : 0) * NB * 512 + lane * 8;                               // padding: results replaced by zeros
     }
+  }
+  int at = 0;
+  auto issue = [&]() {
+    const int kb = at < a.RB ? at : a.RB - 1;                        // past K: a valid address, not multiplied
+    elt* dst = lsm + (at & (LE_STAGES - 1)) * F * 512 + wave * LQ * 512;
+#pragma unroll
+    for (int q = 0; q < LQ; ++q)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[q] + kb * 512),
+                                       (__attribute__((address_space(3))) void*)(dst + q * 512), 16, 0, 0);
+    ++at;
+  };
+  const int wn = wave >> 2, wt = wave & 3;                           // the waves of a SIMD: the two halves of the rows
+  f32x4 acc[WN][WT];
+#pragma unroll
+  for (int i = 0; i < WN; ++i)
+#pragma unroll
+    for (int j = 0; j < WT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto products = [&](auto V) {
+    issue();
+    issue();
+    issue();
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * LQ) : "memory");    // the first step of this wave has landed
+    bare_barrier();
+    if (wn) bare_barrier();                                          // the second group: half a step behind the first
+    for (int kb = 0; kb < a.RB; ++kb) {
+      const elt* st = lsm + (kb & (LE_STAGES - 1)) * F * 512 + lane * 8;
+      eltx8 w[WN], c[WT];
+#pragma unroll
+      for (int j = 0; j < WT; ++j) c[j] = ld8(st + (RT + wt * WT + j) * 512);
+#pragma unroll
+      for (int i = 0; i < WN; ++i) w[i] = ld8(st + (wn * WN + i) * 512);
+      issue();                                                       // into the slot that both groups have done with
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(2 * LQ) : "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      bare_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int i = 0; i < WN; ++i)
+#pragma unroll
+        for (int j = 0; j < WT; ++j) acc[i][j] = decltype(V)::value ? mfma_16x16x32(c[j], w[i], acc[i][j]) : mfma_16x16x32(w[i], c[j], acc[i][j]);
+      __builtin_amdgcn_s_setprio(0);
+      __builtin_amdgcn_sched_barrier(0);
+      bare_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (!wn) bare_barrier();
   };
   if (val) products(std::true_type());
   else products(std::false_type());
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                   // loads past the last step must not outlive the workgroup's LDS
   const int r16 = lane & 15, g = lane >> 4;
 #pragma unroll
-  for (int i = 0; i < LE_ROWS; ++i) {
-    const int nt = nt0 + i;
-    if (nt >= tiles) continue;
+  for (int j = 0; j < WT; j += 2) {
+    const int p = pg0 + wt * WT + j;                                 // pages come in whole fours: an even page is followed by one
+    if (p >= a.pages) continue;
+    const bool e0 = page_of(p) >= 0, e1 = page_of(p + 1) >= 0;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const f32x4 s = page[j] >= 0 ? acc[i][j] : f32x4{0.f, 0.f, 0.f, 0.f};
-      const eltx4 o = eltx4{(elt)s[0], (elt)s[1], (elt)s[2], (elt)s[3]};
-      if (val) {                                                     // s[r] = token 4 g + r, dim r16 of the tile
-        const int h = nt / a.VB, db = nt - h * a.VB, p = pg0 + j;
-        *reinterpret_cast<eltx4*>(a.v + (((size_t)h * (a.pages / 2) + p / 2) * a.VB + db) * 512 + lane * 8 + (p & 1) * 4) = o;
+    for (int i = 0; i < WN; ++i) {
+      const int nt = nt0 + wn * WN + i;
+      if (nt >= tiles) continue;
+      const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f}, s = e0 ? acc[i][j] : zero, u = e1 ? acc[i][j + 1] : zero;
+      if (val) {                                                     // s[r] = token 4 g + r, dim r16 of the tile; u the same of the odd page
+        const int h = nt / a.VB, db = nt - h * a.VB;
+        st8(a.v + (((size_t)h * (a.pages / 2) + p / 2) * a.VB + db) * 512 + lane * 8,
+            eltx8{(elt)s[0], (elt)s[1], (elt)s[2], (elt)s[3], (elt)u[0], (elt)u[1], (elt)u[2], (elt)u[3]});
       } else {                                                       // s[r] = dim 4 g + r of the tile, token r16
         const int h = nt / (2 * a.KN), d = (nt - h * 2 * a.KN) * 16 + g * 4;
-        *reinterpret_cast<eltx4*>(a.k + (((size_t)h * a.pages + pg0 + j) * a.KN + (d >> 5)) * 512 + ((d >> 3) & 3) * 128 + r16 * 8 + (d & 7)) = o;
+        elt* o = a.k + (((size_t)h * a.pages + p) * a.KN + (d >> 5)) * 512 + ((d >> 3) & 3) * 128 + r16 * 8 + (d & 7);
+        *reinterpret_cast<eltx4*>(o) = eltx4{(elt)s[0], (elt)s[1], (elt)s[2], (elt)s[3]};
+        *reinterpret_cast<eltx4*>(o + (size_t)a.KN * 512) = eltx4{(elt)u[0], (elt)u[1], (elt)u[2], (elt)u[3]};
       }
     }
   }
@@ -1401,10 +1430,12 @@ extern "C" int mlora_latent_prefill(void* out, int out_layout, int ld_out, const
   e.v = e.k + (size_t)H * pages * e.KN * 512;
   e.r = e.v + (size_t)H * (pages / 2) * e.VB * 512;
   e.cache = (const elt*)cache; e.phys = phys; e.uk = (const elt*)uk; e.uv = (const elt*)uv;
-  e.kb_blocks = ceil_div(H * e.KN * 2, 4 * LE_ROWS);
-  e.vb_blocks = ceil_div(H * e.VB, 4 * LE_ROWS);
   hipStream_t s = (hipStream_t)stream;
-  hipLaunchKernelGGL(latent_expand_kernel, dim3((e.kb_blocks + e.vb_blocks + 1 + 7) / 8 * 8, ceil_div(pages, 8)), dim3(512), 0, s, e);   // whole eights: a weight row stays on one XCD
+  e.kb_blocks = ceil_div(H * e.KN * 2, LE_ROWS);
+  e.vb_blocks = ceil_div(H * e.VB, LE_ROWS);
+  constexpr size_t lds = (size_t)LE_STAGES * 2 * LE_ROWS * 512 * sizeof(elt);
+  static_assert(lds <= 64 * 1024, "no attribute needed");
+  hipLaunchKernelGGL(latent_expand_kernel, dim3((e.kb_blocks + e.vb_blocks + 1 + 7) / 8 * 8, ceil_div(pages, LE_ROWS)), dim3(512), lds, s, e);   // whole eights: a weight row stays on one XCD
   LatentPrefill a = {};
   a.out = (elt*)out; a.frag_tt = out_layout == MLORA_FRAG ? mlora_frag_tiles(T) : 0; a.ld_out = ld_out;
   a.q = (const elt*)q; a.ld_q = ld_q; a.qr = (const elt*)q_rot; a.k = e.k; a.v = e.v; a.r = e.r; a.tiles = (const int4*)tiles;
