@@ -576,20 +576,32 @@ __global__ __launch_bounds__(LP_WAVES* WAVE, 2) void latent_prefill_kernel(Laten
   const elt* kh = a.k + ((size_t)kvh * a.pages + tile.z) * KN * 512 + lane * 8;
   const elt* vh = a.v + ((size_t)kvh * (a.pages / 2) + tile.z / 2) * VB * 512 + lane * 8;
   const elt* rh = a.r + (size_t)tile.z * KR * 512 + lane * 8;
-  // piece i of a block: page p = i / KB, fragment i % KB of it for i < 4 KB; then the pairs' V pieces
+  // Pieces of a block in LDS: page p's fragments at p KB + f, the page pairs' V pieces behind them.  Wave p brings page p and a quarter of V, so
+  // that an address is a base, the block's step and a constant.  Worked out per piece from its number, which was divided by KB, they were 580 scalar
+  // instructions of a wave per block: where a workgroup has a compute unit to itself, one prompt of 1000 tokens under 16 heads, 50 -> 42 us, of 4000
+  // 203 -> 178; two workgroups on a unit (32 heads, 4000 tokens, 290 us) hide them.
   auto issue = [&](int b) {
     elt* dst = lsm + (b & 1) * PIECES * 512;
-    for (int i = wave; i < PIECES; i += LP_WAVES) {                  // uniform
-      const elt* src;
-      if (i < 4 * KB) {
-        const int p = i / KB, f = i - p * KB;
-        src = f < KN ? kh + ((size_t)(4 * b + p) * KN + f) * 512 : rh + ((size_t)(4 * b + p) * KR + f - KN) * 512;
-      } else {
-        src = vh + ((size_t)(2 * b) * VB + i - 4 * KB) * 512;
-      }
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                       (__attribute__((address_space(3))) void*)(dst + i * 512), 16, 0, 0);
+    auto bring = [&](elt* to, const elt* src) {
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src, (__attribute__((address_space(3))) void*)to, 16, 0, 0);
+    };
+    const elt* kp = kh + (size_t)(4 * b + wave) * KN * 512;
+    elt* kd = dst + wave * KB * 512;
+#pragma unroll
+    for (int f = 0; f < KB_; ++f) {
+      if (f < KN) bring(kd + f * 512, kp + f * 512);                 // uniform
     }
+    if constexpr (!TIED) {
+      const elt* rp = rh + (size_t)(4 * b + wave) * KR * 512;
+#pragma unroll
+      for (int f = 0; f < KB_; ++f)
+        if (f < KR) bring(kd + (KN + f) * 512, rp + f * 512);        // uniform
+    }
+    const elt* vp = vh + (size_t)b * 2 * VB * 512 + wave * (VB / 2) * 512;
+    elt* vd = dst + (4 * KB + wave * (VB / 2)) * 512;
+#pragma unroll
+    for (int f = 0; f < VB_ / 2; ++f)
+      if (EXACT || f < VB / 2) bring(vd + f * 512, vp + f * 512);
   };
   int b0 = 0;
   if constexpr (TIED) {                                              // the first block within reach of any of the queries
@@ -630,15 +642,17 @@ __global__ __launch_bounds__(LP_WAVES* WAVE, 2) void latent_prefill_kernel(Laten
     if (!act[0] && !act[1]) continue;
     f32x4 st[LP_QT][4];                                              // st[u][p][r] = S[key 4 g + r of page p][query qi of tile u]
 #pragma unroll
-    for (int p = 0; p < 4; ++p) {
+    for (int p = 0; p < 4; p += 2) {                                 // two pages together: four sums, so that none waits for its last product
 #pragma unroll
-      for (int u = 0; u < LP_QT; ++u) st[u][p] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int u = 0; u < LP_QT; ++u) st[u][p] = st[u][p + 1] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int kb = 0; kb < KB_; ++kb) {
         if (EXACT || kb < KB) {
-          const eltx8 kf = ld8(ks + (p * KB + kb) * 512);
+          const eltx8 k0 = ld8(ks + (p * KB + kb) * 512), k1 = ld8(ks + ((p + 1) * KB + kb) * 512);
 #pragma unroll
-          for (int u = 0; u < LP_QT; ++u) st[u][p] = mfma_16x16x32(kf, qf[u][kb], st[u][p]);
+          for (int u = 0; u < LP_QT; ++u) st[u][p] = mfma_16x16x32(k0, qf[u][kb], st[u][p]);
+#pragma unroll
+          for (int u = 0; u < LP_QT; ++u) st[u][p + 1] = mfma_16x16x32(k1, qf[u][kb], st[u][p + 1]);
         }
       }
     }
@@ -694,14 +708,17 @@ __global__ __launch_bounds__(LP_WAVES* WAVE, 2) void latent_prefill_kernel(Laten
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int db = 0; db < VB_; ++db) {
+      for (int db = 0; db < VB_; db += 2) {                          // VB is even; a sum's hi and lo product four apart
         if (EXACT || db < VB) {
-          const eltx8 vf = ld8(vs + (j * VB + db) * 512);
+          const eltx8 v0 = ld8(vs + (j * VB + db) * 512), v1 = ld8(vs + (j * VB + db + 1) * 512);
 #pragma unroll
-          for (int u = 0; u < LP_QT; ++u) {
-            O[u][db] = mfma_16x16x32(vf, ph[u][j], O[u][db]);
-            O[u][db] = mfma_16x16x32(vf, pl[u][j], O[u][db]);        // O^T[dim 16 db + 4 g + r][query qi of tile u]
-          }
+          for (int u = 0; u < LP_QT; ++u) O[u][db] = mfma_16x16x32(v0, ph[u][j], O[u][db]);        // O^T[dim 16 db + 4 g + r][query qi of tile u]
+#pragma unroll
+          for (int u = 0; u < LP_QT; ++u) O[u][db + 1] = mfma_16x16x32(v1, ph[u][j], O[u][db + 1]);
+#pragma unroll
+          for (int u = 0; u < LP_QT; ++u) O[u][db] = mfma_16x16x32(v0, pl[u][j], O[u][db]);
+#pragma unroll
+          for (int u = 0; u < LP_QT; ++u) O[u][db + 1] = mfma_16x16x32(v1, pl[u][j], O[u][db + 1]);
         }
       }
   }
