@@ -73,15 +73,23 @@ class LatentAttention:
         self.o_rows = padded(o, Hp, H, self.vp).reshape(Hp, self.out_cols)      # the output projection, for the layer to place
 
     def prompt_form_pays(self, seqs) -> bool:
-        """Whether a pass (per sequence: appended tokens, context length) is cheaper with keys and values made: products on
-        the matrix cores for that form, cache bytes through the second-level caches for the other (they are read once per
-        token and 16 heads)."""
+        """Whether a pass (per sequence: appended tokens, context length) is cheaper with keys and values made.  Both sums are microseconds,
+        fitted to 225 passes of 8 to 3000 tokens at contexts up to 5000 under 8, 16 and 32 heads of 128 + 64 dims over rank 512.  Lifted: the launches,
+        the two products per token and head, the cache bytes (read once per token and 16 heads), and above 256 tokens the second
+        product in a launch of its own.  Made: the launches, the longest context in blocks of 64 keys (a workgroup goes through them one after the
+        other), keys and values, scores, queries and outputs.  The lesser sum is the slower form in 3 of the 225, by 9 % at most;
+        4 us more are asked for because the host makes a plan.  lifted / made: 16 heads, one prompt of 90 23.5 / 21.3, 250 32.8 / 27.7, 500
+        69 / 40, 1000 130 / 58; eight of 40 54 / 20; 20 tokens behind 500 24 / 40, 300 behind 1000 95 / 70."""
         if self.uk is None:
             return False
-        H = self.spec.heads
-        lifted = sum(n * (c - n / 2) for n, c in seqs) * -(-H // 16) * self.q_cols * 2 / 8e12
-        made = sum(c * self.rank_p * (self.dp + self.vp) + n * c * (self.dp + self.q_cols - self.rank_p + 2 * self.vp) for n, c in seqs) * 2 * H / 4e14
-        return made + 2e-5 < lifted
+        H, image = self.spec.heads, self.rank_p * (self.dp + self.vp)
+        rot = self.q_cols - self.rank_p
+        T, far = sum(n for n, _ in seqs), max(c for _, c in seqs)
+        pairs = sum(n * (c - n / 2) for n, c in seqs)
+        lifted = 18.8 + 2.7e-8 * T * H * image + 1.43e-7 * pairs * -(-H // 16) * self.q_cols + (18.8 if T > 256 else 0.0) + 0.0079 * far
+        made = 17.1 + 0.0314 * far + 2.76e-9 * sum(c for _, c in seqs) * H * image + 4e-10 * pairs * H * (self.dp + rot + 2 * self.vp) \
+            + 7.3e-7 * T * H * (self.dp + rot + self.vp)
+        return made + 4.0 < lifted
 
     def attend(self, qkv, pages, block_table, tok_seq, tok_pos, cos, sin, max_ctx, store, plan=None, out=None):
         """plan: a PrefillPlan of the pass for the prompt form, None for the lifted form."""
