@@ -575,6 +575,9 @@ typedef struct mlora_decode_plan {
   size_t lora_ws_bytes;
   float* ksplit_ws;           /* partials of the K-split o_proj / down_proj GEMVs, or NULL (no split) */
   size_t ksplit_ws_bytes;     /* >= mlora_gemv_ksplit_bytes over both projections (with their appended rows) */
+  int lora_segments;          /* up to 64 sequences: the deltas as launches of their own (mlora_gather_mm_segments) instead of riding in the
+                               * linear, attention and norm launches - for larger ranks, and few adapters of many tokens.  With lora_dense
+                               * only those of gate and up.  Needs what mlora_gather_mm_segments needs of the shapes */
 } mlora_decode_plan;
 
 int mlora_decode_step(const mlora_decode_plan* plan, void* stream);

@@ -113,7 +113,7 @@ class DecodePlan(C.Structure):
                 ("block_table", _p), ("max_blocks", _i), ("n_pages", _i), ("n_seq", _i),
                 ("T", _i), ("tokens", _p), ("rows", _p), ("pos", _p), ("ctx", _p), ("tok_adapter", _p),
                 ("resid", _p), ("xn", _p), ("qkv", _p), ("attn", _p), ("gate_up", _p), ("act", _p), ("logits", _p),
-                ("lora_ws", _p), ("lora_ws_bytes", _z), ("ksplit_ws", _p), ("ksplit_ws_bytes", _z)]
+                ("lora_ws", _p), ("lora_ws_bytes", _z), ("ksplit_ws", _p), ("ksplit_ws_bytes", _z), ("lora_segments", _i)]
 
 
 SIGNATURES["mlora_decode_step"] = (_i, [C.POINTER(DecodePlan), _p])

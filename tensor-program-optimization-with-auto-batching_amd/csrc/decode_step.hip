@@ -151,6 +151,8 @@ extern "C" int mlora_decode_step(const mlora_decode_plan* p, void* stream) {
   const int q_sz = Hq * D, kv_sz = Hkv * D, qkv_sz = q_sz + 2 * kv_sz;
   const bool lora = p->tok_adapter != nullptr && p->lora_r > 0;
   const bool dense = lora && p->lora_dense != 0;
+  // deltas as launches of their own: all of them, or beside appended rows those of gate and up
+  const bool segs = lora && !dense && p->lora_segments, gu_segs = lora && p->lora_segments;
   const int r = p->lora_r, n_ad = p->lora_n_ad;
   const float sc = p->lora_scaling;
   // the o projection's delta from riders of its GEMV launch (o_p is then the base weight alone)
@@ -176,6 +178,19 @@ extern "C" int mlora_decode_step(const mlora_decode_plan* p, void* stream) {
   void* ws_o = ws + (size_t)3 * kq * slot;
   void* ws_down = ws + (size_t)(3 * kq + 1) * slot;
   const size_t down_bytes = lora ? p->lora_ws_bytes - (size_t)(3 * kq + 1) * slot : 0;   // (a smaller K may take more than the largest)
+  auto seg_deltas = [&](void* y, int y_dtype, int ldy, const void* x, int K, const mlora_lora_proj* lp, const int32_t* col, const int32_t* ncol, int n) -> int {
+    mlora_lora_bucket bk[3];
+    int32_t c[3], nc[3];
+    int live = 0;
+    for (int i = 0; i < n; ++i)
+      if (lp[i].A) {
+        bk[live] = mlora_lora_bucket{lp[i].A, lp[i].B, r, n_ad, sc};
+        c[live] = col[i];
+        nc[live++] = ncol[i];
+      }
+    if (live == 0) return MLORA_OK;
+    return mlora_gather_mm_segments(y, y_dtype, ldy, x, MLORA_FRAG, bk, live, c, nc, p->tok_adapter, T, K, p->lora_ws, p->lora_ws_bytes, stream);
+  };
   auto delta = [&](void* y, int y_dtype, int ldy, const void* x, const mlora_lora_proj& lp, int K, int N) -> int {
     if (!lora || !lp.A) return MLORA_OK;
     return mlora_gather_mm(y, y_dtype, ldy, x, MLORA_FRAG, lp.A, lp.B, p->tok_adapter, sc, T, K, N, r, n_ad, ws_down, down_bytes, stream);
@@ -186,13 +201,13 @@ extern "C" int mlora_decode_step(const mlora_decode_plan* p, void* stream) {
   // units ends with a second round on a few of them).
   auto ksplit_of = [&](int K, bool has_lora) -> int {
     const int ld_part = H + (dense && has_lora ? n_ad * r : 0);
-    const int n_total = ld_part + (!dense && has_lora ? mlora_gemv_shrink_rows(K, 1, n_ad) : 0);
+    const int n_total = ld_part + (!dense && !segs && has_lora ? mlora_gemv_shrink_rows(K, 1, n_ad) : 0);
     const int ks = p->ksplit_ws ? mlora_gemv_ksplit(T, K, n_total) : 1;
     return ks > 1 && mlora_gemv_ksplit_bytes(T, ld_part, ks) <= p->ksplit_ws_bytes ? ks : 1;
   };
   // o_proj / down_proj: resid += x . W^T with the adapter's shrink riding along (dense: appended rows; else shrink units)
   auto acc_gemv = [&](const void* x, const void* Wp, int K, const mlora_lora_proj& lp, void* v_ws, int ks) -> int {
-    const bool has = lora && lp.A;
+    const bool has = lora && !segs && lp.A;
     const void* A1[1] = {lp.A};
     if (has && dense)
       return mlora_gemv_frag_acc_ksplit(p->resid, (float*)v_ws, p->ksplit_ws, ks, x, Wp, T, K, H, n_ad * r, nullptr, nullptr, 0,
@@ -217,8 +232,8 @@ extern "C" int mlora_decode_step(const mlora_decode_plan* p, void* stream) {
     const mlora_layer& L = p->layers[l];
     if (l == 0) STEP(mlora_embed_rmsnorm(p->xn, p->resid, p->embed, p->tokens, p->vocab, L.ln1, p->eps, T, H, stream));
     else STEP(norm(L.ln1, pending_B, ws_down, I, pending_ks));
-    const bool qkv_lora = lora && (L.lora[MLORA_Q].A || L.lora[MLORA_K].A || L.lora[MLORA_V].A);
-    const bool o_lora = lora && L.lora[MLORA_O].A;
+    const bool qkv_lora = lora && !segs && (L.lora[MLORA_Q].A || L.lora[MLORA_K].A || L.lora[MLORA_V].A);
+    const bool o_lora = lora && !segs && L.lora[MLORA_O].A;
     const bool o_via_ride = o_lora && o_ride;   // the attention launch writes the o shrink's head shares, riders of the o GEMV expand them
     if (qkv_lora) {
       const void* A3[3] = {L.lora[MLORA_Q].A, L.lora[MLORA_K].A, L.lora[MLORA_V].A};
@@ -236,6 +251,11 @@ extern "C" int mlora_decode_step(const mlora_decode_plan* p, void* stream) {
                                     dense ? kq : 0, B3, p->tok_adapter, sc, H, r, n_ad, stream));
     } else {
       STEP(mlora_gemv_frag(qkv, MLORA_F16, MLORA_STORE, p->xn, L.qkv_p, T, H, qkv_sz, stream));
+      if (segs) {
+        const mlora_lora_proj lp[3] = {L.lora[MLORA_Q], L.lora[MLORA_K], L.lora[MLORA_V]};
+        const int32_t col[3] = {0, q_sz, q_sz + kv_sz}, ncol[3] = {q_sz, kv_sz, kv_sz};
+        STEP(seg_deltas(qkv, MLORA_F16, qkv_sz, p->xn, H, lp, col, ncol, 3));
+      }
       if (o_via_ride)
         STEP(mlora_rope_attn_decode_oshrink(p->attn, MLORA_FRAG, qkv, L.k_cache, L.v_cache, p->block_table, p->max_blocks, p->rows,
                                             p->pos, p->ctx, p->rope_cos, p->rope_sin, p->max_pos, T, Hq, Hkv, D, p->n_pages, p->n_seq,
@@ -254,6 +274,10 @@ extern "C" int mlora_decode_step(const mlora_decode_plan* p, void* stream) {
     } else {
       const int ks_o = ksplit_of(q_sz, o_lora);
       STEP(acc_gemv(p->attn, L.o_p, q_sz, L.lora[MLORA_O], ws_o, ks_o));
+      if (segs) {
+        const int32_t col[1] = {0}, ncol[1] = {H};
+        STEP(seg_deltas(p->resid, MLORA_F32, H, p->attn, q_sz, &L.lora[MLORA_O], col, ncol, 1));
+      }
       STEP(norm(L.ln2, o_lora ? L.lora[MLORA_O].B : nullptr, ws_o, q_sz, ks_o));
     }
     const bool gu_lora = lora && (L.lora[MLORA_GATE].A || L.lora[MLORA_UP].A);
@@ -261,13 +285,23 @@ extern "C" int mlora_decode_step(const mlora_decode_plan* p, void* stream) {
       STEP(mlora_gemv_frag_silu(p->act, p->xn, L.gate_up_il_p, T, H, I, stream));
     } else {
       STEP(mlora_gemv_frag(gu, MLORA_F16, MLORA_STORE, p->xn, L.gate_up_p, T, H, 2 * I, stream));
-      STEP(delta(gu, MLORA_F16, 2 * I, p->xn, L.lora[MLORA_GATE], H, I));
-      STEP(delta(gu + I, MLORA_F16, 2 * I, p->xn, L.lora[MLORA_UP], H, I));
+      if (gu_segs) {
+        const mlora_lora_proj lp[2] = {L.lora[MLORA_GATE], L.lora[MLORA_UP]};
+        const int32_t col[2] = {0, I}, ncol[2] = {I, I};
+        STEP(seg_deltas(gu, MLORA_F16, 2 * I, p->xn, H, lp, col, ncol, 2));
+      } else {
+        STEP(delta(gu, MLORA_F16, 2 * I, p->xn, L.lora[MLORA_GATE], H, I));
+        STEP(delta(gu + I, MLORA_F16, 2 * I, p->xn, L.lora[MLORA_UP], H, I));
+      }
       STEP(mlora_silu_mul(p->act, MLORA_FRAG, gu, gu + I, 2 * I, T, I, stream));
     }
-    const bool down_lora = lora && L.lora[MLORA_DOWN].A;
+    const bool down_lora = lora && !segs && L.lora[MLORA_DOWN].A;
     pending_ks = ksplit_of(I, down_lora);
     STEP(acc_gemv(p->act, L.down_p, I, L.lora[MLORA_DOWN], ws_down, pending_ks));
+    if (segs) {
+      const int32_t col[1] = {0}, ncol[1] = {H};
+      STEP(seg_deltas(p->resid, MLORA_F32, H, p->act, I, &L.lora[MLORA_DOWN], col, ncol, 1));
+    }
     pending_B = down_lora ? L.lora[MLORA_DOWN].B : nullptr;   // expanded inside the next RMSNorm launch
   }
   STEP(norm(p->norm, pending_B, ws_down, I, pending_ks));

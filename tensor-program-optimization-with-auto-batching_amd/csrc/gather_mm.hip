@@ -1380,7 +1380,9 @@ static int gather_mm_impl(void* y, int y_dtype, int ldy, const void* x, int x_la
     const GmmSet one = {y, (const f16*)x, (const f16*)A, (const f16*)B};
     return gmm_one_launch(one, nullptr, 1, y_dtype, ldy, x_layout, tok_adapter, scaling, T, K, N, r, n_ad, (hipStream_t)stream, bf);
   }
-  if (gmm_segments_fit(y, ldy, x_layout, T, K, N)) {
+  // (more than 64 tokens, or ranks whose partial sums do not fit the one launch: 40 tokens of rank 64 by the pair of kernels below 274 us with one adapter,
+  // 29 with sixteen; here 14 and 22.  64 of rank 32 298 and 24; 11 and 15)
+  if (T > 0 && gmm_segments_serve(y, ldy, x_layout, K, N)) {
     MLORA_CHECK(y && x && A && B && tok_adapter, MLORA_ERR_INVALID, "gather_mm: null pointer");
     MLORA_CHECK(y_dtype == MLORA_F16 || y_dtype == MLORA_F32, MLORA_ERR_INVALID, "gather_mm: bad y_dtype %d", y_dtype);
     MLORA_CHECK(ldy >= N, MLORA_ERR_INVALID, "gather_mm: need ldy >= N (ldy=%d N=%d)", ldy, N);

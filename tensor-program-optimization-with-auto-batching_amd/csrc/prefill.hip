@@ -159,7 +159,7 @@ extern "C" int mlora_prefill(const mlora_prefill_plan* p, void* stream) {
       return p->tok_rest ? deltas(y, y_dtype, N, x, K, pj, n, p->tok_rest) : MLORA_OK;
     }
     if (ks && part) {
-      const int riding = T <= 64 && n > 0 ? mlora_gemv_shrink_rows(K, 1, 1) : 0;
+      const int riding = T <= 64 && n > 0 && !p->segments ? mlora_gemv_shrink_rows(K, 1, 1) : 0;
       const int k = mlora_gemv_ksplit(T, K, N + riding);
       *ks = k > 1 && mlora_gemv_ksplit_bytes(T, N, k) <= at.ksplit_bytes ? k : 1;
       STEP(mlora_gemv_frag_acc_ksplit((float*)y, nullptr, *ks > 1 ? part : nullptr, *ks, x, W, T, K, N, 0, nullptr, nullptr, 0, nullptr, 0, 0, stream));

@@ -252,13 +252,15 @@ class LlamaForCausalLM(CausalLM):
             self._ws = torch.empty(need, dtype=torch.float32, device=self.device)
         return self._ws
 
-    def _segments_pay(self, T, n_seq, tok_adapter):
-        """Whether the deltas of a prompt pass of up to 64 tokens go to the matrix cores, where a launch takes as long whatever the tokens
-        share; the one-launch kernel works an adapter's tokens off one after the other.  Three projections of 4096 x 4096, one adapter,
-        us, one launch / matrix cores: rank 8, 8 and 16 tokens 13.1 / 13.0, 22.4 / 12.7; 16, 4 and 8 tokens 11.2 / 12.3, 16.6 / 12.4; 32, 4
-        tokens 17.0 / 12.3; 64, 40 tokens 822 / 14.4; four adapters, rank 16, 16 and 40 tokens 11.2 / 14.3, 20.1 / 13.7; 64, 8 tokens 21.9 / 18.3."""
-        (tid, _), = tok_adapter.items()
-        return T * self.lora_types[tid].r >= 128 * n_seq
+    def segments_pay(self, T, most, tid):
+        """Whether the deltas of up to 64 tokens, of which `most` name one adapter (a prompt pass: its longest sequence), go to the matrix cores
+        in launches of their own, which take as long whatever the tokens share.  The units that ride in a decode step's launches, and the
+        one-launch kernel, work an adapter's tokens off one after the other.  Decode steps of two 7B layers, q, k, v and o adapted, us, riding /
+        launches: rank 8, one adapter, 8 tokens 295 / 288, 64 tokens 563 / 369, sixteen of 64 361 / 393; rank 16, one, 4 tokens 285 / 281, 16 tokens
+        349 / 290; two of 8 290 / 300; four of 32 359 / 310 (two of 32), eight of 32 314 / 331; rank 32, one token 301 / 277, 8 of 8 309 / 316, 64 of
+        64 503 / 455; rank 64, one 352 / 297, 64 of one 1732 / 396, 64 of 64 603 / 515."""
+        s, r = self.shape, self.lora_types[tid].r
+        return not (s.hidden_size % 32 or s.q_size % 32 or s.intermediate_size % 32 or s.kv_size % 16) and 0 < T <= 64 and (r >= 32 or most * r >= 96)
 
     def _lora(self, y, x, l, proj, tok_adapter, segments=False):
         """y += delta for every adapter type that targets (l, proj); tok_adapter: {tid: ids [T] int32}, or the merged
@@ -367,8 +369,12 @@ class LlamaForCausalLM(CausalLM):
         # the RMSNorm that reads the residual next adds the partial results (the same kernels and slice counts as the
         # native decode step)
         ks_ws = self._ksplit_ws(T) if dec_frag or (frag and (T <= 256 or is_decode)) else None
-        segs = (T <= 64 and frag and not is_decode and kv._cur is not None and len(tok_adapter) == 1 and "multi" not in tok_adapter
-                and self._segments_pay(T, len(kv._cur[0]), tok_adapter))
+        segs = False
+        if T <= 64 and kv._cur is not None and len(tok_adapter) == 1 and "multi" not in tok_adapter and (host_ids is not None or not is_decode):
+            (tid, _), = tok_adapter.items()
+            segs = self.segments_pay(T, most_of_one(host_ids[tid]) if is_decode else max(kv._cur[1]), tid)
+        # (what rides along in a decode step's launches counts as rows there; nothing does where the deltas are launches of their own)
+        riding = (lambda *a: 0) if segs else self._riding_rows
         # a prefill-sized pass of one adapter type of rank 32 or 64: where a 256-token block agrees on one adapter its
         # deltas ride in the base GEMM as extra k-steps; `rest` names the tokens that still need the separate call
         # (a prefill pass only: where the ids are known on the device only, the choice needs a read-back, which a decode
@@ -409,14 +415,14 @@ class LlamaForCausalLM(CausalLM):
                 o_sh = o_shares[0].tables[(l, "o_proj")]
             if o_sh is not None:
                 attn, vpart = kv.attention_with_fused_qkv(l, qkv, s.num_attention_heads, frag=frag, o_shrink=(o_sh[0], o_shares[1]))
-                parts = self._linear_acc(attn, L["o"], resid, ks_ws, self._riding_rows(l, "o_proj", lora_tids, T, q_sz))
+                parts = self._linear_acc(attn, L["o"], resid, ks_ws, riding(l, "o_proj", lora_tids, T, q_sz))
                 ops.lora_expand_shares(resid, vpart, o_sh[1], o_shares[1], o_shares[0].scaling)
             else:
                 attn = kv.attention_with_fused_qkv(l, qkv, s.num_attention_heads, frag=frag)
                 if fuse and self._fused_linear(fuse, attn, L["o"], l, (("o_proj", 0, H),), resid=resid) is not None:
                     parts = None
                 else:
-                    parts = self._linear_acc(attn, L["o"], resid, ks_ws, self._riding_rows(l, "o_proj", lora_tids, T, q_sz))
+                    parts = self._linear_acc(attn, L["o"], resid, ks_ws, riding(l, "o_proj", lora_tids, T, q_sz))
                     if tok_adapter:
                         self._lora(resid, attn, l, "o_proj", tok_adapter, segs)
             xn = ops.rmsnorm(resid, L["ln2"], s.rms_norm_eps, frag=frag, parts=parts)
@@ -438,7 +444,7 @@ class LlamaForCausalLM(CausalLM):
             if fuse and self._fused_linear(fuse, act, L["down"], l, (("down_proj", 0, H),), resid=resid) is not None:
                 parts = None
             else:
-                parts = self._linear_acc(act, L["down"], resid, ks_ws, self._riding_rows(l, "down_proj", lora_tids, T, I))
+                parts = self._linear_acc(act, L["down"], resid, ks_ws, riding(l, "down_proj", lora_tids, T, I))
                 if tok_adapter:
                     self._lora(resid, act, l, "down_proj", tok_adapter, segs)
         if logits_rows is not None:
@@ -550,7 +556,7 @@ class LlamaForCausalLM(CausalLM):
             d_ids = ops.upload(torch.from_numpy(ids), self.device)
             p.lora_r, p.lora_n_ad, p.lora_scaling, p.tok_adapter = lt.r, lt.n_adapters, lt.scaling, ptr(d_ids, i32)
             if T <= 64:
-                p.segments = self._segments_pay(T, len(kv._cur[0]), {tid: None})
+                p.segments = self.segments_pay(T, max(kv._cur[1]), tid)
             elif lt.r in (32, 64) and ops.gemm_frag_preferred(T, s.hidden_size, s.hidden_size):
                 blk, rest = (ops.upload(torch.from_numpy(a), self.device) if a is not None else None for a in block_adapters(ids, lt.n_adapters))
                 p.blk_adapter, p.tok_rest = ptr(blk, i32), None if rest is None else ptr(rest, i32)
@@ -624,7 +630,8 @@ class LlamaForCausalLM(CausalLM):
         return super().prefill_no_adapter(h, kv)
 
     def decode_a(self, tid, h, kv, wids):
-        return self.forward(h, kv, self._ids(h.shape[0], {tid: (None, wids)})), kv
+        ids = self._ids(h.shape[0], {tid: (None, wids)}, host=True)
+        return self.forward(h, kv, {t: ops.upload(torch.from_numpy(a), self.device) for t, a in ids.items()}, host_ids=ids), kv
 
     def mixed_decode(self, tids, h, kv, *params):
         """params = sids_i, wids_i, sids_j, wids_j, ... for the adapter types in `tids`
@@ -659,6 +666,11 @@ class LlamaForCausalLM(CausalLM):
         s = self.shape
         per_layer = sum(np.prod(linear_dims(s, p)) for p in LINEARS)
         return int(2 * (per_layer * s.num_hidden_layers + s.vocab_size * s.hidden_size))
+
+
+def most_of_one(ids) -> int:
+    """How many of the tokens of ids [T] (host) name the adapter that most of them name."""
+    return int(np.unique(ids[ids >= 0], return_counts=True)[1].max(initial=0))
 
 
 def block_adapters(ids, n_ad):

@@ -303,3 +303,39 @@ def test_native_step_begins_and_ends_as_its_operators(hidden, requests, vocab):
     for a, b in zip(*[g[0] for g in got]):
         assert np.array_equal(a, b)
     assert torch.equal(got[0][1], got[1][1]) and torch.equal(got[0][2], got[1][2])
+
+
+ALL = ("q_proj", "k_proj", "v_proj", "o_proj", "gate_proj", "up_proj", "down_proj")
+
+
+@pytest.mark.parametrize("B,r,targets,dense", [(1, 32, ("q_proj", "v_proj"), False), (6, 16, ALL, False), (17, 8, ALL, False), (33, 64, ALL, False), (64, 32, ("o_proj", "down_proj"), False),
+                                               (48, 16, ("q_proj", "up_proj"), False), (20, 16, ALL, True)])
+def test_native_step_with_deltas_in_launches_of_their_own(B, r, targets, dense):
+    """Steps whose tokens share adapters, on both sides of the rule: tokens and the whole K cache of the per-operator path, bit for bit, and logits that
+    agree with the riding forms to rounding; beside appended rows, gate and up alone."""
+    synth, llama, dsm = load_pkg("synth"), load_pkg("llama"), load_pkg("decode_session")
+    shape = synth.LlamaShape(hidden_size=1024, intermediate_size=1408, num_attention_heads=8, num_key_value_heads=4, num_hidden_layers=2, head_dim=128, vocab_size=600)
+    model = llama.LlamaForCausalLM.from_synthetic(9, shape, [synth.LoraSpec(r=r, alpha=r / 2, n_adapters=4, targets=targets)], DEV)
+    ids = (np.arange(B) % 7 // 6).astype(np.int32)             # most name adapter 0
+    ids[B // 2] = -1 if B > 1 else 0
+    most = llama.most_of_one(ids)
+    assert most == (ids == 0).sum() and model.segments_pay(B, most, 0) == (r >= 32 or most * r >= 96)
+    got = {}
+    for kind in ("py", "native", "graph", "riding"):
+        kv = model.create_paged_kv_cache(B, B * 64, 32, 16, max_seq_len=64)
+        first = _prefill(model, kv, synth.randint(2, "own", (B, 20), 600).numpy(), ids)
+        if kind == "py":
+            s = dsm.DecodeSession(model, kv, list(range(B)), {0: ids}, first)
+        else:
+            s = dsm.NativeDecodeSession(model, kv, list(range(B)), ids, first, use_graph=kind == "graph", dense_lora=dense)
+            if kind == "riding":
+                s.plan.lora_segments = 0
+        toks = [s.step().cpu().numpy().copy()]
+        logits = None if kind == "py" else s.buf["logits"].clone()
+        toks += [s.step().cpu().numpy().copy() for _ in range(3)]
+        got[kind] = (np.stack(toks), kv.k.clone(), logits)
+    if not dense:
+        assert np.array_equal(got["py"][0], got["native"][0]) and torch.equal(got["py"][1], got["native"][1])
+    assert np.array_equal(got["graph"][0], got["native"][0]) and torch.equal(got["graph"][1], got["native"][1])
+    a, b = got["native"][2], got["riding"][2]
+    assert float((a - b).abs().max() / b.std()) <= 1e-2
