@@ -622,6 +622,10 @@ int mlora_prefill(const mlora_prefill_plan* plan, void* stream);
  * (persistent GEMM shapes) and mlora_silu_mul. */
 int mlora_gemv_frag_clipglu(void* act, const void* xf, const void* Wil_p, int T, int K, int I, float scale, float limit, float alpha, void* stream);
 int mlora_linear_frag_clipglu(void* act, const void* xf, const void* Wp, int T, int K, int I, float scale, float limit, float alpha, void* stream);
+/* Either gated product (kind: MLORA_GLU_*; scale, limit, alpha: of the clipped one) for more than 64 tokens, on the kernel that mlora_linear_frag
+ * takes at that size (mid-size or persistent).  K and I in whole 32, operands 16-byte aligned. */
+int mlora_linear_frag_glu(void* act, const void* xf, const void* Wp, int T, int K, int I, int kind, float scale, float limit, float alpha,
+                          void* stream);
 int mlora_clipglu_mul(void* out, int out_layout, const void* gate, const void* up, int ld, int T, int I, float scale, float limit, float alpha,
                       void* stream);
 

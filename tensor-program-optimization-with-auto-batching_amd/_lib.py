@@ -17,6 +17,7 @@ GLU_SILU, GLU_CLIPPED = 0, 1
 ACT_NONE, ACT_RELU2, ACT_GLU = 0, 1, 2
 MOE_UP, MOE_DOWN = 0, 1
 ROWMAJOR, FRAG = 0, 1
+GLU_SILU, GLU_CLIPPED = 0, 1
 STORE, ACCUMULATE = 0, 1
 PAGE_SIZE = 16
 
@@ -57,6 +58,7 @@ SIGNATURES = {
     "mlora_gemv_frag_lora": (_i, [_p, _i, _i, _p, _p, _i, _i, _i, _p, _p, _i, _p, _i, _i, _p]),
     "mlora_gemv_frag_silu": (_i, [_p, _p, _p, _i, _i, _i, _p]),
     "mlora_gemv_frag_clipglu": (_i, [_p, _p, _p, _i, _i, _i, _f, _f, _f, _p]),
+    "mlora_linear_frag_glu": (_i, [_p, _p, _p, _i, _i, _i, _i, _f, _f, _f, _p]),
     "mlora_linear_frag_clipglu": (_i, [_p, _p, _p, _i, _i, _i, _f, _f, _f, _p]),
     "mlora_clipglu_mul": (_i, [_p, _i, _p, _p, _i, _i, _i, _f, _f, _f, _p]),
     "mlora_gemv_frag_split": (_i, [_p, _i, _i, _p, _p, _p, _i, _i, _i, _i, _p]),

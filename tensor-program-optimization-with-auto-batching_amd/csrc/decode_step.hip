@@ -99,13 +99,15 @@ int decode_step_wide(const mlora_decode_plan* p, void* stream) {
       STEP(deltas(p->resid, MLORA_F32, H, p->attn, q_sz, lp, col, ncol, 1));
     }
     STEP(norm(L.ln2, ks_o));
-    STEP(mlora_linear_frag(gu, MLORA_F16, MLORA_STORE, p->xn, L.gate_up_p, T, H, 2 * I, stream));
-    {
+    if (lora && (L.lora[MLORA_GATE].A || L.lora[MLORA_UP].A)) {
+      STEP(mlora_linear_frag(gu, MLORA_F16, MLORA_STORE, p->xn, L.gate_up_p, T, H, 2 * I, stream));
       const mlora_lora_proj* lp[2] = {&L.lora[MLORA_GATE], &L.lora[MLORA_UP]};
       const int32_t col[2] = {0, I}, ncol[2] = {I, I};
       STEP(deltas(gu, MLORA_F16, 2 * I, p->xn, H, lp, col, ncol, 2));
+      STEP(mlora_silu_mul(p->act, MLORA_FRAG, gu, gu + I, 2 * I, T, I, stream));
+    } else {
+      STEP(mlora_linear_frag_glu(p->act, p->xn, L.gate_up_p, T, H, I, MLORA_GLU_SILU, 0.f, 0.f, 0.f, stream));
     }
-    STEP(mlora_silu_mul(p->act, MLORA_FRAG, gu, gu + I, 2 * I, T, I, stream));
     pending_ks = ksplit_of(I);
     STEP(mlora_gemv_frag_acc_ksplit(p->resid, nullptr, p->ksplit_ws, pending_ks, p->act, L.down_p, T, I, H, 0, nullptr, nullptr, 0, nullptr, 0,
                                     0, stream));

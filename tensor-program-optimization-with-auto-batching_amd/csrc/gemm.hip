@@ -786,10 +786,15 @@ constexpr int MID_KS = 2;                      // 32-k steps per stage
 constexpr int mid_stages(int FT) { return FT == 16 ? 3 : 4; }
 
 // GX: the rows are groups of gx_rows (a multiple of 16 FN) that read activations of their own, gx_stride elements apart.
+// A gated product (OUT_SILU, OUT_CLIP): Wp is the fused [2 I, K] matrix (N = 2 I), a block FN / 2 tiles of gate rows and the up rows of the same
+// channels, so that the waves wn = 0 hold the one and wn = 1 the other; they exchange halves through LDS, rounded to elements as a linear
+// would store them, and leave the product in fragment order.
 template <int OUT, int FT, int FN, bool GX = false>
 __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_mid_kernel(void* __restrict__ yv, float* __restrict__ part, int ld_part,
                                                                     const elt* __restrict__ xf, int x_tt, const elt* __restrict__ Wp,
-                                                                    int T, int K, int N, int gx_rows = 0, long gx_stride = 0) {
+                                                                    int T, int K, int N, int gx_rows = 0, long gx_stride = 0,
+                                                                    GluArgs ga = GluArgs()) {
+  constexpr bool GLU = OUT == OUT_SILU || OUT == OUT_CLIP;
   constexpr int MID_STAGES = mid_stages(FT);
   constexpr int SF = FN + FT;                  // fragments of one 32-k step: weights, then tokens
   constexpr int LF = MID_KS * SF;              // fragments per stage
@@ -805,7 +810,12 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_mid_kernel(void* __res
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int KB = K / 32;
   const int tiles = (N + 15) / 16;
-  const int n0 = blockIdx.x * FN * 16, t0 = blockIdx.z * FT * 16;
+  const int n0 = blockIdx.x * FN * (GLU ? 8 : 16), t0 = blockIdx.z * FT * 16;       // GLU: the first channel
+  const int I = N / 2, itiles = I / 16;
+  auto tile_row = [&](int f) {                 // the 16-row tile of W that is weight fragment f of the block (it may lie past the end)
+    if constexpr (GLU) return f < FN / 2 ? n0 / 16 + f : itiles + n0 / 16 + f - FN / 2;
+    return n0 / 16 + f;
+  };
   if constexpr (GX) xf += (n0 / gx_rows) * gx_stride;
   const int per = (KB + gridDim.y - 1) / gridDim.y;
   const int kb0 = blockIdx.y * per;
@@ -820,8 +830,8 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_mid_kernel(void* __res
     const int f = (wave + PP_WAVES * q) % SF;  // uniform (past LF for the last q of a wave with one fewer: set up, never issued)
     kso[q] = (wave + PP_WAVES * q) / SF;
     if (f < FN) {
-      int nt = n0 / 16 + f;
-      nt = nt < tiles ? nt : tiles - 1;        // rows past N: a valid fragment, results dropped
+      int nt = tile_row(f);
+      nt = nt < tiles ? nt : tiles - 1;        // rows past N: a valid fragment, results dropped (past the gate's: the up part's first ones)
       src[q] = Wp + (size_t)nt * KB * 512 + lane * 8;
       step[q] = 512;
     } else {
@@ -960,6 +970,49 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_mid_kernel(void* __res
     }
     return;
   }
+  if constexpr (GLU) {
+    // waves wn = 0 finish the first token fragments of a pair of waves, wn = 1 the others
+    constexpr int H0 = (WTF + 1) / 2;
+    eltx4* ex = reinterpret_cast<eltx4*>(smem) + (size_t)wt * WNF * WTF * WAVE + lane;
+    auto give = [&](auto J0, auto J1) {
+#pragma unroll
+      for (int i = 0; i < WNF; ++i)
+#pragma unroll
+        for (int j = decltype(J0)::value; j < decltype(J1)::value; ++j)
+          ex[(i * WTF + j) * WAVE] = eltx4{(elt)acc[i][j][0], (elt)acc[i][j][1], (elt)acc[i][j][2], (elt)acc[i][j][3]};
+    };
+    auto finish = [&](auto J0, auto J1, auto GATE) {
+#pragma unroll
+      for (int j = decltype(J0)::value; j < decltype(J1)::value; ++j) {
+        const int t = t0 + (wt * WTF + j) * 16 + r16;
+        if ((t >> 4) >= x_tt) continue;        // the token tile does not exist
+#pragma unroll
+        for (int i = 0; i < WNF; ++i) {
+          const int c = n0 + i * 16 + gq * 4;
+          if (c >= I) continue;
+          const eltx4 other = ex[(i * WTF + j) * WAVE];
+          eltx4 o = eltx4{0, 0, 0, 0};         // rows past T inside the last tile: zeros, as the separate kernel writes them
+          if (t < T) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const float own = (float)(elt)acc[i][j][r], oth = (float)other[r];
+              o[r] = (elt)glu<OUT == OUT_CLIP ? MLORA_GLU_CLIPPED : MLORA_GLU_SILU>(decltype(GATE)::value ? own : oth, decltype(GATE)::value ? oth : own, ga);
+            }
+          }
+          *reinterpret_cast<eltx4*>((elt*)yv + ((size_t)(c >> 5) * x_tt + (t >> 4)) * 512 + ((c & 31) >> 3) * 128 + (t & 15) * 8 + (c & 7)) = o;
+        }
+      }
+    };
+    typedef std::integral_constant<int, 0> Z;
+    typedef std::integral_constant<int, H0> Hf;
+    typedef std::integral_constant<int, WTF> W;
+    if (wn == 0) give(Hf(), W());
+    else give(Z(), Hf());
+    __syncthreads();
+    if (wn == 0) finish(Z(), Hf(), std::true_type());
+    else finish(Hf(), W(), std::false_type());
+    return;
+  }
   if constexpr (OUT == OUT_F16) {
     // 16 tokens x (16 WNF) columns at a time through the wave's staging buffer: D[n][t] fragments in, token rows out
     elt* ostage = smem + wave * PP_OUT_ELEMS;
@@ -1056,34 +1109,34 @@ MidShape gemm_mid_shape(int T, int K, int N, int ksplit_max) {
 
 template <int OUT, int FT, int FN, bool GX = false>
 int launch_gemm_mid_shape(void* y, float* part, int ld_part, int ksplit, const elt* xf, int x_tt, const elt* Wp, int T, int K, int N,
-                          hipStream_t s, int gx_rows = 0, long gx_stride = 0) {
+                          hipStream_t s, int gx_rows = 0, long gx_stride = 0, const GluArgs& ga = GluArgs()) {
   constexpr size_t lds = (size_t)mid_stages(FT) * MID_KS * (FN + FT) * 512 * sizeof(elt);
   static_assert(lds >= (size_t)PP_WAVES * PP_OUT_ELEMS * sizeof(elt), "the output staging fits the ring");
   static const hipError_t configured =               // the attribute is per kernel, set once per process, by one thread
       hipFuncSetAttribute((const void*)gemm_mid_kernel<OUT, FT, FN, GX>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (configured != hipSuccess)
     return mlora_set_error(MLORA_ERR_LAUNCH, "linear_frag: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(configured));
-  const dim3 grid(ceil_div(N, FN * 16), ksplit, ceil_div(T, FT * 16));
-  hipLaunchKernelGGL((gemm_mid_kernel<OUT, FT, FN, GX>), grid, dim3(PP_WAVES * WAVE), lds, s, y, part, ld_part, xf, x_tt, Wp, T, K, N, gx_rows, gx_stride);
+  const dim3 grid(ceil_div(N, FN * 16), ksplit, ceil_div(T, FT * 16));       // (a gated product: ceil(I / (8 FN)) is the same)
+  hipLaunchKernelGGL((gemm_mid_kernel<OUT, FT, FN, GX>), grid, dim3(PP_WAVES * WAVE), lds, s, y, part, ld_part, xf, x_tt, Wp, T, K, N, gx_rows, gx_stride, ga);
   return MLORA_OK;
 }
 
 template <int OUT>
 int launch_gemm_mid(void* y, float* part, int ld_part, const MidShape& m, const elt* xf, int x_tt, const elt* Wp, int T, int K, int N,
-                    hipStream_t s) {
-  if (m.ft == 8) {
-    if (m.fn == 4) return launch_gemm_mid_shape<OUT, 8, 4>(y, part, ld_part, m.ksplit, xf, x_tt, Wp, T, K, N, s);
-    if (m.fn == 6) return launch_gemm_mid_shape<OUT, 8, 6>(y, part, ld_part, m.ksplit, xf, x_tt, Wp, T, K, N, s);
-    return launch_gemm_mid_shape<OUT, 8, 8>(y, part, ld_part, m.ksplit, xf, x_tt, Wp, T, K, N, s);
-  }
-  if (m.ft == 12) {
-    if (m.fn == 4) return launch_gemm_mid_shape<OUT, 12, 4>(y, part, ld_part, m.ksplit, xf, x_tt, Wp, T, K, N, s);
-    if (m.fn == 6) return launch_gemm_mid_shape<OUT, 12, 6>(y, part, ld_part, m.ksplit, xf, x_tt, Wp, T, K, N, s);
-    return launch_gemm_mid_shape<OUT, 12, 8>(y, part, ld_part, m.ksplit, xf, x_tt, Wp, T, K, N, s);
-  }
-  if (m.fn == 4) return launch_gemm_mid_shape<OUT, 16, 4>(y, part, ld_part, m.ksplit, xf, x_tt, Wp, T, K, N, s);
-  if (m.fn == 6) return launch_gemm_mid_shape<OUT, 16, 6>(y, part, ld_part, m.ksplit, xf, x_tt, Wp, T, K, N, s);
-  return launch_gemm_mid_shape<OUT, 16, 8>(y, part, ld_part, m.ksplit, xf, x_tt, Wp, T, K, N, s);
+                    hipStream_t s, const GluArgs& ga = GluArgs()) {
+#define MLORA_MID(FT, FN) \
+  if (m.ft == FT && m.fn == FN) return launch_gemm_mid_shape<OUT, FT, FN>(y, part, ld_part, m.ksplit, xf, x_tt, Wp, T, K, N, s, 0, 0, ga)
+  MLORA_MID(8, 4);
+  MLORA_MID(8, 6);
+  MLORA_MID(8, 8);
+  MLORA_MID(12, 4);
+  MLORA_MID(12, 6);
+  MLORA_MID(12, 8);
+  MLORA_MID(16, 4);
+  MLORA_MID(16, 6);
+  MLORA_MID(16, 8);
+#undef MLORA_MID
+  return mlora_set_error(MLORA_ERR_UNSUPPORTED, "linear_frag: no block of %d x %d fragments", m.ft, m.fn);
 }
 
 template <int OUT, int FT, int FN, int WT_, int WN_>
@@ -1224,9 +1277,33 @@ extern "C" int mlora_linear_frag_clipglu(void* act, const void* xf, const void* 
               "linear_frag_clipglu: need I %% 32 == 0 (T=%d K=%d I=%d)", T, K, I);
   MLORA_CHECK(mlora_gemm_frag_preferred(T, K, 2 * I) && (((uintptr_t)xf | (uintptr_t)act) & 15) == 0, MLORA_ERR_UNSUPPORTED,
               "linear_frag_clipglu: only shapes of the persistent GEMM (mlora_gemm_frag_preferred; T=%d K=%d N=%d)", T, K, 2 * I);
-  const int e = launch_gemm_pp<OUT_CLIP>(act, (const elt*)xf, 0, mlora_frag_tiles(T), (const elt*)Wp, T, K, 2 * I, (hipStream_t)stream,
-                                         PPLora(), GluArgs{scale, limit, alpha});
-  return e ? e : mlora_launch_status("linear_frag_clipglu");
+  return mlora_linear_frag_glu(act, xf, Wp, T, K, I, MLORA_GLU_CLIPPED, scale, limit, alpha, stream);
+}
+
+// act = the gated product of [gate | up] = xf . Wp^T for more than 64 tokens, on the kernel that the plain linear takes at that size.  A product
+// behind the linear writes and reads T x 2 I elements once more and costs a launch (a floor of 2.5 us); what is left in its place is the exchange
+// of half a block through LDS.  Linear and product behind it -> here, in a row of launches (K, I): 512, 1376 at 65 / 512 / 1024 tokens 7.6 / 9.9 /
+// 13.3 -> 6.3 / 6.7 / 8.9 us; 2048, 5632: 14.7 / 34.8 / 52.3 -> 13.1 / 31.3 / 49.3; 2880, 2880: 17.4 / 28.6 / 42.7 -> 15.9 / 25.1 / 39.8; 4096,
+// 11008 at 65 / 512: 31.6 / 87.7 -> 30.0 / 82.9 (weights from HBM each time).  Never slower on the mid-size kernel, so there is no rule.
+extern "C" int mlora_linear_frag_glu(void* act, const void* xf, const void* Wp, int T, int K, int I, int kind, float scale, float limit, float alpha,
+                                     void* stream) {
+  MLORA_CHECK(act && xf && Wp, MLORA_ERR_INVALID, "linear_frag_glu: null pointer");
+  MLORA_CHECK(kind == MLORA_GLU_SILU || kind == MLORA_GLU_CLIPPED, MLORA_ERR_INVALID, "linear_frag_glu: bad kind %d", kind);
+  MLORA_CHECK(T > 64 && K > 0 && K % 32 == 0 && I > 0 && I % 32 == 0 && I <= (1 << 29) && (((uintptr_t)xf | (uintptr_t)act) & 15) == 0,
+              MLORA_ERR_UNSUPPORTED, "linear_frag_glu: more than 64 tokens, K and I in whole 32, aligned operands (T=%d K=%d I=%d)", T, K, I);
+  const GluArgs ga{scale, limit, alpha};
+  const elt *x = (const elt*)xf, *W = (const elt*)Wp;
+  const int tt = mlora_frag_tiles(T);
+  hipStream_t s = (hipStream_t)stream;
+  int e;
+  if (mlora_gemm_frag_preferred(T, K, 2 * I) || persistent_pays(T, K, 2 * I, false)) {
+    e = kind == MLORA_GLU_SILU ? launch_gemm_pp<OUT_SILU>(act, x, 0, tt, W, T, K, 2 * I, s) : launch_gemm_pp<OUT_CLIP>(act, x, 0, tt, W, T, K, 2 * I, s, PPLora(), ga);
+  } else {
+    MLORA_CHECK(ceil_div(T, 128) <= 65535, MLORA_ERR_UNSUPPORTED, "linear_frag_glu: T=%d too large", T);
+    const MidShape m = gemm_mid_shape(T, K, 2 * I, 1);
+    e = kind == MLORA_GLU_SILU ? launch_gemm_mid<OUT_SILU>(act, nullptr, 0, m, x, tt, W, T, K, 2 * I, s) : launch_gemm_mid<OUT_CLIP>(act, nullptr, 0, m, x, tt, W, T, K, 2 * I, s, ga);
+  }
+  return e ? e : mlora_launch_status("linear_frag_glu");
 }
 
 #ifndef MLORA_ELT_BF16      // the adapter kernels are fp16

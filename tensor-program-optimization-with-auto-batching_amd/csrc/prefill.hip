@@ -191,10 +191,12 @@ extern "C" int mlora_prefill(const mlora_prefill_plan* p, void* stream) {
     const int n_gl = live_of(gate_up, 2, gl);
     if (T <= 64 && L.gate_up_il_p && n_gl == 0) {
       STEP(mlora_gemv_frag_silu(act, xn, L.gate_up_il_p, T, H, I, stream));
-    } else if (T > 64 && mlora_gemm_frag_preferred(T, H, 2 * I) && (n_gl == 0 || (p->blk_adapter && !p->tok_rest))) {
+    } else if (T > 64 && n_gl == 0) {
+      STEP(mlora_linear_frag_glu(act, xn, L.gate_up_p, T, H, I, MLORA_GLU_SILU, 0.f, 0.f, 0.f, stream));
+    } else if (T > 64 && mlora_gemm_frag_preferred(T, H, 2 * I) && p->blk_adapter && !p->tok_rest) {
       mlora_fused_lora f[MAXP];
-      if (n_gl) STEP(halves(xn, H, gl, n_gl, f));
-      STEP(mlora_linear_frag_silu(act, xn, L.gate_up_p, T, H, I, n_gl ? f : nullptr, n_gl, n_gl ? p->blk_adapter : nullptr, n_gl ? r : 0, stream));
+      STEP(halves(xn, H, gl, n_gl, f));
+      STEP(mlora_linear_frag_silu(act, xn, L.gate_up_p, T, H, I, f, n_gl, p->blk_adapter, r, stream));
     } else {
       STEP(linear(gu, MLORA_F16, MLORA_STORE, xn, L.gate_up_p, H, 2 * I, gate_up, 2, nullptr));
       STEP(mlora_silu_mul(act, MLORA_FRAG, gu, gu + I, 2 * I, T, I, stream));

@@ -230,8 +230,8 @@ def gate_up_clipglu(x, W, W_il, scale, limit, alpha, out):
         if T <= 64:
             check(L.mlora_gemv_frag_clipglu(out.data.data_ptr(), x.data.data_ptr(), W_il.data.data_ptr(), *args), x.dtype)
             return out
-        if ops._size(x.dtype, "mlora_gemm_frag_preferred", T, K, I2):
-            check(L.mlora_linear_frag_clipglu(out.data.data_ptr(), x.data.data_ptr(), W.data.data_ptr(), *args), x.dtype)
+        if K % 32 == 0 and I2 % 64 == 0:
+            check(L.mlora_linear_frag_glu(out.data.data_ptr(), x.data.data_ptr(), W.data.data_ptr(), *args[:3], ops.GLU_CLIPPED, *args[3:]), x.dtype)
             return out
     return clipglu_mul(ops.linear(x, W), scale, limit, alpha, out)
 
@@ -257,8 +257,8 @@ def gate_up_silu(x, W, W_il, out):
         if T <= 64:
             check(L.mlora_gemv_frag_silu(out.data.data_ptr(), x.data.data_ptr(), W_il.data.data_ptr(), T, K, I2 // 2, _stream()), x.dtype)
             return out
-        if ops._size(x.dtype, "mlora_gemm_frag_preferred", T, K, I2):
-            check(L.mlora_linear_frag_silu(out.data.data_ptr(), x.data.data_ptr(), W.data.data_ptr(), T, K, I2 // 2, None, 0, None, 0, _stream()),
+        if K % 32 == 0 and I2 % 64 == 0:
+            check(L.mlora_linear_frag_glu(out.data.data_ptr(), x.data.data_ptr(), W.data.data_ptr(), T, K, I2 // 2, ops.GLU_SILU, 0.0, 0.0, 0.0, _stream()),
                   x.dtype)
             return out
     return silu_mul(ops.linear(x, W), out)

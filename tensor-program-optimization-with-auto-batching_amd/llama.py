@@ -482,16 +482,18 @@ class LlamaForCausalLM(CausalLM):
         return y
 
     def _gate_up_silu(self, fuse, x, W, l, projs, adapters):
-        """silu(gate) * up in fragment order out of the persistent GEMM of the fused gate/up projection: without
-        adapters on these projections, or with their deltas as extra k-steps when every 256-token block of the pass
+        """silu(gate) * up in fragment order out of the GEMM of the fused gate/up projection: without
+        adapters on these projections, or (the persistent kernel) with their deltas as extra k-steps when every 256-token block of the pass
         agrees on one adapter.  Returns None where that does not apply (shape, a block that mixes adapters, a rank
         or a mix of adapter types that the extra k-steps do not take)."""
         T, K = x.shape
         N = W.shape[0]
-        if not isinstance(x, ops.FragActivation) or not isinstance(W, ops.PackedWeight) or (N // 2) % 32 or not ops.gemm_frag_preferred(T, K, N):
+        if not isinstance(x, ops.FragActivation) or not isinstance(W, ops.PackedWeight) or (N // 2) % 32:
             return None
         if not adapters or not self._targets(l, *(p for p, _, _ in projs)):
-            return ops.linear_frag_silu(x, W)
+            return ops.linear_frag_glu(x, W)
+        if not ops.gemm_frag_preferred(T, K, N):
+            return None
         if fuse is None or fuse[3] is not None:
             return None
         lt, ids, blk, _ = fuse

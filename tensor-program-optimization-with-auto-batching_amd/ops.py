@@ -12,7 +12,7 @@ import struct
 import torch
 
 from . import _lib
-from ._lib import F16, F32, ROWMAJOR, FRAG, STORE, ACCUMULATE, lib
+from ._lib import F16, F32, ROWMAJOR, FRAG, STORE, ACCUMULATE, GLU_SILU, GLU_CLIPPED, lib
 
 _BUCKET = struct.Struct("@PPiif4x")          # mlora_lora_bucket
 _LIB_OF = {torch.float16: "float16", torch.bfloat16: "bfloat16", torch.float32: "float32"}
@@ -496,6 +496,19 @@ def linear_frag_silu(x: FragActivation, W: PackedWeight, projs=(), blk_adapter=N
     check(lib().mlora_linear_frag_silu(out.data.data_ptr(), x.data.data_ptr(), W.data.data_ptr(), T, K, I,
                                        C.cast(arr, C.c_void_p) if projs else None, len(projs),
                                        _dev(blk_adapter, torch.int32) if projs else None, r, _stream()))
+    return out
+
+
+def linear_frag_glu(x: FragActivation, W: PackedWeight) -> FragActivation:
+    """silu(gate) * up of the fused gate/up projection `W` [2I, K] for more than 64 tokens, in fragment order: the product leaves whichever
+    kernel `linear(x, W)` takes (same bits as that and `silu_mul`)."""
+    T, K = x.shape
+    N, K2 = W.shape
+    if K2 != K or N % 2:
+        raise ValueError(f"linear_frag_glu: x{x.shape} vs W{W.shape}")
+    out = FragActivation(T, N // 2, x.device, dtype=x.dtype)
+    check(lib_of(W.dtype).mlora_linear_frag_glu(out.data.data_ptr(), x.data.data_ptr(), W.data.data_ptr(), T, K, N // 2, GLU_SILU, 0.0, 0.0, 0.0, _stream()),
+          W.dtype)
     return out
 
 

@@ -1677,3 +1677,34 @@ def test_gather_mm_segments_of_few_tokens(ops, T, segs, r, y32):
         assert bool(((y.double() - want).abs() <= room).all())
         assert torch.equal(y[~live], y0[~live]) and torch.equal(y[:, :32], y0[:, :32]) and torch.equal(y[:, -24:], y0[:, -24:])
         assert torch.equal(y[:, 32 + cols[0]:offs[1]], y0[:, 32 + cols[0]:offs[1]])
+
+
+@pytest.mark.parametrize("T", [65, 129, 144, 177, 193, 300, 520])
+@pytest.mark.parametrize("K,I", [(96, 32), (1056, 5600), (64, 11008), (2048, 1408), (2080, 2816)])
+@pytest.mark.parametrize("dt,kind", [(torch.float16, "silu"), (torch.bfloat16, "silu"), (torch.bfloat16, "clip")])
+def test_gated_product_out_of_the_linear(ops, T, K, I, dt, kind):
+    """Every block shape of the mid-size kernel, ragged tokens and channels: the bits of the linear and the separate product, zeros for the tokens
+    past T of the last tile; nothing behind it."""
+    D = load_pkg("decoder_ops")
+    g = torch.Generator(device=DEV).manual_seed(T + K + I)
+    x = torch.randn((T, K), generator=g, device=DEV).to(dt)
+    W = ops.PackedWeight((torch.randn((2 * I, K), generator=g, device=DEV) * K ** -0.5 * 2).to(dt))
+    f = ops.FragActivation.pack(x)
+    n = f.data.numel() // K * I
+    room = torch.full((n + 4096,), float("nan"), dtype=dt, device=DEV)
+    out = ops.FragActivation(T, I, DEV, data=room[:n])
+    if kind == "silu":
+        D.gate_up_silu(f, W, None, out)
+        want = D.silu_mul(ops.linear(f, W), ops.FragActivation(T, I, DEV, dtype=dt))
+    else:
+        D.gate_up_clipglu(f, W, None, 0.8, 1.5, 1.702, out)
+        want = D.clipglu_mul(ops.linear(f, W), 0.8, 1.5, 1.702, ops.FragActivation(T, I, DEV, dtype=dt))
+    torch.cuda.synchronize()
+    if kind == "clip" and T * 2 * I > 128 * 65536:       # the persistent kernel takes the clipped product of unrounded sums
+        a, b = out.data.float(), want.data.float()       # |d/dg|, |d/du| of it are below 2.5 here (g, u up to 1.5): two roundings of at most 1.5 * 2^-9, and two of the product
+        assert bool(((a - b).abs() <= 2 * 2.5 * 1.5 * 2.0 ** -9 + 2.0 ** -8 * b.abs()).all())
+    else:
+        assert torch.equal(out.data, want.data)
+    assert bool(room[n:].isnan().all())
+    if kind == "silu" and dt == torch.float16:
+        assert torch.equal(ops.linear_frag_glu(f, W).data, want.data)
