@@ -271,6 +271,22 @@ int mlora_lora_shrink_split(void* const* v_hi, void* const* v_lo, const void* x,
 int mlora_linear_frag_lora(void* y, int y_dtype, int mode, const void* xf, const void* Wp, int T, int K, int N,
                            const mlora_fused_lora* projs, int n_proj, const int32_t* blk_adapter, int r, void* stream);
 
+/* The linear of the mid-size kernel's shapes (more than 64 tokens, below the persistent one's) with the LoRA deltas of any mix of adapters in its
+ * accumulators: y (=|+=) xf . Wp^T + scaling * B[id] (A[id] x) for the rows n_begin[p] .. n_begin[p] + n_rows[p] of up to three projections (of one
+ * rank in {8, 16, 32, 64}, n_ad and scaling), behind the matrix-core shrink of mlora_gather_mm; rounded once.  workspace: n_proj *
+ * mlora_gather_mm_workspace_bytes(T, K, r) bytes.
+ *   mlora_linear_frag_deltas_pay   - whether a shape is served, and faster so than by mlora_linear_frag and mlora_gather_mm where the tokens of the
+ *                                    pass name n_distinct adapters (accumulate: the mode);
+ *   mlora_linear_frag_deltas       - ks > 1 (accumulating only): K slices as mlora_gemv_frag_acc_ksplit, slices 1.. into part[ks - 1][T][N];
+ *   mlora_linear_frag_silu_deltas  - act = silu(gate) * up in fragment order, of the sums rounded to fp16. */
+int mlora_linear_frag_deltas_pay(int T, int K, int N, int accumulate, int r, int n_distinct);
+int mlora_linear_frag_deltas(void* y, int y_dtype, int mode, float* part, int ks, const void* xf, const void* Wp, int T, int K, int N,
+                             const mlora_lora_bucket* projs, int n_proj, const int32_t* n_begin, const int32_t* n_rows,
+                             const int32_t* tok_adapter, void* workspace, size_t workspace_bytes, void* stream);
+int mlora_linear_frag_silu_deltas(void* act, const void* xf, const void* Wp, int T, int K, int I, const mlora_lora_bucket* projs, int n_proj,
+                                  const int32_t* n_begin, const int32_t* n_rows, const int32_t* tok_adapter, void* workspace,
+                                  size_t workspace_bytes, void* stream);
+
 /* Gate/up projection of a prefill-sized token block with the SiLU product in the epilogue of the persistent GEMM:
  *   act = f16( silu(f16(gate)) * f16(up) ),  [gate | up] = xf . Wp^T (+ the LoRA deltas as in mlora_linear_frag_lora),
  * written in MLORA_FRAG order for the down projection; the [T, 2I] projection output never reaches memory.
@@ -612,6 +628,7 @@ typedef struct mlora_prefill_plan {
   void* ws;
   size_t ws_bytes;
   int max_pos, max_blocks, n_pages, n_seq, T, n_rows;
+  int n_distinct;             /* > 0: the adapters that the tokens name, for mlora_linear_frag_deltas where it pays (more than 64 tokens) */
 } mlora_prefill_plan;
 
 size_t mlora_prefill_workspace_bytes(const mlora_prefill_plan* plan);

@@ -54,6 +54,9 @@ SIGNATURES = {
     "mlora_lora_block_adapters": (_i, [_p, _p, _p, _i, _i, _p]),
     "mlora_lora_shrink_split": (_i, [_p, _p, _p, _i, _p, _i, _p, _f, _i, _i, _i, _i, _p, _z, _p]),
     "mlora_linear_frag_lora": (_i, [_p, _i, _i, _p, _p, _i, _i, _i, _p, _i, _p, _i, _p]),
+    "mlora_linear_frag_deltas_pay": (_i, [_i, _i, _i, _i, _i, _i]),
+    "mlora_linear_frag_deltas": (_i, [_p, _i, _i, _p, _i, _p, _p, _i, _i, _i, _p, _i, _p, _p, _p, _p, _z, _p]),
+    "mlora_linear_frag_silu_deltas": (_i, [_p, _p, _p, _i, _i, _i, _p, _i, _p, _p, _p, _p, _z, _p]),
     "mlora_linear_frag_silu": (_i, [_p, _p, _p, _i, _i, _i, _p, _i, _p, _i, _p]),
     "mlora_gemv_frag_lora": (_i, [_p, _i, _i, _p, _p, _i, _i, _i, _p, _p, _i, _p, _i, _i, _p]),
     "mlora_gemv_frag_silu": (_i, [_p, _p, _p, _i, _i, _i, _p]),
@@ -126,7 +129,7 @@ class PrefillPass(C.Structure):
                 ("lora_r", _i), ("lora_n_ad", _i), ("lora_scaling", _f), ("segments", _i), ("layers", _p), ("norm", _p), ("lm_head_p", _p),
                 ("rope_cos", _p), ("rope_sin", _p), ("block_table", _p), ("tok_seq", _p), ("tok_pos", _p), ("tok_adapter", _p), ("blk_adapter", _p),
                 ("tok_rest", _p), ("logits_rows", _p), ("resid", _p), ("logits", _p), ("ws", _p), ("ws_bytes", _z),
-                ("max_pos", _i), ("max_blocks", _i), ("n_pages", _i), ("n_seq", _i), ("T", _i), ("n_rows", _i)]
+                ("max_pos", _i), ("max_blocks", _i), ("n_pages", _i), ("n_seq", _i), ("T", _i), ("n_rows", _i), ("n_distinct", _i)]
 
 
 SIGNATURES["mlora_prefill_workspace_bytes"] = (_z, [C.POINTER(PrefillPass)])

@@ -1223,7 +1223,7 @@ extern "C" int mlora_gather_mm_batch(const void* const* sets, int n_sets, int y_
 // (`splits`) whose partial sums a reader adds in range order.
 template <int R>
 static int gmm_segments_shrink_r(const SegProjs& pj, const f16* x, int frag_tt, const int32_t* ids, int T, int K, int n_ad, float* v,
-                                 BucketFilter bf, hipStream_t s) {
+                                 BucketFilter bf, hipStream_t s, int most = LORA_MAX_KC) {
   const int tiles = ceil_div(T, 16);
   // few token tiles: split K over workgroups so that the shrink still covers the chip (partials fit the workspace,
   // which holds lora_k_split(K).kc slices of [T, r] per projection); the same split whatever the number of
@@ -1231,6 +1231,7 @@ static int gmm_segments_shrink_r(const SegProjs& pj, const f16* x, int frag_tt, 
   int splits = 512 / tiles;
   const int kc = lora_k_split(K).kc;
   if (splits > kc) splits = kc;
+  if (splits > most) splits = most;
   if (splits > K / 128) splits = K / 128;
   if (splits < 1) splits = 1;
   // Up to 1024 tokens the call is taken to be a decode batch (one token per sequence, tiles that mix many adapters);
@@ -1244,6 +1245,7 @@ static int gmm_segments_shrink_r(const SegProjs& pj, const f16* x, int frag_tt, 
     const int quads = ceil_div(tiles, 4);
     splits = 256 / quads;                        // few K ranges: the expand adds the ranges' partial sums per token
     if (splits > kc) splits = kc;
+    if (splits > most) splits = most;
     if (splits > K / 128) splits = K / 128;
     if (splits < 1) splits = 1;
     hipLaunchKernelGGL((lora_shrink_quad_mfma_kernel<R>), dim3(quads, splits, pj.n), dim3(SEG_WAVES * WAVE), 0, s, v, x, frag_tt, pj, ids, T,
@@ -1637,6 +1639,25 @@ extern "C" int mlora_lora_block_adapters(int32_t* blk_adapter, int32_t* tok_rest
   return mlora_launch_status("lora_block_adapters");
 }
 
+// the shrink on the matrix cores of projections that read x into v [n_proj][K ranges][T][r]: the number of ranges (at most `most`)
+static int shrink_ranges(const void* const* A, int n_proj, const f16* x, int frag_tt, const int32_t* ids, int T, int K, int r, int n_ad, float* v, int most,
+                         hipStream_t s) {
+  SegProjs pj = {};
+  for (int i = 0; i < n_proj; ++i) pj.A[i] = (const f16*)A[i];
+  pj.n = n_proj;
+  const BucketFilter bf{nullptr, 0};
+  switch (r) {
+    case 8: return gmm_segments_shrink_r<8>(pj, x, frag_tt, ids, T, K, n_ad, v, bf, s, most);
+    case 16: return gmm_segments_shrink_r<16>(pj, x, frag_tt, ids, T, K, n_ad, v, bf, s, most);
+    case 32: return gmm_segments_shrink_r<32>(pj, x, frag_tt, ids, T, K, n_ad, v, bf, s, most);
+    default: return gmm_segments_shrink_r<64>(pj, x, frag_tt, ids, T, K, n_ad, v, bf, s, most);
+  }
+}
+int mlora_lora_shrink_ranges(const void* const* A, int n_proj, const void* xf, const int32_t* tok_adapter, int T, int K, int r, int n_ad, float* v, int most,
+                             void* stream) {
+  return shrink_ranges(A, n_proj, (const f16*)xf, mlora_frag_tiles(T), tok_adapter, T, K, r, n_ad, v, most, (hipStream_t)stream);
+}
+
 extern "C" int mlora_lora_shrink_split(void* const* v_hi, void* const* v_lo, const void* x, int x_layout, const void* const* A, int n_proj,
                                        const int32_t* tok_adapter, float scaling, int T, int K, int r, int n_ad, void* workspace,
                                        size_t workspace_bytes, void* stream) {
@@ -1647,19 +1668,12 @@ extern "C" int mlora_lora_shrink_split(void* const* v_hi, void* const* v_lo, con
               "lora_shrink_split: needs T > 64, K %% 32 == 0 (T=%d K=%d layout=%d)", T, K, x_layout);
   MLORA_CHECK(workspace && workspace_bytes >= (size_t)n_proj * mlora_gather_mm_workspace_bytes(T, K, r), MLORA_ERR_WORKSPACE,
               "lora_shrink_split: workspace of %zu bytes given, %zu needed", workspace_bytes, (size_t)n_proj * mlora_gather_mm_workspace_bytes(T, K, r));
-  SegProjs pj = {};
   for (int i = 0; i < n_proj; ++i) {
     MLORA_CHECK(A[i] && v_hi[i] && v_lo[i], MLORA_ERR_INVALID, "lora_shrink_split: null table or output of projection %d", i);
-    pj.A[i] = (const f16*)A[i];
   }
-  pj.n = n_proj;
   hipStream_t s = (hipStream_t)stream;
-  const int frag_tt = x_layout == MLORA_FRAG ? mlora_frag_tiles(T) : 0;
   float* v = (float*)workspace;
-  const BucketFilter bf{nullptr, 0};
-  int splits;
-  if (r == 32) splits = gmm_segments_shrink_r<32>(pj, (const f16*)x, frag_tt, tok_adapter, T, K, n_ad, v, bf, s);
-  else splits = gmm_segments_shrink_r<64>(pj, (const f16*)x, frag_tt, tok_adapter, T, K, n_ad, v, bf, s);
+  const int splits = shrink_ranges(A, n_proj, (const f16*)x, x_layout == MLORA_FRAG ? mlora_frag_tiles(T) : 0, tok_adapter, T, K, r, n_ad, v, LORA_MAX_KC, s);
   VSplitOut vo = {};
   for (int i = 0; i < n_proj; ++i) {
     vo.vh[i] = (f16*)v_hi[i];

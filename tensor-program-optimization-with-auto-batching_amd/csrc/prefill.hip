@@ -115,15 +115,19 @@ extern "C" int mlora_prefill(const mlora_prefill_plan* p, void* stream) {
     return live;
   };
   // deltas of projections that read x and own column ranges of y, for the tokens of ids
+  struct Buckets { mlora_lora_bucket bk[MAXP]; int32_t c[MAXP], nc[MAXP]; };
+  auto buckets_of = [&](const Proj* pj, int n) {
+    Buckets b = {};
+    for (int i = 0; i < n; ++i) {
+      b.bk[i] = mlora_lora_bucket{pj[i].t->A, pj[i].t->B, r, n_ad, sc};
+      b.c[i] = pj[i].c0;
+      b.nc[i] = pj[i].n;
+    }
+    return b;
+  };
   auto deltas = [&](void* y, int y_dtype, int ldy, const void* x, int K, const Proj* pj, int n, const int32_t* ids) -> int {
     if (n == 0) return MLORA_OK;
-    mlora_lora_bucket bk[MAXP];
-    int32_t c[MAXP], nc[MAXP];
-    for (int i = 0; i < n; ++i) {
-      bk[i] = mlora_lora_bucket{pj[i].t->A, pj[i].t->B, r, n_ad, sc};
-      c[i] = pj[i].c0;
-      nc[i] = pj[i].n;
-    }
+    const auto [bk, c, nc] = buckets_of(pj, n);
     if (p->segments)
       return mlora_gather_mm_segments(y, y_dtype, ldy, x, MLORA_FRAG, bk, n, c, nc, ids, T, K, lora_ws, at.lora_bytes, stream);
     if (n >= 2)
@@ -144,7 +148,8 @@ extern "C" int mlora_prefill(const mlora_prefill_plan* p, void* stream) {
     }
     return mlora_lora_shrink_split(hi, lo, x, MLORA_FRAG, A, n, p->tok_adapter, sc, T, K, r, n_ad, lora_ws, at.lora_bytes, stream);
   };
-  // y (=|+=) x . W^T with the deltas of pj: inside the GEMM for the blocks that agree on an adapter where the shape has that form.  ks (added
+  // y (=|+=) x . W^T with the deltas of pj: inside the GEMM where the shape has that form - of the persistent kernel for the blocks that agree
+  // on an adapter, of the mid-size one for all where that pays.  ks (added
   // to fp32 only): the K slices whose partials the next norm adds.
   auto linear = [&](void* y, int y_dtype, int mode, const void* x, const void* W, int K, int N, const Proj* all, int n_all, int* ks) -> int {
     Proj pj[MAXP];
@@ -157,6 +162,14 @@ extern "C" int mlora_prefill(const mlora_prefill_plan* p, void* stream) {
       STEP(halves(x, K, pj, n, f));
       STEP(mlora_linear_frag_lora(y, y_dtype, mode, x, W, T, K, N, f, n, p->blk_adapter, r, stream));
       return p->tok_rest ? deltas(y, y_dtype, N, x, K, pj, n, p->tok_rest) : MLORA_OK;
+    }
+    if (n > 0 && p->n_distinct > 0 && mlora_linear_frag_deltas_pay(T, K, N, mode == MLORA_ACCUMULATE, r, p->n_distinct)) {
+      if (ks && part) {
+        const int k = mlora_gemv_ksplit(T, K, N);
+        *ks = k > 1 && mlora_gemv_ksplit_bytes(T, N, k) <= at.ksplit_bytes ? k : 1;
+      }
+      const Buckets b = buckets_of(pj, n);
+      return mlora_linear_frag_deltas(y, y_dtype, mode, part, ks ? *ks : 1, x, W, T, K, N, b.bk, n, b.c, b.nc, p->tok_adapter, lora_ws, at.lora_bytes, stream);
     }
     if (ks && part) {
       const int riding = T <= 64 && n > 0 && !p->segments ? mlora_gemv_shrink_rows(K, 1, 1) : 0;
@@ -197,6 +210,9 @@ extern "C" int mlora_prefill(const mlora_prefill_plan* p, void* stream) {
       mlora_fused_lora f[MAXP];
       STEP(halves(xn, H, gl, n_gl, f));
       STEP(mlora_linear_frag_silu(act, xn, L.gate_up_p, T, H, I, f, n_gl, p->blk_adapter, r, stream));
+    } else if (p->n_distinct > 0 && mlora_linear_frag_deltas_pay(T, H, 2 * I, 0, r, p->n_distinct)) {
+      const Buckets b = buckets_of(gl, n_gl);
+      STEP(mlora_linear_frag_silu_deltas(act, xn, L.gate_up_p, T, H, I, b.bk, n_gl, b.c, b.nc, p->tok_adapter, lora_ws, at.lora_bytes, stream));
     } else {
       STEP(linear(gu, MLORA_F16, MLORA_STORE, xn, L.gate_up_p, H, 2 * I, gate_up, 2, nullptr));
       STEP(mlora_silu_mul(act, MLORA_FRAG, gu, gu + I, 2 * I, T, I, stream));

@@ -392,6 +392,11 @@ class LlamaForCausalLM(CausalLM):
                     blk, rest = ops.lora_block_adapters(ids, lt.n_adapters)
                     rest = rest if bool((rest >= 0).any()) else None
                 fuse = (lt, ids, blk, None if rest is None else {tid: rest})
+        # below the persistent kernel's sizes the mid-size one takes any mix of adapters, where the host knows that they are few
+        near = None
+        if host_ids is not None and tok_adapter and "multi" not in tok_adapter and len(tok_adapter) == 1 and frag and T > 64 and not is_decode:
+            (tid, ids), = tok_adapter.items()
+            near = (self.lora_types[tid], ids, distinct_adapters(host_ids[tid], self.lora_types[tid].n_adapters))
         o_shares = None
         if tok_adapter and "multi" not in tok_adapter and len(tok_adapter) == 1 and is_decode and T > 64 and frag:
             (tid, ids), = tok_adapter.items()
@@ -403,6 +408,8 @@ class LlamaForCausalLM(CausalLM):
             xn = ops.rmsnorm(resid, L["ln1"], s.rms_norm_eps, frag=frag, parts=parts)
             qkv_projs = (("q_proj", 0, q_sz), ("k_proj", q_sz, kv_sz), ("v_proj", q_sz + kv_sz, kv_sz))
             qkv = self._fused_linear(fuse, xn, L["qkv"], l, qkv_projs) if fuse else None
+            if qkv is None and near:
+                qkv = (self._delta_linear(near, xn, L["qkv"], l, qkv_projs) or (None,))[0]
             if qkv is None:
                 qkv = ops.linear(xn, L["qkv"])
                 if tok_adapter:
@@ -419,7 +426,10 @@ class LlamaForCausalLM(CausalLM):
                 ops.lora_expand_shares(resid, vpart, o_sh[1], o_shares[1], o_shares[0].scaling)
             else:
                 attn = kv.attention_with_fused_qkv(l, qkv, s.num_attention_heads, frag=frag)
-                if fuse and self._fused_linear(fuse, attn, L["o"], l, (("o_proj", 0, H),), resid=resid) is not None:
+                done = self._delta_linear(near, attn, L["o"], l, (("o_proj", 0, H),), resid, ks_ws) if near else None
+                if done is not None:
+                    parts = done[1]
+                elif fuse and self._fused_linear(fuse, attn, L["o"], l, (("o_proj", 0, H),), resid=resid) is not None:
                     parts = None
                 else:
                     parts = self._linear_acc(attn, L["o"], resid, ks_ws, riding(l, "o_proj", lora_tids, T, q_sz))
@@ -433,7 +443,7 @@ class LlamaForCausalLM(CausalLM):
             else:
                 gu_projs = (("gate_proj", 0, I), ("up_proj", I, I))
                 # a prefill-sized pass: the SiLU product leaves the GEMM itself wherever no token needs a separate delta
-                act = self._gate_up_silu(fuse, xn, L["gate_up"], l, gu_projs, bool(tok_adapter)) if frag and T > 64 else None
+                act = self._gate_up_silu(fuse, near, xn, L["gate_up"], l, gu_projs, bool(tok_adapter)) if frag and T > 64 else None
                 if act is None:
                     gu = self._fused_linear(fuse, xn, L["gate_up"], l, gu_projs) if fuse else None
                     if gu is None:
@@ -441,7 +451,10 @@ class LlamaForCausalLM(CausalLM):
                         if tok_adapter:
                             self._lora_group(gu, xn, l, gu_projs, tok_adapter, segs)
                     act = ops.silu_mul(gu, frag=frag)
-            if fuse and self._fused_linear(fuse, act, L["down"], l, (("down_proj", 0, H),), resid=resid) is not None:
+            done = self._delta_linear(near, act, L["down"], l, (("down_proj", 0, H),), resid, ks_ws) if near else None
+            if done is not None:
+                parts = done[1]
+            elif fuse and self._fused_linear(fuse, act, L["down"], l, (("down_proj", 0, H),), resid=resid) is not None:
                 parts = None
             else:
                 parts = self._linear_acc(act, L["down"], resid, ks_ws, riding(l, "down_proj", lora_tids, T, I))
@@ -481,7 +494,20 @@ class LlamaForCausalLM(CausalLM):
                 self._lora_group(y, x, l, projs, rest)
         return y
 
-    def _gate_up_silu(self, fuse, x, W, l, projs, adapters):
+    def _delta_linear(self, near, x, W, l, projs, resid=None, ks_ws=None):
+        """The base linear of `projs` with the deltas of whatever adapters the tokens name inside the mid-size kernel: (y, K-slice
+        partials or None), or None where that does not serve the shape or does not pay."""
+        lt, ids, n_distinct = near
+        T, K = x.shape
+        live = [(c0, n, lt.tables.get((l, proj))) for proj, c0, n in projs]
+        live = [e for e in live if e[2] is not None]
+        if not live or not n_distinct or not ops.linear_frag_deltas_pay(T, K, W.shape[0], resid is not None, lt.r, n_distinct):
+            return None
+        fused = [(*tab, lt.scaling, c0, n) for c0, n, tab in live]
+        return ops.linear_frag_deltas(x, W, fused, ids, self._workspace(T, K, lt.r), out=resid, accumulate=resid is not None,
+                                      ks_ws=ks_ws if resid is not None else None)
+
+    def _gate_up_silu(self, fuse, near, x, W, l, projs, adapters):
         """silu(gate) * up in fragment order out of the GEMM of the fused gate/up projection: without
         adapters on these projections, or (the persistent kernel) with their deltas as extra k-steps when every 256-token block of the pass
         agrees on one adapter.  Returns None where that does not apply (shape, a block that mixes adapters, a rank
@@ -492,6 +518,12 @@ class LlamaForCausalLM(CausalLM):
             return None
         if not adapters or not self._targets(l, *(p for p, _, _ in projs)):
             return ops.linear_frag_glu(x, W)
+        if near and near[2] and ops.linear_frag_deltas_pay(T, K, N, False, near[0].r, near[2]):
+            lt, ids, _ = near
+            live = [(c0, n, lt.tables.get((l, proj))) for proj, c0, n in projs]
+            live = [e for e in live if e[2] is not None]
+            if live:
+                return ops.linear_frag_silu_deltas(x, W, [(*tab, lt.scaling, c0, n) for c0, n, tab in live], ids, self._workspace(T, K, lt.r))
         if not ops.gemm_frag_preferred(T, K, N):
             return None
         if fuse is None or fuse[3] is not None:
@@ -557,6 +589,7 @@ class LlamaForCausalLM(CausalLM):
         if lt is not None:
             d_ids = ops.upload(torch.from_numpy(ids), self.device)
             p.lora_r, p.lora_n_ad, p.lora_scaling, p.tok_adapter = lt.r, lt.n_adapters, lt.scaling, ptr(d_ids, i32)
+            p.n_distinct = distinct_adapters(ids, lt.n_adapters)
             if T <= 64:
                 p.segments = self.segments_pay(T, max(kv._cur[1]), tid)
             elif lt.r in (32, 64) and ops.gemm_frag_preferred(T, s.hidden_size, s.hidden_size):
@@ -683,6 +716,11 @@ def block_adapters(ids, n_ad):
     blk = np.where((pad == pad[:, :1]).all(1), pad[:, 0], -1).astype(np.int32)
     rest = np.where(np.repeat(blk, 256)[:T] >= 0, -1, ids).astype(np.int32)
     return blk, rest if (rest >= 0).any() else None
+
+
+def distinct_adapters(ids, n_ad):
+    """How many adapters the tokens of ids (host) name."""
+    return int(np.unique(ids[(ids >= 0) & (ids < n_ad)]).size)
 
 
 def _host_i32(a):

@@ -473,6 +473,60 @@ def linear_frag_lora(x: FragActivation, W: PackedWeight, projs, blk_adapter, r: 
     return out
 
 
+def linear_frag_deltas_pay(T: int, K: int, N: int, accumulate: bool, r: int, n_distinct: int) -> bool:
+    """Whether `linear_frag_deltas` serves a shape and is the faster form for tokens that name n_distinct adapters."""
+    return bool(lib().mlora_linear_frag_deltas_pay(T, K, N, int(accumulate), r, n_distinct))
+
+
+def _delta_args(who, x, W, projs, tok_adapter, workspace):
+    import ctypes as C
+    from ._lib import LoraBucket
+    T, K = x.shape
+    N, K2 = W.shape
+    n_ad, r, _ = projs[0][0].shape
+    n = len(projs)
+    b, c, nc = (LoraBucket * n)(), (C.c_int32 * n)(), (C.c_int32 * n)()
+    if K2 != K or tok_adapter.shape != (T,):
+        raise ValueError(f"{who}: x{x.shape} vs W{W.shape}, {tuple(tok_adapter.shape)} token ids")
+    for i, (A, B, scaling, n0, rows) in enumerate(projs):
+        if A.shape != (n_ad, r, K) or B.shape != (n_ad, rows, r):
+            raise ValueError(f"{who}: A{tuple(A.shape)} B{tuple(B.shape)} for {rows} rows of K={K}")
+        b[i].A, b[i].B, b[i].r, b[i].n_ad, b[i].scaling, c[i], nc[i] = _dev(A, torch.float16, "A"), _dev(B, torch.float16, "B"), r, n_ad, float(scaling), n0, rows
+    return (C.cast(b, C.c_void_p), n, C.cast(c, C.c_void_p), C.cast(nc, C.c_void_p), _dev(tok_adapter, torch.int32), _dev(workspace, torch.float32),
+            workspace.numel() * 4, _stream())
+
+
+def linear_frag_deltas(x: FragActivation, W: PackedWeight, projs, tok_adapter, workspace, out=None, out_dtype=torch.float16, accumulate=False, ks_ws=None):
+    """`linear(x, W)` with the LoRA deltas of `projs` = [(A [n_ad, r, K], B [n_ad, rows, r], scaling, first row, rows), ...] of tokens that name any
+    adapters, inside the GEMM (shapes of the mid-size kernel).  accumulate: into `out`; with fp32 scratch `ks_ws` K may be split as in
+    `linear_acc_ksplit`.  Returns (out, KSplitParts or None)."""
+    T, K = x.shape
+    N = W.shape[0]
+    if out is None and not accumulate:
+        out = torch.empty((T, N), dtype=out_dtype, device=x.device)
+    if out is None or out.shape != (T, N):
+        raise ValueError(f"linear_frag_deltas: out for {(T, N)}")
+    args = _delta_args("linear_frag_deltas", x, W, projs, tok_adapter, workspace)
+    ks = _size(W.dtype, "mlora_gemv_ksplit", T, K, N) if ks_ws is not None else 1
+    if ks > 1 and ks_ws.numel() * 4 < _size(W.dtype, "mlora_gemv_ksplit_bytes", T, N, ks):
+        ks = 1
+    check(lib().mlora_linear_frag_deltas(_dev(out), _dt(out), ACCUMULATE if accumulate else STORE, _dev(ks_ws, torch.float32) if ks > 1 else None, ks,
+                                         x.data.data_ptr(), W.data.data_ptr(), T, K, N, *args))
+    return out, KSplitParts(ks_ws, ks, N) if ks > 1 else None
+
+
+def linear_frag_silu_deltas(x: FragActivation, W: PackedWeight, projs, tok_adapter, workspace) -> FragActivation:
+    """silu(gate) * up of the fused gate/up projection with the deltas of gate and / or up rows, as `linear_frag_deltas`; in fragment order."""
+    T, K = x.shape
+    N = W.shape[0]
+    if N % 2:
+        raise ValueError(f"linear_frag_silu_deltas: W{W.shape}")
+    args = _delta_args("linear_frag_silu_deltas", x, W, projs, tok_adapter, workspace)
+    out = FragActivation(T, N // 2, x.device)
+    check(lib().mlora_linear_frag_silu_deltas(out.data.data_ptr(), x.data.data_ptr(), W.data.data_ptr(), T, K, N // 2, *args))
+    return out
+
+
 def linear_frag_silu(x: FragActivation, W: PackedWeight, projs=(), blk_adapter=None, r: int = 0, out: FragActivation = None) -> FragActivation:
     """silu(gate) * up of the fused gate/up projection `W` [2I, K] in the epilogue of the persistent GEMM, in fragment
     order.  `projs` as for linear_frag_lora, over the gate rows (first row 0) and / or the up rows (first row I); every

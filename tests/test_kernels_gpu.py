@@ -1708,3 +1708,51 @@ def test_gated_product_out_of_the_linear(ops, T, K, I, dt, kind):
     assert bool(room[n:].isnan().all())
     if kind == "silu" and dt == torch.float16:
         assert torch.equal(ops.linear_frag_glu(f, W).data, want.data)
+
+
+@pytest.mark.parametrize("T,K,rows", [(65, 256, (32, 16, 32)), (130, 1056, (2048, 512, 528)), (137, 4096, (4096,)), (193, 288, (11008,)), (300, 2080, (1024, 1040)),
+                                      (260, 512, (2752, 2752)), (385, 320, (4096, 4096))])
+@pytest.mark.parametrize("r,who", [(8, "one"), (16, "one"), (16, "mixed"), (32, "segments"), (64, "segments"), (64, "mixed")])
+def test_deltas_inside_the_mid_size_linear(ops, T, K, rows, r, who):
+    """Block shapes of the mid-size kernel, ranks, blocks that several projections share (or a part without adapter), one adapter, several in segments,
+    one of nine per token: against fp64, with the bits of the plain linear where no delta belongs."""
+    n_ad, scaling, eps, g = 9, 0.5, 2.0 ** -24, torch.Generator(device=DEV).manual_seed(T + K + r)
+    rnd = lambda *s: torch.randn(s, generator=g, device=DEV)
+    x, A, B = rnd(T, K).half(), [(rnd(n_ad, r, K) * K ** -0.5).half() for _ in rows], [rnd(n_ad, n, r).half() for n in rows]
+    N, at = sum(rows) + 48, 16                                  # sixteen rows ahead and thirty-two behind that no projection has
+    Wd = (rnd(N, K) * K ** -0.5).half()
+    W, t = ops.PackedWeight(Wd), np.arange(T)
+    ids = {"one": np.where(t % 7 == 3, -1, 4), "segments": np.where(t < 40, -1, t // 50), "mixed": t * 5 % 11 - 1}[who].astype(np.int32)
+    d_ids, f = torch.from_numpy(ids).to(DEV), ops.FragActivation.pack(x)
+    ok = (d_ids >= 0) & (d_ids < n_ad)
+    want = x.double() @ Wd.double().T
+    slack = x.double().abs() @ Wd.double().abs().T * K * eps    # K fp32 additions, whatever their order
+    projs = []
+    for A_, B_, n in zip(A, B, rows):
+        for i in range(n_ad):
+            m = d_ids == i
+            a, b = A_[i].double(), B_[i].double()
+            v = scaling * (x[m].double() @ a.T)
+            dv = scaling * (x[m].double().abs() @ a.abs().T) * K * eps + v.abs() * 2.0 ** -21 + eps      # ... of the shrink, the halves' 22 bits, and their smallest step
+            want[m, at:at + n] += v @ b.T
+            slack[m, at:at + n] += dv @ b.abs().T + v.abs() @ b.abs().T * (2 * r) * eps
+        projs.append((A_, B_, scaling, at, n))
+        at += n
+    slack += want.abs() * (2 * r) * eps                         # the delta's products join a sum of about the result's size
+    lora_ws = torch.full((3 * ops._size(torch.float16, "mlora_gather_mm_workspace_bytes", T, K, r) // 4,), float("nan"), device=DEV)
+    y, parts = ops.linear_frag_deltas(f, W, projs, d_ids, lora_ws)
+    assert parts is None and bool(((y.double() - want).abs() <= slack + want.abs() * 2.0 ** -11 + eps).all())
+    plain = ops.linear(f, W)
+    assert torch.equal(y[~ok], plain[~ok]) and torch.equal(y[:, :16], plain[:, :16]) and torch.equal(y[:, at:], plain[:, at:])
+    resid, ws = rnd(T, N), torch.empty(3 * T * N, dtype=torch.float32, device=DEV)
+    for scratch in (None, ws):
+        acc, parts = ops.linear_frag_deltas(f, W, projs, d_ids, lora_ws, out=resid.clone(), accumulate=True, ks_ws=scratch)
+        if parts is not None:
+            acc = acc + ws[:(parts.ks - 1) * T * N].view(parts.ks - 1, T, N).sum(0)
+        assert bool(((acc.double() - resid.double() - want).abs() <= slack + (resid.double().abs() + want.abs()) * 8 * eps).all())
+    if len(rows) == 2 and rows[0] == rows[1]:
+        I = rows[0]
+        W2 = ops.PackedWeight((rnd(2 * I, K) * K ** -0.5).half())
+        gu = [(*p[:3], i * I, I) for i, p in enumerate(projs)]
+        y2, _ = ops.linear_frag_deltas(f, W2, gu, d_ids, lora_ws)
+        assert torch.equal(ops.linear_frag_silu_deltas(f, W2, gu, d_ids, lora_ws).data, ops.silu_mul(y2, frag=True).data)
