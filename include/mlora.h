@@ -271,8 +271,8 @@ int mlora_lora_shrink_split(void* const* v_hi, void* const* v_lo, const void* x,
 int mlora_linear_frag_lora(void* y, int y_dtype, int mode, const void* xf, const void* Wp, int T, int K, int N,
                            const mlora_fused_lora* projs, int n_proj, const int32_t* blk_adapter, int r, void* stream);
 
-/* The linear of the mid-size kernel's shapes (more than 64 tokens, below the persistent one's) with the LoRA deltas of any mix of adapters in its
- * accumulators: y (=|+=) xf . Wp^T + scaling * B[id] (A[id] x) for the rows n_begin[p] .. n_begin[p] + n_rows[p] of up to three projections (of one
+/* The linear of up to 64 tokens (N in whole 16) or of the mid-size kernel's shapes (below the persistent one's) with the LoRA deltas of any mix of
+ * adapters in its accumulators: y (=|+=) xf . Wp^T + scaling * B[id] (A[id] x) for the rows n_begin[p] .. n_begin[p] + n_rows[p] of up to three projections (of one
  * rank in {8, 16, 32, 64}, n_ad and scaling), behind the matrix-core shrink of mlora_gather_mm; rounded once.  workspace: n_proj *
  * mlora_gather_mm_workspace_bytes(T, K, r) bytes.
  *   mlora_linear_frag_deltas_pay   - whether a shape is served, and faster so than by mlora_linear_frag and mlora_gather_mm where the tokens of the
@@ -591,9 +591,10 @@ typedef struct mlora_decode_plan {
   size_t lora_ws_bytes;
   float* ksplit_ws;           /* partials of the K-split o_proj / down_proj GEMVs, or NULL (no split) */
   size_t ksplit_ws_bytes;     /* >= mlora_gemv_ksplit_bytes over both projections (with their appended rows) */
-  int lora_segments;          /* up to 64 sequences: the deltas as launches of their own (mlora_gather_mm_segments) instead of riding in the
-                               * linear, attention and norm launches - for larger ranks, and few adapters of many tokens.  With lora_dense
-                               * only those of gate and up.  Needs what mlora_gather_mm_segments needs of the shapes */
+  int lora_segments;          /* > 0 (how many adapters the tokens name): up to 64 sequences, the deltas of a linear behind a shrink launch of their own, in the linear
+                               * (mlora_linear_frag_deltas) or after it (mlora_gather_mm_segments), instead of riding in the linear, attention
+                               * and norm launches - for larger ranks, and few adapters of many tokens.  With lora_dense only those of gate
+                               * and up.  Needs what those need of the shapes */
 } mlora_decode_plan;
 
 int mlora_decode_step(const mlora_decode_plan* plan, void* stream);

@@ -180,6 +180,22 @@ extern "C" int mlora_decode_step(const mlora_decode_plan* p, void* stream) {
   void* ws_o = ws + (size_t)3 * kq * slot;
   void* ws_down = ws + (size_t)(3 * kq + 1) * slot;
   const size_t down_bytes = lora ? p->lora_ws_bytes - (size_t)(3 * kq + 1) * slot : 0;   // (a smaller K may take more than the largest)
+  // a linear with them: inside the linear behind the shrink where that pays (done is then set), else nothing yet
+  auto seg_linear = [&](void* y, int y_dtype, int mode, int ks, const void* x, const void* W, int K, int N, const mlora_lora_proj* lp, const int32_t* col,
+                        const int32_t* ncol, int n, bool& done) -> int {
+    mlora_lora_bucket bk[3];
+    int32_t c[3], nc[3];
+    int live = 0;
+    for (int i = 0; i < n; ++i)
+      if (lp[i].A) {
+        bk[live] = mlora_lora_bucket{lp[i].A, lp[i].B, r, n_ad, sc};
+        c[live] = col[i];
+        nc[live++] = ncol[i];
+      }
+    done = live > 0 && mlora_linear_frag_deltas_pay(T, K, N, mode == MLORA_ACCUMULATE, r, p->lora_segments);
+    if (!done) return MLORA_OK;
+    return mlora_linear_frag_deltas(y, y_dtype, mode, p->ksplit_ws, ks, x, W, T, K, N, bk, live, c, nc, p->tok_adapter, p->lora_ws, p->lora_ws_bytes, stream);
+  };
   auto seg_deltas = [&](void* y, int y_dtype, int ldy, const void* x, int K, const mlora_lora_proj* lp, const int32_t* col, const int32_t* ncol, int n) -> int {
     mlora_lora_bucket bk[3];
     int32_t c[3], nc[3];
@@ -252,11 +268,13 @@ extern "C" int mlora_decode_step(const mlora_decode_plan* p, void* stream) {
                                     p->ctx, p->rope_cos, p->rope_sin, p->max_pos, T, Hq, Hkv, D, p->n_pages, p->n_seq, ws_qkv,
                                     dense ? kq : 0, B3, p->tok_adapter, sc, H, r, n_ad, stream));
     } else {
-      STEP(mlora_gemv_frag(qkv, MLORA_F16, MLORA_STORE, p->xn, L.qkv_p, T, H, qkv_sz, stream));
-      if (segs) {
-        const mlora_lora_proj lp[3] = {L.lora[MLORA_Q], L.lora[MLORA_K], L.lora[MLORA_V]};
-        const int32_t col[3] = {0, q_sz, q_sz + kv_sz}, ncol[3] = {q_sz, kv_sz, kv_sz};
-        STEP(seg_deltas(qkv, MLORA_F16, qkv_sz, p->xn, H, lp, col, ncol, 3));
+      const mlora_lora_proj lp[3] = {L.lora[MLORA_Q], L.lora[MLORA_K], L.lora[MLORA_V]};
+      const int32_t col[3] = {0, q_sz, q_sz + kv_sz}, ncol[3] = {q_sz, kv_sz, kv_sz};
+      bool done = false;
+      if (segs) STEP(seg_linear(qkv, MLORA_F16, MLORA_STORE, 1, p->xn, L.qkv_p, H, qkv_sz, lp, col, ncol, 3, done));
+      if (!done) {
+        STEP(mlora_gemv_frag(qkv, MLORA_F16, MLORA_STORE, p->xn, L.qkv_p, T, H, qkv_sz, stream));
+        if (segs) STEP(seg_deltas(qkv, MLORA_F16, qkv_sz, p->xn, H, lp, col, ncol, 3));
       }
       if (o_via_ride)
         STEP(mlora_rope_attn_decode_oshrink(p->attn, MLORA_FRAG, qkv, L.k_cache, L.v_cache, p->block_table, p->max_blocks, p->rows,
@@ -275,10 +293,12 @@ extern "C" int mlora_decode_step(const mlora_decode_plan* p, void* stream) {
                                 0.f, 0, 0, 0, stream));
     } else {
       const int ks_o = ksplit_of(q_sz, o_lora);
-      STEP(acc_gemv(p->attn, L.o_p, q_sz, L.lora[MLORA_O], ws_o, ks_o));
-      if (segs) {
-        const int32_t col[1] = {0}, ncol[1] = {H};
-        STEP(seg_deltas(p->resid, MLORA_F32, H, p->attn, q_sz, &L.lora[MLORA_O], col, ncol, 1));
+      const int32_t col[1] = {0}, ncol[1] = {H};
+      bool done = false;
+      if (segs) STEP(seg_linear(p->resid, MLORA_F32, MLORA_ACCUMULATE, ks_o, p->attn, L.o_p, q_sz, H, &L.lora[MLORA_O], col, ncol, 1, done));
+      if (!done) {
+        STEP(acc_gemv(p->attn, L.o_p, q_sz, L.lora[MLORA_O], ws_o, ks_o));
+        if (segs) STEP(seg_deltas(p->resid, MLORA_F32, H, p->attn, q_sz, &L.lora[MLORA_O], col, ncol, 1));
       }
       STEP(norm(L.ln2, o_lora ? L.lora[MLORA_O].B : nullptr, ws_o, q_sz, ks_o));
     }
@@ -286,10 +306,13 @@ extern "C" int mlora_decode_step(const mlora_decode_plan* p, void* stream) {
     if (L.gate_up_il_p && !gu_lora) {
       STEP(mlora_gemv_frag_silu(p->act, p->xn, L.gate_up_il_p, T, H, I, stream));
     } else {
-      STEP(mlora_gemv_frag(gu, MLORA_F16, MLORA_STORE, p->xn, L.gate_up_p, T, H, 2 * I, stream));
-      if (gu_segs) {
-        const mlora_lora_proj lp[2] = {L.lora[MLORA_GATE], L.lora[MLORA_UP]};
-        const int32_t col[2] = {0, I}, ncol[2] = {I, I};
+      const mlora_lora_proj lp[2] = {L.lora[MLORA_GATE], L.lora[MLORA_UP]};
+      const int32_t col[2] = {0, I}, ncol[2] = {I, I};
+      bool done = false;
+      if (gu_segs) STEP(seg_linear(gu, MLORA_F16, MLORA_STORE, 1, p->xn, L.gate_up_p, H, 2 * I, lp, col, ncol, 2, done));
+      if (!done) STEP(mlora_gemv_frag(gu, MLORA_F16, MLORA_STORE, p->xn, L.gate_up_p, T, H, 2 * I, stream));
+      if (done) {
+      } else if (gu_segs) {
         STEP(seg_deltas(gu, MLORA_F16, 2 * I, p->xn, H, lp, col, ncol, 2));
       } else {
         STEP(delta(gu, MLORA_F16, 2 * I, p->xn, L.lora[MLORA_GATE], H, I));
@@ -299,10 +322,12 @@ extern "C" int mlora_decode_step(const mlora_decode_plan* p, void* stream) {
     }
     const bool down_lora = lora && !segs && L.lora[MLORA_DOWN].A;
     pending_ks = ksplit_of(I, down_lora);
-    STEP(acc_gemv(p->act, L.down_p, I, L.lora[MLORA_DOWN], ws_down, pending_ks));
-    if (segs) {
-      const int32_t col[1] = {0}, ncol[1] = {H};
-      STEP(seg_deltas(p->resid, MLORA_F32, H, p->act, I, &L.lora[MLORA_DOWN], col, ncol, 1));
+    const int32_t col[1] = {0}, ncol[1] = {H};
+    bool done = false;
+    if (segs) STEP(seg_linear(p->resid, MLORA_F32, MLORA_ACCUMULATE, pending_ks, p->act, L.down_p, I, H, &L.lora[MLORA_DOWN], col, ncol, 1, done));
+    if (!done) {
+      STEP(acc_gemv(p->act, L.down_p, I, L.lora[MLORA_DOWN], ws_down, pending_ks));
+      if (segs) STEP(seg_deltas(p->resid, MLORA_F32, H, p->act, I, &L.lora[MLORA_DOWN], col, ncol, 1));
     }
     pending_B = down_lora ? L.lora[MLORA_DOWN].B : nullptr;   // expanded inside the next RMSNorm launch
   }

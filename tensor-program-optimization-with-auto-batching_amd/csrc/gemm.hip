@@ -11,7 +11,7 @@
 // bits.
 #include <type_traits>
 
-#include "common.h"
+#include "lora_device.h"
 #include "moe.h"
 
 int mlora_check_linear(const char* who, const void* y, int y_dtype, int mode, const void* x, int ldx, const void* W,
@@ -785,21 +785,9 @@ int launch_gemm_pp(void* y, const elt* x, int ldx, int x_tt, const elt* Wp, int 
 constexpr int MID_KS = 2;                      // 32-k steps per stage
 constexpr int mid_stages(int FT) { return FT == 16 ? 3 : 4; }
 
-// LORA: the deltas of any mix of adapters, y = x . W^T + v . B[id]^T, come into the accumulators ahead of the first step, while the ring fills: a
-// wave takes the adapters of its own tokens in turn, with v - the sum of the shrink's K ranges - as fp16 hi and lo halves and zeros for the
-// tokens of the others, straight from memory into registers.  Behind the last step, as further steps of the ring, the same took 11 us: cold code
-// and addresses that nothing hides.  Projections are row ranges of the fused weight.  137 tokens of one adapter of rank 16, us: q, k, v (K 4096,
-// N 12288) linear 31.0, shrink 5.4, expand 7.7 -> shrink 6.5, linear 35.0; o (N 4096, four K slices) 15.6, 5.0, 8.3 -> 6.5, 18.4.
-constexpr int MID_MAX_RANGES = 4;             // of the shrink's K: as many as are in flight together in registers
-struct MidLora {
-  const elt* B[3];            // [n_ad][n_rows][r]
-  int n_begin[3], n_rows[3];
-  const float* v;             // [n_proj][ranges][T][r], rows of tokens without adapter not written
-  const int32_t* ids;         // [T]: outside 0 .. n_ad - 1 no adapter
-  float scaling;
-  int n_proj, r, n_ad, ranges;
-};
-
+// LORA: the deltas of any mix of adapters (linear_add_deltas) come into the accumulators ahead of the first step, while the ring fills.  Behind
+// the last step, as further steps of the ring, the same took 11 us: cold code and addresses that nothing hides.  137 tokens of one adapter of rank
+// 16, us: q, k, v (K 4096, N 12288) linear 31.0, shrink 5.4, expand 7.7 -> shrink 6.5, linear 35.0; o (N 4096, four K slices) 15.6, 5.0, 8.3 -> 6.5, 18.4.
 // GX: the rows are groups of gx_rows (a multiple of 16 FN) that read activations of their own, gx_stride elements apart.
 // A gated product (OUT_SILU, OUT_CLIP): Wp is the fused [2 I, K] matrix (N = 2 I), a block FN / 2 tiles of gate rows and the up rows of the same
 // channels, so that the waves wn = 0 hold the one and wn = 1 the other; they exchange halves through LDS, rounded to elements as a linear
@@ -808,7 +796,7 @@ template <int OUT, int FT, int FN, bool GX = false, bool LORA = false>
 __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_mid_kernel(void* __restrict__ yv, float* __restrict__ part, int ld_part,
                                                                     const elt* __restrict__ xf, int x_tt, const elt* __restrict__ Wp,
                                                                     int T, int K, int N, int gx_rows = 0, long gx_stride = 0,
-                                                                    GluArgs ga = GluArgs(), MidLora lo = MidLora()) {
+                                                                    GluArgs ga = GluArgs(), LinearDeltas lo = LinearDeltas()) {
   constexpr bool GLU = OUT == OUT_SILU || OUT == OUT_CLIP;
   constexpr int MID_STAGES = mid_stages(FT);
   constexpr int SF = FN + FT;                  // fragments of one 32-k step: weights, then tokens
@@ -957,66 +945,10 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_mid_kernel(void* __res
   for (int i = 0; i < MID_STAGES - 1; ++i) issue();
   if constexpr (LORA) {
     if (blockIdx.y == 0 && t0 + wt * WTF * 16 < T) {             // uniform: slice 0, a wave with tokens
-      const int r16 = lane & 15, g8 = (lane >> 4) * 8, row0 = tile_row(wn * WNF) * 16;
+      int row0[WNF];
 #pragma unroll
-      for (int j = 0; j < WTF; ++j) left[j] = left[j] < lo.n_ad ? left[j] : -1;
-      for (;;) {
-        int a = -1;
-#pragma unroll
-        for (int j = 0; j < WTF; ++j) {
-          const unsigned long long todo = __ballot(left[j] >= 0);
-          if (a < 0 && todo) a = __builtin_amdgcn_readlane(left[j], __builtin_ctzll(todo));
-        }
-        if (a < 0) break;
-        for (int p = 0; p < lo.n_proj; ++p) {
-          // projection p's, by masks: the compiler turns a choice into an address that depends on p, and `lo` would live in scratch memory
-          const unsigned long long m0 = 0ull - (p == 0), m1 = 0ull - (p == 1), m2 = 0ull - (p == 2);
-          const elt* Bp = (const elt*)(((uintptr_t)lo.B[0] & m0) | ((uintptr_t)lo.B[1] & m1) | ((uintptr_t)lo.B[2] & m2));
-          const int begin = (lo.n_begin[0] & (int)m0) | (lo.n_begin[1] & (int)m1) | (lo.n_begin[2] & (int)m2);
-          const int rows = (lo.n_rows[0] & (int)m0) | (lo.n_rows[1] & (int)m1) | (lo.n_rows[2] & (int)m2);
-          if (row0 >= begin + rows || row0 + WNF * 16 <= begin) continue;      // uniform
-          const float* vp = lo.v + (size_t)p * lo.ranges * T * lo.r;
-          for (int c0 = 0; c0 < lo.r; c0 += 32) {
-            const int c = c0 + g8;             // this lane's eight ranks (past r: zeros)
-            eltx8 bf[WNF], hi[WTF], low[WTF];
-#pragma unroll
-            for (int i = 0; i < WNF; ++i) {
-              const int row = row0 + i * 16 + r16 - begin;
-              bf[i] = c < lo.r && row >= 0 && row < rows ? ld8(Bp + ((size_t)a * rows + row) * lo.r + c) : eltx8{0, 0, 0, 0, 0, 0, 0, 0};
-            }
-#pragma unroll
-            for (int j = 0; j < WTF; ++j) {
-              const int t = t0 + (wt * WTF + j) * 16 + r16;
-              const float* q = vp + (size_t)(t < T ? t : T - 1) * lo.r + (c < lo.r ? c : 0);
-              f32x4 x0[MID_MAX_RANGES], x1[MID_MAX_RANGES], s0 = f32x4{0.f, 0.f, 0.f, 0.f}, s1 = s0;
-#pragma unroll
-              for (int s = 0; s < MID_MAX_RANGES; ++s) {         // (past the last range: that one again, not added)
-                const float* qs = q + (size_t)(s < lo.ranges ? s : lo.ranges - 1) * T * lo.r;
-                x0[s] = *reinterpret_cast<const f32x4*>(qs);
-                x1[s] = *reinterpret_cast<const f32x4*>(qs + 4);
-              }
-#pragma unroll
-              for (int s = 0; s < MID_MAX_RANGES; ++s) {
-                s0 = s < lo.ranges ? s0 + x0[s] : s0;
-                s1 = s < lo.ranges ? s1 + x1[s] : s1;
-              }
-              const bool mine = left[j] == a && c < lo.r;        // (others': whatever lies there is replaced)
-#pragma unroll
-              for (int e = 0; e < 8; ++e) {
-                const float f = mine ? (e < 4 ? s0[e & 3] : s1[e & 3]) * lo.scaling : 0.f;
-                hi[j][e] = (elt)f;
-                low[j][e] = (elt)(f - (float)hi[j][e]);
-              }
-            }
-#pragma unroll
-            for (int i = 0; i < WNF; ++i)
-#pragma unroll
-              for (int j = 0; j < WTF; ++j) acc[i][j] = mfma_16x16x32(bf[i], low[j], mfma_16x16x32(bf[i], hi[j], acc[i][j]));
-          }
-        }
-#pragma unroll
-        for (int j = 0; j < WTF; ++j) left[j] = left[j] == a ? -1 : left[j];
-      }
+      for (int i = 0; i < WNF; ++i) row0[i] = tile_row(wn * WNF + i) * 16;
+      linear_add_deltas<WNF, WTF>(acc, lo, left, T, t0 + wt * WTF * 16, row0, lane, 0, 1);
     }
   }
   wait_next();
@@ -1196,7 +1128,7 @@ MidShape gemm_mid_shape(int T, int K, int N, int ksplit_max) {
 
 template <int OUT, int FT, int FN, bool GX = false, bool LORA = false>
 int launch_gemm_mid_shape(void* y, float* part, int ld_part, int ksplit, const elt* xf, int x_tt, const elt* Wp, int T, int K, int N,
-                          hipStream_t s, int gx_rows = 0, long gx_stride = 0, const GluArgs& ga = GluArgs(), const MidLora& lo = MidLora()) {
+                          hipStream_t s, int gx_rows = 0, long gx_stride = 0, const GluArgs& ga = GluArgs(), const LinearDeltas& lo = LinearDeltas()) {
   constexpr size_t lds = (size_t)mid_stages(FT) * MID_KS * (FN + FT) * 512 * sizeof(elt);
   static_assert(lds >= (size_t)PP_WAVES * PP_OUT_ELEMS * sizeof(elt), "the output staging fits the ring");
   static const hipError_t configured =               // the attribute is per kernel, set once per process, by one thread
@@ -1211,7 +1143,7 @@ int launch_gemm_mid_shape(void* y, float* part, int ld_part, int ksplit, const e
 
 template <int OUT, bool LORA = false>
 int launch_gemm_mid(void* y, float* part, int ld_part, const MidShape& m, const elt* xf, int x_tt, const elt* Wp, int T, int K, int N,
-                    hipStream_t s, const GluArgs& ga = GluArgs(), const MidLora& lo = MidLora()) {
+                    hipStream_t s, const GluArgs& ga = GluArgs(), const LinearDeltas& lo = LinearDeltas()) {
 #define MLORA_MID(FT, FN) \
   if (m.ft == FT && m.fn == FN) return launch_gemm_mid_shape<OUT, FT, FN, false, LORA>(y, part, ld_part, m.ksplit, xf, x_tt, Wp, T, K, N, s, 0, 0, ga, lo)
   MLORA_MID(8, 4);
@@ -1400,18 +1332,24 @@ static bool mid_deltas_serve(int T, int K, int N, bool accumulate) {
   return T > 64 && ceil_div(T, 128) <= 65535 && K >= 32 && K % 32 == 0 && !mlora_gemm_frag_preferred(T, K, N) && !persistent_pays(T, K, N, accumulate);
 }
 
-// What the deltas cost in there is a round trip to memory per 32 ranks and adapter, ahead of the first step; on their own they are a launch that reads and
+// What the deltas cost in there is a round trip to memory per 32 ranks and adapter (up to 64 tokens: per tile of 16, and shared by eight waves); on their own they are a launch that reads and
 // writes y.  Passes of two layers, us, on their own / in the linear, by rounds: 1 (7B, q, k, v and o, rank 16, 80 tokens) 423 / 404, (600 tokens) 1066 /
 // 1012, (hidden 1024, all seven, 200 tokens) 314 / 285; 2 (7B, all, rank 64, 300 tokens) 915 / 829; 3 (rank 16, 8 x 60 tokens, q, k, v, o) 774 / 737; 6
 // (rank 64, 4 x 90, all) 1022 / 1004; 7 (rank 16, 8 x 60) 778 / 752; 14 (rank 64, 8 x 50, all) 1002 / 1010, (hidden 1024, 8 x 150) 548 / 559.
+// Decode steps by rounds x tiles: 1 (7B, rank 32, 2 requests, all) 407 / 371; 2 (rank 64, one, all) 385 / 340, (hidden 1024) 197 / 145; 4 (rank 16, 64 of
+// one adapter, q, k, v, o) 408 / 408; 6 (rank 32, 16) 340 / 331; 15 (hidden 1024, rank 32, 40) 170 / 160; 28 (rank 64, 32 of seven) 391 / 387; 56
+// (rank 64, 32 of fourteen) 431 / 448, (hidden 1024) 216 / 202; 64 (64 of eight, all) 675 / 750; 120 (rank 32, 64 of thirty) 497 / 600.
 extern "C" int mlora_linear_frag_deltas_pay(int T, int K, int N, int accumulate, int r, int n_distinct) {
-  return mid_deltas_serve(T, K, N, accumulate != 0) && n_distinct > 0 && (long)ceil_div(r, 32) * n_distinct <= 8;
+  const long rounds = (long)ceil_div(r, 32) * n_distinct;
+  if (T <= 64) return T > 0 && K > 0 && K % 32 == 0 && N % 16 == 0 && rounds > 0 && rounds * ceil_div(T, 16) <= 32;
+  return mid_deltas_serve(T, K, N, accumulate != 0) && rounds > 0 && rounds <= 8;
 }
 
 // the shrink of the projections into the workspace (gather_mm.hip), and what the kernel above reads of it
 int mlora_lora_shrink_ranges(const void* const* A, int n_proj, const void* xf, const int32_t* tok_adapter, int T, int K, int r, int n_ad, float* v, int most,
                              void* stream);
-static int mid_lora(const char* who, MidLora& lo, const mlora_lora_bucket* projs, int n_proj, const int32_t* n_begin, const int32_t* n_rows, const void* xf,
+int mlora_gemv_deltas(void* y, int y_dtype, int mode, float* part, int ks, const void* xf, const void* Wp, int T, int K, int N, const LinearDeltas& ld, void* stream);
+static int mid_lora(const char* who, LinearDeltas& lo, const mlora_lora_bucket* projs, int n_proj, const int32_t* n_begin, const int32_t* n_rows, const void* xf,
                     const int32_t* ids, int T, int K, int N, void* workspace, size_t workspace_bytes, void* stream) {
   MLORA_CHECK(projs && n_begin && n_rows && ids && n_proj >= 1 && n_proj <= 3, MLORA_ERR_INVALID, "%s: null pointer or n_proj=%d outside 1..3", who, n_proj);
   const int r = projs[0].r, n_ad = projs[0].n_ad;
@@ -1432,7 +1370,7 @@ static int mid_lora(const char* who, MidLora& lo, const mlora_lora_bucket* projs
   }
   lo.v = (const float*)workspace; lo.ids = ids; lo.scaling = projs[0].scaling;
   lo.n_proj = n_proj; lo.r = r; lo.n_ad = n_ad;
-  lo.ranges = mlora_lora_shrink_ranges(A, n_proj, xf, ids, T, K, r, n_ad, (float*)workspace, MID_MAX_RANGES, stream);
+  lo.ranges = mlora_lora_shrink_ranges(A, n_proj, xf, ids, T, K, r, n_ad, (float*)workspace, DELTA_RANGES, stream);
   return MLORA_OK;
 }
 
@@ -1440,12 +1378,13 @@ extern "C" int mlora_linear_frag_deltas(void* y, int y_dtype, int mode, float* p
                                         const mlora_lora_bucket* projs, int n_proj, const int32_t* n_begin, const int32_t* n_rows,
                                         const int32_t* tok_adapter, void* workspace, size_t workspace_bytes, void* stream) {
   if (int e = mlora_check_linear("linear_frag_deltas", y, y_dtype, mode, xf, K, Wp, T, K, N)) return e;
-  MLORA_CHECK(mid_deltas_serve(T, K, N, mode == MLORA_ACCUMULATE) && ((uintptr_t)xf & 15) == 0, MLORA_ERR_UNSUPPORTED,
-              "linear_frag_deltas: only shapes of the mid-size kernel (mlora_linear_frag_deltas_pay; T=%d K=%d N=%d)", T, K, N);
-  MLORA_CHECK(ks == 1 || (ks > 1 && ks <= 4 && part && mode == MLORA_ACCUMULATE && K / 32 / ks >= 1), MLORA_ERR_INVALID,
+  MLORA_CHECK((T <= 64 ? T > 0 && K % 32 == 0 && N % 16 == 0 : mid_deltas_serve(T, K, N, mode == MLORA_ACCUMULATE)) && ((uintptr_t)xf & 15) == 0,
+              MLORA_ERR_UNSUPPORTED, "linear_frag_deltas: up to 64 tokens, or shapes of the mid-size kernel (mlora_linear_frag_deltas_pay; T=%d K=%d N=%d)", T, K, N);
+  MLORA_CHECK(ks == 1 || (ks > 1 && ks <= 4 && part && mode == MLORA_ACCUMULATE && K / 32 / ks >= (T <= 64 ? 8 : 1)), MLORA_ERR_INVALID,
               "linear_frag_deltas: ks=%d slices (accumulating only), or no partials buffer", ks);
-  MidLora lo = {};
+  LinearDeltas lo = {};
   if (int e = mid_lora("linear_frag_deltas", lo, projs, n_proj, n_begin, n_rows, xf, tok_adapter, T, K, N, workspace, workspace_bytes, stream)) return e;
+  if (T <= 64) return mlora_gemv_deltas(y, y_dtype, mode, part, ks, xf, Wp, T, K, N, lo, stream);
   hipStream_t s = (hipStream_t)stream;
   MidShape m = gemm_mid_shape(T, K, N, ks);
   m.ksplit = ks;                               // the caller's partial buffers were sized for ks slices
@@ -1464,7 +1403,7 @@ extern "C" int mlora_linear_frag_silu_deltas(void* act, const void* xf, const vo
   MLORA_CHECK(act && xf && Wp, MLORA_ERR_INVALID, "linear_frag_silu_deltas: null pointer");
   MLORA_CHECK(I > 0 && I % 32 == 0 && I <= (1 << 29) && mid_deltas_serve(T, K, 2 * I, false) && (((uintptr_t)xf | (uintptr_t)act) & 15) == 0,
               MLORA_ERR_UNSUPPORTED, "linear_frag_silu_deltas: only shapes of the mid-size kernel, I in whole 32 (T=%d K=%d I=%d)", T, K, I);
-  MidLora lo = {};
+  LinearDeltas lo = {};
   if (int e = mid_lora("linear_frag_silu_deltas", lo, projs, n_proj, n_begin, n_rows, xf, tok_adapter, T, K, 2 * I, workspace, workspace_bytes, stream)) return e;
   const int e = launch_gemm_mid<OUT_SILU, true>(act, nullptr, 0, gemm_mid_shape(T, K, 2 * I, 1), (const elt*)xf, mlora_frag_tiles(T), (const elt*)Wp, T, K, 2 * I,
                                                 (hipStream_t)stream, GluArgs(), lo);

@@ -13,6 +13,8 @@
 //       Wp[n/16][k/32][(k%32)/8][n%16][k%8],
 //     so the fragment of (16 rows, 32 k) is one contiguous 1 KiB block and a wave streams consecutive
 //     blocks: every load is a full DRAM page and consecutive k-steps are consecutive addresses.
+#include <type_traits>
+
 #include "lora_device.h"
 
 namespace {
@@ -125,12 +127,16 @@ __global__ __launch_bounds__(GEMV_WAVES* WAVE) void lora_expand_shares_kernel(Lo
 // GX (fragment order): the rows are groups of gx_rows (a multiple of 16 NT) that read activations of their own, gx_stride elements apart;
 // those behind n_main are cut into gx_kq ranges of K, each a workgroup that leaves a block of y2 (so that no unit gets a whole
 // workgroup more than the others).
-template <int NT, int TT, int OUT, bool PACKED, bool XFRAG, bool SHRINK, int PIPE = 4, bool GX = false>   // PIPE: k-steps in flight per wave
+// DELTA: adapter deltas (linear_add_deltas) join the waves' sums behind their last step, a wave every eighth round.  An expand launch of its own takes
+// 7 to 9 us, mostly its way to the first byte; here the rounds take 1 to 2.
+struct NoDeltas {};
+template <int NT, int TT, int OUT, bool PACKED, bool XFRAG, bool SHRINK, int PIPE = 4, bool GX = false, bool DELTA = false>   // PIPE: k-steps in flight per wave
 __global__ __launch_bounds__(GEMV_WAVES* WAVE, (NT * TT > 8 ? 2 : 4)) void gemv_kernel(void* __restrict__ yv, const elt* __restrict__ x, int ldx,
                                                                 const elt* __restrict__ W, int T, int K, int N,
                                                                 LoraShrinkBatch sb, int shrink_blocks, int n_main,
                                                                 float* __restrict__ y2, int ksplit, float* __restrict__ part,
-                                                                LoraDeltaRide dr, int ride_blocks, GluArgs ga, int gx_rows = 0, long gx_stride = 0, int gx_kq = 1) {
+                                                                LoraDeltaRide dr, int ride_blocks, GluArgs ga, int gx_rows = 0, long gx_stride = 0, int gx_kq = 1,
+                                                                std::conditional_t<DELTA, LinearDeltas, NoDeltas> ld = {}) {
   constexpr int TILES = NT * TT;
   constexpr int HT = TILES > 8 ? TILES / 2 : TILES;   // accumulator tiles summed per pass through LDS (64 KiB holds 8)
   constexpr bool RIDE = OUT == OUT_ACC_F32 && PACKED && XFRAG && !SHRINK;   // the launches that may carry delta riders
@@ -225,6 +231,11 @@ __global__ __launch_bounds__(GEMV_WAVES* WAVE, (NT * TT > 8 ? 2 : 4)) void gemv_
     }
   }
   const int S = (kb1 - kb0 - wave + GEMV_WAVES - 1) / GEMV_WAVES;
+  int ids[TT];
+  if constexpr (DELTA) {                           // asked for ahead of the operands
+#pragma unroll
+    for (int j = 0; j < TT; ++j) ids[j] = j * 16 + r16 < T ? ld.ids[j * 16 + r16] : -1;
+  }
   eltx8 a[PIPE][NT], b[PIPE][TT];
   auto load_stage = [&](int u, int s) {
     const bool in = s < S;
@@ -247,6 +258,14 @@ __global__ __launch_bounds__(GEMV_WAVES* WAVE, (NT * TT > 8 ? 2 : 4)) void gemv_
 #pragma unroll
         for (int j = 0; j < TT; ++j) acc[i][j] = mfma_16x16x32(a[u][i], b[u][j], acc[i][j]);
       load_stage(u, s0 + u + PIPE);
+    }
+  }
+  if constexpr (DELTA) {
+    if (slice == 0) {                              // uniform
+      int row0[NT];
+#pragma unroll
+      for (int i = 0; i < NT; ++i) row0[i] = n0 + i * 16;
+      linear_add_deltas<NT, TT, TILES <= 8 && (TT == 4 || NT * TT == 8)>(acc, ld, ids, T, 0, row0, lane, wave, GEMV_WAVES);
     }
   }
 
@@ -530,15 +549,19 @@ __global__ __launch_bounds__(256) void pack_activation_kernel(elt* __restrict__ 
   st8(dst + (size_t)c * 8, v);
 }
 
-template <int NT, int TT, bool PACKED, bool XFRAG, bool SHRINK, int PIPE = 4>
+template <int NT, int TT, bool PACKED, bool XFRAG, bool SHRINK, bool DELTA = false, int PIPE = 4>
 void launch_gemv(void* y, int out, const elt* x, int ldx, const elt* W, int T, int K, int N, hipStream_t s,
-                 const LoraShrinkBatch& sb, int n_main, float* y2, int ksplit = 1, float* part = nullptr,
+                 const std::conditional_t<DELTA, LinearDeltas, NoDeltas>& ld, const LoraShrinkBatch& sb, int n_main, float* y2, int ksplit = 1, float* part = nullptr,
                  const LoraDeltaRide& dr = LoraDeltaRide(), int rblocks = 0) {
   const int sblocks = SHRINK ? ceil_div(lora_shrink_units(sb), GEMV_WAVES) : 0;
   const dim3 grid(ceil_div(N, 16 * NT) * ksplit + sblocks + rblocks), block(GEMV_WAVES * WAVE);
-  if (out == OUT_F16) hipLaunchKernelGGL((gemv_kernel<NT, TT, OUT_F16, PACKED, XFRAG, SHRINK, PIPE>), grid, block, 0, s, y, x, ldx, W, T, K, N, sb, sblocks, n_main, y2, ksplit, part, dr, 0, GluArgs());
-  else if (out == OUT_F32) hipLaunchKernelGGL((gemv_kernel<NT, TT, OUT_F32, PACKED, XFRAG, SHRINK, PIPE>), grid, block, 0, s, y, x, ldx, W, T, K, N, sb, sblocks, n_main, y2, ksplit, part, dr, 0, GluArgs());
-  else hipLaunchKernelGGL((gemv_kernel<NT, TT, OUT_ACC_F32, PACKED, XFRAG, SHRINK, PIPE>), grid, block, 0, s, y, x, ldx, W, T, K, N, sb, sblocks, n_main, y2, ksplit, part, dr, rblocks, GluArgs());
+#define MLORA_GEMV(OUT, RB) \
+  hipLaunchKernelGGL((gemv_kernel<NT, TT, OUT, PACKED, XFRAG, SHRINK, PIPE, false, DELTA>), grid, block, 0, s, y, x, ldx, W, T, K, N, sb, sblocks, n_main, y2, \
+                     ksplit, part, dr, RB, GluArgs(), 0, 0l, 1, ld)
+  if (out == OUT_F16) MLORA_GEMV(OUT_F16, 0);
+  else if (out == OUT_F32) MLORA_GEMV(OUT_F32, 0);
+  else MLORA_GEMV(OUT_ACC_F32, rblocks);
+#undef MLORA_GEMV
 }
 
 // Rows per workgroup.  Every workgroup reads the whole token block, so its L2 traffic is T / (16 NT) of the weight
@@ -564,10 +587,11 @@ int gemv_split_tiles(int tiles, int ksplit) {
   return 4;
 }
 
-template <bool PACKED, bool XFRAG, bool SHRINK = false>
+template <bool PACKED, bool XFRAG, bool SHRINK = false, bool DELTA = false>
 int gemv_dispatch(void* y, int y_dtype, int mode, const void* x, int ldx, const void* W, int T, int K, int N, void* stream,
                   const LoraShrinkBatch& sb = LoraShrinkBatch(), int n_main = -1, float* y2 = nullptr, int ksplit = 1,
-                  float* part = nullptr, const LoraDeltaRide& dr = LoraDeltaRide(), int rblocks = 0) {
+                  float* part = nullptr, const LoraDeltaRide& dr = LoraDeltaRide(), int rblocks = 0,
+                  const std::conditional_t<DELTA, LinearDeltas, NoDeltas>& ld = {}) {
   if (n_main < 0) n_main = N;
   const int out = mode == MLORA_ACCUMULATE ? OUT_ACC_F32 : (y_dtype == MLORA_F32 ? OUT_F32 : OUT_F16);
   hipStream_t s = (hipStream_t)stream;
@@ -577,15 +601,15 @@ int gemv_dispatch(void* y, int y_dtype, int mode, const void* x, int ldx, const 
   if constexpr (PACKED && XFRAG) {
     const int nt = ksplit > 1 && T <= 64 ? gemv_split_tiles(tiles, ksplit) : 4;
     if (nt == 1) {
-      if (T <= 16) launch_gemv<1, 1, PACKED, XFRAG, SHRINK, 4>(y, out, xp, ldx, Wp, T, K, N, s, sb, n_main, y2, ksplit, part, dr, rblocks);
-      else if (T <= 32) launch_gemv<1, 2, PACKED, XFRAG, SHRINK, 4>(y, out, xp, ldx, Wp, T, K, N, s, sb, n_main, y2, ksplit, part, dr, rblocks);
-      else launch_gemv<1, 4, PACKED, XFRAG, SHRINK, 4>(y, out, xp, ldx, Wp, T, K, N, s, sb, n_main, y2, ksplit, part, dr, rblocks);
+      if (T <= 16) launch_gemv<1, 1, PACKED, XFRAG, SHRINK, DELTA, 4>(y, out, xp, ldx, Wp, T, K, N, s, ld, sb, n_main, y2, ksplit, part, dr, rblocks);
+      else if (T <= 32) launch_gemv<1, 2, PACKED, XFRAG, SHRINK, DELTA, 4>(y, out, xp, ldx, Wp, T, K, N, s, ld, sb, n_main, y2, ksplit, part, dr, rblocks);
+      else launch_gemv<1, 4, PACKED, XFRAG, SHRINK, DELTA, 4>(y, out, xp, ldx, Wp, T, K, N, s, ld, sb, n_main, y2, ksplit, part, dr, rblocks);
       return mlora_launch_status("gemv");
     }
     if (nt == 2) {
-      if (T <= 16) launch_gemv<2, 1, PACKED, XFRAG, SHRINK, 4>(y, out, xp, ldx, Wp, T, K, N, s, sb, n_main, y2, ksplit, part, dr, rblocks);
-      else if (T <= 32) launch_gemv<2, 2, PACKED, XFRAG, SHRINK, 4>(y, out, xp, ldx, Wp, T, K, N, s, sb, n_main, y2, ksplit, part, dr, rblocks);
-      else launch_gemv<2, 4, PACKED, XFRAG, SHRINK, 2>(y, out, xp, ldx, Wp, T, K, N, s, sb, n_main, y2, ksplit, part, dr, rblocks);
+      if (T <= 16) launch_gemv<2, 1, PACKED, XFRAG, SHRINK, DELTA, 4>(y, out, xp, ldx, Wp, T, K, N, s, ld, sb, n_main, y2, ksplit, part, dr, rblocks);
+      else if (T <= 32) launch_gemv<2, 2, PACKED, XFRAG, SHRINK, DELTA, 4>(y, out, xp, ldx, Wp, T, K, N, s, ld, sb, n_main, y2, ksplit, part, dr, rblocks);
+      else launch_gemv<2, 4, PACKED, XFRAG, SHRINK, DELTA, 2>(y, out, xp, ldx, Wp, T, K, N, s, ld, sb, n_main, y2, ksplit, part, dr, rblocks);
       return mlora_launch_status("gemv");
     }
     if (T <= 32 && (ksplit > 1 || tiles >= 768)) {
@@ -593,12 +617,12 @@ int gemv_dispatch(void* y, int y_dtype, int mode, const void* x, int ldx, const 
       // 256 units: with four tiles a quarter of the units would stay idle and the others set the time); same bits
       const int n_cu = gemv_n_cu();
       if (ksplit == 1 && n_cu > 0 && tiles % 3 == 0 && tiles / 3 <= n_cu && ceil_div(tiles, 4) < tiles / 3) {
-        if (T <= 16) launch_gemv<3, 1, PACKED, XFRAG, SHRINK, 4>(y, out, xp, ldx, Wp, T, K, N, s, sb, n_main, y2, ksplit, part);
-        else launch_gemv<3, 2, PACKED, XFRAG, SHRINK, 4>(y, out, xp, ldx, Wp, T, K, N, s, sb, n_main, y2, ksplit, part);
+        if (T <= 16) launch_gemv<3, 1, PACKED, XFRAG, SHRINK, DELTA, 4>(y, out, xp, ldx, Wp, T, K, N, s, ld, sb, n_main, y2, ksplit, part);
+        else launch_gemv<3, 2, PACKED, XFRAG, SHRINK, DELTA, 4>(y, out, xp, ldx, Wp, T, K, N, s, ld, sb, n_main, y2, ksplit, part);
         return mlora_launch_status("gemv");
       }
-      if (T <= 16) launch_gemv<4, 1, PACKED, XFRAG, SHRINK, 4>(y, out, xp, ldx, Wp, T, K, N, s, sb, n_main, y2, ksplit, part, dr, rblocks);
-      else launch_gemv<4, 2, PACKED, XFRAG, SHRINK, 3>(y, out, xp, ldx, Wp, T, K, N, s, sb, n_main, y2, ksplit, part, dr, rblocks);
+      if (T <= 16) launch_gemv<4, 1, PACKED, XFRAG, SHRINK, DELTA, 4>(y, out, xp, ldx, Wp, T, K, N, s, ld, sb, n_main, y2, ksplit, part, dr, rblocks);
+      else launch_gemv<4, 2, PACKED, XFRAG, SHRINK, DELTA, 3>(y, out, xp, ldx, Wp, T, K, N, s, ld, sb, n_main, y2, ksplit, part, dr, rblocks);
       return mlora_launch_status("gemv");
     }
   }
@@ -607,25 +631,25 @@ int gemv_dispatch(void* y, int y_dtype, int mode, const void* x, int ldx, const 
   // (just above 256 tiles, one tile per workgroup would leave a second, nearly empty round of workgroups)
   const bool wide = (tiles >= 512 && (!PACKED || tiles % 2 == 0)) || (PACKED && tiles > 256 && tiles < 512);
   if (T <= 16) {
-    if (wide) launch_gemv<2, 1, PACKED, XFRAG, SHRINK>(y, out, xp, ldx, Wp, T, K, N, s, sb, n_main, y2);
-    else launch_gemv<1, 1, PACKED, XFRAG, SHRINK>(y, out, xp, ldx, Wp, T, K, N, s, sb, n_main, y2);
+    if (wide) launch_gemv<2, 1, PACKED, XFRAG, SHRINK, DELTA>(y, out, xp, ldx, Wp, T, K, N, s, ld, sb, n_main, y2);
+    else launch_gemv<1, 1, PACKED, XFRAG, SHRINK, DELTA>(y, out, xp, ldx, Wp, T, K, N, s, ld, sb, n_main, y2);
   } else if (T <= 32) {
-    if (wide) launch_gemv<2, 2, PACKED, XFRAG, SHRINK>(y, out, xp, ldx, Wp, T, K, N, s, sb, n_main, y2);
-    else launch_gemv<1, 2, PACKED, XFRAG, SHRINK>(y, out, xp, ldx, Wp, T, K, N, s, sb, n_main, y2);
+    if (wide) launch_gemv<2, 2, PACKED, XFRAG, SHRINK, DELTA>(y, out, xp, ldx, Wp, T, K, N, s, ld, sb, n_main, y2);
+    else launch_gemv<1, 2, PACKED, XFRAG, SHRINK, DELTA>(y, out, xp, ldx, Wp, T, K, N, s, ld, sb, n_main, y2);
   } else {
     // 33..64 tokens: four token tiles leave registers for two row tiles per wave (x traffic is then twice the weight
     // traffic instead of four times): 5.3 -> 4.4 ms of GEMV per decode step at T = 64
     if constexpr (PACKED && XFRAG) {
       if (ksplit > 1 || tiles >= 768) {           // one workgroup per unit with four row tiles: the token block is read once per unit
-        launch_gemv<4, 4, PACKED, XFRAG, SHRINK, 2>(y, out, xp, ldx, Wp, T, K, N, s, sb, n_main, y2, ksplit, part, dr, rblocks);
+        launch_gemv<4, 4, PACKED, XFRAG, SHRINK, DELTA, 2>(y, out, xp, ldx, Wp, T, K, N, s, ld, sb, n_main, y2, ksplit, part, dr, rblocks);
         return mlora_launch_status("gemv");
       }
       if (tiles > 256) {                          // 257..511 tiles as one-tile workgroups would need a second, thin round
-        launch_gemv<2, 4, PACKED, XFRAG, SHRINK, 2>(y, out, xp, ldx, Wp, T, K, N, s, sb, n_main, y2, ksplit, part);
+        launch_gemv<2, 4, PACKED, XFRAG, SHRINK, DELTA, 2>(y, out, xp, ldx, Wp, T, K, N, s, ld, sb, n_main, y2, ksplit, part);
         return mlora_launch_status("gemv");
       }
     }
-    launch_gemv<1, 4, PACKED, XFRAG, SHRINK>(y, out, xp, ldx, Wp, T, K, N, s, sb, n_main, y2);
+    launch_gemv<1, 4, PACKED, XFRAG, SHRINK, DELTA>(y, out, xp, ldx, Wp, T, K, N, s, ld, sb, n_main, y2);
   }
   return mlora_launch_status("gemv");
 }
@@ -763,6 +787,13 @@ extern "C" int mlora_gemv_frag_acc_ksplit(float* y, float* y2, float* part, int 
 }
 
 // ranges of K of the last group's rows: whole rounds of a workgroup's waves
+#ifndef MLORA_ELT_BF16
+// y (=|+=) xf . Wp^T + the deltas for up to 64 tokens (K slices: accumulating, slice 0 carries them)
+int mlora_gemv_deltas(void* y, int y_dtype, int mode, float* part, int ks, const void* xf, const void* Wp, int T, int K, int N, const LinearDeltas& ld, void* stream) {
+  return gemv_dispatch<true, true, false, true>(y, y_dtype, mode, xf, K, Wp, T, K, N, stream, LoraShrinkBatch(), N, nullptr, ks, part, LoraDeltaRide(), 0, ld);
+}
+#endif
+
 extern "C" int mlora_gemv_groups_parts(int K) {
   const int by_k = K / KSTEP / GEMV_WAVES;
   return by_k < 1 ? 1 : by_k < 8 ? by_k : 8;

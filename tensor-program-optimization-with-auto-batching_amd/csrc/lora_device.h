@@ -234,3 +234,94 @@ __device__ __forceinline__ float lora_row_dot(const f16* __restrict__ brow, cons
     for (int q = 0; q < n / 2; ++q) g[q] = g[2 * q] + g[2 * q + 1];
   return g[0];
 }
+
+#ifndef MLORA_ELT_F32
+// ---------------------------------------------------------------------------------------------
+// The deltas of any mix of adapters in the accumulators of a linear, y = x . W^T + v . B[id]^T with v = scaling * (sum of the shrink's K ranges) as
+// fp16 hi and lo halves.  Projections are row ranges of the fused weight.
+// ---------------------------------------------------------------------------------------------
+constexpr int DELTA_RANGES = 4;                // K ranges of the shrink: as many as are in flight together in registers
+struct LinearDeltas {
+  const elt* B[3];            // [n_ad][n_rows][r]
+  int n_begin[3], n_rows[3];
+  const float* v;             // [n_proj][ranges][T][r], rows of tokens without adapter not written
+  const int32_t* ids;         // [T]: outside 0 .. n_ad - 1 no adapter
+  float scaling;
+  int n_proj, r, n_ad, ranges;
+};
+
+// acc [NN][TT]: 16-row tiles of W (row0: their first rows) x tiles of 16 tokens from t0 on, as mfma_16x16x32 leaves them; left: the ids of this lane's
+// tokens (-1 past T).  A wave takes the adapters of these tokens in turn, with zeros for the tokens of the others, and of the rounds - an adapter,
+// a projection, 32 ranks - every step-th.  Both operands come straight from memory.
+template <int NN, int TT, bool SERIAL = false>    // SERIAL: the ranges of one token tile in flight at a time
+__device__ __forceinline__ void linear_add_deltas(f32x4 (&acc)[NN][TT], const LinearDeltas& lo, int (&left)[TT], int T, int t0, const int (&row0)[NN], int lane,
+                                                  int first, int step) {
+  const int r16 = lane & 15, g8 = (lane >> 4) * 8;
+#pragma unroll
+  for (int j = 0; j < TT; ++j) left[j] = left[j] < lo.n_ad ? left[j] : -1;
+  int turn = 0;
+  for (;;) {
+    int a = -1;
+#pragma unroll
+    for (int j = 0; j < TT; ++j) {
+      const unsigned long long todo = __ballot(left[j] >= 0);
+      if (a < 0 && todo) a = __builtin_amdgcn_readlane(left[j], __builtin_ctzll(todo));
+    }
+    if (a < 0) break;
+    for (int p = 0; p < lo.n_proj; ++p) {
+      // projection p's, by masks: the compiler turns a choice into an address that depends on p, and `lo` would live in scratch memory
+      const unsigned long long m0 = 0ull - (p == 0), m1 = 0ull - (p == 1), m2 = 0ull - (p == 2);
+      const elt* Bp = (const elt*)(((uintptr_t)lo.B[0] & m0) | ((uintptr_t)lo.B[1] & m1) | ((uintptr_t)lo.B[2] & m2));
+      const int begin = (lo.n_begin[0] & (int)m0) | (lo.n_begin[1] & (int)m1) | (lo.n_begin[2] & (int)m2);
+      const int rows = (lo.n_rows[0] & (int)m0) | (lo.n_rows[1] & (int)m1) | (lo.n_rows[2] & (int)m2);
+      bool has = false;
+#pragma unroll
+      for (int i = 0; i < NN; ++i) has = has || (row0[i] < begin + rows && row0[i] + 16 > begin);
+      if (!has) continue;                      // uniform
+      const float* vp = lo.v + (size_t)p * lo.ranges * T * lo.r;
+      for (int c0 = 0; c0 < lo.r; c0 += 32) {
+        const bool mine = turn == first;       // uniform
+        turn = turn + 1 == step ? 0 : turn + 1;
+        if (!mine) continue;
+        const int c = c0 + g8;                 // this lane's eight ranks (past r: zeros)
+        eltx8 bf[NN];
+#pragma unroll
+        for (int i = 0; i < NN; ++i) {
+          const int row = row0[i] + r16 - begin;
+          bf[i] = c < lo.r && row >= 0 && row < rows ? ld8(Bp + ((size_t)a * rows + row) * lo.r + c) : eltx8{0, 0, 0, 0, 0, 0, 0, 0};
+        }
+#pragma unroll
+        for (int j = 0; j < TT; ++j) {
+          const int t = t0 + j * 16 + r16;
+          const float* q = vp + (size_t)(t < T ? t : T - 1) * lo.r + (c < lo.r ? c : 0);
+          f32x4 x0[DELTA_RANGES], x1[DELTA_RANGES], s0 = f32x4{0.f, 0.f, 0.f, 0.f}, s1 = s0;
+#pragma unroll
+          for (int s = 0; s < DELTA_RANGES; ++s) {               // (past the last range: that one again, not added)
+            const float* qs = q + (size_t)(s < lo.ranges ? s : lo.ranges - 1) * T * lo.r;
+            x0[s] = *reinterpret_cast<const f32x4*>(qs);
+            x1[s] = *reinterpret_cast<const f32x4*>(qs + 4);
+          }
+#pragma unroll
+          for (int s = 0; s < DELTA_RANGES; ++s) {
+            s0 = s < lo.ranges ? s0 + x0[s] : s0;
+            s1 = s < lo.ranges ? s1 + x1[s] : s1;
+          }
+          eltx8 hi, low;
+          const bool of_a = left[j] == a && c < lo.r;            // (others': whatever lies there is replaced)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float f = of_a ? (e < 4 ? s0[e & 3] : s1[e & 3]) * lo.scaling : 0.f;
+            hi[e] = (elt)f;
+            low[e] = (elt)(f - (float)hi[e]);
+          }
+#pragma unroll
+          for (int i = 0; i < NN; ++i) acc[i][j] = mfma_16x16x32(bf[i], low, mfma_16x16x32(bf[i], hi, acc[i][j]));
+          if constexpr (SERIAL) asm volatile("" ::: "memory");
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < TT; ++j) left[j] = left[j] == a ? -1 : left[j];
+  }
+}
+#endif

@@ -163,7 +163,7 @@ extern "C" int mlora_prefill(const mlora_prefill_plan* p, void* stream) {
       STEP(mlora_linear_frag_lora(y, y_dtype, mode, x, W, T, K, N, f, n, p->blk_adapter, r, stream));
       return p->tok_rest ? deltas(y, y_dtype, N, x, K, pj, n, p->tok_rest) : MLORA_OK;
     }
-    if (n > 0 && p->n_distinct > 0 && mlora_linear_frag_deltas_pay(T, K, N, mode == MLORA_ACCUMULATE, r, p->n_distinct)) {
+    if (n > 0 && p->n_distinct > 0 && (T > 64 || p->segments) && mlora_linear_frag_deltas_pay(T, K, N, mode == MLORA_ACCUMULATE, r, p->n_distinct)) {
       if (ks && part) {
         const int k = mlora_gemv_ksplit(T, K, N);
         *ks = k > 1 && mlora_gemv_ksplit_bytes(T, N, k) <= at.ksplit_bytes ? k : 1;
@@ -210,7 +210,7 @@ extern "C" int mlora_prefill(const mlora_prefill_plan* p, void* stream) {
       mlora_fused_lora f[MAXP];
       STEP(halves(xn, H, gl, n_gl, f));
       STEP(mlora_linear_frag_silu(act, xn, L.gate_up_p, T, H, I, f, n_gl, p->blk_adapter, r, stream));
-    } else if (p->n_distinct > 0 && mlora_linear_frag_deltas_pay(T, H, 2 * I, 0, r, p->n_distinct)) {
+    } else if (T > 64 && p->n_distinct > 0 && mlora_linear_frag_deltas_pay(T, H, 2 * I, 0, r, p->n_distinct)) {
       const Buckets b = buckets_of(gl, n_gl);
       STEP(mlora_linear_frag_silu_deltas(act, xn, L.gate_up_p, T, H, I, b.bk, n_gl, b.c, b.nc, p->tok_adapter, lora_ws, at.lora_bytes, stream));
     } else {

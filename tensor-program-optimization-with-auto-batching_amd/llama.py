@@ -258,7 +258,8 @@ class LlamaForCausalLM(CausalLM):
         one-launch kernel, work an adapter's tokens off one after the other.  Decode steps of two 7B layers, q, k, v and o adapted, us, riding /
         launches: rank 8, one adapter, 8 tokens 295 / 288, 64 tokens 563 / 369, sixteen of 64 361 / 393; rank 16, one, 4 tokens 285 / 281, 16 tokens
         349 / 290; two of 8 290 / 300; four of 32 359 / 310 (two of 32), eight of 32 314 / 331; rank 32, one token 301 / 277, 8 of 8 309 / 316, 64 of
-        64 503 / 455; rank 64, one 352 / 297, 64 of one 1732 / 396, 64 of 64 603 / 515."""
+        64 503 / 455; rank 64, one 352 / 297, 64 of one 1732 / 396, 64 of 64 603 / 515.  (Launches of a shrink and an expand; where the expand
+        goes into the linear, `linear_frag_deltas_pay`, they take up to a quarter less.)"""
         s, r = self.shape, self.lora_types[tid].r
         return not (s.hidden_size % 32 or s.q_size % 32 or s.intermediate_size % 32 or s.kv_size % 16) and 0 < T <= 64 and (r >= 32 or most * r >= 96)
 
@@ -392,9 +393,9 @@ class LlamaForCausalLM(CausalLM):
                     blk, rest = ops.lora_block_adapters(ids, lt.n_adapters)
                     rest = rest if bool((rest >= 0).any()) else None
                 fuse = (lt, ids, blk, None if rest is None else {tid: rest})
-        # below the persistent kernel's sizes the mid-size one takes any mix of adapters, where the host knows that they are few
+        # below the persistent kernel's sizes the linears themselves take any mix of adapters, where the host knows that they are few
         near = None
-        if host_ids is not None and tok_adapter and "multi" not in tok_adapter and len(tok_adapter) == 1 and frag and T > 64 and not is_decode:
+        if host_ids is not None and tok_adapter and "multi" not in tok_adapter and len(tok_adapter) == 1 and frag and (segs or T > 64 and not is_decode):
             (tid, ids), = tok_adapter.items()
             near = (self.lora_types[tid], ids, distinct_adapters(host_ids[tid], self.lora_types[tid].n_adapters))
         o_shares = None
@@ -408,7 +409,7 @@ class LlamaForCausalLM(CausalLM):
             xn = ops.rmsnorm(resid, L["ln1"], s.rms_norm_eps, frag=frag, parts=parts)
             qkv_projs = (("q_proj", 0, q_sz), ("k_proj", q_sz, kv_sz), ("v_proj", q_sz + kv_sz, kv_sz))
             qkv = self._fused_linear(fuse, xn, L["qkv"], l, qkv_projs) if fuse else None
-            if qkv is None and near:
+            if qkv is None and near is not None:
                 qkv = (self._delta_linear(near, xn, L["qkv"], l, qkv_projs) or (None,))[0]
             if qkv is None:
                 qkv = ops.linear(xn, L["qkv"])
@@ -446,6 +447,8 @@ class LlamaForCausalLM(CausalLM):
                 act = self._gate_up_silu(fuse, near, xn, L["gate_up"], l, gu_projs, bool(tok_adapter)) if frag and T > 64 else None
                 if act is None:
                     gu = self._fused_linear(fuse, xn, L["gate_up"], l, gu_projs) if fuse else None
+                    if gu is None and near is not None:
+                        gu = (self._delta_linear(near, xn, L["gate_up"], l, gu_projs) or (None,))[0]
                     if gu is None:
                         gu = ops.linear(xn, L["gate_up"])
                         if tok_adapter:
@@ -495,7 +498,7 @@ class LlamaForCausalLM(CausalLM):
         return y
 
     def _delta_linear(self, near, x, W, l, projs, resid=None, ks_ws=None):
-        """The base linear of `projs` with the deltas of whatever adapters the tokens name inside the mid-size kernel: (y, K-slice
+        """The base linear of `projs` with the deltas of whatever adapters the tokens name inside the linear: (y, K-slice
         partials or None), or None where that does not serve the shape or does not pay."""
         lt, ids, n_distinct = near
         T, K = x.shape
@@ -518,7 +521,7 @@ class LlamaForCausalLM(CausalLM):
             return None
         if not adapters or not self._targets(l, *(p for p, _, _ in projs)):
             return ops.linear_frag_glu(x, W)
-        if near and near[2] and ops.linear_frag_deltas_pay(T, K, N, False, near[0].r, near[2]):
+        if near and near[2] and T > 64 and ops.linear_frag_deltas_pay(T, K, N, False, near[0].r, near[2]):
             lt, ids, _ = near
             live = [(c0, n, lt.tables.get((l, proj))) for proj, c0, n in projs]
             live = [e for e in live if e[2] is not None]

@@ -1711,10 +1711,11 @@ def test_gated_product_out_of_the_linear(ops, T, K, I, dt, kind):
 
 
 @pytest.mark.parametrize("T,K,rows", [(65, 256, (32, 16, 32)), (130, 1056, (2048, 512, 528)), (137, 4096, (4096,)), (193, 288, (11008,)), (300, 2080, (1024, 1040)),
-                                      (260, 512, (2752, 2752)), (385, 320, (4096, 4096))])
+                                      (260, 512, (2752, 2752)), (385, 320, (4096, 4096)), (1, 1024, (1024, 512, 512)), (16, 4096, (4096,)), (17, 11008, (4096,)),
+                                      (31, 4096, (4096, 4096, 4096)), (33, 1024, (1024, 48)), (50, 4096, (4096,)), (64, 544, (11008, 5552)), (64, 512, (8192,))])
 @pytest.mark.parametrize("r,who", [(8, "one"), (16, "one"), (16, "mixed"), (32, "segments"), (64, "segments"), (64, "mixed")])
-def test_deltas_inside_the_mid_size_linear(ops, T, K, rows, r, who):
-    """Block shapes of the mid-size kernel, ranks, blocks that several projections share (or a part without adapter), one adapter, several in segments,
+def test_deltas_inside_the_linear(ops, T, K, rows, r, who):
+    """Block shapes of the mid-size kernel and of the one for up to 64 tokens, ranks, blocks that several projections share (or a part without adapter), one adapter, several in segments,
     one of nine per token: against fp64, with the bits of the plain linear where no delta belongs."""
     n_ad, scaling, eps, g = 9, 0.5, 2.0 ** -24, torch.Generator(device=DEV).manual_seed(T + K + r)
     rnd = lambda *s: torch.randn(s, generator=g, device=DEV)
@@ -1750,7 +1751,7 @@ def test_deltas_inside_the_mid_size_linear(ops, T, K, rows, r, who):
         if parts is not None:
             acc = acc + ws[:(parts.ks - 1) * T * N].view(parts.ks - 1, T, N).sum(0)
         assert bool(((acc.double() - resid.double() - want).abs() <= slack + (resid.double().abs() + want.abs()) * 8 * eps).all())
-    if len(rows) == 2 and rows[0] == rows[1]:
+    if len(rows) == 2 and rows[0] == rows[1]:               # (more than 64 tokens)
         I = rows[0]
         W2 = ops.PackedWeight((rnd(2 * I, K) * K ** -0.5).half())
         gu = [(*p[:3], i * I, I) for i, p in enumerate(projs)]
