@@ -573,17 +573,16 @@ class LlamaForCausalLM(CausalLM):
 
     # ------------------------------------------------------------------ a prompt pass in one call
     def _native_prefill_serves(self, h, kv):
-        """Whether `mlora_prefill` takes a pass: not a decode step, activations in fragment order."""
+        """Whether `mlora_prefill` takes a pass: not a decode step, activations in fragment order, a cache of at least the model's layers."""
         s = self.shape
         return (kv._cur is not None and not kv._cur[2] and h.dim() == 2 and h.shape[0] > 0 and h.is_cuda and h.dtype == torch.float32
-                and h.is_contiguous() and not s.hidden_size % 32 and not s.q_size % 32 and not s.intermediate_size % 32)
+                and h.is_contiguous() and not s.hidden_size % 32 and not s.q_size % 32 and not s.intermediate_size % 32
+                and tuple(h.shape) == (sum(kv._cur[1]), s.hidden_size) and kv.n_layers >= len(self.layers))
 
     def _native_prefill(self, h, kv, logits_rows, tid=None, ids=None):
         """`forward` of a prompt pass - the same launches - queued by one call: the host takes 4 us a layer for their addresses instead of 14 us a
         launch.  tid, ids: adapter type and host ids of the tokens."""
         s, T = self.shape, h.shape[0]
-        if sum(kv._cur[1]) != T or h.shape[1] != s.hidden_size or kv.n_layers != len(self.layers):
-            raise ValueError(f"prefill: {tuple(h.shape)} rows for {sum(kv._cur[1])} announced tokens")
         kv._join()
         f16, i32, ptr = torch.float16, torch.int32, ops._dev
         lt = self.lora_types[tid] if tid is not None else None

@@ -503,3 +503,26 @@ def test_prompt_pass_in_one_call(lens, r, targets, decoded):
     assert bool(torch.isfinite(got[0][0]).all())
     for a, b in zip(*got):
         assert torch.equal(a, b)
+
+
+def test_prompt_pass_of_fewer_layers_than_the_cache():
+    """A model cut off after a layer, on a cache of both: prefill_a0 takes it as `forward` does, with the same bits."""
+    synth, llama, ops = load_pkg("synth"), load_pkg("llama"), load_pkg("ops")
+    shape = synth.LlamaShape(hidden_size=512, intermediate_size=544, num_attention_heads=4, num_key_value_heads=4, num_hidden_layers=2, head_dim=128, vocab_size=520)
+    model = llama.LlamaForCausalLM.from_synthetic(5, shape, [synth.LoraSpec(r=16, alpha=32.0, n_adapters=2, targets=ALL_LINEARS)], DEV)
+    tokens, wids, got = synth.randint(3, "cut", (90,), shape.vocab_size), np.array([1], np.int32), []
+    model.layers = model.layers[:1]
+    for native in (True, False):
+        kv = model.create_paged_kv_cache(1, 96, 96, 16)
+        kv.add_sequence(0)
+        kv.begin_forward([0], [90])
+        h = model.embed(tokens)
+        if native:
+            logits, _ = model["prefill_a0"](h, kv, wids)
+        else:
+            ids = {0: np.repeat(wids, 90)}
+            logits = model.forward(h, kv, {0: torch.from_numpy(ids[0]).to(DEV)}, torch.tensor([89], device=DEV), ids)
+        kv.end_forward()
+        got.append((logits, kv.k, h))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
