@@ -180,7 +180,8 @@ class NativeDecodeSession:
             p.lora_r, p.lora_n_ad, p.lora_scaling = lt.r, lt.n_adapters, lt.scaling
             p.lora_dense = (2 if self.o_delta_ride else 1) if self.dense_lora else 0
             # (of one type: the union of several adds exact zeros to the sums of each, which matrix-core sums of another rank are not)
-            p.lora_segments = distinct_adapters(ids, model.lora_types[tid].n_adapters) if not isinstance(tid, tuple) and model.segments_pay(T, most_of_one(ids), tid) else 0
+            if not isinstance(tid, tuple) and model.segments_pay(T, most_of_one(ids), tid, bool(self.dense_lora)):
+                p.lora_segments = distinct_adapters(ids, lt.n_adapters)
         p.layers = C.cast(layers, C.POINTER(_lib.Layer))
         p.embed, p.norm, p.lm_head_p = model.embed_tokens.data_ptr(), model.norm.data_ptr(), model.lm_head.data.data_ptr()
         p.rope_cos, p.rope_sin, p.max_pos = kv.rope_cos.data_ptr(), kv.rope_sin.data_ptr(), kv.max_pos

@@ -252,16 +252,19 @@ class LlamaForCausalLM(CausalLM):
             self._ws = torch.empty(need, dtype=torch.float32, device=self.device)
         return self._ws
 
-    def segments_pay(self, T, most, tid):
+    def segments_pay(self, T, most, tid, beside_rows=False):
         """Whether the deltas of up to 64 tokens, of which `most` name one adapter (a prompt pass: its longest sequence), go to the matrix cores
         in launches of their own, which take as long whatever the tokens share.  The units that ride in a decode step's launches, and the
         one-launch kernel, work an adapter's tokens off one after the other.  Decode steps of two 7B layers, q, k, v and o adapted, us, riding /
         launches: rank 8, one adapter, 8 tokens 295 / 288, 64 tokens 563 / 369, sixteen of 64 361 / 393; rank 16, one, 4 tokens 285 / 281, 16 tokens
         349 / 290; two of 8 290 / 300; four of 32 359 / 310 (two of 32), eight of 32 314 / 331; rank 32, one token 301 / 277, 8 of 8 309 / 316, 64 of
         64 503 / 455; rank 64, one 352 / 297, 64 of one 1732 / 396, 64 of 64 603 / 515.  (Launches of a shrink and an expand; where the expand
-        goes into the linear, `linear_frag_deltas_pay`, they take up to a quarter less.)"""
+        goes into the linear, `linear_frag_deltas_pay`, they take up to a quarter less.)  beside_rows: the shrink of the other linears is appended to
+        their weights, and what is asked for is gate and up, each a one-launch kernel otherwise; steps with all linears adapted, us, those / these:
+        rank 16, one of two adapters 310 / 299, 8 of sixteen 346 / 318, 32 of sixty-four 479 / 407; rank 8, two of one 310 / 302, 16 of thirty-two 351
+        / 337, 64 of four 570 / 482; hidden 1024, rank 16, 4 of four 139 / 127, rank 8, 32 of sixteen 158 / 160."""
         s, r = self.shape, self.lora_types[tid].r
-        return not (s.hidden_size % 32 or s.q_size % 32 or s.intermediate_size % 32 or s.kv_size % 16) and 0 < T <= 64 and (r >= 32 or most * r >= 96)
+        return not (s.hidden_size % 32 or s.q_size % 32 or s.intermediate_size % 32 or s.kv_size % 16) and 0 < T <= 64 and (r >= 32 or most * r >= 96 or beside_rows)
 
     def _lora(self, y, x, l, proj, tok_adapter, segments=False):
         """y += delta for every adapter type that targets (l, proj); tok_adapter: {tid: ids [T] int32}, or the merged
