@@ -278,11 +278,15 @@ int mlora_linear_frag_lora(void* y, int y_dtype, int mode, const void* xf, const
  *   mlora_linear_frag_deltas_pay   - whether a shape is served, and faster so than by mlora_linear_frag and mlora_gather_mm where the tokens of the
  *                                    pass name n_distinct adapters (accumulate: the mode);
  *   mlora_linear_frag_deltas       - ks > 1 (accumulating only): K slices as mlora_gemv_frag_acc_ksplit, slices 1.. into part[ks - 1][T][N];
- *   mlora_linear_frag_silu_deltas  - act = silu(gate) * up in fragment order, of the sums rounded to fp16. */
+ *   mlora_linear_frag_silu_deltas  - act = silu(gate) * up in fragment order, of the sums rounded to fp16 (more than 64 tokens);
+ *   mlora_gemv_frag_silu_deltas    - the same up to 64 tokens, of interleaved tiles (mlora_gemv_frag_silu). */
 int mlora_linear_frag_deltas_pay(int T, int K, int N, int accumulate, int r, int n_distinct);
 int mlora_linear_frag_deltas(void* y, int y_dtype, int mode, float* part, int ks, const void* xf, const void* Wp, int T, int K, int N,
                              const mlora_lora_bucket* projs, int n_proj, const int32_t* n_begin, const int32_t* n_rows,
                              const int32_t* tok_adapter, void* workspace, size_t workspace_bytes, void* stream);
+int mlora_gemv_frag_silu_deltas(void* act, const void* xf, const void* Wil_p, int T, int K, int I, const mlora_lora_bucket* projs, int n_proj,
+                                const int32_t* n_begin, const int32_t* n_rows, const int32_t* tok_adapter, void* workspace,
+                                size_t workspace_bytes, void* stream);
 int mlora_linear_frag_silu_deltas(void* act, const void* xf, const void* Wp, int T, int K, int I, const mlora_lora_bucket* projs, int n_proj,
                                   const int32_t* n_begin, const int32_t* n_rows, const int32_t* tok_adapter, void* workspace,
                                   size_t workspace_bytes, void* stream);

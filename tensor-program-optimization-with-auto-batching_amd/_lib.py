@@ -56,6 +56,7 @@ SIGNATURES = {
     "mlora_linear_frag_lora": (_i, [_p, _i, _i, _p, _p, _i, _i, _i, _p, _i, _p, _i, _p]),
     "mlora_linear_frag_deltas_pay": (_i, [_i, _i, _i, _i, _i, _i]),
     "mlora_linear_frag_deltas": (_i, [_p, _i, _i, _p, _i, _p, _p, _i, _i, _i, _p, _i, _p, _p, _p, _p, _z, _p]),
+    "mlora_gemv_frag_silu_deltas": (_i, [_p, _p, _p, _i, _i, _i, _p, _i, _p, _p, _p, _p, _z, _p]),
     "mlora_linear_frag_silu_deltas": (_i, [_p, _p, _p, _i, _i, _i, _p, _i, _p, _p, _p, _p, _z, _p]),
     "mlora_linear_frag_silu": (_i, [_p, _p, _p, _i, _i, _i, _p, _i, _p, _i, _p]),
     "mlora_gemv_frag_lora": (_i, [_p, _i, _i, _p, _p, _i, _i, _i, _p, _p, _i, _p, _i, _i, _p]),

@@ -181,8 +181,9 @@ extern "C" int mlora_decode_step(const mlora_decode_plan* p, void* stream) {
   void* ws_down = ws + (size_t)(3 * kq + 1) * slot;
   const size_t down_bytes = lora ? p->lora_ws_bytes - (size_t)(3 * kq + 1) * slot : 0;   // (a smaller K may take more than the largest)
   // a linear with them: inside the linear behind the shrink where that pays (done is then set), else nothing yet
+  // (interleaved: the gate / up weights whose linear leaves the product, y)
   auto seg_linear = [&](void* y, int y_dtype, int mode, int ks, const void* x, const void* W, int K, int N, const mlora_lora_proj* lp, const int32_t* col,
-                        const int32_t* ncol, int n, bool& done) -> int {
+                        const int32_t* ncol, int n, bool& done, const void* interleaved = nullptr) -> int {
     mlora_lora_bucket bk[3];
     int32_t c[3], nc[3];
     int live = 0;
@@ -194,6 +195,8 @@ extern "C" int mlora_decode_step(const mlora_decode_plan* p, void* stream) {
       }
     done = live > 0 && mlora_linear_frag_deltas_pay(T, K, N, mode == MLORA_ACCUMULATE, r, p->lora_segments);
     if (!done) return MLORA_OK;
+    if (interleaved)
+      return mlora_gemv_frag_silu_deltas(y, x, interleaved, T, K, N / 2, bk, live, c, nc, p->tok_adapter, p->lora_ws, p->lora_ws_bytes, stream);
     return mlora_linear_frag_deltas(y, y_dtype, mode, p->ksplit_ws, ks, x, W, T, K, N, bk, live, c, nc, p->tok_adapter, p->lora_ws, p->lora_ws_bytes, stream);
   };
   auto seg_deltas = [&](void* y, int y_dtype, int ldy, const void* x, int K, const mlora_lora_proj* lp, const int32_t* col, const int32_t* ncol, int n) -> int {
@@ -309,7 +312,11 @@ extern "C" int mlora_decode_step(const mlora_decode_plan* p, void* stream) {
       const mlora_lora_proj lp[2] = {L.lora[MLORA_GATE], L.lora[MLORA_UP]};
       const int32_t col[2] = {0, I}, ncol[2] = {I, I};
       bool done = false;
-      if (gu_segs) STEP(seg_linear(gu, MLORA_F16, MLORA_STORE, 1, p->xn, L.gate_up_p, H, 2 * I, lp, col, ncol, 2, done));
+      // the product out of the linear as well, up to 16 tokens and three workgroups of two tiles on a compute unit; two layers with all linears
+      // adapted, us, product behind / out of it: 7B, one request at rank 64 339 / 325, 8 at rank 16 317 / 304, hidden 1024, 4 125 / 122; 20 requests
+      // 370 / 373, hidden 1024, 32 159 / 162, 8 of intermediate 14336 443 / 448
+      const void* il = T <= 16 && I <= 3 * 256 * 16 ? L.gate_up_il_p : nullptr;
+      if (gu_segs) STEP(seg_linear(il ? p->act : gu, MLORA_F16, MLORA_STORE, 1, p->xn, L.gate_up_p, H, 2 * I, lp, col, ncol, 2, done, il));
       if (!done) STEP(mlora_gemv_frag(gu, MLORA_F16, MLORA_STORE, p->xn, L.gate_up_p, T, H, 2 * I, stream));
       if (done) {
       } else if (gu_segs) {
@@ -318,7 +325,7 @@ extern "C" int mlora_decode_step(const mlora_decode_plan* p, void* stream) {
         STEP(delta(gu, MLORA_F16, 2 * I, p->xn, L.lora[MLORA_GATE], H, I));
         STEP(delta(gu + I, MLORA_F16, 2 * I, p->xn, L.lora[MLORA_UP], H, I));
       }
-      STEP(mlora_silu_mul(p->act, MLORA_FRAG, gu, gu + I, 2 * I, T, I, stream));
+      if (!done || !il) STEP(mlora_silu_mul(p->act, MLORA_FRAG, gu, gu + I, 2 * I, T, I, stream));
     }
     const bool down_lora = lora && !segs && L.lora[MLORA_DOWN].A;
     pending_ks = ksplit_of(I, down_lora);

@@ -1397,6 +1397,18 @@ extern "C" int mlora_linear_frag_deltas(void* y, int y_dtype, int mode, float* p
   return e ? e : mlora_launch_status("linear_frag_deltas");
 }
 
+int mlora_gemv_silu_deltas(void* act, const void* xf, const void* Wil_p, int T, int K, int I, const LinearDeltas& ld, void* stream);
+extern "C" int mlora_gemv_frag_silu_deltas(void* act, const void* xf, const void* Wil_p, int T, int K, int I, const mlora_lora_bucket* projs, int n_proj,
+                                           const int32_t* n_begin, const int32_t* n_rows, const int32_t* tok_adapter, void* workspace,
+                                           size_t workspace_bytes, void* stream) {
+  MLORA_CHECK(act && xf && Wil_p, MLORA_ERR_INVALID, "gemv_frag_silu_deltas: null pointer");
+  MLORA_CHECK(T > 0 && T <= 64 && K > 0 && K % 32 == 0 && I > 0 && I % 32 == 0 && I <= (1 << 29) && (((uintptr_t)xf | (uintptr_t)act) & 15) == 0,
+              MLORA_ERR_UNSUPPORTED, "gemv_frag_silu_deltas: up to 64 tokens, K and I in whole 32, aligned operands (T=%d K=%d I=%d)", T, K, I);
+  LinearDeltas lo = {};
+  if (int e = mid_lora("gemv_frag_silu_deltas", lo, projs, n_proj, n_begin, n_rows, xf, tok_adapter, T, K, 2 * I, workspace, workspace_bytes, stream)) return e;
+  return mlora_gemv_silu_deltas(act, xf, Wil_p, T, K, I, lo, stream);
+}
+
 extern "C" int mlora_linear_frag_silu_deltas(void* act, const void* xf, const void* Wp, int T, int K, int I, const mlora_lora_bucket* projs, int n_proj,
                                              const int32_t* n_begin, const int32_t* n_rows, const int32_t* tok_adapter, void* workspace,
                                              size_t workspace_bytes, void* stream) {

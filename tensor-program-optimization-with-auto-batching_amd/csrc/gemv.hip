@@ -264,7 +264,10 @@ __global__ __launch_bounds__(GEMV_WAVES* WAVE, (NT * TT > 8 ? 2 : 4)) void gemv_
     if (slice == 0) {                              // uniform
       int row0[NT];
 #pragma unroll
-      for (int i = 0; i < NT; ++i) row0[i] = n0 + i * 16;
+      for (int i = 0; i < NT; ++i) {
+        const int g = bid * NT + i;                // (a gated product: tiles of gate and up in turn)
+        row0[i] = OUT == OUT_SILU_FRAG ? (g & 1) * (N / 2) + (g >> 1) * 16 : g * 16;
+      }
       linear_add_deltas<NT, TT, TILES <= 8 && (TT == 4 || NT * TT == 8)>(acc, ld, ids, T, 0, row0, lane, wave, GEMV_WAVES);
     }
   }
@@ -954,6 +957,22 @@ static int gemv_frag_glu(const char* who, void* act, const void* xf, const void*
   else hipLaunchKernelGGL((gemv_kernel<2, 4, OUT, true, true, false, 2>), grid, block, 0, s, act, xp, K, Wp, T, K, 2 * I, sb, 0, 2 * I, nullptr, 1, nullptr, LoraDeltaRide(), 0, ga);
   return mlora_launch_status(who);
 }
+
+#ifndef MLORA_ELT_BF16
+// act = silu(gate) * up of the sums with their deltas, rounded to fp16 (up to 64 tokens; interleaved tiles): the bits of the linear and the product
+int mlora_gemv_silu_deltas(void* act, const void* xf, const void* Wil_p, int T, int K, int I, const LinearDeltas& ld, void* stream) {
+  const elt *x = (const elt*)xf, *W = (const elt*)Wil_p;
+  const LoraShrinkBatch sb = LoraShrinkBatch();
+#define MLORA_SILU_DELTAS(TT, PIPE) \
+  hipLaunchKernelGGL((gemv_kernel<2, TT, OUT_SILU_FRAG, true, true, false, PIPE, false, true>), dim3(I / 16), dim3(GEMV_WAVES * WAVE), 0, (hipStream_t)stream, act, x, \
+                     K, W, T, K, 2 * I, sb, 0, 2 * I, nullptr, 1, nullptr, LoraDeltaRide(), 0, GluArgs(), 0, 0l, 1, ld)
+  if (T <= 16) MLORA_SILU_DELTAS(1, 4);
+  else if (T <= 32) MLORA_SILU_DELTAS(2, 4);
+  else MLORA_SILU_DELTAS(4, 2);
+#undef MLORA_SILU_DELTAS
+  return mlora_launch_status("gemv_frag_silu_deltas");
+}
+#endif
 
 extern "C" int mlora_gemv_frag_silu(void* act, const void* xf, const void* Wil_p, int T, int K, int I, void* stream) {
   return gemv_frag_glu<MLORA_GLU_SILU>("gemv_frag_silu", act, xf, Wil_p, T, K, I, GluArgs(), stream);

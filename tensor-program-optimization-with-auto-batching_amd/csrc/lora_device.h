@@ -252,14 +252,14 @@ struct LinearDeltas {
 
 // acc [NN][TT]: 16-row tiles of W (row0: their first rows) x tiles of 16 tokens from t0 on, as mfma_16x16x32 leaves them; left: the ids of this lane's
 // tokens (-1 past T).  A wave takes the adapters of these tokens in turn, with zeros for the tokens of the others, and of the rounds - an adapter,
-// a projection, 32 ranks - every step-th.  Both operands come straight from memory.
+// 32 ranks - every step-th (a power of two).  Both operands come straight from memory.
 template <int NN, int TT, bool SERIAL = false>    // SERIAL: the ranges of one token tile in flight at a time
 __device__ __forceinline__ void linear_add_deltas(f32x4 (&acc)[NN][TT], const LinearDeltas& lo, int (&left)[TT], int T, int t0, const int (&row0)[NN], int lane,
                                                   int first, int step) {
   const int r16 = lane & 15, g8 = (lane >> 4) * 8;
 #pragma unroll
   for (int j = 0; j < TT; ++j) left[j] = left[j] < lo.n_ad ? left[j] : -1;
-  int turn = 0;
+  int round = 0;                               // an adapter's first: which wave does it depends on the ids and r alone, not on the rows of a block
   for (;;) {
     int a = -1;
 #pragma unroll
@@ -280,9 +280,7 @@ __device__ __forceinline__ void linear_add_deltas(f32x4 (&acc)[NN][TT], const Li
       if (!has) continue;                      // uniform
       const float* vp = lo.v + (size_t)p * lo.ranges * T * lo.r;
       for (int c0 = 0; c0 < lo.r; c0 += 32) {
-        const bool mine = turn == first;       // uniform
-        turn = turn + 1 == step ? 0 : turn + 1;
-        if (!mine) continue;
+        if ((round + c0 / 32) % step != first) continue;         // uniform
         const int c = c0 + g8;                 // this lane's eight ranks (past r: zeros)
         eltx8 bf[NN];
 #pragma unroll
@@ -322,6 +320,7 @@ __device__ __forceinline__ void linear_add_deltas(f32x4 (&acc)[NN][TT], const Li
     }
 #pragma unroll
     for (int j = 0; j < TT; ++j) left[j] = left[j] == a ? -1 : left[j];
+    round += (lo.r + 31) / 32;
   }
 }
 #endif

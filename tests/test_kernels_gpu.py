@@ -1751,6 +1751,16 @@ def test_deltas_inside_the_linear(ops, T, K, rows, r, who):
         if parts is not None:
             acc = acc + ws[:(parts.ks - 1) * T * N].view(parts.ks - 1, T, N).sum(0)
         assert bool(((acc.double() - resid.double() - want).abs() <= slack + (resid.double().abs() + want.abs()) * 8 * eps).all())
+    if T <= 64 and rows[0] % 32 == 0:                           # gate and up, or up alone, of one linear
+        I = rows[0]
+        W2 = ops.PackedWeight((rnd(2 * I, K) * K ** -0.5).half())
+        il = ops.interleave_gate_up(W2.unpack())
+        gu = [(A[0], B[0], scaling, 0, I), (A[0], B[0].flip(1).contiguous(), scaling, I, I)][T % 2:]
+        y2, _ = ops.linear_frag_deltas(f, W2, gu, d_ids, lora_ws)
+        act = ops.FragActivation(T, I, DEV)
+        ops.check(ops.lib().mlora_gemv_frag_silu_deltas(act.data.data_ptr(), f.data.data_ptr(), il.data.data_ptr(), T, K, I,
+                                                        *ops._delta_args("silu", f, W2, gu, d_ids, lora_ws)))
+        assert torch.equal(act.unpack(), ops.silu_mul(y2, frag=True).unpack())
     if len(rows) == 2 and rows[0] == rows[1]:               # (more than 64 tokens)
         I = rows[0]
         W2 = ops.PackedWeight((rnd(2 * I, K) * K ** -0.5).half())
