@@ -251,8 +251,9 @@ struct LinearDeltas {
 };
 
 // acc [NN][TT]: 16-row tiles of W (row0: their first rows) x tiles of 16 tokens from t0 on, as mfma_16x16x32 leaves them; left: the ids of this lane's
-// tokens (-1 past T).  A wave takes the adapters of these tokens in turn, with zeros for the tokens of the others, and of the rounds - an adapter,
-// 32 ranks - every step-th (a power of two).  Both operands come straight from memory.
+// tokens (-1 past T).  A wave takes the adapters of these tokens in turn and of the rounds - an adapter, 32 ranks - every step-th (a power of two);
+// both operands come straight from memory.  A product's columns are tokens, so a lane keeps the sums of a round where its own token names the adapter and the
+// row is the projection's, and its accumulators as they were otherwise: what an adapter's tables hold, infinities and NaN too, stays with its tokens.
 template <int NN, int TT, bool SERIAL = false>    // SERIAL: the ranges of one token tile in flight at a time
 __device__ __forceinline__ void linear_add_deltas(f32x4 (&acc)[NN][TT], const LinearDeltas& lo, int (&left)[TT], int T, int t0, const int (&row0)[NN], int lane,
                                                   int first, int step) {
@@ -313,7 +314,16 @@ __device__ __forceinline__ void linear_add_deltas(f32x4 (&acc)[NN][TT], const Li
             low[e] = (elt)(f - (float)hi[e]);
           }
 #pragma unroll
-          for (int i = 0; i < NN; ++i) acc[i][j] = mfma_16x16x32(bf[i], low, mfma_16x16x32(bf[i], hi, acc[i][j]));
+          for (int i = 0; i < NN; ++i) {
+            if (row0[i] >= begin + rows || row0[i] + 16 <= begin) continue;      // uniform
+            const f32x4 sum = mfma_16x16x32(bf[i], low, mfma_16x16x32(bf[i], hi, acc[i][j]));
+            if (row0[i] >= begin && row0[i] + 16 <= begin + rows) {              // uniform: all rows of the tile are the projection's
+              acc[i][j] = left[j] == a ? sum : acc[i][j];
+            } else {
+#pragma unroll
+              for (int q = 0; q < 4; ++q) acc[i][j][q] = left[j] == a && (unsigned)(row0[i] + g8 / 2 + q - begin) < (unsigned)rows ? sum[q] : acc[i][j][q];
+            }
+          }
           if constexpr (SERIAL) asm volatile("" ::: "memory");
         }
       }

@@ -1767,3 +1767,54 @@ def test_deltas_inside_the_linear(ops, T, K, rows, r, who):
         gu = [(*p[:3], i * I, I) for i, p in enumerate(projs)]
         y2, _ = ops.linear_frag_deltas(f, W2, gu, d_ids, lora_ws)
         assert torch.equal(ops.linear_frag_silu_deltas(f, W2, gu, d_ids, lora_ws).data, ops.silu_mul(y2, frag=True).data)
+
+
+def _delta_case(ops, T, K, rows, r, n_ad, seed):
+    """Tables, packed weight and fragment-ordered tokens of a linear whose projections lie behind each other."""
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    rnd = lambda *s: torch.randn(s, generator=g, device=DEV)
+    x = rnd(T, K).half()
+    tabs = [((rnd(n_ad, r, K) * K ** -0.5).half(), rnd(n_ad, n, r).half()) for n in rows]
+    W = ops.PackedWeight((rnd(sum(rows), K) * K ** -0.5).half())
+    ws = torch.full((3 * ops._size(torch.float16, "mlora_gather_mm_workspace_bytes", T, K, r) // 4,), float("nan"), device=DEV)
+    return x, tabs, W, ws
+
+
+@pytest.mark.parametrize("T", [1, 16, 40, 64, 137])
+@pytest.mark.parametrize("r", [8, 64])
+def test_bad_weights_of_an_adapter_stay_with_its_tokens(ops, T, r):
+    """Infinities and NaN in A or B of some adapters, and a token whose activations overflow: the tokens that do not name them keep the bits
+    that they have with good tables, in every form that takes the deltas of several adapters in one product."""
+    K, rows, n_ad = 544, (64, 64), 6
+    x, tabs, W, ws = _delta_case(ops, T, K, rows, r, n_ad, T + r)
+    ids = torch.arange(T, device=DEV, dtype=torch.int32) % 7 - 1
+    if T == 1:
+        ids[0] = 2
+    ill = (ids == 0) | (ids == 3) | (ids == 5)
+    bad = [(A.clone(), B.clone()) for A, B in tabs]
+    for A, B in bad:
+        B[0], B[3, ::3], A[5, 0, 7] = float("inf"), float("nan"), float("inf")
+    xb = x.clone()
+    if T > 6:
+        xb[6, 3] = float("inf")
+        ill[6] = True
+    il = ops.interleave_gate_up(W.unpack())
+    out = []
+    for xx, tt in ((x, tabs), (xb, bad)):
+        f, projs, got = ops.FragActivation.pack(xx), [(A, B, 0.5, 64 * i, 64) for i, (A, B) in enumerate(tt)], []
+        y0 = torch.ones((T, 128), device=DEV)
+        got.append(ops.linear_frag_deltas(f, W, projs, ids, ws)[0])
+        got.append(ops.linear_frag_deltas(f, W, projs, ids, ws, out=y0.clone(), accumulate=True)[0])
+        got.append(ops.gather_mm_segments(y0.clone(), f, tt, [0, 64], [64, 64], ids, 0.5, ws))
+        got.append(ops.gather_mm(y0[:, :64].contiguous(), xx, *tt[0], ids, 0.5, ws))
+        if T <= 64:
+            act = ops.FragActivation(T, 64, DEV)
+            ops.check(ops.lib().mlora_gemv_frag_silu_deltas(act.data.data_ptr(), f.data.data_ptr(), il.data.data_ptr(), T, K, 64,
+                                                            *ops._delta_args("silu", f, W, projs, ids, ws)))
+            got.append(act.unpack())
+        else:
+            got.append(ops.linear_frag_silu_deltas(f, W, projs, ids, ws).unpack())
+        out.append(got)
+    torch.cuda.synchronize()
+    for a, b in zip(*out):
+        assert bool(torch.isfinite(a).all()) and torch.equal(a[~ill], b[~ill])
