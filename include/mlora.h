@@ -274,7 +274,8 @@ int mlora_linear_frag_lora(void* y, int y_dtype, int mode, const void* xf, const
 /* The linear of up to 64 tokens (N in whole 16) or of the mid-size kernel's shapes (below the persistent one's) with the LoRA deltas of any mix of
  * adapters in its accumulators: y (=|+=) xf . Wp^T + scaling * B[id] (A[id] x) for the rows n_begin[p] .. n_begin[p] + n_rows[p] of up to three projections (of one
  * rank in {8, 16, 32, 64}, n_ad and scaling), behind the matrix-core shrink of mlora_gather_mm; rounded once.  workspace: n_proj *
- * mlora_gather_mm_workspace_bytes(T, K, r) bytes.
+ * mlora_gather_mm_workspace_bytes(T, K, r) bytes.  Up to 64 tokens v = scaling * A x keeps the bits of fp32, as it does in mlora_gather_mm and
+ * mlora_gather_mm_segments there; for more tokens these, and the forms with extra k-steps, take it as two fp16 halves (22 bits, steps of 2^-24, up to 65504).
  *   mlora_linear_frag_deltas_pay   - whether a shape is served, and faster so than by mlora_linear_frag and mlora_gather_mm where the tokens of the
  *                                    pass name n_distinct adapters (accumulate: the mode);
  *   mlora_linear_frag_deltas       - ks > 1 (accumulating only): K slices as mlora_gemv_frag_acc_ksplit, slices 1.. into part[ks - 1][T][N];

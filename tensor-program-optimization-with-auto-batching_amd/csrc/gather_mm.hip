@@ -401,14 +401,15 @@ __global__ __launch_bounds__(GMM_THREADS, (GR == 8 ? 4 : 2)) void gather_mm_deco
 }
 
 // ---------------------------------------------------------------------------------------------
-// Prefill-sized gather-matmul (T > 64) on the matrix cores.  Tokens arrive grouped in adapter segments, so a tile
+// Gather-matmul on the matrix cores: T > 64, and fewer tokens that come in segments or whose partial sums do not fit one launch.  Tokens arrive grouped in adapter segments, so a tile
 // of 16 consecutive tokens holds one adapter, two at a segment boundary; a tile is processed once per distinct
 // adapter in it and rows of other adapters are masked at the store.
 //   shrink: workgroup per token tile, 4 waves split K;  V^T[r, 16 tok] = A[a] . X^T  with A[a] as the A operand
 //           (rows = rank index) and the token tile as the B operand, so a lane ends up with 4 consecutive rank
 //           entries of one token (one 16-byte store of v[t, 4g..4g+3]); fixed-order LDS sum of the 4 waves.
 //   expand: wave per (token tile, 64 output columns);  D[n, tok] = B[a] . V^T with v split into fp16 hi + lo halves
-//           (two MFMAs, ~22 mantissa bits of v); a lane read-modify-writes 4 consecutive y elements of one token.
+//           (two MFMAs, ~22 mantissa bits of v, steps of 2^-24, up to 65504); up to 64 tokens, where the kernels beside these hold v in
+//           fp32, into three scaled parts (Col32).  A lane read-modify-writes 4 consecutive y elements of one token.
 // v is [T, r] fp32 (one full sum per token, no K-slices).
 // ---------------------------------------------------------------------------------------------
 constexpr int SEG_WAVES = 4;
@@ -485,7 +486,8 @@ __device__ __forceinline__ f32x4 sum_ranges(const float* __restrict__ p, int spl
   return sum;
 }
 
-template <int R>
+// SUMS 2: the steps of a wave go to two sums in turn, added at the end - half the roundings behind each other.
+template <int R, int SUMS>
 __device__ __forceinline__ void shrink_tile_mfma(float* __restrict__ v, const f16* __restrict__ x, int frag_tt, const f16* __restrict__ A,
                                                  const int32_t* __restrict__ ids, int T, int K, int n_ad,
                                                  const int32_t* __restrict__ bucket_of, int bucket, int t0, int kb0, int kb1,
@@ -503,11 +505,13 @@ __device__ __forceinline__ void shrink_tile_mfma(float* __restrict__ v, const f1
 #pragma unroll
   for (int g0 = 0; g0 < 16; g0 += GA) {
     if (g0 < ta.n && (only_group < 0 || g0 == only_group * GA)) {   // uniform
-      f32x4 acc[GA][NT];
+      f32x4 acc[SUMS][GA][NT];
 #pragma unroll
-      for (int u = 0; u < GA; ++u)
+      for (int c = 0; c < SUMS; ++c)
 #pragma unroll
-        for (int i = 0; i < NT; ++i) acc[u][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int u = 0; u < GA; ++u)
+#pragma unroll
+          for (int i = 0; i < NT; ++i) acc[c][u][i] = f32x4{0.f, 0.f, 0.f, 0.f};
       // two register sets: the k-step after this one is requested before this one is multiplied
       f16x8 xf[2], af[2][GA][NT];
       auto load = [&](int s, int kb) {
@@ -531,7 +535,7 @@ __device__ __forceinline__ void shrink_tile_mfma(float* __restrict__ v, const f1
           if (g0 + u < ta.n) {
 #pragma unroll
             for (int i = 0; i < NT; ++i)
-              acc[u][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[s][u][i], xf[s], acc[u][i], 0, 0, 0);   // rows: rank index, cols: tokens
+              acc[s % SUMS][u][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[s][u][i], xf[s], acc[s % SUMS][u][i], 0, 0, 0);   // rows: rank index, cols: tokens
           }
         }
       };
@@ -548,7 +552,7 @@ __device__ __forceinline__ void shrink_tile_mfma(float* __restrict__ v, const f1
 #pragma unroll
       for (int u = 0; u < GA; ++u)
 #pragma unroll
-        for (int i = 0; i < NT; ++i) red[wave][u * NT + i][lane] = acc[u][i];
+        for (int i = 0; i < NT; ++i) red[wave][u * NT + i][lane] = SUMS == 2 ? acc[0][u][i] + acc[SUMS - 1][u][i] : acc[0][u][i];
       __syncthreads();
       // wave w sums and stores the adapters u = w, w + 4, ... of the group (fixed order over the four K parts)
 #pragma unroll
@@ -569,7 +573,7 @@ __device__ __forceinline__ void shrink_tile_mfma(float* __restrict__ v, const f1
   }
 }
 
-template <int R>
+template <int R, int SUMS>
 __global__ __launch_bounds__(SEG_WAVES * WAVE) void lora_shrink_mfma_kernel(float* __restrict__ v, const f16* __restrict__ x, int frag_tt,
                                                                             SegProjs pj,
                                                                             const int32_t* __restrict__ ids, int T, int K,
@@ -590,7 +594,7 @@ __global__ __launch_bounds__(SEG_WAVES * WAVE) void lora_shrink_mfma_kernel(floa
   const int per = (KB + gridDim.y - 1) / gridDim.y;
   const int kb0 = blockIdx.y * per, kb1 = min(KB, kb0 + per);
   v += ((size_t)proj * gridDim.y + blockIdx.y) * T * R;
-  shrink_tile_mfma<R>(v, x, frag_tt, A, ids, T, K, n_ad, bucket_of, bucket, blockIdx.x * 16, kb0, kb1, red, group);
+  shrink_tile_mfma<R, SUMS>(v, x, frag_tt, A, ids, T, K, n_ad, bucket_of, bucket, blockIdx.x * 16, kb0, kb1, red, group);
 }
 
 // Prefill-sized shrink: FOUR token tiles per workgroup.  When all adapted tokens of the four tiles use one adapter (an
@@ -625,7 +629,7 @@ __global__ __launch_bounds__(SEG_WAVES * WAVE, 2) void lora_shrink_quad_mfma_ker
   const bool same = __ballot(idl == a) == have;
   if (!same) {
     for (int u = 0; u < QT; ++u)
-      if (tq + u * 16 < T) shrink_tile_mfma<R>(v, x, frag_tt, A, ids, T, K, n_ad, bucket_of, bucket, tq + u * 16, kb0, kb1, red);
+      if (tq + u * 16 < T) shrink_tile_mfma<R, 1>(v, x, frag_tt, A, ids, T, K, n_ad, bucket_of, bucket, tq + u * 16, kb0, kb1, red);
     return;
   }
   const f16* __restrict__ Aa = A + (size_t)a * R * K + g * 8;
@@ -891,10 +895,11 @@ __global__ __launch_bounds__(SEG_WAVES * WAVE, 2) void lora_expand_pair_mfma_ker
   }
 }
 
-// Expand for token tiles that mix many adapters (decode batches).  Per block of 16 output columns every adapter of the tile contributes B[a] . v^T (two MFMAs: hi and lo half of
-// v); a token's column of the result is taken from the product of its own adapter, so all adapters are worked off before
-// the one read-modify-write of y.  The B fragments of up to GB adapters are requested together.
-template <int R, typename YT>
+// Expand for token tiles that mix many adapters (decode batches).  Per block of 16 output columns every adapter of the tile contributes B[a] . v^T; a
+// token's column of the result is taken from the product of its own adapter, so all adapters are worked off before
+// the one read-modify-write of y.  The B fragments of up to GB adapters are requested together.  V32 (up to 64 tokens): v with
+// the bits of fp32 (two 7B layers, 64 requests of thirty adapters at rank 64 557 us, with halves 553, on the fp32 matrix instruction 629).
+template <int R, typename YT, bool V32>
 __global__ __launch_bounds__(SEG_WAVES * WAVE) void lora_expand_mixed_mfma_kernel(SegProjs pj, const float* __restrict__ v,
                                                                             const int32_t* __restrict__ ids, float scaling,
                                                                             int T, int ldy, int n_ad,
@@ -929,8 +934,9 @@ __global__ __launch_bounds__(SEG_WAVES * WAVE) void lora_expand_mixed_mfma_kerne
   const int a_first = __builtin_amdgcn_readfirstlane(__shfl(id, __builtin_ctz(all), WAVE));
   const bool one_adapter = ((unsigned)__ballot(id == a_first) & 0xffffu) == all;
   const TileAdapters ta = tile_adapters(id);                     // the tile's distinct adapters and their rows, found once
-  // the token tile of v as the B operand, hi and lo halves: lane holds v[token col][ks*32 + 8g .. +7]
+  // the token tile of v as the B operand, in parts: lane holds v[token col][ks*32 + 8g .. +7]
   f16x8 vh[KS], vl[KS];
+  Col32 vc[KS];
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) {
     const int j = ks * 32 + g * 8;
@@ -948,13 +954,25 @@ __global__ __launch_bounds__(SEG_WAVES * WAVE) void lora_expand_mixed_mfma_kerne
         f[4 + e] = hi[e] * scaling;
       }
     }
+    if constexpr (V32) {
+      vc[ks] = col32_of(f);
+    } else {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const f16 h = (f16)f[e];
-      vh[ks][e] = h;
-      vl[ks][e] = (f16)(f[e] - (float)h);
+      for (int e = 0; e < 8; ++e) {
+        const f16 h = (f16)f[e];
+        vh[ks][e] = h;
+        vl[ks][e] = (f16)(f[e] - (float)h);
+      }
     }
   }
+  auto product = [&](const f16x8 bf, int ks, f32x4 c) -> f32x4 {       // rows: output column, cols: tokens
+    if constexpr (V32) {
+      return mfma_16x16x32_col32(bf, vc[ks], c);
+    } else {
+      c = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf, vh[ks], c, 0, 0, 0);
+      return __builtin_amdgcn_mfma_f32_16x16x32_f16(bf, vl[ks], c, 0, 0, 0);
+    }
+  };
   // write-back role of the lane: token lane / 4, the 16 columns of column tile lane % 4 (contiguous in y)
   const int wt = lane >> 2, wc = lane & 3;
   // SINGLE: the tile holds one adapter (a prefill segment) - the products accumulate directly, no per-token selection
@@ -975,8 +993,7 @@ __global__ __launch_bounds__(SEG_WAVES * WAVE) void lora_expand_mixed_mfma_kerne
             for (int ks = 0; ks < KS; ++ks) {
               const int j = ks * 32 + g * 8;
               const f16x8 bf = j < R ? ld8(Ba + (size_t)(nb + col) * R + ks * 32) : f16x8{0, 0, 0, 0, 0, 0, 0, 0};
-              acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf, vh[ks], acc, 0, 0, 0);    // rows: output column, cols: tokens
-              acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf, vl[ks], acc, 0, 0, 0);
+              acc = product(bf, ks, acc);
             }
           } else {
             // the tile's adapters GB at a time (ranks up to 32: all sixteen at once): their B fragments are requested
@@ -999,10 +1016,7 @@ __global__ __launch_bounds__(SEG_WAVES * WAVE) void lora_expand_mixed_mfma_kerne
                   if (g0 + u < ta.n) {
                     f32x4 d = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                    for (int ks = 0; ks < KS; ++ks) {
-                      d = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf[u][ks], vh[ks], d, 0, 0, 0);
-                      d = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf[u][ks], vl[ks], d, 0, 0, 0);
-                    }
+                    for (int ks = 0; ks < KS; ++ks) d = product(bf[u][ks], ks, d);
                     if ((ta.rows[g0 + u] >> col) & 1u) acc = d;
                   }
                 }
@@ -1239,8 +1253,14 @@ static int gmm_segments_shrink_r(const SegProjs& pj, const f16* x, int frag_tt, 
   // workgroup, about two workgroups per compute unit.  Either set of kernels is correct for either input.
   if (T <= 1024) {
     constexpr int NG = 16 / (8 / ((R + 15) / 16));   // adapter groups of a tile, each with its own workgroup
-    hipLaunchKernelGGL((lora_shrink_mfma_kernel<R>), dim3(tiles, splits, pj.n * NG), dim3(SEG_WAVES * WAVE), 0, s, v, x, frag_tt, pj, ids, T, K,
-                       n_ad, bf.bucket_of, bf.bucket);
+    // (up to 64 tokens, and with fewer ranges than there might be: two sums, so that a sum's error is that of the vector units' and of eight ranges; against
+    // fp64, K 11008, rank 64, 1e-7: vector units 1.33, one sum 1.47 in eight ranges, 1.86 in four)
+#define MLORA_SHRINK(SUMS)                                                                                                                    \
+  hipLaunchKernelGGL((lora_shrink_mfma_kernel<R, SUMS>), dim3(tiles, splits, pj.n * NG), dim3(SEG_WAVES * WAVE), 0, s, v, x, frag_tt, pj, ids, \
+                     T, K, n_ad, bf.bucket_of, bf.bucket)
+    if (T <= 64 || most < LORA_MAX_KC) MLORA_SHRINK(2);
+    else MLORA_SHRINK(1);
+#undef MLORA_SHRINK
   } else {
     const int quads = ceil_div(tiles, 4);
     splits = 256 / quads;                        // few K ranges: the expand adds the ranges' partial sums per token
@@ -1271,14 +1291,16 @@ static void gmm_segments_r(const SegProjs& pj, int y_dtype, int ldy, const f16* 
     nit = nit < 1 ? 1 : (nit > 8 ? 8 : nit);
   }
   const dim3 grid(mixed ? tiles : ceil_div(tiles, 2), ceil_div(N, SEG_WAVES * 64 * nit), pj.n);
-#define MLORA_EXPAND_MFMA(KERNEL, YT)                                                                                       \
-  hipLaunchKernelGGL((KERNEL<R, YT>), grid, dim3(SEG_WAVES * WAVE), 0, s, pj, v, ids, scaling, T, ldy, n_ad, \
+#define MLORA_EXPAND_MFMA(KERNEL, ...)                                                                                      \
+  hipLaunchKernelGGL((KERNEL<R, __VA_ARGS__>), grid, dim3(SEG_WAVES * WAVE), 0, s, pj, v, ids, scaling, T, ldy, n_ad, \
                      bf.bucket_of, bf.bucket, splits, nit)
   if (y_dtype == MLORA_F16) {
-    if (mixed) MLORA_EXPAND_MFMA(lora_expand_mixed_mfma_kernel, f16);
+    if (T <= 64) MLORA_EXPAND_MFMA(lora_expand_mixed_mfma_kernel, f16, true);
+    else if (mixed) MLORA_EXPAND_MFMA(lora_expand_mixed_mfma_kernel, f16, false);
     else MLORA_EXPAND_MFMA(lora_expand_pair_mfma_kernel, f16);
   } else {
-    if (mixed) MLORA_EXPAND_MFMA(lora_expand_mixed_mfma_kernel, float);
+    if (T <= 64) MLORA_EXPAND_MFMA(lora_expand_mixed_mfma_kernel, float, true);
+    else if (mixed) MLORA_EXPAND_MFMA(lora_expand_mixed_mfma_kernel, float, false);
     else MLORA_EXPAND_MFMA(lora_expand_pair_mfma_kernel, float);
   }
 #undef MLORA_EXPAND_MFMA

@@ -948,7 +948,7 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_mid_kernel(void* __res
       int row0[WNF];
 #pragma unroll
       for (int i = 0; i < WNF; ++i) row0[i] = tile_row(wn * WNF + i) * 16;
-      linear_add_deltas<WNF, WTF>(acc, lo, left, T, t0 + wt * WTF * 16, row0, lane, 0, 1);
+      linear_add_deltas<WNF, WTF, false>(acc, lo, left, T, t0 + wt * WTF * 16, row0, lane, 0, 1);
     }
   }
   wait_next();
@@ -1370,7 +1370,8 @@ static int mid_lora(const char* who, LinearDeltas& lo, const mlora_lora_bucket* 
   }
   lo.v = (const float*)workspace; lo.ids = ids; lo.scaling = projs[0].scaling;
   lo.n_proj = n_proj; lo.r = r; lo.n_ad = n_ad;
-  lo.ranges = mlora_lora_shrink_ranges(A, n_proj, xf, ids, T, K, r, n_ad, (float*)workspace, DELTA_RANGES, stream);
+  // (a long K up to 64 tokens: twice the ranges, so that the sums are as exact as elsewhere; a second round of loads, 1 us)
+  lo.ranges = mlora_lora_shrink_ranges(A, n_proj, xf, ids, T, K, r, n_ad, (float*)workspace, T <= 64 && K > 8192 ? 2 * DELTA_RANGES : DELTA_RANGES, stream);
   return MLORA_OK;
 }
 

@@ -268,7 +268,7 @@ __global__ __launch_bounds__(GEMV_WAVES* WAVE, (NT * TT > 8 ? 2 : 4)) void gemv_
         const int g = bid * NT + i;                // (a gated product: tiles of gate and up in turn)
         row0[i] = OUT == OUT_SILU_FRAG ? (g & 1) * (N / 2) + (g >> 1) * 16 : g * 16;
       }
-      linear_add_deltas<NT, TT, TILES <= 8 && (TT == 4 || NT * TT == 8)>(acc, ld, ids, T, 0, row0, lane, wave, GEMV_WAVES);
+      linear_add_deltas<NT, TT, true, TILES <= 8 && (TT == 4 || NT * TT == 8)>(acc, ld, ids, T, 0, row0, lane, wave, GEMV_WAVES);
     }
   }
 

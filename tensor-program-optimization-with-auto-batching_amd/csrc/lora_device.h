@@ -237,10 +237,49 @@ __device__ __forceinline__ float lora_row_dot(const f16* __restrict__ brow, cons
 
 #ifndef MLORA_ELT_F32
 // ---------------------------------------------------------------------------------------------
-// The deltas of any mix of adapters in the accumulators of a linear, y = x . W^T + v . B[id]^T with v = scaling * (sum of the shrink's K ranges) as
-// fp16 hi and lo halves.  Projections are row ranges of the fused weight.
+// The deltas of any mix of adapters in the accumulators of a linear, y = x . W^T + v . B[id]^T with v = scaling * (sum of the shrink's K ranges).  Projections
+// are row ranges of the fused weight.
 // ---------------------------------------------------------------------------------------------
-constexpr int DELTA_RANGES = 4;                // K ranges of the shrink: as many as are in flight together in registers
+
+// The second operand of mfma_16x16x32 with the bits of fp32: eight values of a column, scaled by a power of two that brings the largest of the column's 32 below
+// 2^15, as three fp16 parts.  11 bits each, the last one's step 2^-24: whole fp32 values down to 2^-14 of the largest, and 2^-39 of it below that.  48 cycles of a
+// SIMD a product, against 256 of the fp32 matrix instruction, and fewer roundings.  (Two parts of the values as they are keep 22 bits, nothing below 2^-24, and
+// make NaN of what is beyond 65504.)
+struct Col32 {
+  eltx8 part[3];
+  float back;                 // the inverse of the scale
+};
+__device__ __forceinline__ Col32 col32_of(const float (&f)[8]) {
+  float m = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) m = fmaxf(m, fabsf(f[e]));
+  m = fmaxf(m, __shfl_xor(m, 16, WAVE));                         // the other k-groups of the column
+  m = fmaxf(m, __shfl_xor(m, 32, WAVE));
+  const int ex = (int)(__float_as_uint(m) >> 23);                // biased; 255: an infinity, for which no part but the first is taken
+  const int sx = 268 - ex < 253 ? 268 - ex : 253;
+  const float scale = __uint_as_float((unsigned)sx << 23);
+  Col32 c;
+  c.back = __uint_as_float((unsigned)(254 - sx) << 23);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float x = f[e] * scale;
+    c.part[0][e] = (elt)x;
+    const float y = ex < 255 ? x - (float)c.part[0][e] : 0.f;
+    c.part[1][e] = (elt)y;
+    c.part[2][e] = (elt)(y - (float)c.part[1][e]);
+  }
+  return c;
+}
+__device__ __forceinline__ f32x4 mfma_16x16x32_col32(eltx8 a, const Col32& b, f32x4 c) {
+  f32x4 d = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int p = 2; p >= 0; --p) d = mfma_16x16x32(a, b.part[p], d);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) c[q] = fmaf(d[q], b.back, c[q]);
+  return c;
+}
+
+constexpr int DELTA_RANGES = 4;                // K ranges of the shrink that are in flight together in registers
 struct LinearDeltas {
   const elt* B[3];            // [n_ad][n_rows][r]
   int n_begin[3], n_rows[3];
@@ -254,7 +293,8 @@ struct LinearDeltas {
 // tokens (-1 past T).  A wave takes the adapters of these tokens in turn and of the rounds - an adapter, 32 ranks - every step-th (a power of two);
 // both operands come straight from memory.  A product's columns are tokens, so a lane keeps the sums of a round where its own token names the adapter and the
 // row is the projection's, and its accumulators as they were otherwise: what an adapter's tables hold, infinities and NaN too, stays with its tokens.
-template <int NN, int TT, bool SERIAL = false>    // SERIAL: the ranges of one token tile in flight at a time
+// V32: v with the bits of fp32 (up to 64 tokens); else as fp16 hi and lo halves.  SERIAL: the ranges of one token tile in flight at a time
+template <int NN, int TT, bool V32, bool SERIAL = false>
 __device__ __forceinline__ void linear_add_deltas(f32x4 (&acc)[NN][TT], const LinearDeltas& lo, int (&left)[TT], int T, int t0, const int (&row0)[NN], int lane,
                                                   int first, int step) {
   const int r16 = lane & 15, g8 = (lane >> 4) * 8;
@@ -291,32 +331,49 @@ __device__ __forceinline__ void linear_add_deltas(f32x4 (&acc)[NN][TT], const Li
         }
 #pragma unroll
         for (int j = 0; j < TT; ++j) {
+          if (!__ballot(left[j] == a)) continue;                 // uniform: no token of this tile names the adapter
           const int t = t0 + j * 16 + r16;
           const float* q = vp + (size_t)(t < T ? t : T - 1) * lo.r + (c < lo.r ? c : 0);
-          f32x4 x0[DELTA_RANGES], x1[DELTA_RANGES], s0 = f32x4{0.f, 0.f, 0.f, 0.f}, s1 = s0;
+          f32x4 s0 = f32x4{0.f, 0.f, 0.f, 0.f}, s1 = s0;
+          auto add_ranges = [&](int first) {
+            f32x4 x0[DELTA_RANGES], x1[DELTA_RANGES];
 #pragma unroll
-          for (int s = 0; s < DELTA_RANGES; ++s) {               // (past the last range: that one again, not added)
-            const float* qs = q + (size_t)(s < lo.ranges ? s : lo.ranges - 1) * T * lo.r;
-            x0[s] = *reinterpret_cast<const f32x4*>(qs);
-            x1[s] = *reinterpret_cast<const f32x4*>(qs + 4);
-          }
+            for (int s = 0; s < DELTA_RANGES; ++s) {             // (past the last range: that one again, not added)
+              const float* qs = q + (size_t)(first + s < lo.ranges ? first + s : lo.ranges - 1) * T * lo.r;
+              x0[s] = *reinterpret_cast<const f32x4*>(qs);
+              x1[s] = *reinterpret_cast<const f32x4*>(qs + 4);
+            }
 #pragma unroll
-          for (int s = 0; s < DELTA_RANGES; ++s) {
-            s0 = s < lo.ranges ? s0 + x0[s] : s0;
-            s1 = s < lo.ranges ? s1 + x1[s] : s1;
+            for (int s = 0; s < DELTA_RANGES; ++s) {
+              s0 = first + s < lo.ranges ? s0 + x0[s] : s0;
+              s1 = first + s < lo.ranges ? s1 + x1[s] : s1;
+            }
+          };
+          add_ranges(0);
+          if constexpr (V32) {
+            if (lo.ranges > DELTA_RANGES) add_ranges(DELTA_RANGES);        // uniform
           }
-          eltx8 hi, low;
           const bool of_a = left[j] == a && c < lo.r;            // (others': whatever lies there is replaced)
+          float f[8];
 #pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const float f = of_a ? (e < 4 ? s0[e & 3] : s1[e & 3]) * lo.scaling : 0.f;
-            hi[e] = (elt)f;
-            low[e] = (elt)(f - (float)hi[e]);
+          for (int e = 0; e < 8; ++e) f[e] = of_a ? (e < 4 ? s0[e & 3] : s1[e & 3]) * lo.scaling : 0.f;
+          eltx8 hi, low;
+          Col32 col;
+          if constexpr (V32) {
+            col = col32_of(f);
+          } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              hi[e] = (elt)f[e];
+              low[e] = (elt)(f[e] - (float)hi[e]);
+            }
           }
 #pragma unroll
           for (int i = 0; i < NN; ++i) {
             if (row0[i] >= begin + rows || row0[i] + 16 <= begin) continue;      // uniform
-            const f32x4 sum = mfma_16x16x32(bf[i], low, mfma_16x16x32(bf[i], hi, acc[i][j]));
+            f32x4 sum;
+            if constexpr (V32) sum = mfma_16x16x32_col32(bf[i], col, acc[i][j]);
+            else sum = mfma_16x16x32(bf[i], low, mfma_16x16x32(bf[i], hi, acc[i][j]));
             if (row0[i] >= begin && row0[i] + 16 <= begin + rows) {              // uniform: all rows of the tile are the projection's
               acc[i][j] = left[j] == a ? sum : acc[i][j];
             } else {

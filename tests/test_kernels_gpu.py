@@ -1818,3 +1818,26 @@ def test_bad_weights_of_an_adapter_stay_with_its_tokens(ops, T, r):
     torch.cuda.synchronize()
     for a, b in zip(*out):
         assert bool(torch.isfinite(a).all()) and torch.equal(a[~ill], b[~ill])
+
+
+@pytest.mark.parametrize("T,segs", [(1, 1), (16, 16), (17, 2), (64, 1), (64, 64)])
+@pytest.mark.parametrize("r", [8, 32, 64])
+@pytest.mark.parametrize("exp", [-24, -16, 14])
+def test_deltas_of_few_tokens_keep_32_bits(ops, T, segs, r, exp):
+    """Up to 64 tokens what comes out of the shrink stays fp32, very small or beyond fp16's largest: the error of a delta against fp64 is bounded
+    by that of fp32 sums, relative to the magnitudes that are added, without a smallest step."""
+    K, n, n_ad = 1056, 272, 64
+    x, ((A, B),), W, ws = _delta_case(ops, T, K, (n,), r, n_ad, T + r)
+    W = ops.PackedWeight(torch.zeros((n, K), device=DEV).half())
+    ids = torch.arange(T, device=DEV, dtype=torch.int32) * segs // T
+    scaling, f = 2.0 ** exp, ops.FragActivation.pack(x)
+    y0 = torch.zeros((T, n), device=DEV)
+    a, b = A[ids.long()].double(), B[ids.long()].double()
+    v, vm = ((t * scaling).squeeze(2) for t in (torch.matmul(a, x.double()[:, :, None]), torch.matmul(a.abs(), x.double().abs()[:, :, None])))
+    want = torch.matmul(b, v[:, :, None])[:, :, 0]
+    # (K + 16) roundings of v's K products and ranges, 2 r + 4 of the products that follow, each of at most 2^-24 of the magnitudes that are added
+    room = (K + 16 + 2 * r + 4) * 2.0 ** -24 * torch.matmul(b.abs(), vm[:, :, None])[:, :, 0]
+    # ... of which a sum in any order comes nowhere near: what fp16 halves of v lose at 2^-24 (their smallest step is 2^-24 itself) is beyond a tenth of it
+    for y in (ops.linear_frag_deltas(f, W, [(A, B, scaling, 0, n)], ids, ws, out_dtype=torch.float32)[0], ops.gather_mm_segments(y0.clone(), f, [(A, B)], [0], [n], ids, scaling, ws),
+              ops.gather_mm(y0.clone(), x, A, B, ids, scaling, ws)):
+        assert bool(((y.double() - want).abs() <= room / 10).all())
