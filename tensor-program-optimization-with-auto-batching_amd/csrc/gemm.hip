@@ -787,7 +787,7 @@ constexpr int mid_stages(int FT) { return FT == 16 ? 3 : 4; }
 
 // LORA: the deltas of any mix of adapters (linear_add_deltas) come into the accumulators ahead of the first step, while the ring fills.  Behind
 // the last step, as further steps of the ring, the same took 11 us: cold code and addresses that nothing hides.  137 tokens of one adapter of rank
-// 16, us: q, k, v (K 4096, N 12288) linear 31.0, shrink 5.4, expand 7.7 -> shrink 6.5, linear 35.0; o (N 4096, four K slices) 15.6, 5.0, 8.3 -> 6.5, 18.4.
+// 16, us: q, k, v (K 4096, N 12288) linear 31.0, shrink 5.4, expand 7.7 -> shrink 6.4, linear 37.8; o (N 4096, four K slices) 15.6, 5.0, 8.3 -> 6.4, 19.2.
 // GX: the rows are groups of gx_rows (a multiple of 16 FN) that read activations of their own, gx_stride elements apart.
 // A gated product (OUT_SILU, OUT_CLIP): Wp is the fused [2 I, K] matrix (N = 2 I), a block FN / 2 tiles of gate rows and the up rows of the same
 // channels, so that the waves wn = 0 hold the one and wn = 1 the other; they exchange halves through LDS, rounded to elements as a linear
@@ -948,7 +948,8 @@ __global__ __launch_bounds__(PP_WAVES* WAVE, 2) void gemm_mid_kernel(void* __res
       int row0[WNF];
 #pragma unroll
       for (int i = 0; i < WNF; ++i) row0[i] = tile_row(wn * WNF + i) * 16;
-      linear_add_deltas<WNF, WTF, false>(acc, lo, left, T, t0 + wt * WTF * 16, row0, lane, 0, 1);
+      int half[WTF];
+      linear_add_deltas<WNF, WTF, false>(acc, lo, left, half, T, t0 + wt * WTF * 16, row0, lane, 0, 1);
     }
   }
   wait_next();

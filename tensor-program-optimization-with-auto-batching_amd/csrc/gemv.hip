@@ -127,11 +127,12 @@ __global__ __launch_bounds__(GEMV_WAVES* WAVE) void lora_expand_shares_kernel(Lo
 // GX (fragment order): the rows are groups of gx_rows (a multiple of 16 NT) that read activations of their own, gx_stride elements apart;
 // those behind n_main are cut into gx_kq ranges of K, each a workgroup that leaves a block of y2 (so that no unit gets a whole
 // workgroup more than the others).
-// DELTA: adapter deltas (linear_add_deltas) join the waves' sums behind their last step, a wave every eighth round.  An expand launch of its own takes
-// 7 to 9 us, mostly its way to the first byte; here the rounds take 1 to 2.
+// DELTA: adapter deltas (linear_add_deltas) behind the waves' last step, a wave every eighth round.  An expand launch of its own takes
+// 7 to 9 us, mostly its way to the first byte; here the rounds take 1 to 2.  They are added behind the sum over the waves, ranks 0 .. 31 and then the others: in the
+// sums of the waves that did them, a token's bits would depend on the rows and the adapters of the others.
 struct NoDeltas {};
 template <int NT, int TT, int OUT, bool PACKED, bool XFRAG, bool SHRINK, int PIPE = 4, bool GX = false, bool DELTA = false>   // PIPE: k-steps in flight per wave
-__global__ __launch_bounds__(GEMV_WAVES* WAVE, (NT * TT > 8 ? 2 : 4)) void gemv_kernel(void* __restrict__ yv, const elt* __restrict__ x, int ldx,
+__global__ __launch_bounds__(GEMV_WAVES* WAVE, (NT * TT > 8 || (DELTA && TT > 1) ? 2 : 4)) void gemv_kernel(void* __restrict__ yv, const elt* __restrict__ x, int ldx,
                                                                 const elt* __restrict__ W, int T, int K, int N,
                                                                 LoraShrinkBatch sb, int shrink_blocks, int n_main,
                                                                 float* __restrict__ y2, int ksplit, float* __restrict__ part,
@@ -260,20 +261,124 @@ __global__ __launch_bounds__(GEMV_WAVES* WAVE, (NT * TT > 8 ? 2 : 4)) void gemv_
       load_stage(u, s0 + u + PIPE);
     }
   }
+  // the results of lane slot sl of a tile pair: the product of gate sums sg and up sums su of channels 16 p .. of token tile j
+  auto store_pair = [&](const f32x4& sg, const f32x4& su, int p, int j, int sl) {
+    constexpr int KIND = OUT == OUT_SILU_FRAG ? MLORA_GLU_SILU : MLORA_GLU_CLIPPED;
+    const int c = (bid * (NT / 2) + p) * 16 + (sl >> 4) * 4;     // output channel of the first of this lane's 4 rows
+    const int t = j * 16 + (sl & 15);
+    if (t < T && c < N / 2) {
+      eltx4 o;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) o[q] = (elt)glu<KIND>(sg[q], su[q], ga);
+      *reinterpret_cast<eltx4*>((elt*)yv + frag_offset(t, c, TT)) = o;
+    }
+  };
+  // ... of lane slot sl of a tile
+  auto store_tile = [&](const f32x4& s, int tile, int sl) {
+    const int i = tile / TT, j = tile % TT;
+    const int n = n0 + i * 16 + (sl >> 4) * 4;     // D[n][t]: lane holds rows 4*(lane/16)..+3, column lane%16
+    const int t = j * 16 + (sl & 15);
+    if (slice > 0) {                               // a K slice other than the first: fp32 partial, summed by the reader of y
+      if (t < T && n < N) *reinterpret_cast<f32x4*>(part + ((size_t)(slice - 1) * T + t) * N + n) = s;
+    } else if (t < T && n >= n_main && n < N) {
+      // rows past n_main are a second result block (adapter shrink rows appended to the weight): fp32, own buffer
+      *reinterpret_cast<f32x4*>(y2 + (size_t)t * (N - n_main) + (n - n_main)) = s;
+    } else if (t < T && n < N) {                   // N % 4 == 0: the 4 rows are inside together
+      const size_t o = (size_t)t * n_main + n;
+      if constexpr (OUT == OUT_F16) {
+        *reinterpret_cast<eltx4*>((elt*)yv + o) = eltx4{(elt)s[0], (elt)s[1], (elt)s[2], (elt)s[3]};
+      } else if constexpr (OUT == OUT_F32) {
+        *reinterpret_cast<f32x4*>((float*)yv + o) = s;
+      } else if constexpr (OUT == OUT_ACC_F32) {
+        f32x4* p = reinterpret_cast<f32x4*>((float*)yv + o);
+        *p = *p + s;
+      }
+    }
+  };
+
   if constexpr (DELTA) {
-    if (slice == 0) {                              // uniform
+    // the waves' sums go to LDS, the rounds into the same registers, then a wave adds up a tile of each pass: the sums and what has been done for it in rounds
+    static_assert(HT <= GEMV_WAVES, "a wave per tile");
+    constexpr int PASSES = TILES / HT;
+    f32x4 sum[PASSES];
+    int half[TT];
+    unsigned adapted = 0;                          // bit j: this lane's token of tile j has an adapter
+    auto give = [&](int h) {
+#pragma unroll
+      for (int i = 0; i < NT; ++i)
+#pragma unroll
+        for (int j = 0; j < TT; ++j) {
+          const int tile = i * TT + j;             // compile-time
+          if (tile / HT == h) red[wave][tile % HT][lane] = acc[i][j];
+        }
+    };
+    auto add_up = [&](int h) {
+      __syncthreads();
+      if (wave < HT) {
+        sum[h] = red[0][wave][lane];
+#pragma unroll
+        for (int w = 1; w < GEMV_WAVES; ++w) sum[h] += red[w][wave][lane];
+      }
+      __syncthreads();
+    };
+    auto rounds = [&]() {
       int row0[NT];
 #pragma unroll
       for (int i = 0; i < NT; ++i) {
         const int g = bid * NT + i;                // (a gated product: tiles of gate and up in turn)
         row0[i] = OUT == OUT_SILU_FRAG ? (g & 1) * (N / 2) + (g >> 1) * 16 : g * 16;
+#pragma unroll
+        for (int j = 0; j < TT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
       }
-      linear_add_deltas<NT, TT, true, TILES <= 8 && (TT == 4 || NT * TT == 8)>(acc, ld, ids, T, 0, row0, lane, wave, GEMV_WAVES);
+#pragma unroll
+      for (int j = 0; j < TT; ++j) adapted |= (unsigned)(ids[j] >= 0 && ids[j] < ld.n_ad) << j;
+      linear_add_deltas<NT, TT, true>(acc, ld, ids, half, T, 0, row0, lane, wave, GEMV_WAVES);
+    };
+    if constexpr (PASSES == 1) {
+      give(0);
+      if (slice == 0) rounds();                    // uniform
+      add_up(0);
+    } else {
+#pragma unroll
+      for (int h = 0; h < PASSES; ++h) {
+        give(h);
+        add_up(h);
+      }
+      if (slice == 0) rounds();
     }
+    if (slice == 0) {
+#pragma unroll
+      for (int h = 0; h < PASSES; ++h) {
+        if (h > 0) __syncthreads();
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+          for (int j = 0; j < TT; ++j) {
+            const int tile = i * TT + j;
+            if (tile / HT == h && half[j] >= 0) red[half[j]][tile % HT][lane] = acc[i][j];
+          }
+        __syncthreads();
+        if (wave < HT && ((adapted >> ((h * HT + wave) % TT)) & 1u)) {
+          sum[h] += red[0][wave][lane];
+          if (ld.r > 32) sum[h] += red[1][wave][lane];
+        }
+      }
+    }
+    if constexpr (OUT == OUT_SILU_FRAG) {
+      static_assert(PASSES == 1 && NT == 2, "one tile pair");
+      __syncthreads();
+      if (wave >= TT && wave < HT) red[0][wave][lane] = sum[0];        // the up tiles' sums to the waves of the gate tiles
+      __syncthreads();
+      if (wave < TT) store_pair(sum[0], red[0][TT + wave][lane], 0, wave, lane);
+    } else {
+#pragma unroll
+      for (int h = 0; h < PASSES; ++h)
+        if (wave < HT) store_tile(sum[h], h * HT + wave, lane);
+    }
+    return;
   }
 
   if constexpr (OUT == OUT_SILU_FRAG || OUT == OUT_CLIP_FRAG) {
-    constexpr int KIND = OUT == OUT_SILU_FRAG ? MLORA_GLU_SILU : MLORA_GLU_CLIPPED;
     // The weight interleaves 16-row tiles of gate and up, so this block's two tiles are gate rows c..c+15 and up
     // rows c..c+15 of the same channels: out[t, c + ..] = silu(elt(gate)) * elt(up), written in fragment order.
     static_assert(NT % 2 == 0 && TILES <= 8, "the SiLU epilogue pairs a gate tile with an up tile and sums all tiles in one pass");
@@ -291,14 +396,7 @@ __global__ __launch_bounds__(GEMV_WAVES* WAVE, (NT * TT > 8 ? 2 : 4)) void gemv_
         sg += red[w][2 * p * TT + j][sl];
         su += red[w][(2 * p + 1) * TT + j][sl];
       }
-      const int c = (bid * (NT / 2) + p) * 16 + (sl >> 4) * 4;   // output channel of the first of this lane's 4 rows
-      const int t = j * 16 + (sl & 15);
-      if (t < T && c < N / 2) {
-        eltx4 o;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) o[q] = (elt)glu<KIND>(sg[q], su[q], ga);
-        *reinterpret_cast<eltx4*>((elt*)yv + frag_offset(t, c, TT)) = o;
-      }
+      store_pair(sg, su, p, j, sl);
     }
     return;
   }
@@ -319,26 +417,7 @@ __global__ __launch_bounds__(GEMV_WAVES* WAVE, (NT * TT > 8 ? 2 : 4)) void gemv_
       f32x4 s = red[0][lt][sl];
 #pragma unroll
       for (int w = 1; w < GEMV_WAVES; ++w) s += red[w][lt][sl];
-      const int tile = h0 + lt;
-      const int i = tile / TT, j = tile % TT;
-      const int n = n0 + i * 16 + (sl >> 4) * 4;   // D[n][t]: lane holds rows 4*(lane/16)..+3, column lane%16
-      const int t = j * 16 + (sl & 15);
-      if (slice > 0) {                             // a K slice other than the first: fp32 partial, summed by the reader of y
-        if (t < T && n < N) *reinterpret_cast<f32x4*>(part + ((size_t)(slice - 1) * T + t) * N + n) = s;
-      } else if (t < T && n >= n_main && n < N) {
-        // rows past n_main are a second result block (adapter shrink rows appended to the weight): fp32, own buffer
-        *reinterpret_cast<f32x4*>(y2 + (size_t)t * (N - n_main) + (n - n_main)) = s;
-      } else if (t < T && n < N) {                 // N % 4 == 0: the 4 rows are inside together
-        const size_t o = (size_t)t * n_main + n;
-        if constexpr (OUT == OUT_F16) {
-          *reinterpret_cast<eltx4*>((elt*)yv + o) = eltx4{(elt)s[0], (elt)s[1], (elt)s[2], (elt)s[3]};
-        } else if constexpr (OUT == OUT_F32) {
-          *reinterpret_cast<f32x4*>((float*)yv + o) = s;
-        } else if constexpr (OUT == OUT_ACC_F32) {
-          f32x4* p = reinterpret_cast<f32x4*>((float*)yv + o);
-          *p = *p + s;
-        }
-      }
+      store_tile(s, h0 + lt, sl);
     }
   }
 }

@@ -290,17 +290,23 @@ struct LinearDeltas {
 };
 
 // acc [NN][TT]: 16-row tiles of W (row0: their first rows) x tiles of 16 tokens from t0 on, as mfma_16x16x32 leaves them; left: the ids of this lane's
-// tokens (-1 past T).  A wave takes the adapters of these tokens in turn and of the rounds - an adapter, 32 ranks - every step-th (a power of two);
-// both operands come straight from memory.  A product's columns are tokens, so a lane keeps the sums of a round where its own token names the adapter and the
-// row is the projection's, and its accumulators as they were otherwise: what an adapter's tables hold, infinities and NaN too, stays with its tokens.
-// V32: v with the bits of fp32 (up to 64 tokens); else as fp16 hi and lo halves.  SERIAL: the ranges of one token tile in flight at a time
-template <int NN, int TT, bool V32, bool SERIAL = false>
-__device__ __forceinline__ void linear_add_deltas(f32x4 (&acc)[NN][TT], const LinearDeltas& lo, int (&left)[TT], int T, int t0, const int (&row0)[NN], int lane,
-                                                  int first, int step) {
+// tokens (-1 past T).  A wave takes the adapters of these tokens in turn and of the rounds - an adapter, 32 ranks - every step-th (a power of two above one, or one);
+// both operands come straight from memory.  A product's columns are tokens, so a lane keeps the sums of a round where its own token names the adapter, and
+// its accumulators as they were otherwise: what an adapter's tables hold, infinities and NaN too, stays with its tokens.  (Without a branch: behind one the loads of
+// a wave's tiles would go out one after the other, 137 tokens x 12288 x 4096 42 instead of 36 us.)  Which wave
+// does a round follows the order of the adapters among the tokens; a token's one or two rounds are different waves', and half[j] says which of them
+// this wave has done for the lane's token (-1: none), so that the caller can add them in an order that does not depend on the other tokens.
+// V32: v with the bits of fp32 (up to 64 tokens); else as fp16 hi and lo halves.
+template <int NN, int TT, bool V32>
+__device__ __forceinline__ void linear_add_deltas(f32x4 (&acc)[NN][TT], const LinearDeltas& lo, int (&left)[TT], int (&half)[TT], int T, int t0, const int (&row0)[NN],
+                                                  int lane, int first, int step) {
   const int r16 = lane & 15, g8 = (lane >> 4) * 8;
 #pragma unroll
-  for (int j = 0; j < TT; ++j) left[j] = left[j] < lo.n_ad ? left[j] : -1;
-  int round = 0;                               // an adapter's first: which wave does it depends on the ids and r alone, not on the rows of a block
+  for (int j = 0; j < TT; ++j) {
+    left[j] = left[j] < lo.n_ad ? left[j] : -1;
+    half[j] = -1;
+  }
+  int round = 0;                               // an adapter's first
   for (;;) {
     int a = -1;
 #pragma unroll
@@ -309,6 +315,11 @@ __device__ __forceinline__ void linear_add_deltas(f32x4 (&acc)[NN][TT], const Li
       if (a < 0 && todo) a = __builtin_amdgcn_readlane(left[j], __builtin_ctzll(todo));
     }
     if (a < 0) break;
+    for (int c0 = 0; c0 < lo.r; c0 += 32) {
+      if ((round + c0 / 32) % step != first) continue;           // uniform
+#pragma unroll
+      for (int j = 0; j < TT; ++j) half[j] = left[j] == a ? c0 / 32 : half[j];
+    }
     for (int p = 0; p < lo.n_proj; ++p) {
       // projection p's, by masks: the compiler turns a choice into an address that depends on p, and `lo` would live in scratch memory
       const unsigned long long m0 = 0ull - (p == 0), m1 = 0ull - (p == 1), m2 = 0ull - (p == 2);
@@ -331,7 +342,6 @@ __device__ __forceinline__ void linear_add_deltas(f32x4 (&acc)[NN][TT], const Li
         }
 #pragma unroll
         for (int j = 0; j < TT; ++j) {
-          if (!__ballot(left[j] == a)) continue;                 // uniform: no token of this tile names the adapter
           const int t = t0 + j * 16 + r16;
           const float* q = vp + (size_t)(t < T ? t : T - 1) * lo.r + (c < lo.r ? c : 0);
           f32x4 s0 = f32x4{0.f, 0.f, 0.f, 0.f}, s1 = s0;
@@ -370,18 +380,12 @@ __device__ __forceinline__ void linear_add_deltas(f32x4 (&acc)[NN][TT], const Li
           }
 #pragma unroll
           for (int i = 0; i < NN; ++i) {
-            if (row0[i] >= begin + rows || row0[i] + 16 <= begin) continue;      // uniform
             f32x4 sum;
             if constexpr (V32) sum = mfma_16x16x32_col32(bf[i], col, acc[i][j]);
             else sum = mfma_16x16x32(bf[i], low, mfma_16x16x32(bf[i], hi, acc[i][j]));
-            if (row0[i] >= begin && row0[i] + 16 <= begin + rows) {              // uniform: all rows of the tile are the projection's
-              acc[i][j] = left[j] == a ? sum : acc[i][j];
-            } else {
-#pragma unroll
-              for (int q = 0; q < 4; ++q) acc[i][j][q] = left[j] == a && (unsigned)(row0[i] + g8 / 2 + q - begin) < (unsigned)rows ? sum[q] : acc[i][j][q];
-            }
+            const bool of_p = row0[i] < begin + rows && row0[i] + 16 > begin;    // uniform
+            acc[i][j] = left[j] == a && of_p ? sum : acc[i][j];
           }
-          if constexpr (SERIAL) asm volatile("" ::: "memory");
         }
       }
     }

@@ -1841,3 +1841,38 @@ def test_deltas_of_few_tokens_keep_32_bits(ops, T, segs, r, exp):
     for y in (ops.linear_frag_deltas(f, W, [(A, B, scaling, 0, n)], ids, ws, out_dtype=torch.float32)[0], ops.gather_mm_segments(y0.clone(), f, [(A, B)], [0], [n], ids, scaling, ws),
               ops.gather_mm(y0.clone(), x, A, B, ids, scaling, ws)):
         assert bool(((y.double() - want).abs() <= room / 10).all())
+
+
+@pytest.mark.parametrize("T", [7, 16, 33, 64, 130])
+@pytest.mark.parametrize("r", [8, 32, 64])
+def test_a_token_keeps_its_bits_in_any_row_beside_any_adapters(ops, T, r):
+    """The deltas of a token do not depend on the row that it has, nor on which adapters the other tokens name and in which order."""
+    K, rows, n_ad = 1056, (96, 64), 20
+    x, tabs, W, ws = _delta_case(ops, T, K, rows, r, n_ad, T + r)
+    W2, projs = ops.PackedWeight(W.unpack()[:128].contiguous()), [(*tabs[0], 0.5, 0, 96), (*tabs[1], 0.5, 96, 64)]
+    gu = [(tabs[1][0], tabs[1][1], 0.5, 0, 64), (tabs[0][0], tabs[0][1][:, :64].contiguous(), 0.5, 64, 64)]
+    il = ops.interleave_gate_up(W2.unpack())
+    ids = (torch.arange(T, device=DEV, dtype=torch.int32) * 7 + 3) % n_ad
+    others = ids.clone()
+    others[1:] = torch.where(torch.arange(1, T, device=DEV) % 3 == 0, ids[1:], (ids[1:] * 3 + 1) % (n_ad + 1) - 1)
+    same = torch.nonzero(others == ids).squeeze(1)
+
+    def run(xx, who):
+        f, out = ops.FragActivation.pack(xx), []
+        out.append(ops.linear_frag_deltas(f, W, projs, who, ws, out_dtype=torch.float32)[0])
+        resid, part = torch.zeros((T, 160), device=DEV), torch.full((3 * T * 160,), float("nan"), device=DEV)
+        acc, parts = ops.linear_frag_deltas(f, W, projs, who, ws, out=resid, accumulate=True, ks_ws=part)
+        out.append(acc)
+        out.append(ops.gather_mm_segments(torch.zeros((T, 160), device=DEV), f, [t for t in tabs], [0, 96], [96, 64], who, 0.5, ws))
+        if T <= 64:
+            act = ops.FragActivation(T, 64, DEV)
+            ops.check(ops.lib().mlora_gemv_frag_silu_deltas(act.data.data_ptr(), f.data.data_ptr(), il.data.data_ptr(), T, K, 64,
+                                                            *ops._delta_args("silu", f, W2, gu, who, ws)))
+            out.append(act.unpack())
+        else:
+            out.append(ops.linear_frag_silu_deltas(f, W2, gu, who, ws).unpack())
+        return out
+    a, c = run(x, ids), run(x, others)
+    for order in (torch.arange(T - 1, -1, -1, device=DEV), torch.randperm(T, generator=torch.Generator(device=DEV).manual_seed(T), device=DEV)):
+        for p, q, s in zip(a, run(x[order].contiguous(), ids[order].contiguous()), c):
+            assert torch.equal(p[order], q) and torch.equal(p[same], s[same])
