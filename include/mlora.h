@@ -596,7 +596,7 @@ typedef struct mlora_decode_plan {
   size_t lora_ws_bytes;
   float* ksplit_ws;           /* partials of the K-split o_proj / down_proj GEMVs, or NULL (no split) */
   size_t ksplit_ws_bytes;     /* >= mlora_gemv_ksplit_bytes over both projections (with their appended rows) */
-  int lora_segments;          /* > 0 (how many adapters the tokens name): up to 64 sequences, the deltas of a linear behind a shrink launch of their own, in the linear
+  int lora_segments;          /* > 0 (how many adapters the tokens may name): up to 64 sequences, the deltas of a linear behind a shrink launch of their own, in the linear
                                * (mlora_linear_frag_deltas) or after it (mlora_gather_mm_segments), instead of riding in the linear, attention
                                * and norm launches - for larger ranks, and few adapters of many tokens.  With lora_dense only those of gate
                                * and up.  Needs what those need of the shapes */

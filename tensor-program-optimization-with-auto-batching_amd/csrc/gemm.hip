@@ -1337,12 +1337,12 @@ static bool mid_deltas_serve(int T, int K, int N, bool accumulate) {
 // writes y.  Passes of two layers, us, on their own / in the linear, by rounds: 1 (7B, q, k, v and o, rank 16, 80 tokens) 423 / 404, (600 tokens) 1066 /
 // 1012, (hidden 1024, all seven, 200 tokens) 314 / 285; 2 (7B, all, rank 64, 300 tokens) 915 / 829; 3 (rank 16, 8 x 60 tokens, q, k, v, o) 774 / 737; 6
 // (rank 64, 4 x 90, all) 1022 / 1004; 7 (rank 16, 8 x 60) 778 / 752; 14 (rank 64, 8 x 50, all) 1002 / 1010, (hidden 1024, 8 x 150) 548 / 559.
-// Decode steps by rounds x tiles: 1 (7B, rank 32, 2 requests, all) 407 / 371; 2 (rank 64, one, all) 385 / 340, (hidden 1024) 197 / 145; 4 (rank 16, 64 of
-// one adapter, q, k, v, o) 408 / 408; 6 (rank 32, 16) 340 / 331; 15 (hidden 1024, rank 32, 40) 170 / 160; 28 (rank 64, 32 of seven) 391 / 387; 56
-// (rank 64, 32 of fourteen) 431 / 448, (hidden 1024) 216 / 202; 64 (64 of eight, all) 675 / 750; 120 (rank 32, 64 of thirty) 497 / 600.
+// Decode steps: (7B, rank 32, 2 requests, all) 407 / 371; (rank 64, one, all) 385 / 340, (hidden 1024) 197 / 145; (rank 32, 16) 340 / 331.  The line is one tile
+// of tokens, whatever they name (a step's bits must not follow its ids): of more tiles (rank 16, 64 of one adapter, q, k, v, o) 408 / 408, (hidden 1024, rank
+// 32, 40) 268 / 280, (rank 64, 32 of seven) 401 / 411, (rank 64, 49 of three) 441 / 460.
 extern "C" int mlora_linear_frag_deltas_pay(int T, int K, int N, int accumulate, int r, int n_distinct) {
   const long rounds = (long)ceil_div(r, 32) * n_distinct;
-  if (T <= 64) return T > 0 && K > 0 && K % 32 == 0 && N % 16 == 0 && rounds > 0 && rounds * ceil_div(T, 16) <= 32;
+  if (T <= 64) return T > 0 && T <= 16 && K > 0 && K % 32 == 0 && N % 16 == 0 && rounds > 0;
   return mid_deltas_serve(T, K, N, accumulate != 0) && rounds > 0 && rounds <= 8;
 }
 

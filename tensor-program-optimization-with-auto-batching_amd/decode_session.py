@@ -11,7 +11,7 @@ import numpy as np
 import torch
 
 from . import ops
-from .llama import distinct_adapters, most_of_one
+from .llama import share_of
 
 
 class DecodeSession:
@@ -41,8 +41,6 @@ class DecodeSession:
             self._inv = torch.from_numpy(np.argsort(order)).to(dev)
         self.seq_ids = list(seq_ids)
         self.tok_adapter = {tid: i32(ids) for tid, ids in tok_adapter.items()}
-        # one type: the ids on the host as well, for the choice that the native step makes from them
-        self.host_ids = {tid: ids.cpu().numpy() for tid, ids in self.tok_adapter.items()} if len(self.tok_adapter) == 1 else None
         if len(self.tok_adapter) > 1:         # several adapter types: merged once here (the check reads back to the host)
             self.tok_adapter = model._merge_types(self.tok_adapter)
         self.tokens = i32(first_tokens).clone()
@@ -56,7 +54,7 @@ class DecodeSession:
 
     def _enqueue(self):
         m = self.model
-        logits = m.forward(m.embed(self.tokens), self.kv, self.tok_adapter, *((None, self.host_ids) if self.host_ids else ()))
+        logits = m.forward(m.embed(self.tokens), self.kv, self.tok_adapter)
         self.tokens.copy_(ops.argmax(logits))
         self.pos.add_(1)
         self.ctx.add_(1)
@@ -179,9 +177,11 @@ class NativeDecodeSession:
         if lt is not None:
             p.lora_r, p.lora_n_ad, p.lora_scaling = lt.r, lt.n_adapters, lt.scaling
             p.lora_dense = (2 if self.o_delta_ride else 1) if self.dense_lora else 0
-            # (of one type: the union of several adds exact zeros to the sums of each, which matrix-core sums of another rank are not)
-            if not isinstance(tid, tuple) and model.segments_pay(T, most_of_one(ids), tid, bool(self.dense_lora)):
-                p.lora_segments = distinct_adapters(ids, lt.n_adapters)
+            # (beside appended rows whatever the types are: the zeros of a padded union leave the bits of each.  Without, one type alone: the union's rank would have
+            # the say over all of them, and the call per step of several types does not take these launches)
+            one = tid[0] if isinstance(tid, tuple) and len(tid) == 1 else tid
+            if model._segments_serve(T) if self.dense_lora else not isinstance(one, tuple) and model.segments_pay(T, share_of(T, lt.n_adapters), one):
+                p.lora_segments = min(T, lt.n_adapters)
         p.layers = C.cast(layers, C.POINTER(_lib.Layer))
         p.embed, p.norm, p.lm_head_p = model.embed_tokens.data_ptr(), model.norm.data_ptr(), model.lm_head.data.data_ptr()
         p.rope_cos, p.rope_sin, p.max_pos = kv.rope_cos.data_ptr(), kv.rope_sin.data_ptr(), kv.max_pos

@@ -253,18 +253,23 @@ class LlamaForCausalLM(CausalLM):
         return self._ws
 
     def segments_pay(self, T, most, tid, beside_rows=False):
-        """Whether the deltas of up to 64 tokens, of which `most` name one adapter (a prompt pass: its longest sequence), go to the matrix cores
-        in launches of their own, which take as long whatever the tokens share.  The units that ride in a decode step's launches, and the
-        one-launch kernel, work an adapter's tokens off one after the other.  Decode steps of two 7B layers, q, k, v and o adapted, us, riding /
+        """Whether the deltas of up to 64 tokens go to the matrix cores in launches of their own, which take as long whatever the tokens share.  The
+        units that ride in a decode step's launches, and the one-launch kernel, work an adapter's tokens off one after the other; `most` is how many that
+        is: of a prompt pass its longest sequence, of a step what an adapter has on average if all of the type are in use (`share_of`).  Nothing here may
+        follow the ids of a batch: the forms round differently, and a request's bits must not depend on what the others name.  That costs steps whose tokens share
+        more than that at ranks 8 and 16, and those that share nothing at rank 32.  Decode steps of two 7B layers, q, k, v and o adapted, us, riding /
         launches: rank 8, one adapter, 8 tokens 295 / 288, 64 tokens 563 / 369, sixteen of 64 361 / 393; rank 16, one, 4 tokens 285 / 281, 16 tokens
         349 / 290; two of 8 290 / 300; four of 32 359 / 310 (two of 32), eight of 32 314 / 331; rank 32, one token 301 / 277, 8 of 8 309 / 316, 64 of
-        64 503 / 455; rank 64, one 352 / 297, 64 of one 1732 / 396, 64 of 64 603 / 515.  (Launches of a shrink and an expand; where the expand
-        goes into the linear, `linear_frag_deltas_pay`, they take up to a quarter less.)  beside_rows: the shrink of the other linears is appended to
+        64 503 / 455; rank 64, one 352 / 297, 64 of one 1732 / 396, 64 of 64 603 / 515.  (Launches of a shrink and an expand; up to 16 tokens the expand
+        goes into the linear, `linear_frag_deltas_pay`, which takes up to a quarter less.)  beside_rows: the shrink of the other linears is appended to
         their weights, and what is asked for is gate and up, each a one-launch kernel otherwise; steps with all linears adapted, us, those / these:
         rank 16, one of two adapters 310 / 299, 8 of sixteen 346 / 318, 32 of sixty-four 479 / 407; rank 8, two of one 310 / 302, 16 of thirty-two 351
-        / 337, 64 of four 570 / 482; hidden 1024, rank 16, 4 of four 139 / 127, rank 8, 32 of sixteen 158 / 160."""
-        s, r = self.shape, self.lora_types[tid].r
-        return not (s.hidden_size % 32 or s.q_size % 32 or s.intermediate_size % 32 or s.kv_size % 16) and 0 < T <= 64 and (r >= 32 or most * r >= 96 or beside_rows)
+        / 337, 64 of four 570 / 482; hidden 1024, rank 16, 4 of four 139 / 127; the only one the other way round, by 1 %, is rank 8, 32 of sixteen 158 / 160."""
+        return self._segments_serve(T) and (self.lora_types[tid].r >= 32 or most * self.lora_types[tid].r >= 96 or beside_rows)
+
+    def _segments_serve(self, T):
+        s = self.shape
+        return 0 < T <= 64 and not (s.hidden_size % 32 or s.q_size % 32 or s.intermediate_size % 32 or s.kv_size % 16)
 
     def _lora(self, y, x, l, proj, tok_adapter, segments=False):
         """y += delta for every adapter type that targets (l, proj); tok_adapter: {tid: ids [T] int32}, or the merged
@@ -374,9 +379,9 @@ class LlamaForCausalLM(CausalLM):
         # native decode step)
         ks_ws = self._ksplit_ws(T) if dec_frag or (frag and (T <= 256 or is_decode)) else None
         segs = False
-        if T <= 64 and kv._cur is not None and len(tok_adapter) == 1 and "multi" not in tok_adapter and (host_ids is not None or not is_decode):
+        if T <= 64 and kv._cur is not None and len(tok_adapter) == 1 and "multi" not in tok_adapter:
             (tid, _), = tok_adapter.items()
-            segs = self.segments_pay(T, most_of_one(host_ids[tid]) if is_decode else max(kv._cur[1]), tid)
+            segs = self.segments_pay(T, share_of(T, self.lora_types[tid].n_adapters) if is_decode else max(kv._cur[1]), tid)
         # (what rides along in a decode step's launches counts as rows there; nothing does where the deltas are launches of their own)
         riding = (lambda *a: 0) if segs else self._riding_rows
         # a prefill-sized pass of one adapter type of rank 32 or 64: where a 256-token block agrees on one adapter its
@@ -396,11 +401,12 @@ class LlamaForCausalLM(CausalLM):
                     blk, rest = ops.lora_block_adapters(ids, lt.n_adapters)
                     rest = rest if bool((rest >= 0).any()) else None
                 fuse = (lt, ids, blk, None if rest is None else {tid: rest})
-        # below the persistent kernel's sizes the linears themselves take any mix of adapters, where the host knows that they are few
+        # below the persistent kernel's sizes the linears themselves take any mix of adapters: a prompt's where the host knows that they are few, and those of up
+        # to 16 tokens whatever they are
         near = None
-        if host_ids is not None and tok_adapter and "multi" not in tok_adapter and len(tok_adapter) == 1 and frag and (segs or T > 64 and not is_decode):
+        if segs or (host_ids is not None and len(tok_adapter) == 1 and "multi" not in tok_adapter and frag and T > 64 and not is_decode):
             (tid, ids), = tok_adapter.items()
-            near = (self.lora_types[tid], ids, distinct_adapters(host_ids[tid], self.lora_types[tid].n_adapters))
+            near = (self.lora_types[tid], ids, 1 if segs else distinct_adapters(host_ids[tid], self.lora_types[tid].n_adapters))
         o_shares = None
         if tok_adapter and "multi" not in tok_adapter and len(tok_adapter) == 1 and is_decode and T > 64 and frag:
             (tid, ids), = tok_adapter.items()
@@ -670,8 +676,7 @@ class LlamaForCausalLM(CausalLM):
         return super().prefill_no_adapter(h, kv)
 
     def decode_a(self, tid, h, kv, wids):
-        ids = self._ids(h.shape[0], {tid: (None, wids)}, host=True)
-        return self.forward(h, kv, {t: ops.upload(torch.from_numpy(a), self.device) for t, a in ids.items()}, host_ids=ids), kv
+        return self.forward(h, kv, self._ids(h.shape[0], {tid: (None, wids)})), kv
 
     def mixed_decode(self, tids, h, kv, *params):
         """params = sids_i, wids_i, sids_j, wids_j, ... for the adapter types in `tids`
@@ -708,9 +713,9 @@ class LlamaForCausalLM(CausalLM):
         return int(2 * (per_layer * s.num_hidden_layers + s.vocab_size * s.hidden_size))
 
 
-def most_of_one(ids) -> int:
-    """How many of the tokens of ids [T] (host) name the adapter that most of them name."""
-    return int(np.unique(ids[ids >= 0], return_counts=True)[1].max(initial=0))
+def share_of(T, n_adapters) -> int:
+    """How many of the T tokens of a step an adapter has where all n_adapters of the type are in use alike."""
+    return -(-T // max(n_adapters, 1))
 
 
 def block_adapters(ids, n_ad):

@@ -318,8 +318,8 @@ def test_native_step_with_deltas_in_launches_of_their_own(B, r, targets, dense):
     model = llama.LlamaForCausalLM.from_synthetic(9, shape, [synth.LoraSpec(r=r, alpha=r / 2, n_adapters=4, targets=targets)], DEV)
     ids = (np.arange(B) % 7 // 6).astype(np.int32)             # most name adapter 0
     ids[B // 2] = -1 if B > 1 else 0
-    most = llama.most_of_one(ids)
-    assert most == (ids == 0).sum() and model.segments_pay(B, most, 0) == (r >= 32 or most * r >= 96)
+    most = llama.share_of(B, 4)
+    assert most * 4 >= B > (most - 1) * 4 and model.segments_pay(B, most, 0) == (r >= 32 or most * r >= 96)
     got = {}
     for kind in ("py", "native", "graph", "riding"):
         kv = model.create_paged_kv_cache(B, B * 64, 32, 16, max_seq_len=64)
@@ -339,3 +339,71 @@ def test_native_step_with_deltas_in_launches_of_their_own(B, r, targets, dense):
     assert np.array_equal(got["graph"][0], got["native"][0]) and torch.equal(got["graph"][1], got["native"][1])
     a, b = got["native"][2], got["riding"][2]
     assert float((a - b).abs().max() / b.std()) <= 1e-2
+
+
+@pytest.mark.parametrize("B,r,targets,n_ad,dense", [(6, 16, ALL, 2, False), (12, 8, ("q_proj", "o_proj"), 3, False), (14, 64, ALL, 9, False), (20, 16, ALL, 1, False), (20, 64, ALL, 30, False),
+                                                    (41, 32, ALL, 16, False), (8, 16, ALL, 12, True), (24, 8, ALL, 7, True)])
+def test_a_request_keeps_its_bits_in_any_row_beside_any_others(B, r, targets, n_ad, dense):
+    """Logits and keys of some requests of a step, in three batches of the same size: as they are, the rows in reverse order, and beside requests that name other
+    adapters, one or none."""
+    synth, llama, dsm = load_pkg("synth"), load_pkg("llama"), load_pkg("decode_session")
+    shape = synth.LlamaShape(hidden_size=1024, intermediate_size=1408, num_attention_heads=8, num_key_value_heads=4, num_hidden_layers=2, head_dim=128, vocab_size=600)
+    model = llama.LlamaForCausalLM.from_synthetic(9, shape, [synth.LoraSpec(r=r, alpha=r / 2, n_adapters=n_ad, targets=targets)], DEV)
+    prompts = synth.randint(2, "bits", (B, 20), 600).numpy()
+    ids = (np.arange(B) * 5 % (n_ad + 1) - 1).astype(np.int32)
+    kept = [0, B // 2, B - 1]
+    got = {}
+    for name in ("as is", "reversed", "one", "others", "none"):
+        who = {"one": np.full(B, n_ad - 1), "others": (np.arange(B) * 3 + 1) % n_ad, "none": np.full(B, -1)}.get(name, ids).astype(np.int32)
+        who[kept] = ids[kept]
+        rows = list(range(B))[::-1] if name == "reversed" else list(range(B))
+        for native in (True, False) if not dense else (True,):
+            kv = model.create_paged_kv_cache(B, B * 64, 32, 16, max_seq_len=64)
+            first = _prefill(model, kv, prompts, who, chunk=1)
+            if native:
+                s = dsm.NativeDecodeSession(model, kv, rows, who[rows], first[rows], use_graph=False, dense_lora=dense)
+            else:
+                s = dsm.DecodeSession(model, kv, rows, {0: who[rows]}, first[rows])
+            logits = []
+            for _ in range(3):
+                s.step()
+                logits += [s.buf["logits"].view(B, -1)[[rows.index(q) for q in kept]]] if native else []
+            pages = torch.tensor(np.stack([kv.table_h[kv.slot[q]][:2] for q in kept]), device=DEV).reshape(-1).long()
+            got.setdefault(native, []).append((kv.k[:, pages].clone(), s.tokens[[rows.index(q) for q in kept]].clone(), *logits))
+    for runs in got.values():
+        for other in runs[1:]:
+            for a, b in zip(runs[0], other):
+                assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("r,B", [(16, 5), (32, 5), (64, 24), (16, 30)])
+def test_requests_without_adapter_beside_one_type(r, B):
+    """One adapter type and rows without: the call per step (`mixed_decode_a0`), the session of the front end and the native step have the same tokens and
+    keys, whether a batch's ids are on the host or not."""
+    synth, llama, dsm, ops = load_pkg("synth"), load_pkg("llama"), load_pkg("decode_session"), load_pkg("ops")
+    shape = synth.LlamaShape(hidden_size=1024, intermediate_size=1408, num_attention_heads=8, num_key_value_heads=4, num_hidden_layers=2, head_dim=128, vocab_size=600)
+    model = llama.LlamaForCausalLM.from_synthetic(9, shape, [synth.LoraSpec(r=r, alpha=r / 2, n_adapters=2, targets=ALL)], DEV)
+    prompts, ids = synth.randint(2, "bare", (B, 20), 600).numpy(), (np.arange(B) % 4 // 3 * 2 - 1).astype(np.int32) * -1
+    ids[1] = -1
+    has, got = np.flatnonzero(ids >= 0), []
+    for kind in ("steps", "session", "native", "native, of a tuple"):
+        kv = model.create_paged_kv_cache(B, B * 64, 32, 16, max_seq_len=64)
+        toks = [_prefill(model, kv, prompts, ids)]
+        rows = list(range(B))
+        if kind == "steps":
+            for _ in range(4):
+                kv.begin_forward(rows, [1] * B)
+                logits, _ = model["mixed_decode_a0"](model.embed(torch.from_numpy(toks[-1])), kv, has, ids[has])
+                kv.end_forward()
+                toks.append(ops.argmax(logits).cpu().numpy())
+        else:
+            if kind == "session":
+                s = dsm.DecodeSession(model, kv, rows, model._ids(B, {0: (has, ids[has])}), toks[0])
+            elif kind == "native":
+                s = dsm.NativeDecodeSession(model, kv, rows, ids, toks[0], dense_lora=False)
+            else:
+                s = dsm.NativeDecodeSession(model, kv, rows, model.union_rows((0,), B, {0: (has, ids[has])}), toks[0], tid=(0,), dense_lora=False)
+            toks += [s.step().cpu().numpy().copy() for _ in range(4)]
+        got.append((np.stack(toks), kv.k.clone()))
+    for toks, k in got[1:]:
+        assert np.array_equal(toks, got[0][0]) and torch.equal(k, got[0][1])
