@@ -325,3 +325,35 @@ def test_adapter_buckets_as_the_library_reads_them(scaling):
     got = bucket.from_buffer_copy(load_pkg("ops")._bucket(1 << 40, 24, 16, 3, scaling))
     want = bucket(1 << 40, 24, 16, 3, float(scaling))
     assert bytes(got) == bytes(want) and got.scaling == ctypes.c_float(float(scaling)).value
+
+
+@pytest.mark.parametrize("n", [1, 4, 127, 128, 212])
+def test_pages_of_a_pass_whichever_way_they_are_looked_up(n, monkeypatch):
+    """A few sequences are looked up one by one and many at once: the pages of each lie where the lengths ask for them and nowhere else, what does not fit is
+    refused with nothing staged, and a step of a few sequences builds no arrays."""
+    kvm, rng = load_pkg("kv_cache"), np.random.default_rng(n)
+    kv = kvm.PagedStateCache([], n * 6, 8, max_seqs=n, max_blocks=8, max_pos=120, dtype=torch.float32, device="cpu")
+    ids = [f"s{i}" for i in range(n)]
+    for s in ids:
+        kv.add_sequence(s)
+    lens = np.zeros(n, int)
+    for _ in range(6):
+        add = rng.integers(0, 15, n)
+        kv.begin_forward(ids, add.tolist())
+        kv.end_forward()
+        lens += add
+        rows = kv.table_h[[kv.slot[s] for s in ids]]
+        assert ((rows >= 0) == (np.arange(8) < -(-lens[:, None] // 16))).all()
+        used = rows[rows >= 0]
+        assert len(set(used.tolist())) == used.size and set(used.tolist()).isdisjoint(kv.free) and used.size + len(kv.free) == n * 6
+        assert [kv.lens[s] for s in ids] == lens.tolist()
+    with pytest.raises(RuntimeError, match="exceeds the cache geometry"):
+        kv.begin_forward(ids, [0] * (n - 1) + [121 - int(lens[-1])])
+    with pytest.raises(KeyError):
+        kv.begin_forward(["unknown"] * n, [1] * n)
+    with pytest.raises(ValueError):
+        kv.begin_forward(ids, [1] * (n + 1))
+    built = []
+    monkeypatch.setattr(kvm.np, "asarray", lambda *a, f=np.asarray, **k: built.append(a) or f(*a, **k))
+    kv.begin_forward(ids, [0] * n, device_meta=(None, None, None))
+    assert n >= 128 or not built
