@@ -332,7 +332,7 @@ def test_pages_of_a_pass_whichever_way_they_are_looked_up(n, monkeypatch):
     """A few sequences are looked up one by one and many at once: the pages of each lie where the lengths ask for them and nowhere else, what does not fit is
     refused with nothing staged, and a step of a few sequences builds no arrays."""
     kvm, rng = load_pkg("kv_cache"), np.random.default_rng(n)
-    kv = kvm.PagedStateCache([], n * 6, 8, max_seqs=n, max_blocks=8, max_pos=120, dtype=torch.float32, device="cpu")
+    kv = kvm.PagedStateCache([], 32, n * 6, max_seqs=n, max_blocks=8, max_pos=120, dtype=torch.float32, device="cpu")
     ids = [f"s{i}" for i in range(n)]
     for s in ids:
         kv.add_sequence(s)
