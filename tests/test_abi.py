@@ -181,6 +181,42 @@ def test_argument_validation_of_fused_and_batched_entry_points():
     assert lib.mlora_decode_step(None, None) == -1
 
 
+def _prefill_plan(lm, T, targets=(), layers=2, **fields):
+    """A plan of the 7B shape with dummy pointers; targets: which of the seven projections have tables."""
+    import ctypes as C
+    p, L = lm.PrefillPass(), (lm.Layer * layers)()
+    for e in L:
+        for f in ("ln1", "ln2", "qkv_p", "o_p", "gate_up_p", "down_p", "k_cache", "v_cache"):
+            setattr(e, f, 256)
+        for j in targets:
+            e.lora[j].A, e.lora[j].B = 256, 256
+    p.n_layers, p.hidden, p.inter, p.n_q_heads, p.n_kv_heads, p.head_dim, p.vocab, p.eps = layers, 4096, 11008, 32, 32, 128, 32000, 1e-5
+    p.T, p.n_rows, p.n_seq, p.max_blocks, p.n_pages, p.max_pos = T, 1, 1, 4096, 4096, 65536
+    for f in ("norm", "lm_head_p", "rope_cos", "rope_sin", "block_table", "tok_seq", "tok_pos", "logits_rows", "resid", "logits", "ws"):
+        setattr(p, f, 256)
+    if targets:
+        p.tok_adapter, p.lora_r, p.lora_n_ad, p.lora_scaling = 256, 16, 4, 0.5
+    p.layers = C.cast(L, C.c_void_p)
+    for k, v in fields.items():
+        setattr(p, k, v)
+    p._keep = L
+    return p
+
+
+def test_workspace_of_a_prompt_pass():
+    """Room for gate and up only where a layer keeps them, in the place of q, k, v and the attention output."""
+    import ctypes as C
+    lm = load_pkg("_lib")
+    need = lambda *a, **k: lm.lib().mlora_prefill_workspace_bytes(C.byref(_prefill_plan(lm, *a, **k)))
+    for T in (300, 4096, 16384):
+        xn, attention, act, gu = T * 4096 * 2, T * 4 * 4096 * 2, T * 11008 * 2, T * 2 * 11008 * 2
+        small = 3 * 8 * T * 16 * 4 + (1 << 17) + 16 * 11008 * 2 * 2      # adapters' scratch, last rows, whole tiles
+        assert xn + attention <= need(T) <= xn + max(attention, act) + small
+        assert need(T, (0, 2)) <= xn + max(attention, act) + small       # q and v
+        assert xn + act + gu <= need(T, (4, 5)) <= xn + act + gu + small # gate and up, nothing known of the adapters
+    assert need(300, (4, 5), n_distinct=1) <= 300 * 5 * 4096 * 2 + 3 * 8 * 300 * 16 * 4 + (1 << 17) + 16 * 11008 * 4
+
+
 def test_ops_refuse_cpu_tensors():
     import torch
     ops = load_pkg("ops")
