@@ -608,7 +608,8 @@ int mlora_decode_step(const mlora_decode_plan* plan, void* stream);
  * adapters as there; resid f32 [T, hidden] holds the embedded tokens and is left as the residual stream; logits f32 [n_rows, vocab] of the tokens
  * logits_rows [n_rows] (int64).  tok_adapter: NULL without adapters.  blk_adapter, tok_rest (mlora_lora_block_adapters): the deltas of ranks 32
  * and 64 as extra k-steps of the GEMMs where a block agrees on an adapter; tok_rest NULL: no token is left over.  segments: the deltas
- * otherwise go to mlora_gather_mm_segments (any T) instead of mlora_gather_mm.  Needs hidden, inter and n_q_heads * head_dim in whole 32.
+ * otherwise go to mlora_gather_mm_segments (any T) instead of mlora_gather_mm.  Needs hidden, inter and n_q_heads * head_dim in whole 32; a plan that is
+ * refused, here or in mlora_decode_step, queues nothing.
  * ws: mlora_prefill_workspace_bytes(plan) bytes (0 for a plan that is refused), 256-byte aligned.
  * Replaces: the batched forward of llama_for_causal_lm.py:79-100,121-144 as the host drives it operator by operator. */
 typedef struct mlora_prefill_plan {

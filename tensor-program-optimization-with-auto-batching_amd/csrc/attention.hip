@@ -1133,7 +1133,9 @@ __global__ __launch_bounds__(PF_WAVES* WAVE, 2) void paged_attn_prefill_block_ke
   }
 }
 
-int check_attn(const char* who, int Hq, int Hkv, int D, int n_pages, int n_seq, int max_blocks) {
+}  // namespace
+
+int mlora_check_attn(const char* who, int Hq, int Hkv, int D, int n_pages, int n_seq, int max_blocks) {
   MLORA_CHECK(D == 64 || D == 128, MLORA_ERR_UNSUPPORTED, "%s: head_dim %d not in {64, 128}", who, D);
   MLORA_CHECK(Hq > 0 && Hkv > 0 && Hq % Hkv == 0, MLORA_ERR_INVALID, "%s: bad heads Hq=%d Hkv=%d", who, Hq, Hkv);
   MLORA_CHECK(n_pages > 0 && n_seq > 0 && max_blocks > 0, MLORA_ERR_INVALID, "%s: bad cache shape n_pages=%d n_seq=%d max_blocks=%d", who, n_pages, n_seq, max_blocks);
@@ -1141,13 +1143,11 @@ int check_attn(const char* who, int Hq, int Hkv, int D, int n_pages, int n_seq, 
   return MLORA_OK;
 }
 
-}  // namespace
-
 static int rope_kv_append_impl(const char* who, void* qkv, void* k_cache, void* v_cache, const int32_t* block_table,
                                int max_blocks, const int32_t* tok_seq, const int32_t* tok_pos, const float* rope_cos,
                                const float* rope_sin, int max_pos, int T, int Hq, int Hkv, int D, int n_pages, int n_seq,
                                const LoraExpandQKV& lx, void* stream) {
-  if (int e = check_attn(who, Hq, Hkv, D, n_pages, n_seq, max_blocks)) return e;
+  if (int e = mlora_check_attn(who, Hq, Hkv, D, n_pages, n_seq, max_blocks)) return e;
   MLORA_CHECK(qkv && k_cache && v_cache && block_table && tok_seq && tok_pos && rope_cos && rope_sin, MLORA_ERR_INVALID, "%s: null pointer", who);
   MLORA_CHECK(T >= 0 && max_pos > 0, MLORA_ERR_INVALID, "%s: bad T=%d max_pos=%d", who, T, max_pos);
   if (T == 0) return MLORA_OK;
@@ -1205,7 +1205,7 @@ static int paged_attn_decode_impl(void* out, int out_layout, const void* qkv, co
                                   const int32_t* block_table, int max_blocks, const int32_t* seq_ids,
                                   const int32_t* ctx_len, int B, int Hq, int Hkv, int D, int n_pages, int n_seq,
                                   const int32_t* tok_adapter, int r, int n_ad, const void* o_A, void* o_vpart, void* stream) {
-  if (int e = check_attn("paged_attn_decode", Hq, Hkv, D, n_pages, n_seq, max_blocks)) return e;
+  if (int e = mlora_check_attn("paged_attn_decode", Hq, Hkv, D, n_pages, n_seq, max_blocks)) return e;
   MLORA_CHECK(out && qkv && k_cache && v_cache && block_table && seq_ids && ctx_len, MLORA_ERR_INVALID, "paged_attn_decode: null pointer");
   MLORA_CHECK(B >= 0 && B <= 65535, MLORA_ERR_INVALID, "paged_attn_decode: bad B=%d (0..65535)", B);
   MLORA_CHECK(out_layout == MLORA_ROWMAJOR || out_layout == MLORA_FRAG, MLORA_ERR_INVALID, "paged_attn_decode: bad out_layout %d", out_layout);
@@ -1277,7 +1277,7 @@ static int rope_attn_decode_impl(void* out, int out_layout, const void* qkv, voi
                                  const float* rope_sin, int max_pos, int B, int Hq, int Hkv, int D, int n_pages, int n_seq,
                                  const void* v_part, int v_dense, const void* const* Bmat, const int32_t* tok_adapter,
                                  float scaling, int K, int r, int n_ad, const void* o_A, void* o_vpart, void* stream) {
-  if (int e = check_attn("rope_attn_decode", Hq, Hkv, D, n_pages, n_seq, max_blocks)) return e;
+  if (int e = mlora_check_attn("rope_attn_decode", Hq, Hkv, D, n_pages, n_seq, max_blocks)) return e;
   MLORA_CHECK(out && qkv && k_cache && v_cache && block_table && seq_ids && tok_pos && ctx_len && rope_cos && rope_sin,
               MLORA_ERR_INVALID, "rope_attn_decode: null pointer");
   MLORA_CHECK(B >= 0 && B <= 65535 && max_pos > 0, MLORA_ERR_INVALID, "rope_attn_decode: bad B=%d (0..65535) max_pos=%d", B, max_pos);
@@ -1367,7 +1367,7 @@ extern "C" int mlora_paged_attn_prefill(void* out, int out_layout, const void* q
                                         const int32_t* block_table, int max_blocks, const int32_t* tok_seq,
                                         const int32_t* tok_pos, int T, int Hq, int Hkv, int D, int n_pages, int n_seq,
                                         void* stream) {
-  if (int e = check_attn("paged_attn_prefill", Hq, Hkv, D, n_pages, n_seq, max_blocks)) return e;
+  if (int e = mlora_check_attn("paged_attn_prefill", Hq, Hkv, D, n_pages, n_seq, max_blocks)) return e;
   MLORA_CHECK(out && qkv && k_cache && v_cache && block_table && tok_seq && tok_pos, MLORA_ERR_INVALID, "paged_attn_prefill: null pointer");
   MLORA_CHECK(T >= 0 && ceil_div(T, PF_WAVES * 16 * PF_QT) <= 65535, MLORA_ERR_INVALID, "paged_attn_prefill: bad T=%d", T);
   MLORA_CHECK(out_layout == MLORA_ROWMAJOR || out_layout == MLORA_FRAG, MLORA_ERR_INVALID, "paged_attn_prefill: bad out_layout %d", out_layout);

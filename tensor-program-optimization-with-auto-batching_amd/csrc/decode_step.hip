@@ -175,6 +175,26 @@ extern "C" int mlora_decode_step(const mlora_decode_plan* p, void* stream) {
   const size_t ws_need = (size_t)(3 * kq + 2) * slot;
   MLORA_CHECK(!lora || (p->lora_ws && p->lora_ws_bytes >= ws_need), MLORA_ERR_WORKSPACE,
               "decode_step: lora_ws of %zu bytes given, %zu needed", p->lora_ws_bytes, ws_need);
+  // ... and what deltas in launches of their own ask of sizes, room and alignment (the projections that are adapted and take them)
+  if (segs || gu_segs) {
+    size_t seg_need = 0;
+    MLORA_CHECK((r == 8 || r == 16 || r == 32 || r == 64) && n_ad > 0 && n_ad <= 65535, MLORA_ERR_UNSUPPORTED,
+                "decode_step: lora_segments: rank %d not in {8,16,32,64} or bad lora_n_ad %d", r, n_ad);
+    const int K_of[7] = {H, H, H, q_sz, H, H, I}, N_of[7] = {q_sz, kv_sz, kv_sz, H, I, I, H}, ld_of[7] = {qkv_sz, qkv_sz, qkv_sz, H, 2 * I, 2 * I, H};
+    for (int l = 0; l < p->n_layers; ++l)
+      for (int j = 0; j < 7; ++j) {
+        if (!p->layers[l].lora[j].A || !(segs || j == MLORA_GATE || j == MLORA_UP)) continue;
+        MLORA_CHECK(K_of[j] % 32 == 0 && N_of[j] % 16 == 0 && ld_of[j] % 8 == 0, MLORA_ERR_UNSUPPORTED,
+                    "decode_step: lora_segments need inputs in whole 32 and outputs in whole 16 (projection %d: %d, %d)", j, K_of[j], N_of[j]);
+        const size_t n = 3 * mlora_gather_mm_workspace_bytes(T, K_of[j], r);
+        seg_need = n > seg_need ? n : seg_need;
+      }
+    MLORA_CHECK(p->lora_ws_bytes >= seg_need, MLORA_ERR_WORKSPACE, "decode_step: lora_ws of %zu bytes given, %zu needed", p->lora_ws_bytes, seg_need);
+    // (inside the linear: what it reads; behind it: what they add to)
+    MLORA_CHECK(T > 16 || ((uintptr_t)p->lora_ws & 15) == 0, MLORA_ERR_WORKSPACE, "decode_step: lora_segments need a 16-byte aligned lora_ws");
+    const uintptr_t of = T <= 16 ? (uintptr_t)p->xn | (uintptr_t)p->attn | (uintptr_t)p->act : (uintptr_t)p->qkv | (uintptr_t)p->gate_up | (uintptr_t)p->resid;
+    MLORA_CHECK((of & 15) == 0, MLORA_ERR_UNSUPPORTED, "decode_step: lora_segments need 16-byte aligned buffers");
+  }
   char* ws = (char*)p->lora_ws;
   void* ws_qkv = ws;
   void* ws_o = ws + (size_t)3 * kq * slot;

@@ -1,7 +1,11 @@
 // A prompt pass of the whole model enqueued natively: the operators of the per-operator path (llama.py, forward) in their order, with the same
 // choices, from one call.  Up to a few hundred tokens a pass is shorter than the host takes to queue it operator by operator (14 us a launch; a
 // launch from here 4): two layers of hidden 1024, 8 prompts of 27 to 54 tokens 422 -> 272 us, two of the 7B shape, 6 to 12 tokens 476 -> 365.
+#include <initializer_list>
+
 #include "common.h"
+
+int mlora_check_attn(const char* who, int Hq, int Hkv, int D, int n_pages, int n_seq, int max_blocks);
 
 namespace {
 
@@ -84,6 +88,26 @@ Slots slots_of(const mlora_prefill_plan* p) {
   return s;
 }
 
+// A projection of a layer: its tables, and which rows of the (fused) weight it has
+constexpr int MAXP = 3;
+struct Proj {
+  const mlora_lora_proj* t;
+  int c0, n;
+};
+// the projections of in[0..n) that have tables
+int live_of(const mlora_prefill_plan* p, const Proj* in, int n, Proj* out) {
+  int live = 0;
+  for (int i = 0; p->tok_adapter && i < n; ++i)
+    if (in[i].t->A) out[live++] = in[i];
+  return live;
+}
+// Whether the deltas of pj ride in the persistent GEMM as further k-steps: a 256-row block must lie in one projection
+bool rides(const mlora_prefill_plan* p, int K, int N, const Proj* pj, int n) {
+  bool r = n > 0 && p->blk_adapter && mlora_gemm_frag_preferred(p->T, K, N);
+  for (int i = 0; i < n; ++i) r = r && pj[i].c0 % 256 == 0 && (pj[i].n % 256 == 0 || pj[i].c0 + pj[i].n == N);
+  return r;
+}
+
 int check_plan(const mlora_prefill_plan* p) {
   MLORA_CHECK(p && p->layers, MLORA_ERR_INVALID, "prefill: null plan");
   MLORA_CHECK(p->T > 0 && p->n_layers >= 0 && p->n_rows > 0 && p->n_q_heads > 0 && p->n_kv_heads > 0 && p->head_dim > 0 && p->hidden > 0 && p->inter > 0 &&
@@ -93,6 +117,10 @@ int check_plan(const mlora_prefill_plan* p) {
               "prefill: hidden, intermediate and q sizes must be multiples of 32");
   MLORA_CHECK(!p->tok_adapter || p->lora_r == 8 || p->lora_r == 16 || p->lora_r == 32 || p->lora_r == 64, MLORA_ERR_UNSUPPORTED,
               "prefill: rank %d not in {8,16,32,64}", p->lora_r);
+  MLORA_CHECK(!p->tok_adapter || (p->lora_n_ad > 0 && p->lora_n_ad <= 65535 && p->T <= (1 << 20)), MLORA_ERR_INVALID, "prefill: bad lora_n_ad %d (T=%d)",
+              p->lora_n_ad, p->T);
+  MLORA_CHECK(ceil_div(p->T, 128) <= 65535 && p->hidden <= 16384 && p->vocab % 4 == 0, MLORA_ERR_UNSUPPORTED,
+              "prefill: T=%d or hidden=%d too large, or vocab %% 4 != 0 (%d)", p->T, p->hidden, p->vocab);
   MLORA_CHECK(!p->blk_adapter || (p->tok_adapter && (p->lora_r == 32 || p->lora_r == 64)), MLORA_ERR_INVALID, "prefill: blk_adapter goes with ranks 32 and 64");
   return MLORA_OK;
 }
@@ -109,13 +137,29 @@ extern "C" int mlora_prefill(const mlora_prefill_plan* p, void* stream) {
                   p->logits && p->ws,
               MLORA_ERR_INVALID, "prefill: null buffer");
   const bool lora = p->tok_adapter != nullptr;
-  // every layer is looked at before the first launch: a rejected call enqueues nothing
+  // every layer, and what the operators ask of its sizes, is looked at before the first launch: a rejected call enqueues nothing
+  STEP(mlora_check_attn("prefill", Hq, Hkv, D, p->n_pages, p->n_seq, p->max_blocks));
+  MLORA_CHECK(T > 256 || H <= 8192 || (mlora_gemv_ksplit(T, q_sz, H) == 1 && mlora_gemv_ksplit(T, I, H) == 1), MLORA_ERR_UNSUPPORTED,
+              "prefill: a pass that splits K needs hidden <= 8192 (%d)", H);
   for (int l = 0; l < p->n_layers; ++l) {
     const mlora_layer& L = p->layers[l];
     MLORA_CHECK(L.ln1 && L.ln2 && L.qkv_p && L.o_p && L.gate_up_p && L.down_p && L.k_cache && L.v_cache, MLORA_ERR_INVALID,
                 "prefill: layer %d has a null weight, norm or cache pointer", l);
     for (int j = 0; lora && j < 7; ++j)
       MLORA_CHECK(!L.lora[j].A || L.lora[j].B, MLORA_ERR_INVALID, "prefill: layer %d projection %d has A but no B table", l, j);
+    MLORA_CHECK(!lora || !p->segments || kv_sz % 16 == 0 || !(L.lora[MLORA_K].A || L.lora[MLORA_V].A), MLORA_ERR_UNSUPPORTED,
+                "prefill: segments need key/value sizes in whole 16 (%d)", kv_sz);
+    auto aligned = [&](int K, int N, std::initializer_list<Proj> all) {
+      Proj pj[MAXP];
+      const int n = live_of(p, all.begin(), (int)all.size(), pj);
+      bool ok = true;
+      for (int i = 0; rides(p, K, N, pj, n) && i < n; ++i) ok = ok && ((uintptr_t)pj[i].t->B & 15) == 0;
+      return ok;
+    };
+    MLORA_CHECK(aligned(H, qkv_sz, {{&L.lora[MLORA_Q], 0, q_sz}, {&L.lora[MLORA_K], q_sz, kv_sz}, {&L.lora[MLORA_V], q_sz + kv_sz, kv_sz}}) &&
+                    aligned(q_sz, H, {{&L.lora[MLORA_O], 0, H}}) && aligned(H, 2 * I, {{&L.lora[MLORA_GATE], 0, I}, {&L.lora[MLORA_UP], I, I}}) &&
+                    aligned(I, H, {{&L.lora[MLORA_DOWN], 0, H}}),
+                MLORA_ERR_INVALID, "prefill: layer %d: the B tables of deltas inside the persistent GEMM must be 16-byte aligned", l);
   }
   const Slots at = slots_of(p);
   MLORA_CHECK(p->ws_bytes >= at.total && ((uintptr_t)p->ws & 255) == 0, MLORA_ERR_WORKSPACE, "prefill: workspace of %zu bytes given, %zu needed (256-byte aligned)",
@@ -126,14 +170,6 @@ extern "C" int mlora_prefill(const mlora_prefill_plan* p, void* stream) {
   float* part = at.ksplit_bytes ? (float*)(ws + at.ksplit) : nullptr;
   const int r = p->lora_r, n_ad = p->lora_n_ad;
   const float sc = p->lora_scaling;
-  struct Proj { const mlora_lora_proj* t; int c0, n; };
-  constexpr int MAXP = 3;
-  auto live_of = [&](const Proj* in, int n, Proj* out) {
-    int live = 0;
-    for (int i = 0; lora && i < n; ++i)
-      if (in[i].t->A) out[live++] = in[i];
-    return live;
-  };
   // deltas of projections that read x and own column ranges of y, for the tokens of ids
   struct Buckets { mlora_lora_bucket bk[MAXP]; int32_t c[MAXP], nc[MAXP]; };
   auto buckets_of = [&](const Proj* pj, int n) {
@@ -173,11 +209,9 @@ extern "C" int mlora_prefill(const mlora_prefill_plan* p, void* stream) {
   // to fp32 only): the K slices whose partials the next norm adds.
   auto linear = [&](void* y, int y_dtype, int mode, const void* x, const void* W, int K, int N, const Proj* all, int n_all, int* ks) -> int {
     Proj pj[MAXP];
-    const int n = live_of(all, n_all, pj);
-    bool rides = n > 0 && p->blk_adapter && mlora_gemm_frag_preferred(T, K, N);
-    for (int i = 0; i < n; ++i) rides = rides && pj[i].c0 % 256 == 0 && (pj[i].n % 256 == 0 || pj[i].c0 + pj[i].n == N);
+    const int n = live_of(p, all, n_all, pj);
     if (ks) *ks = 1;
-    if (rides) {
+    if (rides(p, K, N, pj, n)) {
       mlora_fused_lora f[MAXP];
       STEP(halves(x, K, pj, n, f));
       STEP(mlora_linear_frag_lora(y, y_dtype, mode, x, W, T, K, N, f, n, p->blk_adapter, r, stream));
@@ -221,7 +255,7 @@ extern "C" int mlora_prefill(const mlora_prefill_plan* p, void* stream) {
     STEP(norm(L.ln2, ks));
     const Proj gate_up[2] = {{&L.lora[MLORA_GATE], 0, I}, {&L.lora[MLORA_UP], I, I}};
     Proj gl[MAXP];
-    const int n_gl = live_of(gate_up, 2, gl);
+    const int n_gl = live_of(p, gate_up, 2, gl);
     switch (gate_up_form(p, L)) {
       case GU_IL: STEP(mlora_gemv_frag_silu(act, xn, L.gate_up_il_p, T, H, I, stream)); break;
       case GU_LINEAR: STEP(mlora_linear_frag_glu(act, xn, L.gate_up_p, T, H, I, MLORA_GLU_SILU, 0.f, 0.f, 0.f, stream)); break;

@@ -203,6 +203,91 @@ def _prefill_plan(lm, T, targets=(), layers=2, **fields):
     return p
 
 
+def test_rejected_passes_queue_nothing():
+    """What the operators of a prompt pass or a step ask of its sizes is refused ahead of the first launch (which would report no device here): the codes are those
+    of the refusal, whichever layer it is about."""
+    import ctypes as C
+    lm = load_pkg("_lib")
+    lib = lm.lib()
+
+    def prefill(T=40, targets=(0, 1, 2, 3, 4, 5, 6), layer1=None, **fields):
+        p = _prefill_plan(lm, T, targets, **fields)
+        p.ws_bytes = 1 << 40
+        if layer1:
+            layer1(p._keep[1])
+        return lib.mlora_prefill(C.byref(p), None), lib.mlora_last_error()
+    assert prefill(head_dim=96)[0] == -2 and prefill(n_kv_heads=5)[0] == -1 and prefill(n_pages=0)[0] == -1
+    assert prefill(lora_r=12)[0] == -2 and prefill(lora_n_ad=0)[0] == -1 and prefill(lora_n_ad=70000)[0] == -1
+    assert prefill(vocab=32002)[0] == -2 and prefill(inter=11000)[0] == -2 and prefill(T=0)[0] == -1 and prefill(n_rows=0)[0] == -1
+    assert prefill(blk_adapter=256)[0] == -1 and prefill(T=4096, lora_r=64, blk_adapter=256, layer1=lambda L: setattr(L.lora[3], "B", 264))[0] == -1
+    assert prefill(layer1=lambda L: setattr(L.lora[6], "B", None))[0] == -1 and prefill(layer1=lambda L: setattr(L, "down_p", None))[0] == -1
+    assert prefill(logits=None)[0] == -1 and prefill(ws=264)[0] == -3
+    small = _prefill_plan(lm, 40, (4,))
+    small.ws_bytes = lib.mlora_prefill_workspace_bytes(C.byref(small)) - 1
+    assert small.ws_bytes > 0 and lib.mlora_prefill(C.byref(small), None) == -3
+    assert lib.mlora_prefill_workspace_bytes(None) == 0 and lib.mlora_prefill(None, None) == -1
+
+    def step(targets=(0, 1, 2, 3, 4, 5, 6), ws=1 << 40, T=8, **fields):
+        p, L = lm.DecodePlan(), (lm.Layer * 2)()
+        for e in L:
+            for f in ("ln1", "ln2", "qkv_p", "o_p", "gate_up_p", "gate_up_il_p", "down_p", "k_cache", "v_cache"):
+                setattr(e, f, 256)
+        for j in targets:                                # of the last layer alone
+            L[1].lora[j].A, L[1].lora[j].B = 256, 256
+        p.n_layers, p.hidden, p.inter, p.n_q_heads, p.n_kv_heads, p.head_dim, p.vocab, p.eps = 2, 1024, 2752, 8, 8, 128, 32000, 1e-5
+        for f in ("tokens", "rows", "pos", "ctx", "resid", "xn", "qkv", "attn", "gate_up", "act", "logits", "embed", "norm", "lm_head_p", "block_table", "rope_cos", "rope_sin",
+                  "tok_adapter", "lora_ws"):
+            setattr(p, f, 256)
+        p.T, p.max_blocks, p.n_pages, p.n_seq, p.max_pos, p.lora_r, p.lora_n_ad, p.lora_scaling, p.lora_ws_bytes, p.lora_segments = T, 4, 64, 8, 64, 32, 4, 0.5, ws, 1
+        p.layers = C.cast(L, C.POINTER(lm.Layer))
+        for k, v in fields.items():
+            setattr(p, k, v)
+        return lib.mlora_decode_step(C.byref(p), None)
+    assert step(lora_r=12) == -2 and step(lora_n_ad=0) == -2
+    assert step(hidden=1008) == -2 and step((4,), inter=2744) == -2 and step((6,), inter=2768) == -2         # K of gate; rows of gate; K of down
+    assert step((1,), n_kv_heads=1, head_dim=8) == -2                                                           # eight rows of k
+    assert step(lora_ws=264) == -3 and step(xn=264) == -2 and step(T=20, resid=264) == -2
+    assert step(ws=5 * lib.mlora_gather_mm_workspace_bytes(8, 2752, 32) - 1) == -3
+
+
+def test_arguments_of_linears_with_deltas():
+    """Every refusal of the entry points that take adapter deltas, or a gated product, into a linear happens on the host."""
+    import ctypes as C
+    lm = load_pkg("_lib")
+    lib = lm.lib()
+    bk, c, n = (lm.LoraBucket * 3)(), (C.c_int32 * 3)(0, 512, 768), (C.c_int32 * 3)(512, 256, 256)
+    for e in bk:
+        e.A, e.B, e.r, e.n_ad, e.scaling = 256, 256, 16, 4, 0.5
+    pt = lambda a: C.cast(a, C.c_void_p)
+
+    def linear(T=8, K=1024, N=1024, mode=0, dt=0, ks=1, part=None, n_proj=3, ids=256, ws=256, wsb=1 << 30, x=256, y=256):
+        return lib.mlora_linear_frag_deltas(y, dt, mode, part, ks, x, 256, T, K, N, pt(bk), n_proj, pt(c), pt(n), ids, ws, wsb, None)
+    assert linear(y=None) == -1 and linear(x=264) == -2 and linear(K=1000) == -2 and linear(N=1032) == -2 and linear(T=0) == -2
+    assert linear(mode=1) == -2 and linear(ks=2, part=256) == -1 and linear(mode=1, dt=1, ks=2) == -1 and linear(mode=1, dt=1, ks=5, part=256) == -1
+    assert linear(mode=1, dt=1, K=256, ks=2, part=256) == -1 and linear(n_proj=0) == -1 and linear(n_proj=4) == -1 and linear(ids=None) == -1
+    assert linear(ws=264) == -3 and linear(wsb=3 * lib.mlora_gather_mm_workspace_bytes(8, 1024, 16) - 1) == -3 and linear(N=1008) == -2      # rows past N
+    assert linear(T=4096, K=4096, N=4096) == -2                                                                                              # the persistent kernel's
+    for field, v, code in (("B", None, -1), ("r", 8, -2), ("n_ad", 5, -2), ("scaling", 1.0, -2)):
+        old = getattr(bk[1], field)
+        setattr(bk[1], field, v)
+        assert linear() == code
+        setattr(bk[1], field, old)
+    silu = lambda fn, T, act=256, I=512, n_proj=2, wsb=1 << 30: getattr(lib, fn)(act, 256, 256, T, 1024, I, pt(bk), n_proj, pt((C.c_int32 * 2)(0, 512)), pt((C.c_int32 * 2)(512, 512)), 256, 256, wsb, None)
+    for fn, T, other in (("mlora_gemv_frag_silu_deltas", 8, 65), ("mlora_linear_frag_silu_deltas", 100, 64)):
+        assert silu(fn, other) == -2 and silu(fn, T, act=None) == -1 and silu(fn, T, act=264) == -2 and silu(fn, T, I=528) == -2 and silu(fn, T, n_proj=4) == -1
+        assert silu(fn, T, I=480) == -2 and silu(fn, T, wsb=64) == -3
+    seg = lambda T=8, K=1024, ldy=1024, y=256, lay=1, dt=0, n_proj=3, wsb=1 << 30, co=c, nc=n: lib.mlora_gather_mm_segments(
+        y, dt, ldy, 256, lay, pt(bk), n_proj, pt(co), pt(nc), 256, T, K, 256, wsb, None)
+    assert seg(n_proj=0) == -1 and seg(n_proj=4) == -1 and seg(y=None) == -1 and seg(dt=7) == -1 and seg(ldy=1000) == -1 and seg(K=1016) == -2 and seg(y=264) == -2
+    assert seg(lay=5) == -2 and seg(nc=(C.c_int32 * 3)(512, 256, 248)) == -2 and seg(co=(C.c_int32 * 3)(0, 516, 768)) == -2 and seg(wsb=64) == -3 and seg(T=0) == 0
+    glu = lambda T=100, K=1024, I=512, act=256, kind=0: lib.mlora_linear_frag_glu(act, 256, 256, T, K, I, kind, 1.0, 1.0, 1.0, None)
+    assert glu(act=None) == -1 and glu(kind=2) == -1 and glu(T=64) == -2 and glu(K=1000) == -2 and glu(I=528) == -2 and glu(act=264) == -2
+    assert lib.mlora_linear_frag_clipglu(256, 256, 256, 100, 1024, 512, 1.0, 1.0, 1.0, None) == -2 and b"persistent" in lib.mlora_last_error()
+    pay = lambda T, r=16, distinct=1, K=1024, N=1024: lib.mlora_linear_frag_deltas_pay(T, K, N, 0, r, distinct)
+    assert pay(16) == 1 and pay(17) == 0 and pay(64) == 0 and pay(0) == 0 and pay(8, distinct=0) == 0 and pay(8, K=1000) == 0 and pay(8, N=1032) == 0
+    assert pay(100, 64, 4) == 1 and pay(100, 64, 5) == 0 and pay(4096, K=4096, N=4096) == 0
+
+
 def test_workspace_of_a_prompt_pass():
     """Room for gate and up only where a layer keeps them, in the place of q, k, v and the attention output."""
     import ctypes as C
