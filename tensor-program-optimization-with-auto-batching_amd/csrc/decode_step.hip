@@ -3,6 +3,7 @@
 #include "common.h"
 
 int mlora_argmax_advance(int32_t* ids, const float* logits, int B, int V, int32_t* pos, int32_t* ctx, void* stream);
+int mlora_check_attn(const char* who, int Hq, int Hkv, int D, int n_pages, int n_seq, int max_blocks);
 int mlora_embed_rmsnorm(void* y, float* resid, const void* table, const int32_t* ids, int V, const void* w, float eps, int T, int H, void* stream);
 
 namespace {
@@ -131,8 +132,14 @@ extern "C" int mlora_decode_step(const mlora_decode_plan* p, void* stream) {
   MLORA_CHECK(p->tokens && p->rows && p->pos && p->ctx && p->resid && p->xn && p->qkv && p->attn && p->gate_up && p->act &&
                   p->logits && p->embed && p->norm && p->lm_head_p && p->block_table && p->rope_cos && p->rope_sin,
               MLORA_ERR_INVALID, "decode_step: null buffer");
-  // every layer of the plan is looked at before the first launch: a rejected call enqueues nothing
-  {
+  // every layer of the plan, and what the operators ask of its sizes, is looked at before the first launch: a rejected call enqueues nothing
+  MLORA_CHECK(H > 0 && H <= 16384 && H % 32 == 0 && p->vocab > 0 && p->vocab % 4 == 0, MLORA_ERR_UNSUPPORTED,
+              "decode_step: hidden in whole 32 up to 16384, vocab in whole 4 (%d, %d)", H, p->vocab);
+  if (p->n_layers > 0) {
+    STEP(mlora_check_attn("decode_step", Hq, Hkv, D, p->n_pages, p->n_seq, p->max_blocks));
+    MLORA_CHECK(Hq / Hkv <= 16 && I > 0 && I % 32 == 0, MLORA_ERR_UNSUPPORTED,
+                "decode_step: at most 16 query heads per kv head, intermediate in whole 32 (%d, %d)", Hq / Hkv, I);
+    MLORA_CHECK(p->max_pos > 0, MLORA_ERR_INVALID, "decode_step: bad max_pos %d", p->max_pos);
     const bool any_lora = p->tok_adapter != nullptr && p->lora_r > 0;
     for (int l = 0; l < p->n_layers; ++l) {
       const mlora_layer& L = p->layers[l];
@@ -141,8 +148,12 @@ extern "C" int mlora_decode_step(const mlora_decode_plan* p, void* stream) {
       const bool gu_lora = any_lora && (L.lora[MLORA_GATE].A || L.lora[MLORA_UP].A);
       MLORA_CHECK(L.gate_up_p || (T <= 64 && L.gate_up_il_p && !gu_lora), MLORA_ERR_INVALID, "decode_step: layer %d needs gate_up_p", l);
       if (any_lora)
-        for (int j = 0; j < 7; ++j)
-          MLORA_CHECK(!L.lora[j].A || L.lora[j].B, MLORA_ERR_INVALID, "decode_step: layer %d projection %d has A but no B table", l, j);
+        for (int j = 0; j < 7; ++j) {
+          MLORA_CHECK(!L.lora[j].A || p->lora_r == 8 || p->lora_r == 16 || p->lora_r == 32 || p->lora_r == 64, MLORA_ERR_UNSUPPORTED,
+                      "decode_step: rank %d not in {8,16,32,64}", p->lora_r);
+          MLORA_CHECK(!L.lora[j].A || (L.lora[j].B && p->lora_n_ad > 0 && p->lora_n_ad <= 65535), MLORA_ERR_INVALID,
+                      "decode_step: layer %d projection %d has A but no B table, or bad lora_n_ad %d", l, j, p->lora_n_ad);
+        }
     }
   }
   if (T > 64) {
@@ -178,8 +189,6 @@ extern "C" int mlora_decode_step(const mlora_decode_plan* p, void* stream) {
   // ... and what deltas in launches of their own ask of sizes, room and alignment (the projections that are adapted and take them)
   if (segs || gu_segs) {
     size_t seg_need = 0;
-    MLORA_CHECK((r == 8 || r == 16 || r == 32 || r == 64) && n_ad > 0 && n_ad <= 65535, MLORA_ERR_UNSUPPORTED,
-                "decode_step: lora_segments: rank %d not in {8,16,32,64} or bad lora_n_ad %d", r, n_ad);
     const int K_of[7] = {H, H, H, q_sz, H, H, I}, N_of[7] = {q_sz, kv_sz, kv_sz, H, I, I, H}, ld_of[7] = {qkv_sz, qkv_sz, qkv_sz, H, 2 * I, 2 * I, H};
     for (int l = 0; l < p->n_layers; ++l)
       for (int j = 0; j < 7; ++j) {

@@ -243,7 +243,8 @@ def test_rejected_passes_queue_nothing():
         for k, v in fields.items():
             setattr(p, k, v)
         return lib.mlora_decode_step(C.byref(p), None)
-    assert step(lora_r=12) == -2 and step(lora_n_ad=0) == -2
+    assert step(lora_r=12) == -2 and step(lora_n_ad=0) == -1 and step(T=65, lora_r=12) == -2 and step(T=65, lora_n_ad=0) == -1
+    assert step(head_dim=96) == -2 and step(n_kv_heads=3) == -1 and step(n_q_heads=136) == -2 and step(vocab=32001) == -2 and step((), inter=2744) == -2 and step(max_pos=0) == -1
     assert step(hidden=1008) == -2 and step((4,), inter=2744) == -2 and step((6,), inter=2768) == -2         # K of gate; rows of gate; K of down
     assert step((1,), n_kv_heads=1, head_dim=8) == -2                                                           # eight rows of k
     assert step(lora_ws=264) == -3 and step(xn=264) == -2 and step(T=20, resid=264) == -2
