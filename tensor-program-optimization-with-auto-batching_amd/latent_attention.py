@@ -80,7 +80,7 @@ class LatentAttention:
         other), keys and values, scores, queries and outputs.  The lesser sum is the slower form in 3 of the 225, by 9 % at most;
         4 us more are asked for because the host makes a plan.  lifted / made: 16 heads, one prompt of 90 23.5 / 21.3, 250 32.8 / 27.7, 500
         69 / 40, 1000 130 / 58; eight of 40 54 / 20; 20 tokens behind 500 24 / 40, 300 behind 1000 95 / 70."""
-        if self.uk is None:
+        if self.uk is None or not seqs:
             return False
         H, image = self.spec.heads, self.rank_p * (self.dp + self.vp)
         rot = self.q_cols - self.rank_p

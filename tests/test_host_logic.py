@@ -357,3 +357,12 @@ def test_pages_of_a_pass_whichever_way_they_are_looked_up(n, monkeypatch):
     monkeypatch.setattr(kvm.np, "asarray", lambda *a, f=np.asarray, **k: built.append(a) or f(*a, **k))
     kv.begin_forward(ids, [0] * n, device_meta=(None, None, None))
     assert n >= 128 or not built
+
+
+def test_latent_form_of_passes_without_sequences():
+    """No sequences: the lifted form, as for a layer that has no other; else the cheaper one by the fitted costs."""
+    import types
+    la = load_pkg("latent_attention").LatentAttention
+    layer = types.SimpleNamespace(uk=1, spec=types.SimpleNamespace(heads=16), rank_p=512, dp=128, vp=128, q_cols=576)
+    assert la.prompt_form_pays(layer, []) is False and la.prompt_form_pays(types.SimpleNamespace(uk=None), [(500, 500)]) is False
+    assert la.prompt_form_pays(layer, [(500, 500)]) and not la.prompt_form_pays(layer, [(20, 520)])
