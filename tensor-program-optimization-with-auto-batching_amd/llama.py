@@ -582,9 +582,10 @@ class LlamaForCausalLM(CausalLM):
 
     # ------------------------------------------------------------------ a prompt pass in one call
     def _native_prefill_serves(self, h, kv):
-        """Whether `mlora_prefill` takes a pass: not a decode step, activations in fragment order, a cache of at least the model's layers."""
+        """Whether `mlora_prefill` takes a pass: not a decode step, activations in fragment order, a cache of at least the model's layers, and `forward` is this
+        class's (whose launches it queues)."""
         s = self.shape
-        return (kv._cur is not None and not kv._cur[2] and h.dim() == 2 and h.shape[0] > 0 and h.is_cuda and h.dtype == torch.float32
+        return (getattr(self.forward, "__func__", None) is LlamaForCausalLM.forward and kv._cur is not None and not kv._cur[2] and h.dim() == 2 and h.shape[0] > 0 and h.is_cuda and h.dtype == torch.float32
                 and h.is_contiguous() and not s.hidden_size % 32 and not s.q_size % 32 and not s.intermediate_size % 32
                 and tuple(h.shape) == (sum(kv._cur[1]), s.hidden_size) and kv.n_layers >= len(self.layers))
 

@@ -366,3 +366,29 @@ def test_latent_form_of_passes_without_sequences():
     layer = types.SimpleNamespace(uk=1, spec=types.SimpleNamespace(heads=16), rank_p=512, dp=128, vp=128, q_cols=576)
     assert la.prompt_form_pays(layer, []) is False and la.prompt_form_pays(types.SimpleNamespace(uk=None), [(500, 500)]) is False
     assert la.prompt_form_pays(layer, [(500, 500)]) and not la.prompt_form_pays(layer, [(20, 520)])
+
+
+def test_prompt_passes_of_a_model_with_its_own_forward(monkeypatch):
+    """prefill_a and prefill_no_adapter call `forward` where a subclass or an instance has its own; the native pass serves the class's own alone."""
+    import types
+    llama, synth = load_pkg("llama"), load_pkg("synth")
+    shape = synth.LlamaShape(hidden_size=64, intermediate_size=64, num_attention_heads=1, num_key_value_heads=1, num_hidden_layers=1, head_dim=64, vocab_size=64)
+    h = types.SimpleNamespace(dim=lambda: 2, shape=(5, 64), is_cuda=True, dtype=torch.float32, is_contiguous=lambda: True)
+    kv = types.SimpleNamespace(_cur=([0], [5], False, None, None, None), n_layers=1)
+    lt = types.SimpleNamespace(rows=lambda w: w, n_adapters=1)
+    calls = []
+
+    class Own(llama.LlamaForCausalLM):
+        def forward(self, *a, **k):
+            calls.append(a)
+            return "own"
+    for cls in (llama.LlamaForCausalLM, Own):
+        m = cls.__new__(cls)
+        m.shape, m.layers, m.lora_types, m.device = shape, [None], [lt], "cpu"
+        monkeypatch.setattr(m, "_last_rows", lambda kv: None, raising=False)
+        monkeypatch.setattr(m, "_native_prefill", lambda *a: "native", raising=False)
+        want = "native" if cls is llama.LlamaForCausalLM else "own"
+        assert m.prefill_no_adapter(h, kv)[0] == want and m.prefill_a(0, h, kv, [0])[0] == want
+    m = llama.LlamaForCausalLM.__new__(llama.LlamaForCausalLM)
+    m.shape, m.layers, m._last_rows, m._native_prefill, m.forward = shape, [None], lambda kv: None, None, lambda *a, **k: "own"
+    assert len(calls) == 2 and m.prefill_no_adapter(h, kv)[0] == "own"
