@@ -3,6 +3,7 @@
 #include "common.h"
 
 int mlora_argmax_advance(int32_t* ids, const float* logits, int B, int V, int32_t* pos, int32_t* ctx, void* stream);
+int mlora_n_cu();        // compute units of the device, 0 if it cannot be asked
 int mlora_check_attn(const char* who, int Hq, int Hkv, int D, int n_pages, int n_seq, int max_blocks);
 int mlora_embed_rmsnorm(void* y, float* resid, const void* table, const int32_t* ids, int V, const void* w, float eps, int T, int H, void* stream);
 
@@ -341,10 +342,10 @@ extern "C" int mlora_decode_step(const mlora_decode_plan* p, void* stream) {
       const mlora_lora_proj lp[2] = {L.lora[MLORA_GATE], L.lora[MLORA_UP]};
       const int32_t col[2] = {0, I}, ncol[2] = {I, I};
       bool done = false;
-      // the product out of the linear as well, up to 16 tokens and three workgroups of two tiles on a compute unit; two layers with all linears
-      // adapted, us, product behind / out of it: 7B, one request at rank 64 339 / 325, 8 at rank 16 317 / 304, hidden 1024, 4 125 / 122; 20 requests
-      // 370 / 373, hidden 1024, 32 159 / 162, 8 of intermediate 14336 443 / 448
-      const void* il = T <= 16 && I <= 3 * 256 * 16 ? L.gate_up_il_p : nullptr;
+      // the product out of the linear as well, up to 16 tokens and three workgroups of two tiles on a compute unit (the same bits); two layers with all linears
+      // adapted, us, product behind / out of it: 7B, one request at rank 64 336 / 323, 8 at rank 16 308 / 296, hidden 1024, 4 124 / 123; 16 of nine
+      // adapters 462 / 464 at rank 32, 523 / 535 at rank 64; 8 of intermediate 14336 438 / 438
+      const void* il = T <= 16 && I <= 3 * 16 * mlora_n_cu() ? L.gate_up_il_p : nullptr;
       if (gu_segs) STEP(seg_linear(il ? p->act : gu, MLORA_F16, MLORA_STORE, 1, p->xn, L.gate_up_p, H, 2 * I, lp, col, ncol, 2, done, il));
       if (!done) STEP(mlora_gemv_frag(gu, MLORA_F16, MLORA_STORE, p->xn, L.gate_up_p, T, H, 2 * I, stream));
       if (done) {

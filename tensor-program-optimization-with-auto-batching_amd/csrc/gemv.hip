@@ -816,6 +816,8 @@ extern "C" int mlora_gemv_frag_lora(void* y, int y_dtype, int mode, const void* 
 int mlora_gemm_mid_ksplit(int T, int K, int N, int ks_max);
 int mlora_gemm_mid_acc(float* resid, float* part, int ld_part, int ks, const void* xf, const void* Wp, int T, int K, int N, void* stream);
 
+int mlora_n_cu() { return gemv_n_cu(); }
+
 extern "C" int mlora_gemv_ksplit(int T, int K, int N_total) {
   if (T <= 0 || K <= 0 || K % 32 || N_total <= 0) return 1;
   if (T > 64) return mlora_gemm_mid_ksplit(T, K, N_total, 4);      // the matrix-core kernel for mid-size token blocks
