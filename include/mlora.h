@@ -277,7 +277,7 @@ int mlora_linear_frag_lora(void* y, int y_dtype, int mode, const void* xf, const
  * mlora_gather_mm_workspace_bytes(T, K, r) bytes.  Up to 64 tokens v = scaling * A x keeps the bits of fp32, as it does in mlora_gather_mm and
  * mlora_gather_mm_segments there; for more tokens these, and the forms with extra k-steps, take it as two fp16 halves (22 bits, steps of 2^-24, up to 65504).
  *   mlora_linear_frag_deltas_pay   - whether a shape is served, and faster so than by mlora_linear_frag and mlora_gather_mm where the tokens of the
- *                                    pass name n_distinct adapters (accumulate: the mode);
+ *                                    pass name n_distinct adapters (accumulate: the mode); up to 64 tokens a matter of T alone;
  *   mlora_linear_frag_deltas       - ks > 1 (accumulating only): K slices as mlora_gemv_frag_acc_ksplit, slices 1.. into part[ks - 1][T][N];
  *   mlora_linear_frag_silu_deltas  - act = silu(gate) * up in fragment order, of the sums rounded to fp16 (more than 64 tokens);
  *   mlora_gemv_frag_silu_deltas    - the same up to 64 tokens, of interleaved tiles (mlora_gemv_frag_silu). */
@@ -635,7 +635,7 @@ typedef struct mlora_prefill_plan {
   void* ws;
   size_t ws_bytes;
   int max_pos, max_blocks, n_pages, n_seq, T, n_rows;
-  int n_distinct;             /* > 0: the adapters that the tokens name, for mlora_linear_frag_deltas where it pays (more than 64 tokens) */
+  int n_distinct;             /* > 0: the adapters that the tokens name, for mlora_linear_frag_deltas where it pays (up to 64 tokens: with segments) */
 } mlora_prefill_plan;
 
 size_t mlora_prefill_workspace_bytes(const mlora_prefill_plan* plan);
@@ -646,8 +646,9 @@ int mlora_prefill(const mlora_prefill_plan* plan, void* stream);
  * (persistent GEMM shapes) and mlora_silu_mul. */
 int mlora_gemv_frag_clipglu(void* act, const void* xf, const void* Wil_p, int T, int K, int I, float scale, float limit, float alpha, void* stream);
 int mlora_linear_frag_clipglu(void* act, const void* xf, const void* Wp, int T, int K, int I, float scale, float limit, float alpha, void* stream);
-/* Either gated product (kind: MLORA_GLU_*; scale, limit, alpha: of the clipped one) for more than 64 tokens, on the kernel that mlora_linear_frag
- * takes at that size (mid-size or persistent).  K and I in whole 32, operands 16-byte aligned. */
+/* Either gated product (kind: MLORA_GLU_*; scale, limit, alpha: of the clipped one) for more than 64 tokens, on the persistent kernel where
+ * mlora_gemm_frag_preferred or mlora_linear_frag takes it, else on the mid-size one.  Of the sums rounded to the element type, as a linear would store them,
+ * except the clipped product on the persistent kernel.  K and I in whole 32, operands 16-byte aligned. */
 int mlora_linear_frag_glu(void* act, const void* xf, const void* Wp, int T, int K, int I, int kind, float scale, float limit, float alpha,
                           void* stream);
 int mlora_clipglu_mul(void* out, int out_layout, const void* gate, const void* up, int ld, int T, int I, float scale, float limit, float alpha,

@@ -17,7 +17,6 @@ GLU_SILU, GLU_CLIPPED = 0, 1
 ACT_NONE, ACT_RELU2, ACT_GLU = 0, 1, 2
 MOE_UP, MOE_DOWN = 0, 1
 ROWMAJOR, FRAG = 0, 1
-GLU_SILU, GLU_CLIPPED = 0, 1
 STORE, ACCUMULATE = 0, 1
 PAGE_SIZE = 16
 

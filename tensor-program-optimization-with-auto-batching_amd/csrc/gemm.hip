@@ -1239,9 +1239,10 @@ extern "C" int mlora_linear_packed(void* y, int y_dtype, int mode, const void* x
 extern "C" int mlora_gemv_frag(void* y, int y_dtype, int mode, const void* xf, const void* Wp, int T, int K, int N, void* stream);
 
 // 256 x 256 output blocks: enough of them to give every compute unit one (the forms with an epilogue of their own - a gated product, LoRA deltas -
-// exist from there on).  K in whole 64, here and wherever the persistent kernel is chosen: its ring walks single steps of 32 k, but an odd number of them
-// has been neither tested nor measured.  256 is the number of compute units; the plain linear is taken from half of that on (persistent_pays), these
-// forms have not been measured there.
+// take it from there on).  K in whole 64, here and wherever the persistent kernel is chosen: its ring walks single steps of 32 k, but an odd number of them
+// has been neither tested nor measured.  256 is the number of compute units; the plain linear and the gated product take the kernel from half of
+// that on (persistent_pays), LoRA stages have not been measured there.  Just above one round the plain linear goes back to the mid-size kernel, by an eighth of a
+// round; the gated product and the LoRA stages stay, they have not been compared there.
 extern "C" int mlora_gemm_frag_preferred(int T, int K, int N) {
   return T > 64 && K > 0 && K % 64 == 0 && N > 0 && (long)ceil_div(T, PP_F * 16) * ceil_div(N, PP_F * 16) >= 256;
 }
@@ -1301,7 +1302,8 @@ extern "C" int mlora_linear_frag_clipglu(void* act, const void* xf, const void* 
   return mlora_linear_frag_glu(act, xf, Wp, T, K, I, MLORA_GLU_CLIPPED, scale, limit, alpha, stream);
 }
 
-// act = the gated product of [gate | up] = xf . Wp^T for more than 64 tokens, on the kernel that the plain linear takes at that size.  A product
+// act = the gated product of [gate | up] = xf . Wp^T for more than 64 tokens: on the persistent kernel where mlora_gemm_frag_preferred or the plain linear takes it
+// (which differ just above one round of its blocks), else on the mid-size one.  The clipped product is of unrounded sums on the first, of rounded ones on the second.  A product
 // behind the linear writes and reads T x 2 I elements once more and costs a launch (a floor of 2.5 us); what is left in its place is the exchange
 // of half a block through LDS.  Linear and product behind it -> here, in a row of launches (K, I): 512, 1376 at 65 / 512 / 1024 tokens 7.6 / 9.9 /
 // 13.3 -> 6.3 / 6.7 / 8.9 us; 2048, 5632: 14.7 / 34.8 / 52.3 -> 13.1 / 31.3 / 49.3; 2880, 2880: 17.4 / 28.6 / 42.7 -> 15.9 / 25.1 / 39.8; 4096,
@@ -1328,7 +1330,7 @@ extern "C" int mlora_linear_frag_glu(void* act, const void* xf, const void* Wp, 
 }
 
 #ifndef MLORA_ELT_BF16      // the adapter kernels are fp16
-// Whether the linears with deltas below serve a shape: where the plain one takes the mid-size kernel.
+// Whether the linears with deltas below serve a shape: where neither the plain one nor the gated product takes the persistent kernel.
 static bool mid_deltas_serve(int T, int K, int N, bool accumulate) {
   return T > 64 && ceil_div(T, 128) <= 65535 && K >= 32 && K % 32 == 0 && !mlora_gemm_frag_preferred(T, K, N) && !persistent_pays(T, K, N, accumulate);
 }

@@ -870,7 +870,6 @@ extern "C" int mlora_gemv_frag_acc_ksplit(float* y, float* y2, float* part, int 
                                           ks, part);
 }
 
-// ranges of K of the last group's rows: whole rounds of a workgroup's waves
 #ifndef MLORA_ELT_BF16
 // y (=|+=) xf . Wp^T + the deltas for up to 64 tokens (K slices: accumulating, slice 0 carries them)
 int mlora_gemv_deltas(void* y, int y_dtype, int mode, float* part, int ks, const void* xf, const void* Wp, int T, int K, int N, const LinearDeltas& ld, void* stream) {
@@ -878,6 +877,7 @@ int mlora_gemv_deltas(void* y, int y_dtype, int mode, float* part, int ks, const
 }
 #endif
 
+// ranges of K of the last group's rows: whole rounds of a workgroup's waves
 extern "C" int mlora_gemv_groups_parts(int K) {
   const int by_k = K / KSTEP / GEMV_WAVES;
   return by_k < 1 ? 1 : by_k < 8 ? by_k : 8;

@@ -498,7 +498,7 @@ def _delta_args(who, x, W, projs, tok_adapter, workspace):
 
 def linear_frag_deltas(x: FragActivation, W: PackedWeight, projs, tok_adapter, workspace, out=None, out_dtype=torch.float16, accumulate=False, ks_ws=None):
     """`linear(x, W)` with the LoRA deltas of `projs` = [(A [n_ad, r, K], B [n_ad, rows, r], scaling, first row, rows), ...] of tokens that name any
-    adapters, inside the GEMM (shapes of the mid-size kernel).  accumulate: into `out`; with fp32 scratch `ks_ws` K may be split as in
+    adapters, inside the GEMM (up to 64 tokens, and shapes of the mid-size kernel).  accumulate: into `out`; with fp32 scratch `ks_ws` K may be split as in
     `linear_acc_ksplit`.  Returns (out, KSplitParts or None)."""
     T, K = x.shape
     N = W.shape[0]

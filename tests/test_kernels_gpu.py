@@ -1876,3 +1876,32 @@ def test_a_token_keeps_its_bits_in_any_row_beside_any_adapters(ops, T, r):
     for order in (torch.arange(T - 1, -1, -1, device=DEV), torch.randperm(T, generator=torch.Generator(device=DEV).manual_seed(T), device=DEV)):
         for p, q, s in zip(a, run(x[order].contiguous(), ids[order].contiguous()), c):
             assert torch.equal(p[order], q) and torch.equal(p[same], s[same])
+
+
+@pytest.mark.parametrize("T", [65, 137, 300])
+@pytest.mark.parametrize("half", [0, 1])
+def test_gated_product_with_deltas_of_gate_or_up_alone(ops, T, half):
+    """More than 64 tokens, one half of a block's waves without a projection ahead of the exchange: the bits of the linear and the separate product."""
+    K, I, n_ad = 1056, 608, 5
+    x, tabs, W, ws = _delta_case(ops, T, K, (I, I), 16, n_ad, T + half)
+    ids = torch.arange(T, device=DEV, dtype=torch.int32) // 40 % (n_ad + 1) - 1
+    f, projs = ops.FragActivation.pack(x), [(*tabs[half], 0.5, half * I, I)]
+    y, _ = ops.linear_frag_deltas(f, W, projs, ids, ws)
+    assert torch.equal(ops.linear_frag_silu_deltas(f, W, projs, ids, ws).data, ops.silu_mul(y, frag=True).data)
+
+
+@pytest.mark.parametrize("T,K,I", [(4096, 128, 2048), (4001, 64, 2080)])
+def test_clipped_product_of_the_persistent_kernel_by_its_own_name(ops, T, K, I):
+    """mlora_linear_frag_clipglu: the shapes of the persistent kernel, the bits of mlora_linear_frag_glu."""
+    dt = torch.bfloat16
+    lib = load_pkg("_lib").lib("bfloat16")
+    assert ops._size(dt, "mlora_gemm_frag_preferred", T, K, 2 * I)
+    g = torch.Generator(device=DEV).manual_seed(T)
+    f = ops.FragActivation.pack(torch.randn((T, K), generator=g, device=DEV).to(dt))
+    W = ops.PackedWeight((torch.randn((2 * I, K), generator=g, device=DEV) * K ** -0.5 * 2).to(dt))
+    a, b = (ops.FragActivation(T, I, DEV, dtype=dt) for _ in range(2))
+    ptrs = lambda o: (o.data.data_ptr(), f.data.data_ptr(), W.data.data_ptr(), T, K, I)
+    s = torch.cuda.current_stream().cuda_stream
+    assert lib.mlora_linear_frag_clipglu(*ptrs(a), 0.8, 1.5, 1.702, s) == 0 and lib.mlora_linear_frag_glu(*ptrs(b), 1, 0.8, 1.5, 1.702, s) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(a.data, b.data) and bool((a.data != 0).any())
